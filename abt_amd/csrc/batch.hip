@@ -1,4 +1,4 @@
-// batch.hip -- orientation-averaged far field of many orientations in one launch.
+// batch.hip -- orientation-averaged far field of many orientations.
 //
 // Replaces the orientation loop of the reference drivers (pbt_seq_mod.f90:146-269,
 // pbt_mpi_mod.f90 over MPI ranks): per orientation diff_main (coherent sums of the
@@ -7,18 +7,24 @@
 // summation (Mueller matrices summed incoherently over orientations,
 // outputs_mod.f90:407-471).
 //
-// Work decomposition.  A work unit is (orientation chunk c, bin tile t): the
-// orientations of chunk c (a contiguous range, chunks balanced by beam count) on
-// BLOCK * BPT bins.  A persistent grid of workgroups takes units from a queue
-// (one global atomic counter).  Inside a unit every lane owns BPT bins and walks
-// the orientations of the chunk in order; per orientation it sums the beam tree
-// and then the ext tree (beam records staged in LDS, TB at a time, as in the
-// single-orientation kernel), applies k, forms the Mueller matrix of the total
-// and adds it to the chunk's partial Mueller sum, and adds the bin's weighted S11
-// values to the orientation's integrals.  Every output element is written by one
-// unit, and every sum has a fixed order (beams in tree order, orientations in
-// order within a chunk, chunks in order, tiles in order), so results do not
-// depend on scheduling and repeat bit for bit.
+// Work decomposition.  Every orientation's two beam lists are cut into segments of one length
+// (the plan's, chosen so that segments x bin tiles are many workgroups per CU however few
+// orientations or bins there are).  A run alternates, over groups of orientations whose segment
+// sums fit the plan's buffer:
+//   k_sweep (far_field.hip)  one workgroup per (segment, bin tile): the segment's coherent sum;
+//   k_combine                one lane per bin: an orientation's segment sums added in beam order and
+//                            finished, x k, the Mueller matrix of the total added to the chunk's
+//                            sum, the bin's weighted S11 values added to the orientation's integrals.
+// The segment sums cost 64 bytes per bin and segment written and read once, against ~10^3 beams of
+// ~150 FP64 instructions in each: under 1 % of the time.  In return the sweep's loop has the
+// registers and LDS to itself (an epilogue inside it held 73 spilled registers and 16 KB), and no
+// shape leaves the chip idle.
+// Against one persistent kernel that summed an orientation's whole beam list per bin tile (same body):
+// 24 orientations x 721 x 180 bins 106.7 -> 100.2 ms, 16 x 361 x 180 in the mixed body 33.2 -> 28.0 ms,
+// one orientation x 451 x 360 bins 12.3 -> 5.7 ms, 4 coarse orientations x 37 x 36 bins 1161 -> 103 us.
+// Every output element is written by one lane, and every sum has a fixed order (beams, segments,
+// orientations of a chunk, chunks, tiles), so results do not depend on scheduling and repeat bit
+// for bit; the cut does not depend on the tile shape, so neither do the results.
 //
 // Per-orientation integrals (for the asymmetry parameters, which are ratios per
 // orientation and so cannot be formed from the summed Mueller matrix):
@@ -31,72 +37,12 @@
 #include <math.h>
 #include <stdint.h>
 
-#include "adjbody.h"
 #include "batch.h"
-#include "ffbody.h"
 #include "mueller.h"
-#include "simpne.h"
 
 namespace abt {
 
 constexpr int BB = 256;   // lanes per workgroup
-
-template <int PREC, int TB, int BPT, bool INC>
-__device__ __forceinline__ void sweep(const BatchArgs& a, const double* __restrict__ recs,
-                                      const double* __restrict__ vrecs, int64_t b0, int64_t b1,
-                                      double* tile, const double* etab, const BinIn* bi, const double* cp,
-                                      const double* sp, double (*acc)[8], double* inc)
-{
-    const int tid = threadIdx.x;
-    for (int64_t t0 = b0; t0 < b1; t0 += TB) {
-        const int nt = (int)min((int64_t)TB, b1 - t0);
-        __syncthreads();
-        const double* src = recs + t0 * REC;
-        for (int q = tid; q < nt * REC; q += BB) tile[q] = src[q];
-        __syncthreads();
-        if (PREC == 1) {
-            // FP32 partial sums over groups of MIXED_GROUP beams (counted from the
-            // orientation's first beam; TB is a multiple), added into FP64
-            for (int g0 = 0; g0 < nt; g0 += MIXED_GROUP) {
-                float accf[BPT][8], incf[BPT];
-#pragma unroll
-                for (int j = 0; j < BPT; j++) {
-                    incf[j] = 0.f;
-#pragma unroll
-                    for (int q = 0; q < 8; q++) accf[j][q] = 0.f;
-                }
-                const int g1 = min(nt, g0 + MIXED_GROUP);
-                for (int bb = g0; bb < g1; bb++) {
-#pragma unroll
-                    for (int j = 0; j < BPT; j++)
-                        beam_bin_mixed_t<INC>(tile + bb * REC, vrecs, a.g, bi[j], a.fast_diff, accf[j], incf[j]);
-                }
-#pragma unroll
-                for (int j = 0; j < BPT; j++) {
-                    if (INC) inc[j] += (double)incf[j];
-#pragma unroll
-                    for (int q = 0; q < 8; q++) acc[j][q] += (double)accf[j][q];
-                }
-            }
-        } else {
-            for (int bb = 0; bb < nt; bb++) {
-#pragma unroll
-                for (int j = 0; j < BPT; j++) {
-                    if (PREC == 0)
-                        beam_bin_fp64(tile + bb * REC, vrecs, a.g, bi[j], etab, a.fast_diff, acc[j]);
-                    else if (PREC == 4)
-                        beam_bin_fp64r(tile + bb * REC, vrecs, a.g, bi[j], etab, a.fast_diff, acc[j]);
-                    else {
-                        AdjBeam B;
-                        adj_beam_from_record(tile + bb * REC, B);
-                        model_bin_fp64(B, bi[j].x, bi[j].y, bi[j].z, bi[j].xt, bi[j].yt, bi[j].rad, a.g.waveno,
-                                       a.g.lambda, acc[j]);
-                    }
-                }
-            }
-        }
-    }
-}
 
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -105,178 +51,108 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// Occupancy: 4 waves per SIMD (128 VGPRs) for the mixed body and for the restructured FP64
-// body with 8-beam tiles (whose LDS, ~39 KB per workgroup, lets 4 workgroups share a CU; its
-// spills are outside the beam loop), else 3.
-// Register budget: the per-orientation beam-tree result waits in LDS (xbs) while
-// the ext tree is summed, and the phi rotation and integral weights are re-read
-// after the sweeps, so the live state across a sweep is the accumulators and the
-// bin position only.
-//
-// MODE == BMODE_EST (mixed only): also the error scale of the FP32 body, the sum over
-// orientations of S11_o * I_o with I_o = k^2 sum_b |A_b|_F^2 the bin's incoherent beam sum,
-// into epart.  MODE == BMODE_LIST: lane slots are positions in the list of bins a.list
-// (*a.list_count of them), whose Mueller sums go to mpart at the list position; no
-// integrals (the mixed pass keeps them).
-template <int PREC, int TB, int BPT, int MODE>
-__global__ __launch_bounds__(BB, (PREC == 1 || (PREC == 4 && TB <= 8)) ? 4 : 3) void k_batch(BatchArgs a)
+// The six integral terms of a workgroup's bins, summed in a fixed order into ip[0..5].
+__device__ __forceinline__ void block_integrals(double v[6], double (*red)[6], double* __restrict__ ip)
 {
-    constexpr bool INC = MODE == BMODE_EST;
-    constexpr bool LIST = MODE == BMODE_LIST;
-    constexpr bool ROT = PREC == 0 || PREC == 1 || PREC == 4;   // temp_rot1 applied after the beam sum
-    __shared__ double tile[TB * REC];
-    // the exponential table and the FP64r body's constants, or the table with its low parts
-    __shared__ double etab[PREC == 4 ? ETAB_LDS : (PREC == 0 ? ETAB_GRID : 1)];
-    __shared__ double xbs[8][BB * BPT];
-    __shared__ double red[BB / 64][6];
-    __shared__ unsigned s_unit;
     const int tid = threadIdx.x;
-    const int nbins = a.g.nbins;
-    const double k = a.g.waveno;
-    if (PREC == 0 || PREC == 4) {   // published by the barrier at the top of the unit loop
-        for (int q = tid; q < (PREC == 4 ? ETAB_DOUBLES : ETAB_GRID); q += BB) etab[q] = a.g.etab[q];
-        if (PREC == 4 && tid == 0) fp64r_constants(a.g, etab + ETAB_DOUBLES);
+#pragma unroll
+    for (int q = 0; q < 6; q++) v[q] = wave_sum(v[q]);
+    __syncthreads();   // the previous orientation's sums have been read
+    if ((tid & 63) == 0) {
+#pragma unroll
+        for (int q = 0; q < 6; q++) red[tid >> 6][q] = v[q];
     }
-    int ntiles = a.ntiles, nunits = a.nunits, nslots = nbins;
-    if (LIST) {
-        nslots = *a.list_count;
-        ntiles = (nslots + BB * BPT - 1) / (BB * BPT);
-        nunits = ntiles * a.nchunks;
-    }
-    for (;;) {
-        __syncthreads();
-        if (tid == 0) s_unit = atomicAdd(a.counter, 1u);
-        __syncthreads();
-        const unsigned u = s_unit;
-        if (u >= (unsigned)nunits) break;   // uniform over the workgroup
-        const int c = (int)(u / (unsigned)ntiles);
-        const int t = (int)(u - (unsigned)c * (unsigned)ntiles);
-        const int slot0 = t * BPT * BB + tid;   // slot of lane j: slot0 + j * BB
+    __syncthreads();
+    if (tid < 6) ip[tid] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
+}
 
-        BinIn bi[BPT];
-        double cp[BPT], sp[BPT];
-        int bins[BPT];
+__device__ __forceinline__ void integral_terms(const double xb[8], const double xe[8], double s11, double w1,
+                                               double w2, double v[6])
+{
+    const double sb = mueller_s11(xb), se = mueller_s11(xe);
+    v[0] = w1 * s11;
+    v[1] = w2 * s11;
+    v[2] = w1 * sb;
+    v[3] = w2 * sb;
+    v[4] = w1 * se;
+    v[5] = w2 * se;
+}
+
+// Grid (ntiles of BB bins, nchunks): chunk c takes the c-th share of the group's orientations, in
+// order, for one bin per lane.  Bandwidth-bound: 64 bytes per bin and segment read.
+template <int PREC, int MODE>
+__global__ __launch_bounds__(BB) void k_combine(CombineArgs a)
+{
+    constexpr bool INC = MODE == SWEEP_INC, LIST = MODE == SWEEP_LIST;
+    __shared__ double red[BB / 64][6];
+    const int nbins = a.g.nbins;
+    const int nslots = LIST ? *a.list_count : nbins;
+    const int t = blockIdx.x, c = blockIdx.y;
+    if (t * BB >= nslots) return;   // uniform over the workgroup
+    const int slot = t * BB + threadIdx.x;
+    const bool live = slot < nslots;
+    const int sc = live ? slot : nslots - 1;
+    const int bc = LIST ? a.list[sc] : sc;
+    const double k = a.g.waveno;
+    const double w1 = LIST ? 0.0 : a.w1[bc], w2 = LIST ? 0.0 : a.w2[bc];
+    double msum[16], esum = 0.0;
 #pragma unroll
-        for (int j = 0; j < BPT; j++) {
-            const int sc = min(slot0 + j * BB, nslots - 1);
-            const int bc = LIST ? a.list[sc] : sc;
-            bins[j] = bc;
-            const int iphi = bc % a.g.nphi;
-            bi[j].x = a.g.x[bc]; bi[j].y = a.g.y[bc]; bi[j].z = a.g.z[bc];
-            const int bt = iphi + a.g.nphi * a.g.theta_i;
-            bi[j].xt = a.g.x[bt]; bi[j].yt = a.g.y[bt]; bi[j].zt = a.g.z[bt];
-            bi[j].rad = (PREC == 3 || PREC == 4) ? a.g.rad[bc] : 0.0;
-            cp[j] = ROT ? 0.0 : a.g.cphi[iphi];   // the other bodies rotate after the sum
-            sp[j] = ROT ? 0.0 : a.g.sphi[iphi];
-        }
-        const int o0 = a.chunk_o[c], o1 = a.chunk_o[c + 1];
-        double* mp = a.mpart + (int64_t)c * 16 * nbins;
-        double* ep = INC ? a.epart + (int64_t)c * nbins : nullptr;
-        for (int o = o0; o < o1; o++) {
-            double acc[BPT][8];
-            double inc[BPT];
+    for (int e = 0; e < 16; e++) msum[e] = 0.0;
+    const int n = a.o1 - a.o0;
+    const int oa = a.o0 + (int)((int64_t)n * c / a.nchunks), ob = a.o0 + (int)((int64_t)n * (c + 1) / a.nchunks);
+    const int sbase = a.seg_off[2 * a.o0];   // the buffer holds the group's segments from its first
+    for (int o = oa; o < ob; o++) {
+        double xb[8], xe[8], xt[8], m[16], inc = 0.0;
 #pragma unroll
-            for (int j = 0; j < BPT; j++) inc[j] = 0.0;
-            // segment 0: the beam tree (result parked in LDS), segment 1: the ext tree
-#pragma nounroll
-            for (int seg = 0; seg < 2; seg++) {
+        for (int tree = 0; tree < 2; tree++) {
+            double acc[8];
 #pragma unroll
-                for (int j = 0; j < BPT; j++)
+            for (int q = 0; q < 8; q++) acc[q] = 0.0;
+            const int s0 = a.seg_off[2 * o + tree] - sbase, s1 = a.seg_off[2 * o + tree + 1] - sbase;
+            for (int s = s0; s < s1; s++) {
+                const double* p = a.part + (int64_t)s * 8 * nbins + sc;
 #pragma unroll
-                    for (int q = 0; q < 8; q++) acc[j][q] = 0.0;
-                const double* recs = seg ? a.recs_e : a.recs_b;
-                const double* vrecs = seg ? a.vrecs_e : a.vrecs_b;
-                const int64_t* off = seg ? a.eoff : a.boff;
-                sweep<PREC, TB, BPT, INC>(a, recs, vrecs, off[o], off[o + 1], tile, etab, bi, cp, sp, acc, inc);
-                if (seg == 1) break;
-#pragma unroll
-                for (int j = 0; j < BPT; j++) {
-                    if (ROT) {
-                        const int iphi = bins[j] % a.g.nphi;
-                        if (PREC == 4) fp64r_finish(acc[j], a.g.cphi[iphi], a.g.sphi[iphi], a.g.kr_rev[bins[j]]);
-                        else if (PREC == 1) mixed_finish(acc[j], a.g.cphi[iphi], a.g.sphi[iphi]);
-                        else apply_temp_rot1(acc[j], a.g.cphi[iphi], a.g.sphi[iphi]);
-                    }
-                    if (PREC == 3) model_finish(acc[j], cp[j], sp[j], a.g.kr_rev[bins[j]]);
-#pragma unroll
-                    for (int q = 0; q < 8; q++)
-                        xbs[q][j * BB + tid] = acc[j][q] * k;   // ampl_far_beam * waveno (outputs_mod.f90:104)
-                }
+                for (int q = 0; q < 8; q++) acc[q] += p[(int64_t)q * nbins];
+                if (INC) inc += a.ipart_inc[(int64_t)s * nbins + sc];
             }
+            finish_sum<PREC>(acc, a.g, bc);
+#pragma unroll
+            for (int q = 0; q < 8; q++) (tree ? xe : xb)[q] = acc[q] * k;   // outputs_mod.f90:104-105
+        }
+#pragma unroll
+        for (int q = 0; q < 8; q++) xt[q] = xb[q] + xe[q];                  // outputs_mod.f90:108
+        mueller16(xt, m);
+#pragma unroll
+        for (int e = 0; e < 16; e++) msum[e] += m[e];
+        if (INC) esum += m[0] * (inc * (k * k));
+        if (live && a.store) {
+            double* so = a.store + (int64_t)o * 16 * nbins + bc;
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                so[(int64_t)q * nbins] = xb[q];
+                so[(int64_t)(8 + q) * nbins] = xe[q];
+            }
+        }
+        if (live && a.ampl_out) {
+            double* ao = a.ampl_out + (int64_t)o * 8 * nbins + bc;
+#pragma unroll
+            for (int q = 0; q < 8; q++) ao[(int64_t)q * nbins] = xt[q];
+        }
+        if (!LIST) {
             double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int j = 0; j < BPT; j++) {
-                const int slot = slot0 + j * BB;
-                const int bc = bins[j];
-                if (ROT) {
-                    const int iphi = bc % a.g.nphi;
-                    if (PREC == 4) fp64r_finish(acc[j], a.g.cphi[iphi], a.g.sphi[iphi], a.g.kr_rev[bc]);
-                    else if (PREC == 1) mixed_finish(acc[j], a.g.cphi[iphi], a.g.sphi[iphi]);
-                    else apply_temp_rot1(acc[j], a.g.cphi[iphi], a.g.sphi[iphi]);
-                }
-                if (PREC == 3) model_finish(acc[j], cp[j], sp[j], a.g.kr_rev[bc]);
-                double xb[8], xe[8], xt[8], m[16];
-#pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    xb[q] = xbs[q][j * BB + tid];
-                    xe[q] = acc[j][q] * k;      // outputs_mod.f90:105
-                    xt[q] = xb[q] + xe[q];      // outputs_mod.f90:108
-                }
-                mueller16(xt, m);
-                if (slot < nslots) {
-                    if (a.store) {
-                        double* so = a.store + (int64_t)o * 16 * nbins + bc;
-#pragma unroll
-                        for (int q = 0; q < 8; q++) {
-                            so[(int64_t)q * nbins] = xb[q];
-                            so[(int64_t)(8 + q) * nbins] = xe[q];
-                        }
-                    }
-                    if (a.ampl_out) {
-                        double* ao = a.ampl_out + (int64_t)o * 8 * nbins + bc;
-#pragma unroll
-                        for (int q = 0; q < 8; q++) ao[(int64_t)q * nbins] = xt[q];
-                    }
-                    double* mo = mp + slot;
-                    if (o == o0) {
-#pragma unroll
-                        for (int e = 0; e < 16; e++) mo[(int64_t)e * nbins] = m[e];
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 16; e++) mo[(int64_t)e * nbins] += m[e];
-                    }
-                    if (INC) {
-                        const double es = m[0] * (inc[j] * (k * k));
-                        if (o == o0) ep[slot] = es; else ep[slot] += es;
-                    }
-                    if (!LIST) {
-                        const double w1 = a.w1[bc], w2 = a.w2[bc];
-                        const double sb = mueller_s11(xb), se = mueller_s11(xe);
-                        v[0] = fma(w1, m[0], v[0]);
-                        v[1] = fma(w2, m[0], v[1]);
-                        v[2] = fma(w1, sb, v[2]);
-                        v[3] = fma(w2, sb, v[3]);
-                        v[4] = fma(w1, se, v[4]);
-                        v[5] = fma(w2, se, v[5]);
-                    }
-                }
-            }
-            if (!LIST) {
-#pragma unroll
-                for (int q = 0; q < 6; q++) v[q] = wave_sum(v[q]);
-                if ((tid & 63) == 0) {
-#pragma unroll
-                    for (int q = 0; q < 6; q++) red[tid >> 6][q] = v[q];
-                }
-                __syncthreads();
-                if (tid == 0) {
-                    double* ip = a.ipart + ((int64_t)o * a.ntiles + t) * 6;
-#pragma unroll
-                    for (int q = 0; q < 6; q++) ip[q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
-                }
-                __syncthreads();
-            }
+            if (live) integral_terms(xb, xe, m[0], w1, w2, v);
+            block_integrals(v, red, a.ipart + ((int64_t)o * gridDim.x + t) * 6);
         }
+    }
+    if (!live) return;
+    if (a.mpart) {
+        double* mo = a.mpart + (int64_t)c * 16 * nbins + slot;
+#pragma unroll
+        for (int e = 0; e < 16; e++) mo[(int64_t)e * nbins] = a.first ? msum[e] : mo[(int64_t)e * nbins] + msum[e];
+    }
+    if (INC) {
+        double* ep = a.epart + (int64_t)c * nbins + slot;
+        *ep = a.first ? esum : *ep + esum;
     }
 }
 
@@ -291,32 +167,35 @@ __global__ __launch_bounds__(BB) void k_batch_reduce_m(const double* __restrict_
     out[i] = s;
 }
 
-// integrals[o][q] = sum over tiles, in tile order
+// integrals[o][q] = sum over tiles: one wave per (orientation, integral), each lane every 64th tile
+// in order, then the lanes (a serial walk over the 507 tiles of a 721 x 180 grid took 79 us)
 __global__ __launch_bounds__(BB) void k_batch_reduce_i(const double* __restrict__ ipart, int ntiles,
                                                        int norient, double* __restrict__ out)
 {
-    const int i = blockIdx.x * BB + threadIdx.x;
+    const int i = blockIdx.x * (BB / 64) + (threadIdx.x >> 6);
     if (i >= norient * 6) return;
     const int o = i / 6, q = i - 6 * o;
     const double* p = ipart + (int64_t)o * ntiles * 6 + q;
     double s = 0.0;
-    for (int t = 0; t < ntiles; t++) s += p[(int64_t)t * 6];
-    out[i] = s;
+    for (int t = threadIdx.x & 63; t < ntiles; t += 64) s += p[(int64_t)t * 6];
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) out[i] = s;
 }
 
-// mueller_1d(theta, e) = simpne over phi of the summed Mueller matrix (get_1d_mueller,
-// outputs_mod.f90:280-329); the reference sums the per-orientation 1-D matrices,
-// which is the same linear map applied before the sum.
-__global__ __launch_bounds__(BB) void k_batch_phi(const double* __restrict__ M, const double* __restrict__ phi,
+// mueller_1d(theta, e) = the phi integral (get_1d_mueller, outputs_mod.f90:280-329) of the summed
+// Mueller matrix; the reference sums the per-orientation 1-D matrices, which is the same linear map
+// applied before the sum.  One wave per (element, theta): the row's values times the nodes' weights.
+__global__ __launch_bounds__(BB) void k_batch_phi(const double* __restrict__ M, const double* __restrict__ wphi,
                                                   int nphi, int ntheta, double* __restrict__ out)
 {
-    const int i = blockIdx.x * BB + threadIdx.x;
-    if (i >= 16 * ntheta) return;
-    const int e = i / ntheta, j = i - e * ntheta;
-    out[i] = simpne_eval(nphi, phi, M + (int64_t)nphi * ntheta * e + (int64_t)nphi * j, 1);
+    const int row = blockIdx.x * (BB / 64) + (threadIdx.x >> 6);
+    if (row >= 16 * ntheta) return;
+    const double* y = M + (int64_t)row * nphi;
+    double s = 0.0;
+    for (int i = threadIdx.x & 63; i < nphi; i += 64) s = fma(wphi[i], y[i], s);
+    s = wave_sum(s);
+    if ((threadIdx.x & 63) == 0) out[row] = s;
 }
-
-__global__ void k_zero_u32(unsigned int* p) { if (threadIdx.x == 0 && blockIdx.x == 0) p[0] = 0u; }
 
 // ---- -scaling (outputs_mod.f90:146-184) ----------------------------------------
 //
@@ -324,7 +203,7 @@ __global__ void k_zero_u32(unsigned int* p) { if (threadIdx.x == 0 && blockIdx.x
 // beam_energy_out) and the ext amplitudes by sqrt(scatt_ext_diff / ext_energy_out), scatt_*
 // being that orientation's own cross sections, then remakes the Mueller matrices and the
 // integrated parameters.  The cross sections need every bin of the orientation, so the
-// persistent pass stores the amplitudes, and this pass divides and sums them.
+// first pass stores the amplitudes, and this pass divides and sums them.
 
 // div[o] = {sqrt(scatt_beam / E_beam), sqrt(scatt_ext / E_ext)} from the unscaled integrals
 __global__ __launch_bounds__(BB) void k_scale_div(const double* __restrict__ raw, const double* __restrict__ eb,
@@ -337,9 +216,9 @@ __global__ __launch_bounds__(BB) void k_scale_div(const double* __restrict__ raw
     div[2 * o + 1] = sqrt(raw[6 * o + 4] / ee[o]);
 }
 
-// grid (ntiles of BB bins, nchunks): the chunk's orientations in order for one bin per lane;
-// mpart[c] and ipart[o][t] (ntiles = ceil(nbins / BB)) as the persistent kernel writes them.
-__global__ __launch_bounds__(BB) void k_batch_scaled(BatchArgs a, const double* __restrict__ div, int ntiles)
+// grid (ntiles of BB bins, nchunks): chunk c's share of the orientations in order for one bin per
+// lane; the Mueller sum into mpart[c] and the integrals into ipart[o][t], as k_combine writes them.
+__global__ __launch_bounds__(BB) void k_batch_scaled(CombineArgs a, const double* __restrict__ div)
 {
     __shared__ double red[BB / 64][6];
     const int tid = threadIdx.x;
@@ -352,7 +231,7 @@ __global__ __launch_bounds__(BB) void k_batch_scaled(BatchArgs a, const double* 
     double msum[16];
 #pragma unroll
     for (int e = 0; e < 16; e++) msum[e] = 0.0;
-    const int o0 = a.chunk_o[c], o1 = a.chunk_o[c + 1];
+    const int o0 = (int)((int64_t)a.o1 * c / a.nchunks), o1 = (int)((int64_t)a.o1 * (c + 1) / a.nchunks);
     for (int o = o0; o < o1; o++) {
         const double db = div[2 * o], de = div[2 * o + 1];
         const double* so = a.store + (int64_t)o * 16 * nbins + b;
@@ -372,30 +251,10 @@ __global__ __launch_bounds__(BB) void k_batch_scaled(BatchArgs a, const double* 
             for (int q = 0; q < 8; q++) ao[(int64_t)q * nbins] = xt[q];
         }
         double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        if (live) {
-            const double sb = mueller_s11(xb), se = mueller_s11(xe);
-            v[0] = w1 * m[0];
-            v[1] = w2 * m[0];
-            v[2] = w1 * sb;
-            v[3] = w2 * sb;
-            v[4] = w1 * se;
-            v[5] = w2 * se;
-        }
-#pragma unroll
-        for (int q = 0; q < 6; q++) v[q] = wave_sum(v[q]);
-        if ((tid & 63) == 0) {
-#pragma unroll
-            for (int q = 0; q < 6; q++) red[tid >> 6][q] = v[q];
-        }
-        __syncthreads();
-        if (tid == 0) {
-            double* ip = a.ipart + ((int64_t)o * ntiles + t) * 6;
-#pragma unroll
-            for (int q = 0; q < 6; q++) ip[q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
-        }
-        __syncthreads();
+        if (live) integral_terms(xb, xe, m[0], w1, w2, v);
+        block_integrals(v, red, a.ipart + ((int64_t)o * gridDim.x + t) * 6);
     }
-    if (live && o1 > o0) {
+    if (live) {
         double* mo = a.mpart + (int64_t)c * 16 * nbins + bc;
 #pragma unroll
         for (int e = 0; e < 16; e++) mo[(int64_t)e * nbins] = msum[e];
@@ -471,131 +330,150 @@ __global__ __launch_bounds__(BB) void k_gate_scatter(const double* __restrict__ 
     out[(int64_t)e * nbins + list[i]] = s;
 }
 
-template <int PREC, int TB, int BPT, int MODE>
-const void* batch_kernel() { return reinterpret_cast<const void*>(&k_batch<PREC, TB, BPT, MODE>); }
-
 }  // namespace abt
 
 // ---------------------------------------------------------------------------
-// launch helpers (called by the runtime)
-using abt::BatchArgs;
-
-extern "C" const void* abt_batch_kernel(int prec, int tb, int bpt, int mode)
-{
-    using namespace abt;
-#define K(P, T, B, M) if (prec == P && tb == T && bpt == B && mode == M) return batch_kernel<P, T, B, M>();
-    K(0, 8, 1, 0) K(0, 16, 1, 0) K(0, 32, 1, 0) K(0, 8, 2, 0) K(0, 16, 2, 0) K(0, 32, 2, 0)
-    K(1, 8, 1, 0) K(1, 16, 1, 0) K(1, 32, 1, 0) K(1, 8, 2, 0) K(1, 16, 2, 0) K(1, 32, 2, 0)
-    K(1, 8, 1, 1) K(1, 16, 1, 1) K(1, 32, 1, 1) K(1, 8, 2, 1) K(1, 16, 2, 1) K(1, 32, 2, 1)
-    K(3, 16, 1, 0)
-    K(4, 8, 1, 0) K(4, 16, 1, 0) K(4, 32, 1, 0) K(4, 8, 2, 0) K(4, 16, 2, 0)
-    K(4, 16, 1, 2)
-#undef K
-    return nullptr;
-}
-
+// launch sequences (called by the plan): kernels only, so callers may capture them in a graph
 namespace {
-int launch_pass(const void* kern, const BatchArgs& a, int wgs, hipStream_t st)
+
+using namespace abt;
+
+unsigned blocks(int64_t n) { return (unsigned)((n + BB - 1) / BB); }
+
+template <int MODE>
+void launch_combine(int prec, const CombineArgs& a, hipStream_t st)
 {
-    hipLaunchKernelGGL(abt::k_zero_u32, dim3(1), dim3(64), 0, st, a.counter);
-    BatchArgs args = a;
-    void* params[] = {&args};
-    return (int)hipLaunchKernel(kern, dim3(wgs), dim3(abt::BB), params, 0, st);
+    const dim3 grid(blocks(a.g.nbins), (unsigned)a.nchunks);
+    if (MODE == SWEEP_INC) hipLaunchKernelGGL((k_combine<1, SWEEP_INC>), grid, dim3(BB), 0, st, a);
+    else if (MODE == SWEEP_LIST) hipLaunchKernelGGL((k_combine<4, SWEEP_LIST>), grid, dim3(BB), 0, st, a);
+    else if (prec == 0) hipLaunchKernelGGL((k_combine<0, SWEEP_PLAIN>), grid, dim3(BB), 0, st, a);
+    else if (prec == 1) hipLaunchKernelGGL((k_combine<1, SWEEP_PLAIN>), grid, dim3(BB), 0, st, a);
+    else if (prec == 3) hipLaunchKernelGGL((k_combine<3, SWEEP_PLAIN>), grid, dim3(BB), 0, st, a);
+    else hipLaunchKernelGGL((k_combine<4, SWEEP_PLAIN>), grid, dim3(BB), 0, st, a);
 }
+
+// Sweep and epilogue of every group of the run's orientations.
+template <int MODE>
+int run_groups(const BatchRun& r, int prec, int tb, int bpt, SweepArgs sw, CombineArgs cb)
+{
+    for (int i = 0; i < r.ngroups; i++) {
+        const BatchGroup& G = r.groups[i];
+        if (G.s1 > G.s0) {   // a group may have no beams at all
+            SweepArgs s = sw;
+            s.segs = r.sweep.segs + G.s0;
+            int e = abt_launch_sweep(&s, G.s1 - G.s0, prec, tb, bpt, MODE, r.st);
+            if (e) return e;
+        }
+        CombineArgs c = cb;
+        c.o0 = G.o0;
+        c.o1 = G.o1;
+        c.nchunks = r.nchunks;
+        c.first = i == 0;
+        launch_combine<MODE>(prec, c, r.st);
+    }
+    return (int)hipGetLastError();
+}
+
+void reduce_mueller(const BatchRun& r)
+{
+    const int64_t n = (int64_t)16 * r.comb.g.nbins;
+    if (r.nchunks > 1)
+        hipLaunchKernelGGL(k_batch_reduce_m, dim3(blocks(n)), dim3(BB), 0, r.st, (const double*)r.mpart, r.nchunks, n,
+                           r.mueller);
+}
+
+void reduce_integrals(const BatchRun& r, double* out)
+{
+    hipLaunchKernelGGL(k_batch_reduce_i, dim3((unsigned)((r.norient * 6 + 3) / 4)), dim3(BB), 0, r.st,
+                       (const double*)r.comb.ipart, (int)blocks(r.comb.g.nbins), r.norient, out);
+}
+
+void phi_integral(const BatchRun& r)
+{
+    const DevGrid& g = r.comb.g;
+    if (r.mueller_1d)
+        hipLaunchKernelGGL(k_batch_phi, dim3((unsigned)((16 * g.ntheta + BB / 64 - 1) / (BB / 64))), dim3(BB), 0, r.st,
+                           (const double*)r.mueller, r.wphi, g.nphi, g.ntheta, r.mueller_1d);
+}
+
+CombineArgs with_mueller(const BatchRun& r)
+{
+    CombineArgs c = r.comb;
+    c.mpart = r.nchunks > 1 ? r.mpart : r.mueller;
+    return c;
+}
+
 }  // namespace
 
-extern "C" int abt_launch_batch_pass(const BatchArgs* a, int prec, int tb, int bpt, int mode, int wgs,
-                                     hipStream_t st)
+extern "C" int abt_launch_batch(const BatchRun* r)
 {
-    const void* kern = abt_batch_kernel(prec, tb, bpt, mode);
-    if (!kern) return (int)hipErrorInvalidValue;
-    int e = launch_pass(kern, *a, wgs, st);
-    return e ? e : (int)hipGetLastError();
-}
-
-extern "C" int abt_launch_batch(const BatchArgs* a, int prec, int tb, int bpt, int wgs, int norient,
-                                double* mueller, double* mueller_1d, double* integrals, hipStream_t st)
-{
-    using namespace abt;
-    const void* kern = abt_batch_kernel(prec, tb, bpt, BMODE_PLAIN);
-    if (!kern) return (int)hipErrorInvalidValue;
-    int e = launch_pass(kern, *a, wgs, st);
+    int e = run_groups<SWEEP_PLAIN>(*r, r->prec, r->tb, r->bpt, r->sweep, with_mueller(*r));
     if (e) return e;
-    const int64_t n = (int64_t)16 * a->g.nbins;
-    hipLaunchKernelGGL(k_batch_reduce_m, dim3((unsigned)((n + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->mpart, a->nchunks, n, mueller);
-    hipLaunchKernelGGL(k_batch_reduce_i, dim3((unsigned)((norient * 6 + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->ipart, a->ntiles, norient, integrals);
-    if (mueller_1d)
-        hipLaunchKernelGGL(k_batch_phi, dim3((unsigned)((16 * a->g.ntheta + BB - 1) / BB)), dim3(BB), 0, st,
-                           (const double*)mueller, a->g.phi, a->g.nphi, a->g.ntheta, mueller_1d);
+    reduce_mueller(*r);
+    reduce_integrals(*r, r->integrals);
+    phi_integral(*r);
     return (int)hipGetLastError();
 }
 
-extern "C" int abt_launch_batch_scaled(const BatchArgs* a, int prec, int tb, int bpt, int wgs, int norient,
-                                       const double* beam_energy, const double* ext_energy, double* raw,
-                                       double* div, double* mueller, double* mueller_1d, double* integrals,
-                                       hipStream_t st)
+extern "C" int abt_launch_batch_scaled(const BatchRun* r, const ScaleBufs* s)
 {
-    using namespace abt;
-    const void* kern = abt_batch_kernel(prec, tb, bpt, BMODE_PLAIN);
-    if (!kern || !a->store) return (int)hipErrorInvalidValue;
-    BatchArgs s = *a;
-    s.ampl_out = nullptr;   // the divided totals are written by the scaling pass
-    int e = launch_pass(kern, s, wgs, st);
+    if (!s->store) return (int)hipErrorInvalidValue;
+    CombineArgs c = r->comb;
+    c.mpart = nullptr;      // formed from the divided amplitudes below
+    c.ampl_out = nullptr;
+    c.store = s->store;
+    int e = run_groups<SWEEP_PLAIN>(*r, r->prec, r->tb, r->bpt, r->sweep, c);
     if (e) return e;
-    hipLaunchKernelGGL(k_batch_reduce_i, dim3((unsigned)((norient * 6 + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->ipart, a->ntiles, norient, raw);
-    hipLaunchKernelGGL(k_scale_div, dim3((unsigned)((norient + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)raw, beam_energy, ext_energy, norient, div);
-    const int nt1 = (a->g.nbins + BB - 1) / BB;
-    hipLaunchKernelGGL(k_batch_scaled, dim3((unsigned)nt1, (unsigned)a->nchunks), dim3(BB), 0, st, *a,
-                       (const double*)div, nt1);
-    const int64_t n = (int64_t)16 * a->g.nbins;
-    hipLaunchKernelGGL(k_batch_reduce_m, dim3((unsigned)((n + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->mpart, a->nchunks, n, mueller);
-    hipLaunchKernelGGL(k_batch_reduce_i, dim3((unsigned)((norient * 6 + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->ipart, nt1, norient, integrals);
-    if (mueller_1d)
-        hipLaunchKernelGGL(k_batch_phi, dim3((unsigned)((16 * a->g.ntheta + BB - 1) / BB)), dim3(BB), 0, st,
-                           (const double*)mueller, a->g.phi, a->g.nphi, a->g.ntheta, mueller_1d);
+    reduce_integrals(*r, s->raw);
+    hipLaunchKernelGGL(k_scale_div, dim3(blocks(r->norient)), dim3(BB), 0, r->st, (const double*)s->raw,
+                       s->beam_energy, s->ext_energy, r->norient, s->div);
+    c = with_mueller(*r);
+    c.store = s->store;
+    c.o0 = 0;
+    c.o1 = r->norient;
+    c.nchunks = r->nchunks;
+    hipLaunchKernelGGL(k_batch_scaled, dim3(blocks(c.g.nbins), (unsigned)r->nchunks), dim3(BB), 0, r->st, c,
+                       (const double*)s->div);
+    reduce_mueller(*r);
+    reduce_integrals(*r, r->integrals);
+    phi_integral(*r);
     return (int)hipGetLastError();
 }
 
-extern "C" int abt_launch_batch_gated(const BatchArgs* a, int tb, int bpt, int wgs, int wgs2, int norient,
-                                      double* est, int32_t* flags, int32_t* list, int32_t* count,
-                                      double* mueller, double* mueller_1d, double* integrals, hipStream_t st)
+extern "C" int abt_launch_batch_est(const BatchRun* r, const GateBufs* q)
 {
-    using namespace abt;
-    const void* k1 = abt_batch_kernel(1, tb, bpt, BMODE_EST);
-    const void* k2 = abt_batch_kernel(4, 16, 1, BMODE_LIST);
-    if (!k1 || !k2) return (int)hipErrorInvalidValue;
-    const int nbins = a->g.nbins;
+    CombineArgs c = with_mueller(*r);
+    c.epart = r->nchunks > 1 ? q->epart : q->est;
+    return run_groups<SWEEP_INC>(*r, 1, r->tb, r->bpt, r->sweep, c);
+}
+
+extern "C" int abt_launch_batch_gated(const BatchRun* r, const GateBufs* q)
+{
     // pass 1: mixed, with the error scale
-    int e = launch_pass(k1, *a, wgs, st);
+    int e = abt_launch_batch_est(r, q);
     if (e) return e;
-    const int64_t n = (int64_t)16 * nbins;
-    hipLaunchKernelGGL(k_batch_reduce_m, dim3((unsigned)((n + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->mpart, a->nchunks, n, mueller);
-    hipLaunchKernelGGL(k_batch_reduce_m, dim3((unsigned)((nbins + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->epart, a->nchunks, (int64_t)nbins, est);
-    hipLaunchKernelGGL(k_batch_reduce_i, dim3((unsigned)((norient * 6 + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->ipart, a->ntiles, norient, integrals);
+    const int nbins = r->comb.g.nbins;
+    reduce_mueller(*r);
+    if (r->nchunks > 1)
+        hipLaunchKernelGGL(k_batch_reduce_m, dim3(blocks(nbins)), dim3(BB), 0, r->st, (const double*)q->epart,
+                           r->nchunks, (int64_t)nbins, q->est);
+    reduce_integrals(*r, r->integrals);
     // the bins whose error bound exceeds the gate
-    hipLaunchKernelGGL(k_gate_flags, dim3((unsigned)((nbins + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)mueller, (const double*)est, nbins, flags);
-    hipLaunchKernelGGL(k_gate_compact, dim3(1), dim3(CB), 0, st, (const int32_t*)flags, nbins, list, count);
+    hipLaunchKernelGGL(k_gate_flags, dim3(blocks(nbins)), dim3(BB), 0, r->st, (const double*)r->mueller,
+                       (const double*)q->est, nbins, q->flags);
+    hipLaunchKernelGGL(k_gate_compact, dim3(1), dim3(CB), 0, r->st, (const int32_t*)q->flags, nbins, q->list, q->count);
     // pass 2: those bins in FP64 (restructured body), written over the mixed sums
-    BatchArgs b = *a;
-    b.list = list;
-    b.list_count = count;
-    e = launch_pass(k2, b, wgs2, st);
+    SweepArgs s = r->sweep;
+    s.list = q->list;
+    s.list_count = q->count;
+    CombineArgs c = r->comb;
+    c.mpart = q->lpart;
+    c.list = q->list;
+    c.list_count = q->count;
+    e = run_groups<SWEEP_LIST>(*r, 4, 16, 1, s, c);
     if (e) return e;
-    hipLaunchKernelGGL(k_gate_scatter, dim3((unsigned)((n + BB - 1) / BB)), dim3(BB), 0, st,
-                       (const double*)a->mpart, a->nchunks, nbins, (const int32_t*)list, (const int32_t*)count,
-                       mueller);
-    if (mueller_1d)
-        hipLaunchKernelGGL(k_batch_phi, dim3((unsigned)((16 * a->g.ntheta + BB - 1) / BB)), dim3(BB), 0, st,
-                           (const double*)mueller, a->g.phi, a->g.nphi, a->g.ntheta, mueller_1d);
+    hipLaunchKernelGGL(k_gate_scatter, dim3(blocks((int64_t)16 * nbins)), dim3(BB), 0, r->st, (const double*)q->lpart,
+                       r->nchunks, nbins, (const int32_t*)q->list, (const int32_t*)q->count, r->mueller);
+    phi_integral(*r);
     return (int)hipGetLastError();
 }

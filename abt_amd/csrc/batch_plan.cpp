@@ -1,5 +1,5 @@
 // batch_plan.cpp -- host side of the orientation-batched far field: plans (orientation
-// offsets, chunking, integral weights, resident workspace), the tile-shape
+// offsets, segments, integral weights, resident workspace), the tile-shape
 // autotuner, the capture-safe launch sequence and its HIP graph.
 #include <hip/hip_runtime.h>
 
@@ -17,36 +17,22 @@
 namespace {
 
 constexpr int LANES = 256;
-// Queue depth per persistent workgroup: bounds the tail (the last units finish at different
-// times).  On 1000 orientations of the rough column: 16 units per workgroup (32 chunks)
-// 3552 ms, 32 (64) 3503 ms, 64 (128) 3473 ms.  Partial sums: 128 B per bin per chunk.
 constexpr int MAX_CHUNKS = 128;
-constexpr int UNITS_PER_WG = 64;
+// Segment sums kept at once: 64 bytes per bin and segment.  Orientations are run in groups whose
+// segments fit; a group's last round of workgroups costs about 512 / (segments x tiles) of its time
+// (0.4 % at 2 GiB).
+constexpr size_t PART_BYTES = (size_t)2 << 30;
+// Workgroups a run is cut into, per CU (4 resident): the last round is then under 1 % of a run, and
+// a few coarse orientations still fill the chip.
+constexpr int64_t UNITS_PER_CU = 256;
+constexpr int64_t MIN_SEG = 32, MAX_SEG = 4096;
 const int TB_CAND[3] = {8, 16, 32};
 const int BPT_CAND[2] = {1, 2};
 
 struct Shape {
     int tb = 16, bpt = 1;
-    int wgs = 0;        // persistent workgroups
-    int ntiles = 0;
-    int nchunks = 0;
+    int wgs = 0;        // workgroups the chip holds at once
 };
-
-// Contiguous orientation ranges with about equal beam counts (beam + ext trees).
-void make_chunks(const int64_t* boff, const int64_t* eoff, int n, int nch, std::vector<int32_t>& out)
-{
-    out.assign(1, 0);
-    const double total = (double)(boff[n] - boff[0] + eoff[n] - eoff[0]);
-    int o = 0;
-    for (int c = 1; c < nch; c++) {
-        const double target = total * c / nch;
-        while (o < n && (double)(boff[o] - boff[0] + eoff[o] - eoff[0]) < target) o++;
-        o = std::max(o, out.back() + 1);
-        o = std::min(o, n - (nch - c));
-        out.push_back(o);
-    }
-    out.push_back(n);
-}
 
 // ABI precision -> kernel variant: ABT_FP64_ACCURATE runs the accurate-phase FP64 body (3),
 // ABT_FP64_FAST the restructured FP64 body (4); ABT_MIXED_GATED's tuned pass is the mixed
@@ -60,7 +46,7 @@ int kernel_prec(int precision)
         default: return precision;
     }
 }
-int kernel_mode(int precision) { return precision == ABT_MIXED_GATED ? abt::BMODE_EST : abt::BMODE_PLAIN; }
+int kernel_mode(int precision) { return precision == ABT_MIXED_GATED ? abt::SWEEP_INC : abt::SWEEP_PLAIN; }
 
 bool shape_allowed(int prec, int tb, int bpt)
 {
@@ -69,20 +55,8 @@ bool shape_allowed(int prec, int tb, int bpt)
     return true;
 }
 
-int kernel_occupancy(const void* k, int* per_cu)
-{
-    int n = 0;
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, LANES, 0));
-    *per_cu = std::max(1, n);
-    return 0;
-}
-
-int occupancy(int prec, int tb, int bpt, int* per_cu)
-{
-    const void* k = abt_batch_kernel(kernel_prec(prec), tb, bpt, kernel_mode(prec));
-    if (!k) return abt_fail(ABT_ERR_ARG, "no batched kernel for beams_per_tile %d, bins_per_thread %d", tb, bpt);
-    return kernel_occupancy(k, per_cu);
-}
+int64_t round_up(int64_t n, int64_t q) { return (n + q - 1) / q * q; }
+int64_t ceil_div(int64_t n, int64_t q) { return (n + q - 1) / q; }
 
 }  // namespace
 
@@ -91,93 +65,130 @@ struct abt_batch_plan {
     int norient = 0, prec = 0, fast_diff = 0, cus = 256;
     std::vector<int64_t> boff, eoff;
     Shape shape;
-    bool tuned = false;
+    // the cut: segments of at most seg_len beams, orientation by orientation (beam tree, ext tree)
+    int64_t seg_len = 0;
+    std::vector<int32_t> seg_off;          // [2 norient + 1]
+    std::vector<abt::BatchGroup> groups;
+    int64_t max_segs = 0;                  // of a group: what the segment-sum buffer holds
+    int nchunks = 1;                       // Mueller partial sums
     // device memory: one allocation
     void* mem = nullptr;
-    int64_t* d_boff = nullptr;
-    int64_t* d_eoff = nullptr;
-    int32_t* d_chunk = nullptr;      // [MAX_CHUNKS + 1] chunk table of the plan's shape
-    int32_t* d_chunk_tune = nullptr; // [MAX_CHUNKS + 1] chunk table of the autotuner's sample
+    size_t mem_bytes = 0;
+    abt::SweepSeg* d_segs = nullptr;
+    int32_t* d_seg_off = nullptr;
     double* d_w1 = nullptr;
     double* d_w2 = nullptr;
-    double* d_mpart = nullptr;       // [max_chunks][16][nbins]
-    double* d_ipart = nullptr;       // [norient][ntiles(bpt=1)][6]
-    unsigned int* d_counter = nullptr;
-    // gated mixed precision: error-scale partials and sums, flags, the list of FP64 bins
-    double* d_epart = nullptr;       // [max_chunks][nbins]
-    double* d_est = nullptr;         // [nbins]
-    int32_t* d_flags = nullptr;      // [nbins]
-    int32_t* d_list = nullptr;       // [nbins]
-    int32_t* d_count = nullptr;
-    int wgs_list = 0;                // persistent workgroups of the FP64 list pass
+    double* d_wphi = nullptr;
+    double* d_part = nullptr;        // [max_segs][8][nbins]
+    double* d_pinc = nullptr;        // [max_segs][nbins] (gated)
+    double* d_mpart = nullptr;       // [nchunks][16][nbins] (nchunks > 1, or gated)
+    double* d_ipart = nullptr;       // [norient][ntiles][6]
+    abt::GateBufs gate = {};
     // -scaling: per-orientation amplitudes, unscaled integrals, divisors; the caller's energies
     void* smem = nullptr;
-    double* d_store = nullptr;       // [norient][16][nbins]
-    double* d_raw = nullptr;         // [norient][6]
-    double* d_div = nullptr;         // [norient][2]
-    const double* beam_energy = nullptr;
-    const double* ext_energy = nullptr;
-    int max_chunks = 1;
+    size_t smem_bytes = 0;
+    abt::ScaleBufs scale = {};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
 
 namespace {
 
-int shape_for(const abt_batch_plan* p, int norient, int tb, int bpt, Shape* s)
+int shape_for(const abt_batch_plan* p, int tb, int bpt, Shape* s)
 {
-    int per_cu = 1;
-    int rc = occupancy(p->prec, tb, bpt, &per_cu);
-    if (rc) return rc;
+    const void* k = abt_sweep_kernel(kernel_prec(p->prec), tb, bpt, kernel_mode(p->prec));
+    if (!k) return abt_fail(ABT_ERR_ARG, "no batched kernel for beams_per_tile %d, bins_per_thread %d", tb, bpt);
+    int n = 0;
+    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, LANES, 0));
     s->tb = tb;
     s->bpt = bpt;
-    s->wgs = per_cu * p->cus;
-    s->ntiles = (int)((p->g->nbins + (int64_t)LANES * bpt - 1) / ((int64_t)LANES * bpt));
-    int64_t want = (int64_t)UNITS_PER_WG * s->wgs;
-    int64_t nch = (want + s->ntiles - 1) / s->ntiles;
-    nch = std::min<int64_t>(nch, std::min(norient, MAX_CHUNKS));
-    s->nchunks = (int)std::max<int64_t>(1, nch);
+    s->wgs = std::max(1, n) * p->cus;
     return 0;
 }
 
-// Launch arguments of the plan's buffers with chunk table `chunk` and shape s.
-void fill_args(const abt_batch_plan* p, const Shape& s, const int32_t* chunk, const double* rb,
-               const double* vb, const double* re, const double* ve, abt::BatchArgs* a)
+// The segment length and table.  A rule of the plan's sizes only (not of the tile shape), so that
+// every shape gives the same sums; lengths are multiples of 32, so that the mixed body's FP32 beam
+// groups are those of the uncut list.
+void make_segments(abt_batch_plan* p, std::vector<abt::SweepSeg>& segs)
 {
-    a->g = p->g->d;
-    a->recs_b = rb;
-    a->vrecs_b = vb ? vb : rb;
-    a->recs_e = re;
-    a->vrecs_e = ve ? ve : re;
-    a->boff = p->d_boff;
-    a->eoff = p->d_eoff;
-    a->chunk_o = chunk;
-    a->w1 = p->d_w1;
-    a->w2 = p->d_w2;
-    a->mpart = p->d_mpart;
-    a->ipart = p->d_ipart;
-    a->counter = p->d_counter;
-    a->ampl_out = nullptr;
-    a->store = p->d_store;
-    a->epart = p->d_epart;
-    a->list = p->d_list;
-    a->list_count = p->d_count;
-    a->nchunks = s.nchunks;
-    a->ntiles = s.ntiles;
-    a->nunits = s.nchunks * s.ntiles;
-    a->fast_diff = p->fast_diff;
+    const int n = p->norient;
+    const int64_t nbins = p->g->nbins, tiles = ceil_div(nbins, LANES);
+    const int64_t total = p->boff[n] + p->eoff[n];
+    const int64_t want = std::max<int64_t>(1, ceil_div(UNITS_PER_CU * p->cus, tiles));
+    int64_t len = std::min(MAX_SEG, std::max(MIN_SEG, round_up(ceil_div(total, want), 32)));
+    // an orientation's segments fit the buffer and one launch
+    const int64_t most = std::max<int64_t>(2, std::min<int64_t>(65535, (int64_t)(PART_BYTES / (64 * (size_t)nbins))));
+    int64_t largest = 1;
+    for (int o = 0; o < n; o++)
+        largest = std::max(largest, p->boff[o + 1] - p->boff[o] + p->eoff[o + 1] - p->eoff[o]);
+    len = std::max(len, most > 2 ? round_up(ceil_div(largest, most - 1), 32) : round_up(largest, 32));
+    p->seg_len = len;
+    p->seg_off.assign(1, 0);
+    for (int o = 0; o < n; o++)
+        for (int tree = 0; tree < 2; tree++) {
+            const std::vector<int64_t>& off = tree ? p->eoff : p->boff;
+            for (int64_t b = off[o]; b < off[o + 1]; b += len)
+                segs.push_back({b, (int32_t)std::min(len, off[o + 1] - b), tree});
+            p->seg_off.push_back((int32_t)segs.size());
+        }
+    // groups of orientations: at most `most` segments each
+    p->max_segs = 1;
+    for (int o = 0; o < n;) {
+        int e = o + 1;
+        while (e < n && p->seg_off[2 * (e + 1)] - p->seg_off[2 * o] <= most) e++;
+        p->groups.push_back({o, e, p->seg_off[2 * o], p->seg_off[2 * e]});
+        p->max_segs = std::max<int64_t>(p->max_segs, p->seg_off[2 * e] - p->seg_off[2 * o]);
+        o = e;
+    }
 }
 
-// Upload the chunk table of the first `norient` orientations for `nchunks` chunks.
-int upload_chunks(const abt_batch_plan* p, int norient, int nchunks, int32_t* dst)
+// The launches over the first `norient` orientations: groups (the plan's, cut at norient).
+std::vector<abt::BatchGroup> groups_of(const abt_batch_plan* p, int norient)
 {
-    std::vector<int32_t> ch;
-    make_chunks(p->boff.data(), p->eoff.data(), norient, nchunks, ch);
-    HIPCHK(hipMemcpy(dst, ch.data(), sizeof(int32_t) * ch.size(), hipMemcpyHostToDevice));
-    return 0;
+    std::vector<abt::BatchGroup> out;
+    for (const abt::BatchGroup& G : p->groups) {
+        if (G.o0 >= norient) break;
+        const int o1 = std::min(G.o1, norient);
+        out.push_back({G.o0, o1, G.s0, p->seg_off[2 * o1]});
+    }
+    return out;
 }
 
-int sync_chunks(abt_batch_plan* p) { return upload_chunks(p, p->norient, p->shape.nchunks, p->d_chunk); }
+// A run of the plan's buffers in shape s.
+abt::BatchRun make_run(const abt_batch_plan* p, const Shape& s, const std::vector<abt::BatchGroup>& groups,
+                       int norient, const double* rb, const double* vb, const double* re, const double* ve,
+                       hipStream_t st)
+{
+    abt::BatchRun r;
+    memset(&r, 0, sizeof(r));
+    r.sweep.g = p->g->d;
+    r.sweep.recs[0] = rb;
+    r.sweep.recs[1] = re;
+    r.sweep.vrecs[0] = vb ? vb : rb;
+    r.sweep.vrecs[1] = ve ? ve : re;
+    r.sweep.segs = p->d_segs;
+    r.sweep.part = p->d_part;
+    r.sweep.ipart = p->d_pinc;
+    r.sweep.fast_diff = p->fast_diff;
+    r.comb.g = p->g->d;
+    r.comb.part = p->d_part;
+    r.comb.ipart_inc = p->d_pinc;
+    r.comb.seg_off = p->d_seg_off;
+    r.comb.w1 = p->d_w1;
+    r.comb.w2 = p->d_w2;
+    r.comb.ipart = p->d_ipart;
+    r.groups = groups.data();
+    r.ngroups = (int)groups.size();
+    r.prec = kernel_prec(p->prec);
+    r.tb = s.tb;
+    r.bpt = s.bpt;
+    r.norient = norient;
+    r.nchunks = p->nchunks;
+    r.mpart = p->d_mpart;
+    r.wphi = p->d_wphi;
+    r.st = st;
+    return r;
+}
 
 int check_recs(const double* rb, const double* re, const abt_batch_plan* p)
 {
@@ -223,39 +234,30 @@ int abt_batch_plan_create(const abt_dev_grid* g, int32_t norient, const int64_t*
     p->cus = cus;
     p->boff.assign(beam_off, beam_off + norient + 1);
     p->eoff.assign(ext_off, ext_off + norient + 1);
-    // largest chunk count over the candidate shapes sizes the partial sums
-    p->max_chunks = 1;
-    for (int tb : TB_CAND)
-        for (int bpt : BPT_CAND) {
-            if (!shape_allowed(precision, tb, bpt)) continue;
-            Shape s;
-            rc = shape_for(p, norient, tb, bpt, &s);
-            if (rc) { delete p; return rc; }
-            p->max_chunks = std::max(p->max_chunks, s.nchunks);
-        }
-    rc = shape_for(p, norient, 16, 1, &p->shape);
+    // (the restructured body's 8-beam tiles hold 4 waves per SIMD)
+    rc = shape_for(p, precision == ABT_FP64_FAST ? 8 : 16, 1, &p->shape);
     if (rc) { delete p; return rc; }
+    std::vector<abt::SweepSeg> segs;
+    make_segments(p, segs);
     const bool gated = precision == ABT_MIXED_GATED;
-    if (gated) {
-        int per_cu = 1;
-        rc = kernel_occupancy(abt_batch_kernel(4, 16, 1, abt::BMODE_LIST), &per_cu);
-        if (rc) { delete p; return rc; }
-        p->wgs_list = per_cu * cus;
-    }
-    const int64_t nbins = g->nbins, ntiles1 = (nbins + LANES - 1) / LANES;
+    const int64_t nbins = g->nbins, ntiles = ceil_div(nbins, LANES);
+    int longest = 1;   // orientations of the largest group
+    for (const abt::BatchGroup& G : p->groups) longest = std::max(longest, G.o1 - G.o0);
+    p->nchunks = (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(4 * cus, ntiles), std::min(longest, MAX_CHUNKS)));
     const int nth = g->d.ntheta, nph = g->d.nphi;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
-    const size_t o_boff = take(sizeof(int64_t) * (norient + 1));
-    const size_t o_eoff = take(sizeof(int64_t) * (norient + 1));
-    const size_t o_chunk = take(sizeof(int32_t) * (MAX_CHUNKS + 1));
-    const size_t o_chunk_t = take(sizeof(int32_t) * (MAX_CHUNKS + 1));
+    const size_t mpart_bytes = sizeof(double) * 16 * nbins * (size_t)p->nchunks;
+    const size_t o_seg = take(sizeof(abt::SweepSeg) * std::max<size_t>(1, segs.size()));
+    const size_t o_so = take(sizeof(int32_t) * p->seg_off.size());
     const size_t o_w1 = take(sizeof(double) * nbins);
     const size_t o_w2 = take(sizeof(double) * nbins);
-    const size_t o_mp = take(sizeof(double) * 16 * nbins * (size_t)p->max_chunks);
-    const size_t o_ip = take(sizeof(double) * 6 * (size_t)ntiles1 * norient);
-    const size_t o_ct = take(sizeof(unsigned int) * 64);
-    const size_t o_ep = gated ? take(sizeof(double) * nbins * (size_t)p->max_chunks) : 0;
+    const size_t o_wp = take(sizeof(double) * nph);
+    const size_t o_pt = take(sizeof(double) * 8 * nbins * (size_t)p->max_segs);
+    const size_t o_mp = p->nchunks > 1 || gated ? take(mpart_bytes) : 0;
+    const size_t o_ip = take(sizeof(double) * 6 * (size_t)ntiles * norient);
+    const size_t o_pi = gated ? take(sizeof(double) * nbins * (size_t)p->max_segs) : 0;
+    const size_t o_ep = gated ? take(sizeof(double) * nbins * (size_t)p->nchunks) : 0;
     const size_t o_est = gated ? take(sizeof(double) * nbins) : 0;
     const size_t o_fl = gated ? take(sizeof(int32_t) * nbins) : 0;
     const size_t o_li = gated ? take(sizeof(int32_t) * nbins) : 0;
@@ -264,22 +266,20 @@ int abt_batch_plan_create(const abt_dev_grid* g, int32_t norient, const int64_t*
         delete p;
         return abt_fail(ABT_ERR_NOMEM, "batched plan: hipMalloc of %zu bytes failed", off);
     }
+    p->mem_bytes = off;
     char* m = (char*)p->mem;
-    p->d_boff = (int64_t*)(m + o_boff);
-    p->d_eoff = (int64_t*)(m + o_eoff);
-    p->d_chunk = (int32_t*)(m + o_chunk);
-    p->d_chunk_tune = (int32_t*)(m + o_chunk_t);
+    p->d_segs = (abt::SweepSeg*)(m + o_seg);
+    p->d_seg_off = (int32_t*)(m + o_so);
     p->d_w1 = (double*)(m + o_w1);
     p->d_w2 = (double*)(m + o_w2);
-    p->d_mpart = (double*)(m + o_mp);
+    p->d_wphi = (double*)(m + o_wp);
+    p->d_part = (double*)(m + o_pt);
+    if (p->nchunks > 1 || gated) p->d_mpart = (double*)(m + o_mp);
     p->d_ipart = (double*)(m + o_ip);
-    p->d_counter = (unsigned int*)(m + o_ct);
     if (gated) {
-        p->d_epart = (double*)(m + o_ep);
-        p->d_est = (double*)(m + o_est);
-        p->d_flags = (int32_t*)(m + o_fl);
-        p->d_list = (int32_t*)(m + o_li);
-        p->d_count = (int32_t*)(m + o_cn);
+        p->d_pinc = (double*)(m + o_pi);
+        p->gate = {(double*)(m + o_ep), (double*)(m + o_est), (int32_t*)(m + o_fl), (int32_t*)(m + o_li),
+                   (int32_t*)(m + o_cn), p->d_mpart};
     }
     // integral weights: simpne over phi, then x sin(theta) / k^2 (x cos(theta)) and simpne over theta
     std::vector<double> th(nth), ph(nph), wt(nth), wp(nph), w1(nbins), w2(nbins);
@@ -300,18 +300,15 @@ int abt_batch_plan_create(const abt_dev_grid* g, int32_t norient, const int64_t*
         e = hipMemcpy(p->d_w1, w1.data(), sizeof(double) * nbins, hipMemcpyHostToDevice);
     }
     if (e == hipSuccess) e = hipMemcpy(p->d_w2, w2.data(), sizeof(double) * nbins, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->d_boff, beam_off, sizeof(int64_t) * (norient + 1), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->d_eoff, ext_off, sizeof(int64_t) * (norient + 1), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(p->d_wphi, wp.data(), sizeof(double) * nph, hipMemcpyHostToDevice);
+    if (e == hipSuccess && !segs.empty())
+        e = hipMemcpy(p->d_segs, segs.data(), sizeof(abt::SweepSeg) * segs.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess)
+        e = hipMemcpy(p->d_seg_off, p->seg_off.data(), sizeof(int32_t) * p->seg_off.size(), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
         (void)hipFree(p->mem);
         delete p;
         return abt_fail(ABT_ERR_HIP, "batched plan upload: %s", hipGetErrorString(e));
-    }
-    rc = sync_chunks(p);
-    if (rc) {
-        (void)hipFree(p->mem);
-        delete p;
-        return rc;
     }
     *out = p;
     return 0;
@@ -340,8 +337,8 @@ int abt_batch_set_scaling(abt_batch_plan* p, const double* beam_energy_out, cons
     if (!beam_energy_out) {
         if (p->smem) (void)hipFree(p->smem);
         p->smem = nullptr;
-        p->d_store = p->d_raw = p->d_div = nullptr;
-        p->beam_energy = p->ext_energy = nullptr;
+        p->smem_bytes = 0;
+        p->scale = {};
         return 0;
     }
     if (!p->smem) {
@@ -352,12 +349,13 @@ int abt_batch_set_scaling(abt_batch_plan* p, const double* beam_energy_out, cons
         if (e != hipSuccess)
             return abt_fail(ABT_ERR_HIP, "abt_batch_set_scaling: %zu bytes: %s", bytes, hipGetErrorString(e));
         p->smem = m;
-        p->d_store = (double*)m;
-        p->d_raw = p->d_store + nstore;
-        p->d_div = p->d_raw + 6 * (size_t)p->norient;
+        p->smem_bytes = bytes;
+        p->scale.store = (double*)m;
+        p->scale.raw = p->scale.store + nstore;
+        p->scale.div = p->scale.raw + 6 * (size_t)p->norient;
     }
-    p->beam_energy = beam_energy_out;
-    p->ext_energy = ext_energy_out;
+    p->scale.beam_energy = beam_energy_out;
+    p->scale.ext_energy = ext_energy_out;
     return 0;
 }
 
@@ -365,12 +363,11 @@ int abt_batch_set_tiles(abt_batch_plan* p, int32_t beams_per_tile, int32_t bins_
 {
     if (!p) return abt_fail(ABT_ERR_ARG, "abt_batch_set_tiles: null plan");
     Shape s;
-    int rc = shape_for(p, p->norient, beams_per_tile, bins_per_thread, &s);
+    int rc = shape_for(p, beams_per_tile, bins_per_thread, &s);
     if (rc) return rc;
     drop_graph(p);   // a captured graph holds the old shape
     p->shape = s;
-    p->tuned = true;
-    return sync_chunks(p);
+    return 0;
 }
 
 int abt_batch_get_tiles(const abt_batch_plan* p, int32_t* beams_per_tile, int32_t* bins_per_thread,
@@ -379,7 +376,7 @@ int abt_batch_get_tiles(const abt_batch_plan* p, int32_t* beams_per_tile, int32_
     if (!p) return abt_fail(ABT_ERR_ARG, "abt_batch_get_tiles: null plan");
     if (beams_per_tile) *beams_per_tile = p->shape.tb;
     if (bins_per_thread) *bins_per_thread = p->shape.bpt;
-    if (chunks) *chunks = p->shape.nchunks;
+    if (chunks) *chunks = p->nchunks;
     if (workgroups) *workgroups = p->shape.wgs;
     return 0;
 }
@@ -402,6 +399,7 @@ int abt_batch_autotune(abt_batch_plan* p, const double* recs_b, const double* vr
     hipEvent_t e0 = nullptr, e1 = nullptr;
     hipError_t he = hipEventCreate(&e0);
     if (he == hipSuccess) he = hipEventCreate(&e1);
+    const std::vector<abt::BatchGroup> groups = groups_of(p, ns);
     float best = 1e30f;
     Shape best_s = p->shape;
     int idx = 0;
@@ -415,22 +413,16 @@ int abt_batch_autotune(abt_batch_plan* p, const double* recs_b, const double* vr
                 continue;
             }
             Shape s;
-            rc = shape_for(p, ns, tb, bpt, &s);
+            rc = shape_for(p, tb, bpt, &s);
             if (rc) break;
-            rc = upload_chunks(p, ns, s.nchunks, p->d_chunk_tune);
-            if (rc) break;
-            abt::BatchArgs a;
-            fill_args(p, s, p->d_chunk_tune, recs_b, vrecs_b, recs_e, vrecs_e, &a);
-            a.store = nullptr;   // the timing is the far-field pass's
+            abt::BatchRun r = make_run(p, s, groups, ns, recs_b, vrecs_b, recs_e, vrecs_e, st);
+            r.mueller = out;
+            r.integrals = out + 16 * nbins;
             float ms = 0.f;
             for (int rep = 0; rep < 2 && !rc; rep++) {   // first launch warms up
                 he = hipEventRecord(e0, st);
-                // gated plans tune their mixed pass (the plain mixed kernel of the same shape
-                // plus the error scale: run the pass alone)
-                int le = kernel_mode(p->prec) == abt::BMODE_EST
-                             ? abt_launch_batch_pass(&a, kernel_prec(p->prec), tb, bpt, kernel_mode(p->prec), s.wgs, st)
-                             : abt_launch_batch(&a, kernel_prec(p->prec), tb, bpt, s.wgs, ns, out, nullptr,
-                                                out + 16 * nbins, st);
+                // gated plans tune their mixed pass with its error scale
+                const int le = p->prec == ABT_MIXED_GATED ? abt_launch_batch_est(&r, &p->gate) : abt_launch_batch(&r);
                 if (le) rc = abt_fail(ABT_ERR_HIP, "batched launch failed: %s", hipGetErrorString((hipError_t)le));
                 if (he == hipSuccess) he = hipEventRecord(e1, st);
                 if (he == hipSuccess) he = hipEventSynchronize(e1);
@@ -449,13 +441,9 @@ int abt_batch_autotune(abt_batch_plan* p, const double* recs_b, const double* vr
     (void)hipFree(out);
     if (rc) return rc;
     if (he != hipSuccess) return abt_fail(ABT_ERR_HIP, "autotune timing: %s", hipGetErrorString(he));
-    Shape s;
-    rc = shape_for(p, p->norient, best_s.tb, best_s.bpt, &s);
-    if (rc) return rc;
     drop_graph(p);
-    p->shape = s;
-    p->tuned = true;
-    return sync_chunks(p);
+    p->shape = best_s;
+    return 0;
 }
 
 int abt_batch_run(const abt_batch_plan* p, const double* recs_b, const double* vrecs_b,
@@ -467,21 +455,14 @@ int abt_batch_run(const abt_batch_plan* p, const double* recs_b, const double* v
     if (rc) return rc;
     rc = abt_ensure_device(nullptr);
     if (rc) return rc;
-    abt::BatchArgs a;
-    fill_args(p, p->shape, p->d_chunk, recs_b, vrecs_b, recs_e, vrecs_e, &a);
-    a.ampl_out = dev_ampl;
-    int e;
-    if (p->beam_energy)
-        e = abt_launch_batch_scaled(&a, kernel_prec(p->prec), p->shape.tb, p->shape.bpt, p->shape.wgs, p->norient,
-                                    p->beam_energy, p->ext_energy, p->d_raw, p->d_div, dev_mueller,
-                                    dev_mueller_1d, dev_integrals, (hipStream_t)stream);
-    else if (p->prec == ABT_MIXED_GATED)
-        e = abt_launch_batch_gated(&a, p->shape.tb, p->shape.bpt, p->shape.wgs, p->wgs_list, p->norient,
-                                   p->d_est, p->d_flags, p->d_list, p->d_count, dev_mueller, dev_mueller_1d,
-                                   dev_integrals, (hipStream_t)stream);
-    else
-        e = abt_launch_batch(&a, kernel_prec(p->prec), p->shape.tb, p->shape.bpt, p->shape.wgs, p->norient,
-                             dev_mueller, dev_mueller_1d, dev_integrals, (hipStream_t)stream);
+    abt::BatchRun r = make_run(p, p->shape, p->groups, p->norient, recs_b, vrecs_b, recs_e, vrecs_e, (hipStream_t)stream);
+    r.comb.ampl_out = dev_ampl;
+    r.mueller = dev_mueller;
+    r.mueller_1d = dev_mueller_1d;
+    r.integrals = dev_integrals;
+    const int e = p->scale.beam_energy       ? abt_launch_batch_scaled(&r, &p->scale)
+                  : p->prec == ABT_MIXED_GATED ? abt_launch_batch_gated(&r, &p->gate)
+                                               : abt_launch_batch(&r);
     if (e) return abt_fail(ABT_ERR_HIP, "batched launch failed: %s", hipGetErrorString((hipError_t)e));
     return 0;
 }
@@ -527,12 +508,7 @@ int abt_batch_launch(const abt_batch_plan* p, void* stream)
 int abt_batch_workspace(const abt_batch_plan* p, size_t* bytes)
 {
     if (!p || !bytes) return abt_fail(ABT_ERR_ARG, "abt_batch_workspace: null argument");
-    const int64_t nbins = p->g->nbins, ntiles1 = (nbins + LANES - 1) / LANES;
-    *bytes = sizeof(double) * (16 * (size_t)nbins * p->max_chunks + 6 * (size_t)ntiles1 * p->norient +
-                               2 * (size_t)nbins);
-    if (p->prec == ABT_MIXED_GATED)
-        *bytes += sizeof(double) * ((size_t)nbins * p->max_chunks + nbins) + sizeof(int32_t) * 2 * (size_t)nbins;
-    if (p->smem) *bytes += sizeof(double) * ((size_t)16 * nbins * p->norient + 8 * (size_t)p->norient);
+    *bytes = p->mem_bytes + p->smem_bytes;
     return 0;
 }
 
@@ -544,7 +520,7 @@ int abt_batch_gate_stats(const abt_batch_plan* p, int32_t* refined_bins, void* s
         return 0;
     }
     hipStream_t st = (hipStream_t)stream;
-    HIPCHK(hipMemcpyAsync(refined_bins, p->d_count, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(refined_bins, p->gate.count, sizeof(int32_t), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     return 0;
 }

@@ -1,88 +1,103 @@
-// far_field.hip -- coherent far-field sum of prepared beams onto the (theta, phi) bins.
+// far_field.hip -- coherent far-field sums of prepared beams onto the (theta, phi) bins.
 //
-// Work decomposition (both kernels): one lane per far-field bin, bins contiguous
-// with phi fastest (the Fortran (nphi, ntheta) layout), 256 lanes per workgroup.
-// Beam records are staged in LDS one tile at a time (cooperative coalesced
-// loads, then broadcast reads) and every lane walks the tile in beam order, so
-// each bin's sum is formed in a fixed order and is run-to-run deterministic.
-// blockIdx.y splits the beam list into chunks so that a launch has many short
-// workgroups (a small last round); chunk partials are then summed in chunk order
-// by k_reduce_chunks.
+// Work decomposition.  One lane per BPT far-field bins, bins contiguous with phi fastest (the
+// Fortran (nphi, ntheta) layout), 256 lanes per workgroup.  A workgroup sums one segment of
+// the beam list on one tile of 256 x BPT bins (grid: tiles x segments): beam records are staged
+// in LDS one tile at a time (cooperative coalesced loads, then broadcast reads) and every lane
+// walks them in beam order.  Segment sums are stored as the body forms them; k_finish_sum
+// (one orientation) or the batched plan's epilogue (batch.hip) adds them in segment order and
+// finishes the sum, so each bin's sum is formed in a fixed order and repeats bit for bit.
+// Cutting the beam list is what fills the chip when there are few bins or few orientations,
+// and it bounds the last round of workgroups when there are many.  A single segment is finished
+// in place.
 //
-// k_ff_fp64  -- the reference's formulas in FP64 (diffraction, diff_mod.f90:576-670;
-//               karczewski :124-198; contour_integral :357-421), every phase formed with
-//               the reference's operations (bit-identical arguments of every sine and
-//               cosine), the amplitude algebra around them reorganised (beam_bin_fp64).
-// k_ff_fp64r -- (PREC 4) the mixed kernel's algorithm below with every step in FP64.
-// k_ff_mixed -- the same quantity restructured for the vector ALUs:
-//               * geometry, phases and their reduction to octants in FP64
-//                 (the bin direction, q = k (prop - khat), vertex phases,
-//                 the k|r - com| ~ 1.2e7 rad far-field phase);
-//               * polarisation (Karczewski-Wolf, scattering-plane rotation)
-//                 and the aperture integral body in FP32: the edge sum is the
-//                 rotation-invariant polygon form factor
-//                   sum_ref = -(1/2pi) sum_j (qx dy_j - qy dx_j)/|q|^2 sinc(K_j/2) e^{i mu_j}
-//                 (q in revolutions/um), which equals the reference's split
-//                 kxx/kyy sum but is singular only at q -> 0;
-//               * near q -> 0 (|q| a < SERIES_QA) an FP64 power series of the
-//                 form factor (complete homogeneous symmetric polynomials of
-//                 the vertex phases);
-//               * the scattering-plane rotation temp_rot1 depends on phi only,
-//                 so it is applied once per bin after the beam sum; the
-//                 polarisation matrix rot4 . diff_ampl has the form g I + h J
-//                 and is folded into two complex weights per beam;
-//               * accumulation in FP64.
+// Bodies (ffbody.h, adjbody.h), by kernel precision:
+//   0  the reference's formulas in FP64 (diffraction, diff_mod.f90:576-670; karczewski :124-198;
+//      contour_integral :357-421), every phase formed with the reference's operations;
+//   1  mixed: geometry, phases and their reduction in FP64, polarisation and the rotation-invariant
+//      polygon form factor in FP32;
+//   2  body 0 summing |amplitude|^2 instead (conditioning diagnostic);
+//   3  the frame-free FP64 model (adjbody.h);
+//   4  the mixed kernel's algorithm with every step in FP64.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
+#include <string.h>
 
-#include "ffbody.h"
+#include "sweep.h"
 
 namespace abt {
 
 constexpr int BLOCK = 256;
 
-// ---------------------------------------------------------------------------
-// The mixed kernel with up to 16-beam tiles is held to 128 VGPRs (4 waves per SIMD), its
-// fastest occupancy on gfx950.
-template <int PREC, int TB>
-__global__ __launch_bounds__(BLOCK, (PREC == 1 && TB <= 16) ? 4 : (PREC == 4 ? 2 : 1))
-void k_far_field(DevGrid g, const double* __restrict__ recs, const double* __restrict__ vrecs,
-                 int64_t nb, int64_t per_chunk, int fast_diff, double* __restrict__ out,
-                 double* __restrict__ work)
+// Bin inputs of one lane slot.
+template <int PREC>
+__device__ __forceinline__ BinIn load_bin(const DevGrid& g, int bc)
 {
-    // Mixed kernel: two record tiles; the next tile's records are loaded into registers
-    // while the current one is summed, then stored to the other buffer (one barrier per
-    // tile).  The FP64 bodies need their registers: one tile, loaded between barriers.
-    constexpr bool DB = PREC == 1;
+    BinIn bi;
+    bi.x = g.x[bc]; bi.y = g.y[bc]; bi.z = g.z[bc];
+    const int bt = bc % g.nphi + g.nphi * g.theta_i;
+    bi.xt = g.x[bt]; bi.yt = g.y[bt]; bi.zt = g.z[bt];
+    bi.rad = PREC >= 3 ? g.rad[bc] : 0.0;
+    return bi;
+}
+
+// Occupancy: 4 waves per SIMD (128 VGPRs) for the mixed body with up to 16-beam tiles and for
+// the restructured FP64 body with 8-beam tiles, else what the registers and LDS give (>= 2).
+template <int PREC, int TB, int BPT, int MODE>
+__global__ __launch_bounds__(BLOCK, (BPT == 1 && ((PREC == 1 && TB <= 16) || (PREC == 4 && TB <= 8))) ? 4 : 2)
+void k_sweep(SweepArgs a)
+{
+    constexpr bool INC = MODE == SWEEP_INC, LIST = MODE == SWEEP_LIST;
+    // Mixed body: two record tiles; the next tile's records are loaded into registers while the
+    // current one is summed, then stored to the other buffer (one barrier per tile).  The FP64
+    // bodies need their registers: one tile, loaded between barriers.
+    constexpr bool DB = PREC == 1 && TB <= 16 && BPT == 1;
     __shared__ double tile[(DB ? 2 : 1) * TB * REC];
     // the exponential table and the FP64r body's constants, or the table with its low parts
-    __shared__ double etab[PREC == 4 ? ETAB_LDS : (PREC != 1 ? ETAB_GRID : 1)];
+    constexpr bool TAB = PREC == 0 || PREC == 2 || PREC == 4;
+    __shared__ double etab[PREC == 4 ? ETAB_LDS : (TAB ? ETAB_GRID : 1)];
     constexpr int PF = DB ? (TB * REC + BLOCK - 1) / BLOCK : 1;   // doubles per lane per tile
+    const DevGrid& g = a.g;
     const int tid = threadIdx.x;
-    if (PREC != 1) {   // published by the barriers of the tile loop before any use
+    const int nslots = LIST ? *a.list_count : g.nbins;
+    const int slot0 = blockIdx.x * (BLOCK * BPT) + tid;   // slot of lane j: slot0 + j * BLOCK
+    if ((int)blockIdx.x * (BLOCK * BPT) >= nslots) return;   // LIST: tiles past the listed bins
+    if (TAB) {   // published by the barriers of the tile loop before any use
         for (int q = tid; q < (PREC == 4 ? ETAB_DOUBLES : ETAB_GRID); q += BLOCK) etab[q] = g.etab[q];
         if (PREC == 4 && tid == 0) fp64r_constants(g, etab + ETAB_DOUBLES);
     }
-    const int bin = blockIdx.x * BLOCK + tid;
-    const bool active = bin < g.nbins;
-    const int bc = active ? bin : g.nbins - 1;
-    const int iphi = bc % g.nphi;
-    BinIn bi;
-    bi.x = g.x[bc]; bi.y = g.y[bc]; bi.z = g.z[bc];
-    const int bt = iphi + g.nphi * g.theta_i;
-    bi.xt = g.x[bt]; bi.yt = g.y[bt]; bi.zt = g.z[bt];
-    bi.rad = PREC == 4 ? g.rad[bc] : 0.0;
-    const double cp = g.cphi[iphi], sp = g.sphi[iphi];
-    double acc[8];
+    BinIn bi[BPT];
 #pragma unroll
-    for (int q = 0; q < 8; q++) acc[q] = 0.0;
-    const int64_t b0 = (int64_t)blockIdx.y * per_chunk;
-    const int64_t b1 = min(nb, b0 + per_chunk);
+    for (int j = 0; j < BPT; j++) {
+        const int sc = min(slot0 + j * BLOCK, nslots - 1);
+        bi[j] = load_bin<PREC>(g, LIST ? a.list[sc] : sc);
+    }
+    double acc[BPT][8], inc[BPT];
+#pragma unroll
+    for (int j = 0; j < BPT; j++) {
+        inc[j] = 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) acc[j][q] = 0.0;
+    }
+    const int seg = blockIdx.y;
+    int64_t b0, b1;
+    int tree = 0;
+    if (a.segs) {
+        const SweepSeg s = a.segs[seg];
+        b0 = s.start;
+        b1 = s.start + s.count;
+        tree = s.tree;
+    } else {
+        b0 = (int64_t)seg * a.per;
+        b1 = min(a.nb, b0 + a.per);
+    }
+    const double* __restrict__ recs = a.recs[tree];
+    const double* __restrict__ vrecs = a.vrecs[tree];
     if (DB) {
         // the bin's inputs must have arrived before the tile loop: a use inside it would make
         // the compiler wait there for the older loads, and with them for the prefetched tile
-        asm volatile("" : "+v"(bi.x), "+v"(bi.y), "+v"(bi.z), "+v"(bi.xt), "+v"(bi.yt), "+v"(bi.zt));
+        asm volatile("" : "+v"(bi[0].x), "+v"(bi[0].y), "+v"(bi[0].z), "+v"(bi[0].xt), "+v"(bi[0].yt), "+v"(bi[0].zt));
     }
     if (DB && b0 < b1) {
         const int nt0 = (int)min((int64_t)TB, b1 - b0);
@@ -109,23 +124,44 @@ void k_far_field(DevGrid g, const double* __restrict__ recs, const double* __res
             __syncthreads();
         }
         const double* cur = tile + buf * (TB * REC);
-        if (active) {
-            if (PREC == 1) {
-                // FP32 partial sums over groups of MIXED_GROUP beams, added into FP64
-                for (int g0 = 0; g0 < nt; g0 += MIXED_GROUP) {
-                    float accf[8];
+        if (PREC == 1) {
+            // FP32 partial sums over groups of MIXED_GROUP beams (segments start at multiples of
+            // it from the tree's first beam), added into FP64
+            for (int g0 = 0; g0 < nt; g0 += MIXED_GROUP) {
+                float accf[BPT][8], incf[BPT];
 #pragma unroll
-                    for (int q = 0; q < 8; q++) accf[q] = 0.f;
-                    const int g1 = min(nt, g0 + MIXED_GROUP);
-                    for (int bb = g0; bb < g1; bb++) beam_bin_mixed(cur + bb * REC, vrecs, g, bi, fast_diff, accf);
+                for (int j = 0; j < BPT; j++) {
+                    incf[j] = 0.f;
 #pragma unroll
-                    for (int q = 0; q < 8; q++) acc[q] += (double)accf[q];
+                    for (int q = 0; q < 8; q++) accf[j][q] = 0.f;
                 }
-            } else if (PREC == 4) {
-                for (int bb = 0; bb < nt; bb++) beam_bin_fp64r(cur + bb * REC, vrecs, g, bi, etab, fast_diff, acc);
-            } else {
-                for (int bb = 0; bb < nt; bb++)
-                    beam_bin_fp64(cur + bb * REC, vrecs, g, bi, etab, fast_diff, acc, PREC == 2);
+                const int g1 = min(nt, g0 + MIXED_GROUP);
+                for (int bb = g0; bb < g1; bb++) {
+#pragma unroll
+                    for (int j = 0; j < BPT; j++)
+                        beam_bin_mixed_t<INC>(cur + bb * REC, vrecs, g, bi[j], a.fast_diff, accf[j], incf[j]);
+                }
+#pragma unroll
+                for (int j = 0; j < BPT; j++) {
+                    if (INC) inc[j] += (double)incf[j];
+#pragma unroll
+                    for (int q = 0; q < 8; q++) acc[j][q] += (double)accf[j][q];
+                }
+            }
+        } else {
+            for (int bb = 0; bb < nt; bb++) {
+#pragma unroll
+                for (int j = 0; j < BPT; j++) {
+                    if (PREC == 4)
+                        beam_bin_fp64r(cur + bb * REC, vrecs, g, bi[j], etab, a.fast_diff, acc[j]);
+                    else if (PREC == 3) {
+                        AdjBeam B;
+                        adj_beam_from_record(cur + bb * REC, B);
+                        model_bin_fp64(B, bi[j].x, bi[j].y, bi[j].z, bi[j].xt, bi[j].yt, bi[j].rad, g.waveno,
+                                       g.lambda, acc[j]);
+                    } else
+                        beam_bin_fp64(cur + bb * REC, vrecs, g, bi[j], etab, a.fast_diff, acc[j], PREC == 2);
+                }
             }
         }
         if (DB) {
@@ -139,52 +175,63 @@ void k_far_field(DevGrid g, const double* __restrict__ recs, const double* __res
             buf ^= 1;
         }
     }
-    if (!active) return;
-    if (PREC == 0) apply_temp_rot1(acc, cp, sp);
-    if (PREC == 1) mixed_finish(acc, cp, sp);
-    if (PREC == 4) fp64r_finish(acc, cp, sp, g.kr_rev[bin]);
     const int nbins = g.nbins;
-    if (PREC == 2) {   // incoherent intensity: one double per bin, never chunked
-        out[bin] = acc[0];
-        return;
-    }
-    if (work == nullptr) {
-        double2* o2 = reinterpret_cast<double2*>(out);
 #pragma unroll
-        for (int q = 0; q < 4; q++) o2[bin + (int64_t)nbins * q] = make_double2(acc[2 * q], acc[2 * q + 1]);
-    } else {
-        double* wc = work + (int64_t)blockIdx.y * 8 * nbins;
+    for (int j = 0; j < BPT; j++) {
+        const int slot = slot0 + j * BLOCK;
+        if (slot >= nslots) continue;
+        if (a.part) {
+            double* p = a.part + (int64_t)seg * 8 * nbins + slot;
 #pragma unroll
-        for (int q = 0; q < 8; q++) wc[(int64_t)q * nbins + bin] = acc[q];
+            for (int q = 0; q < 8; q++) p[(int64_t)q * nbins] = acc[j][q];
+            if (INC) a.ipart[(int64_t)seg * nbins + slot] = inc[j];
+        } else if (PREC == 2) {   // incoherent intensity: one double per bin
+            a.out[slot] = acc[j][0];
+        } else {
+            finish_sum<PREC>(acc[j], g, slot);
+            double2* o2 = reinterpret_cast<double2*>(a.out);
+#pragma unroll
+            for (int q = 0; q < 4; q++) o2[slot + (int64_t)nbins * q] = make_double2(acc[j][2 * q], acc[j][2 * q + 1]);
+        }
     }
 }
 
-// Sum chunk partials in chunk order: work[(c*8 + comp)*nbins + bin] -> out.
-__global__ __launch_bounds__(BLOCK) void k_reduce_chunks(const double* __restrict__ work,
-                                                         int nchunks, int nbins,
-                                                         double* __restrict__ out)
+// One orientation: the segment sums of a bin in segment order, finished, in the Fortran layout.
+// Reads 64 bytes per bin and segment: bandwidth-bound.
+template <int PREC>
+__global__ __launch_bounds__(BLOCK) void k_finish_sum(DevGrid g, const double* __restrict__ part, int nseg,
+                                                      double* __restrict__ out)
 {
-    const int64_t idx = (int64_t)blockIdx.x * BLOCK + threadIdx.x;   // over 8*nbins
-    if (idx >= (int64_t)8 * nbins) return;
-    const int comp = (int)(idx / nbins);
-    const int bin = (int)(idx - (int64_t)comp * nbins);
-    double s = 0.0;
-    for (int c = 0; c < nchunks; c++) s = s + work[((int64_t)c * 8 + comp) * nbins + bin];
-    const int q = comp >> 1, ri = comp & 1;
-    out[2 * (bin + (int64_t)nbins * q) + ri] = s;
+    const int bin = blockIdx.x * BLOCK + threadIdx.x;
+    if (bin >= g.nbins) return;
+    const int64_t nbins = g.nbins;
+    double acc[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) acc[q] = 0.0;
+    for (int s = 0; s < nseg; s++) {
+        const double* p = part + (int64_t)s * 8 * nbins + bin;
+#pragma unroll
+        for (int q = 0; q < 8; q++) acc[q] += p[q * nbins];
+    }
+    finish_sum<PREC>(acc, g, bin);
+    double2* o2 = reinterpret_cast<double2*>(out);
+#pragma unroll
+    for (int q = 0; q < 4; q++) o2[bin + nbins * q] = make_double2(acc[2 * q], acc[2 * q + 1]);
 }
 
-}  // namespace abt
-
-// ---------------------------------------------------------------------------
-// launch helpers (called by the runtime)
-namespace abt {
 __global__ __launch_bounds__(BLOCK) void k_fill_zero(double* __restrict__ out, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
     if (i < n) out[i] = 0.0;
 }
+
+template <int PREC, int TB, int BPT, int MODE>
+const void* sweep_kernel() { return reinterpret_cast<const void*>(&k_sweep<PREC, TB, BPT, MODE>); }
+
 }  // namespace abt
+
+// ---------------------------------------------------------------------------
+// launch helpers (called by the runtime and the batched plan)
 
 // Zero-fill of n doubles (a kernel, not hipMemsetAsync, so callers may capture it in a graph).
 extern "C" int abt_launch_zero(double* out, int64_t n, hipStream_t st)
@@ -195,35 +242,63 @@ extern "C" int abt_launch_zero(double* out, int64_t n, hipStream_t st)
     return (int)hipGetLastError();
 }
 
+extern "C" const void* abt_sweep_kernel(int prec, int tb, int bpt, int mode)
+{
+    using namespace abt;
+#define K(P, T, B, M) if (prec == P && tb == T && bpt == B && mode == M) return sweep_kernel<P, T, B, M>();
+    K(0, 8, 1, 0) K(0, 16, 1, 0) K(0, 32, 1, 0) K(0, 8, 2, 0) K(0, 16, 2, 0) K(0, 32, 2, 0)
+    K(1, 8, 1, 0) K(1, 16, 1, 0) K(1, 32, 1, 0) K(1, 8, 2, 0) K(1, 16, 2, 0) K(1, 32, 2, 0)
+    K(1, 8, 1, 1) K(1, 16, 1, 1) K(1, 32, 1, 1) K(1, 8, 2, 1) K(1, 16, 2, 1) K(1, 32, 2, 1)
+    K(2, 16, 1, 0)
+    K(3, 16, 1, 0)
+    K(4, 8, 1, 0) K(4, 16, 1, 0) K(4, 32, 1, 0) K(4, 8, 2, 0) K(4, 16, 2, 0)
+    K(4, 16, 1, 2)
+#undef K
+    return nullptr;
+}
+
+extern "C" int abt_launch_sweep(const abt::SweepArgs* a, int nseg, int prec, int tb, int bpt, int mode,
+                                hipStream_t st)
+{
+    const void* kern = abt_sweep_kernel(prec, tb, bpt, mode);
+    if (!kern || nseg < 1 || nseg > 65535) return (int)hipErrorInvalidValue;
+    abt::SweepArgs args = *a;
+    void* params[] = {&args};
+    const int64_t lanes = (int64_t)abt::BLOCK * bpt;
+    const dim3 grid((unsigned)((a->g.nbins + lanes - 1) / lanes), (unsigned)nseg);
+    return (int)hipLaunchKernel(kern, grid, dim3(abt::BLOCK), params, 0, st);
+}
+
+// One orientation's far field of nb prepared beams in nseg segments of `per` beams (a multiple
+// of 32, so that the mixed body's FP32 beam groups do not depend on the cut); prec: the ABI's
+// (0 plain FP64, 1 mixed, 3 restructured FP64) or 2, the incoherent sum (one segment).
+// work: nseg * 64 bytes per bin when nseg > 1.
 extern "C" int abt_launch_far_field(const abt::DevGrid* g, const double* recs, const double* vrecs,
-                                    int64_t nb, int prec, int tb, int fast_diff, int nchunks,
-                                    double* out, double* work, hipStream_t st)
+                                    int64_t nb, int prec, int fast_diff, int64_t per, double* out, double* work,
+                                    hipStream_t st)
 {
     using namespace abt;
     if (g->nbins <= 0) return 0;
-    // chunk lengths are multiples of the largest tile (32 beams), so the mixed kernel's
-    // FP32 beam groups do not depend on the chunking
-    int64_t per_chunk = (nb + nchunks - 1) / nchunks;
-    per_chunk = per_chunk < 32 ? 32 : (per_chunk + 31) / 32 * 32;
-    nchunks = (int)((nb + per_chunk - 1) / per_chunk);
-    if (nchunks < 1) nchunks = 1;
-    dim3 grid((g->nbins + BLOCK - 1) / BLOCK, nchunks);
-    double* w = nchunks > 1 ? work : nullptr;
-#define L(P, T) hipLaunchKernelGGL((k_far_field<P, T>), grid, dim3(BLOCK), 0, st, *g, recs, vrecs, nb, per_chunk, fast_diff, out, w)
-    if (prec == 0) {
-        if (tb == 8) L(0, 8); else if (tb == 32) L(0, 32); else L(0, 16);
-    } else if (prec == 1) {
-        if (tb == 8) L(1, 8); else if (tb == 32) L(1, 32); else L(1, 16);
-    } else if (prec == 3) {   // ABT_FP64_FAST: the restructured FP64 body
-        L(4, 16);
-    } else {
-        L(2, 16);
-    }
-#undef L
-    if (nchunks > 1) {
-        const int64_t n = (int64_t)8 * g->nbins;
-        hipLaunchKernelGGL(k_reduce_chunks, dim3((unsigned)((n + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0,
-                           st, work, nchunks, g->nbins, out);
+    const int kprec = prec == 3 ? 4 : prec;
+    const int nseg = (int)((nb + per - 1) / per);
+    SweepArgs a;
+    memset(&a, 0, sizeof(a));
+    a.g = *g;
+    a.recs[0] = a.recs[1] = recs;
+    a.vrecs[0] = a.vrecs[1] = vrecs;
+    a.nb = nb;
+    a.per = per;
+    a.part = nseg > 1 ? work : nullptr;
+    a.out = out;
+    a.fast_diff = fast_diff;
+    int e = abt_launch_sweep(&a, nseg, kprec, kprec == 4 ? 8 : 16, 1, SWEEP_PLAIN, st);
+    if (e) return e;
+    if (nseg > 1) {
+        const dim3 grid((g->nbins + BLOCK - 1) / BLOCK);
+        const double* w = work;
+        if (kprec == 0) hipLaunchKernelGGL(k_finish_sum<0>, grid, dim3(BLOCK), 0, st, *g, w, nseg, out);
+        else if (kprec == 1) hipLaunchKernelGGL(k_finish_sum<1>, grid, dim3(BLOCK), 0, st, *g, w, nseg, out);
+        else hipLaunchKernelGGL(k_finish_sum<4>, grid, dim3(BLOCK), 0, st, *g, w, nseg, out);
     }
     return (int)hipGetLastError();
 }

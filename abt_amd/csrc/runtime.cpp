@@ -26,8 +26,8 @@
 #include "rt_internal.h"
 
 extern "C" int abt_launch_far_field(const abt::DevGrid* g, const double* recs, const double* vrecs,
-                                    int64_t nb, int prec, int tb, int fast_diff, int nchunks,
-                                    double* out, double* work, hipStream_t st);
+                                    int64_t nb, int prec, int fast_diff, int64_t per, double* out,
+                                    double* work, hipStream_t st);
 extern "C" int abt_launch_zero(double* out, int64_t n, hipStream_t st);
 extern "C" int abt_launch_finalise(const abt::DevGrid* g, double* ab, double* ae, double* tot,
                                    double* M, double* m1d, double* tmp, double* params,
@@ -73,7 +73,8 @@ struct DevBuf {
 // per-thread staging: the host entry points may run concurrently on several threads
 struct ThreadState {
     hipStream_t st = nullptr;
-    DevBuf bufs[9];   // [8]: the visibility entry points
+    DevBuf bufs[9];   // [7]: abt_far_field_dev without a workspace; [8]: the visibility entry points
+    hipEvent_t ff_done = nullptr;   // the last use of bufs[7], which calls on any stream share
     std::vector<double> hrec;
 };
 
@@ -160,22 +161,43 @@ int theta_i_of(int64_t nth, const double* th)
     return (int)(nth - 1);
 }
 
-int choose_chunks(int64_t nbins, int64_t nb, int cus)
+// How one orientation's beam list is cut: segments of `per` beams (a multiple of 32), nseg of them.
+struct Cut {
+    int64_t per = 0;
+    int nseg = 1;
+    size_t work(int64_t nbins) const { return nseg > 1 ? sizeof(double) * 8 * (size_t)nbins * nseg : 0; }
+};
+
+Cut cut_into(int64_t nb, int64_t c)
 {
-    // ~320 workgroups per CU (80 rounds at 4 resident per CU): the last round's partly filled
-    // CUs, and the slower forward-fallback rows, are then a small share of the launch.  Measured
-    // on the 200,000-aperture stress test (2533 bin tiles, mixed kernel): 4 chunks run 9 % faster
-    // than 1, 16 a further 3 %, 32 and 64 a further 0.7 % and 1 %.  Chunks keep >= 512 beams;
-    // at most 32 (the workspace is 64 B per bin per chunk).
-    const int64_t tiles = (nbins + 255) / 256;
-    const int64_t want = (int64_t)cus * 320;
-    int64_t c = (want + tiles - 1) / tiles;
-    c = std::min<int64_t>(c, std::max<int64_t>(1, nb / 512));
-    c = std::max<int64_t>(1, std::min<int64_t>(c, 32));
-    return (int)c;
+    c = std::max<int64_t>(1, std::min<int64_t>(c, 32));   // the workspace is 64 B per bin per segment
+    Cut k;
+    k.per = std::max<int64_t>(32, ((nb + c - 1) / c + 31) / 32 * 32);
+    k.nseg = (int)std::max<int64_t>(1, (nb + k.per - 1) / k.per);
+    return k;
 }
 
-int tile_beams(int prec) { return prec == ABT_FP64 ? 16 : 16; }
+// ~320 workgroups per CU (80 rounds at 4 resident per CU): the last round's partly filled
+// CUs, and the slower forward-fallback rows, are then a small share of the launch.  Measured
+// on the 200,000-aperture stress test (2533 bin tiles, mixed kernel): 4 segments run 9 % faster
+// than 1, 16 a further 3 %, 32 and 64 a further 0.7 % and 1 %.  Segments keep >= 512 beams.
+Cut cut_long(int64_t nbins, int64_t nb, int cus)
+{
+    const int64_t tiles = (nbins + 255) / 256;
+    const int64_t want = ((int64_t)cus * 320 + tiles - 1) / tiles;
+    return cut_into(nb, std::min<int64_t>(want, nb / 512));
+}
+
+// The cut where a workspace for it is at hand.  When the segments of cut_long leave the chip with
+// fewer than 8 workgroups per CU, shorter ones (down to 32 beams) fill it: the default column's
+// 2838 + 864 beams on 64,980 bins (254 tiles), plain FP64, 8.1 -> 7.6 ms a diff_main call.
+Cut cut_beams(int64_t nbins, int64_t nb, int cus)
+{
+    const int64_t tiles = (nbins + 255) / 256;
+    const Cut l = cut_long(nbins, nb, cus);
+    const int64_t fill = ((int64_t)cus * 8 + tiles - 1) / tiles;
+    return fill > l.nseg ? cut_into(nb, std::min<int64_t>(fill, nb / 32)) : l;
+}
 
 }  // namespace
 
@@ -464,15 +486,14 @@ static int run_host_tree(const DevGrid& g, const abt_beams* b, double fov_value,
     double* drec = (double*)ts.bufs[slot].p;
     double* dvrec = poly ? drec + abt::REC * n : drec;
     HIPCHK(hipMemcpyAsync(drec, hrec, rec_bytes + vrec_bytes, hipMemcpyHostToDevice, st));
-    const int nch = choose_chunks(g.nbins, n, g_ctx.cus);
+    const Cut cut = cut_beams(g.nbins, n, g_ctx.cus);
     double* work = nullptr;
-    if (nch > 1) {
-        rc = buf_ensure(ts.bufs[slot + 1], sizeof(double) * 8 * (size_t)g.nbins * nch);
+    if (cut.nseg > 1) {
+        rc = buf_ensure(ts.bufs[slot + 1], cut.work(g.nbins));
         if (rc) return rc;
         work = (double*)ts.bufs[slot + 1].p;
     }
-    int e = abt_launch_far_field(&g, drec, dvrec, n, prec, tile_beams(prec), fast_diff, nch, dev_out,
-                                 work, st);
+    int e = abt_launch_far_field(&g, drec, dvrec, n, prec, fast_diff, cut.per, dev_out, work, st);
     if (e) return fail(ABT_ERR_HIP, "far-field launch failed: %s", hipGetErrorString((hipError_t)e));
     return 0;
 }
@@ -513,6 +534,8 @@ int abt_finalize(void)
         }
         if (ts->st) (void)hipStreamDestroy(ts->st);
         ts->st = nullptr;
+        if (ts->ff_done) (void)hipEventDestroy(ts->ff_done);
+        ts->ff_done = nullptr;
     }
     return 0;
 }
@@ -579,8 +602,7 @@ size_t abt_far_field_workspace(const abt_dev_grid* g, int64_t nb, int precision)
     (void)precision;
     if (!g) return 0;
     if (ensure_device()) return 0;
-    const int nch = choose_chunks(g->nbins, nb, g_ctx.cus);
-    return nch > 1 ? sizeof(double) * 8 * (size_t)g->nbins * nch : 0;
+    return cut_beams(g->nbins, nb, g_ctx.cus).work(g->nbins);
 }
 
 int abt_far_field_dev(const abt_dev_grid* g, const double* dev_recs, const double* dev_vrecs,
@@ -600,18 +622,34 @@ int abt_far_field_dev(const abt_dev_grid* g, const double* dev_recs, const doubl
         return 0;
     }
     if (!dev_recs) return fail(ABT_ERR_ARG, "abt_far_field_dev: null records");
-    const int nch = choose_chunks(g->nbins, nb, g_ctx.cus);
-    const size_t need = nch > 1 ? sizeof(double) * 8 * (size_t)g->nbins * nch : 0;
+    // The long segments where the finer cut has no memory: a caller's own smaller workspace, or none
+    // inside a graph capture (nothing is allocated there for lists under 1024 beams).
+    Cut cut = cut_beams(g->nbins, nb, g_ctx.cus);
     void* work = dev_work;
+    bool capturing = false;
+    if (!work) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        HIPCHK(hipStreamIsCapturing(st, &cs));
+        capturing = cs != hipStreamCaptureStatusNone;
+    }
+    if (work ? work_bytes < cut.work(g->nbins) : capturing) cut = cut_long(g->nbins, nb, g_ctx.cus);
+    const size_t need = cut.work(g->nbins);
+    ThreadState* shared = nullptr;
     if (need && (!work || work_bytes < need)) {
         if (work) return fail(ABT_ERR_ARG, "workspace of %zu bytes is smaller than the %zu needed", work_bytes, need);
         ThreadState& ts = tstate();
         rc = buf_ensure(ts.bufs[7], need);
         if (rc) return rc;
         work = ts.bufs[7].p;
+        if (!capturing) {   // a call of this thread on another stream may still be reading the buffer
+            if (!ts.ff_done) HIPCHK(hipEventCreateWithFlags(&ts.ff_done, hipEventDisableTiming));
+            else HIPCHK(hipStreamWaitEvent(st, ts.ff_done, 0));
+            shared = &ts;
+        }
     }
     int e = abt_launch_far_field(&g->d, dev_recs, dev_vrecs ? dev_vrecs : dev_recs, nb, precision,
-                                 tile_beams(precision), is_fast_diff, nch, dev_out, (double*)work, st);
+                                 is_fast_diff, cut.per, dev_out, (double*)work, st);
+    if (shared) HIPCHK(hipEventRecord(shared->ff_done, st));
     if (e) return fail(ABT_ERR_HIP, "far-field launch failed: %s", hipGetErrorString((hipError_t)e));
     return 0;
 }
@@ -630,8 +668,8 @@ int abt_far_field_incoherent_dev(const abt_dev_grid* g, const double* dev_recs,
         return 0;
     }
     if (!dev_recs) return fail(ABT_ERR_ARG, "abt_far_field_incoherent_dev: null records");
-    int e = abt_launch_far_field(&g->d, dev_recs, dev_vrecs ? dev_vrecs : dev_recs, nb, 2, 16,
-                                 is_fast_diff, 1, dev_intensity, nullptr, (hipStream_t)stream);
+    int e = abt_launch_far_field(&g->d, dev_recs, dev_vrecs ? dev_vrecs : dev_recs, nb, 2, is_fast_diff, nb,
+                                 dev_intensity, nullptr, (hipStream_t)stream);
     if (e) return fail(ABT_ERR_HIP, "far-field launch failed: %s", hipGetErrorString((hipError_t)e));
     return 0;
 }

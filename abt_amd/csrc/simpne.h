@@ -50,17 +50,23 @@ __host__ __device__ inline double simpne_eval(int n, const double* __restrict__ 
     return result - sum1 / (del[0] * del[1] * del[2]);
 }
 
-// w[i] = simpne_eval(n, x, e_i): the quadrature weights of the nodes x (n >= 3).
+// w[i] = simpne_eval(n, x, e_i): the quadrature weights of the nodes x (n >= 3), panel by panel.
 inline void simpne_weights(int n, const double* x, double* w)
 {
-    double* y = new double[n];
-    for (int i = 0; i < n; i++) y[i] = 0.0;
-    for (int i = 0; i < n; i++) {
-        y[i] = 1.0;
-        w[i] = simpne_eval(n, x, y, 1);
-        y[i] = 0.0;
-    }
-    delete[] y;
+#pragma clang fp contract(off)
+    for (int i = 0; i < n; i++) w[i] = 0.0;
+    const auto panel = [&](int m, double lo, double hi) {   // the parabola through x[m-1..m+1] over [lo, hi]
+#pragma clang fp contract(off)
+        const double x1 = x[m - 1], x2 = x[m], x3 = x[m + 1];
+        const double e = hi * hi - lo * lo, f = hi * hi * hi - lo * lo * lo, fe = hi - lo;
+        const double del[3] = {x3 - x2, x1 - x3, x2 - x1};
+        const double g[3] = {x2 + x3, x1 + x3, x1 + x2};
+        const double p[3] = {x2 * x3, x1 * x3, x1 * x2};
+        for (int i = 0; i < 3; i++)
+            w[m - 1 + i] -= del[i] * (f / 3.0 - g[i] * 0.5 * e + p[i] * fe) / (del[0] * del[1] * del[2]);
+    };
+    for (int m = 1; m < n - 1; m += 2) panel(m, x[m - 1], x[m + 1]);
+    if (n % 2 == 0) panel(n - 2, x[n - 2], x[n - 1]);
 }
 
 }  // namespace abt

@@ -153,12 +153,14 @@ int abt_grid_destroy(abt_dev_grid* g);
 int64_t abt_grid_bins(const abt_dev_grid* g);
 
 /* Workspace bytes abt_far_field_dev needs for nb beams (0 when none): 64 bytes per bin
- * per beam chunk, at most 32 chunks of >= 512 beams (2048 bytes per bin). */
+ * per beam segment, at most 32 segments of >= 32 beams (2048 bytes per bin).  With less than this
+ * the call still runs on segments of >= 512 beams where their sums fit. */
 size_t abt_far_field_workspace(const abt_dev_grid* g, int64_t nb, int precision);
 
 /* Coherent far-field sum of nb prepared beams: dev_out (complex, Fortran layout,
  * 8*nbins doubles) overwritten.  dev_work: abt_far_field_workspace bytes (NULL:
- * the library allocates). */
+ * a buffer of the calling thread, ordered between the streams of its calls; nothing is
+ * allocated while the stream is being captured and nb < 1024). */
 int abt_far_field_dev(const abt_dev_grid* g, const double* dev_recs, const double* dev_vrecs,
                       int64_t nb, int precision, int is_fast_diff, double* dev_out,
                       void* dev_work, size_t work_bytes, void* stream);
@@ -201,7 +203,7 @@ int abt_finalise_dev(const abt_dev_grid* g, double* dev_ampl_beam, double* dev_a
  * pbt_mpi_mod.f90 spreads it over MPI ranks): for every orientation diff_main of
  * the beam tree and of the ext tree, finalise (x k, total = beam + ext, Mueller
  * matrix, integrals; outputs_mod.f90:63-278) and summation (outputs_mod.f90:407-471),
- * as one persistent kernel over all orientations.
+ * as a short sequence of launches over groups of orientations.
  *
  * Records: the prepared records (abt_prepare_beams_*) of every orientation's
  * beam tree back to back, and likewise for the ext trees (prepared with
@@ -228,12 +230,14 @@ int abt_batch_plan_create(const abt_dev_grid* g, int32_t norient, const int64_t*
                           const int64_t* ext_off, int precision, int is_fast_diff,
                           abt_batch_plan** out);
 int abt_batch_plan_destroy(abt_batch_plan* plan);
-/* Device bytes the plan holds (partial sums: 128 bytes per bin per orientation chunk, up to
- * 128 chunks; weights, tables). */
+/* Device bytes the plan holds (sums of beam segments: 64 bytes per bin per segment, up to 2 GiB
+ * where one orientation's fit; Mueller partial sums; weights, tables). */
 int abt_batch_workspace(const abt_batch_plan* plan, size_t* bytes);
 /* Tile shape: beams staged per LDS tile (8, 16, 32) and bins per lane (1, 2).
- * Default 16 x 1 until set or autotuned (ABT_FP64_ACCURATE: 16 x 1 only; ABT_FP64_FAST:
- * 2 bins per lane with 8 or 16 beams per tile only). */
+ * Default 16 x 1 (ABT_FP64_FAST 8 x 1) until set or autotuned (ABT_FP64_ACCURATE: 16 x 1 only;
+ * ABT_FP64_FAST: 2 bins per lane with 8 or 16 beams per tile only).  Results do not depend on
+ * it.  get_tiles: chunks is the number of Mueller partial sums, workgroups what the chip holds
+ * at once. */
 int abt_batch_set_tiles(abt_batch_plan* plan, int32_t beams_per_tile, int32_t bins_per_thread);
 int abt_batch_get_tiles(const abt_batch_plan* plan, int32_t* beams_per_tile,
                         int32_t* bins_per_thread, int32_t* chunks, int32_t* workgroups);
