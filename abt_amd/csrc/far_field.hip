@@ -43,9 +43,10 @@ __device__ __forceinline__ BinIn load_bin(const DevGrid& g, int bc)
 }
 
 // Occupancy: 4 waves per SIMD (128 VGPRs) for the mixed body with up to 16-beam tiles and for
-// the restructured FP64 body with 8-beam tiles, else what the registers and LDS give (>= 2).
+// the FP64 bodies with 8-beam tiles, whose LDS (plain body: table with low parts 32 KB + tile 7 KB)
+// lets 4 workgroups share a CU; else what the registers and LDS give (>= 2).
 template <int PREC, int TB, int BPT, int MODE>
-__global__ __launch_bounds__(BLOCK, (BPT == 1 && ((PREC == 1 && TB <= 16) || (PREC == 4 && TB <= 8))) ? 4 : 2)
+__global__ __launch_bounds__(BLOCK, (BPT == 1 && ((PREC == 1 && TB <= 16) || (PREC != 1 && TB <= 8))) ? 4 : 2)
 void k_sweep(SweepArgs a)
 {
     constexpr bool INC = MODE == SWEEP_INC, LIST = MODE == SWEEP_LIST;
@@ -160,7 +161,7 @@ void k_sweep(SweepArgs a)
                         model_bin_fp64(B, bi[j].x, bi[j].y, bi[j].z, bi[j].xt, bi[j].yt, bi[j].rad, g.waveno,
                                        g.lambda, acc[j]);
                     } else
-                        beam_bin_fp64(cur + bb * REC, vrecs, g, bi[j], etab, a.fast_diff, acc[j], PREC == 2);
+                        beam_bin_fp64p<PREC == 2>(cur + bb * REC, vrecs, g, bi[j], etab, a.fast_diff, acc[j]);
                 }
             }
         }
@@ -208,6 +209,7 @@ __global__ __launch_bounds__(BLOCK) void k_finish_sum(DevGrid g, const double* _
     double acc[8];
 #pragma unroll
     for (int q = 0; q < 8; q++) acc[q] = 0.0;
+#pragma unroll 4
     for (int s = 0; s < nseg; s++) {
         const double* p = part + (int64_t)s * 8 * nbins + bin;
 #pragma unroll
@@ -291,7 +293,7 @@ extern "C" int abt_launch_far_field(const abt::DevGrid* g, const double* recs, c
     a.part = nseg > 1 ? work : nullptr;
     a.out = out;
     a.fast_diff = fast_diff;
-    int e = abt_launch_sweep(&a, nseg, kprec, kprec == 4 ? 8 : 16, 1, SWEEP_PLAIN, st);
+    int e = abt_launch_sweep(&a, nseg, kprec, kprec == 4 || kprec == 0 ? 8 : 16, 1, SWEEP_PLAIN, st);
     if (e) return e;
     if (nseg > 1) {
         const dim3 grid((g->nbins + BLOCK - 1) / BLOCK);

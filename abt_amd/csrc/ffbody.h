@@ -133,6 +133,17 @@ __host__ __device__ __forceinline__ void expi_pi(double t, float* c, float* s)
     *c = flipsign(cospi_poly(z), sg);
 }
 
+// An integer field of a beam record (the same in every lane of a wave) in a scalar register, so that
+// branches on it are scalar and a polygon's vertex records come through scalar loads.
+__host__ __device__ __forceinline__ int record_int(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_readfirstlane((int)x);
+#else
+    return (int)x;
+#endif
+}
+
 constexpr float SERIES_QA2 = 2.25f;  // (|q_perp| a)^2 below which the FP64 series is used
 constexpr int SERIES_N = 16;         // truncation < 3e-12 relative at |q| a = 1.5
 
@@ -448,6 +459,69 @@ __host__ __device__ __forceinline__ double rsq64_1(double x)
     return fma(0.5 * y, fma(-x * y, y, 1.0), y);
 }
 
+// Hardware approximations in FP64 (relative error below 2^-24 and 2^-24 on gfx950, measured on 10^9
+// values); one costs as much as the FP32 one with its two conversions.
+__host__ __device__ __forceinline__ double rcp_seed(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rcp(x);
+#else
+    return 1.0 / x;
+#endif
+}
+__host__ __device__ __forceinline__ double rsq_seed(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rsq(x);
+#else
+    return 1.0 / sqrt(x);
+#endif
+}
+
+// The functions below work on normal values whose squares and reciprocals are normal too, as the
+// kernels' are, without the scaling that a general division or square root carries.
+
+// 1 / x correctly rounded: two Newton steps from the approximation (2^-24 -> 2^-48 -> 2^-96 before
+// the last rounding).  Equal to the IEEE quotient on 10^9 random values; 5 instructions for ~11.
+__host__ __device__ __forceinline__ double rcp_cr(double x)
+{
+    double y = rcp_seed(x);
+    y = fma(y, fma(-x, y, 1.0), y);
+    return fma(y, fma(-x, y, 1.0), y);
+}
+
+// 1 / x from an approximation y good to a few ulp, correctly rounded
+__host__ __device__ __forceinline__ double rcp_from(double x, double y) { return fma(y, fma(-x, y, 1.0), y); }
+
+// sqrt(s) from y = 1 / sqrt(s) to a few ulp, correctly rounded: the residual of s y decides the last bit
+__host__ __device__ __forceinline__ double sqrt_from(double s, double y)
+{
+    const double g = s * y;
+    return fma(fma(-g, g, s), 0.5 * y, g);
+}
+
+// sqrt(s) and the reciprocal of that root, both correctly rounded (10^9 random values): one coupled
+// step for g = sqrt(s) and h = 1 / (2 g), then the residuals.
+__host__ __device__ __forceinline__ double sqrt_cr(double s, double* inv)
+{
+    const double q = rsq_seed(s);
+    double g = s * q, h = 0.5 * q;
+    const double t = fma(-h, g, 0.5);
+    g = fma(g, t, g);
+    h = fma(h, t, h);
+    g = fma(fma(-g, g, s), h, g);
+    *inv = rcp_from(g, h + h);
+    return g;
+}
+
+// 1 / sqrt(x) to ~1 ulp: one third-order step, e^3 ~ 2^-70
+__host__ __device__ __forceinline__ double rsq64_3(double x)
+{
+    const double y = rsq_seed(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
 // The table of e^{i pi j / ETAB_N} (DevGrid::etab, ETAB_GRID doubles), built by the host in x87
 // extended precision (64-bit significands): each angle reduced exactly to at most pi/4 (quarter
 // turns, and the reflection a -> pi/2 - a within a quarter), so the extended-precision angle is
@@ -538,21 +612,46 @@ constexpr double SINCOS_SHIFT = 6755399441055744.0;                   // 1.5 * 2
 constexpr double N_OVER_PI = (double)ETAB_N / 3.141592653589793;
 constexpr double PI_OVER_N_HI = 3.141592653589793 / (double)ETAB_N;   // exact: a power-of-two scaling
 constexpr double PI_OVER_N_LO = 1.2246467991473532e-16 / (double)ETAB_N;
-__host__ __device__ __forceinline__ void sincos_tab64(double x, const double* __restrict__ tab, double* s,
-                                                      double* c)
+struct SinCos {
+    double c0, s0;   // the table's high parts
+    double cl, sl;   // corrections: cos = c0 + cl, sin = s0 + sl
+    __host__ __device__ __forceinline__ double c() const { return c0 + cl; }
+    __host__ __device__ __forceinline__ double s() const { return s0 + sl; }
+};
+__host__ __device__ __forceinline__ SinCos sincos_parts64(double x, const double* __restrict__ tab)
 {
     const double t = fma(x, N_OVER_PI, SINCOS_SHIFT);
     const double n = t - SINCOS_SHIFT;
     double r = fma(-n, PI_OVER_N_HI, x);
     r = fma(-n, PI_OVER_N_LO, r);
     const int j = (int)(uint32_t)__builtin_bit_cast(uint64_t, t) & (2 * ETAB_N - 1);
-    const double c0 = tab[2 * j], s0 = tab[2 * j + 1];
+    SinCos o;
+    o.c0 = tab[2 * j];
+    o.s0 = tab[2 * j + 1];
     const double cl = tab[ETAB_LO + 2 * j], sl = tab[ETAB_LO + 2 * j + 1];
     const double z = r * r;
     const double sr = fma(r * z, fma(z, 1.0 / 120.0, -1.0 / 6.0), r);
     const double cm1 = z * fma(z, 1.0 / 24.0, -0.5);                   // cos r - 1
-    *s = s0 + fma(c0, sr, fma(s0, cm1, sl));
-    *c = c0 + fma(-s0, sr, fma(c0, cm1, cl));
+    o.sl = fma(o.c0, sr, fma(o.s0, cm1, sl));
+    o.cl = fma(-o.s0, sr, fma(o.c0, cm1, cl));
+    return o;
+}
+__host__ __device__ __forceinline__ void sincos_tab64(double x, const double* __restrict__ tab, double* s,
+                                                      double* c)
+{
+    const SinCos v = sincos_parts64(x, tab);
+    *s = v.s();
+    *c = v.c();
+}
+
+// sin and cos of x + e, |e| <= SHIFT_MAX, from those of x: first order in e, summed into the
+// corrections, so the result is rounded as sincos_tab64(x + e) is (e^2 / 2 < 5e-19).
+constexpr double SHIFT_MAX = 9.313225746154785e-10;   // 2^-30
+__host__ __device__ __forceinline__ void sincos_shift64(const SinCos& v, double c, double s, double e, double* se,
+                                                        double* ce)
+{
+    *se = v.s0 + fma(e, c, v.sl);
+    *ce = v.c0 + fma(-e, s, v.cl);
 }
 
 // a / b given y = 1 / b correctly rounded: q = a y, r = a - b q (exact), q + r y.  Equal to the
@@ -570,29 +669,41 @@ __host__ __device__ __forceinline__ double div_by(double a, double b, double y)
 // and its rotation into the aperture frame, bvk = k |x3|, kxx and kyy with their clamps, and per
 // edge delta, delta1, delta2, omega1, omega2 and the sums delta + omega -- is formed with the
 // reference's operations in its order, without contraction, so the phases are the reference's
-// doubles bit for bit (the quotients through div_by equal the divisions).  The amplitude algebra
-// around them is reorganised; each step there changes a result by a few ulp at most:
-//   * sines and cosines from the table (sincos_tab64);
-//   * the Karczewski direction normalised by reciprocal square roots, the ratio
-//     sqrt((1 - k_y^2) / (1 - K_y^2)) from the record's 1 / sqrt(1 - K_y^2);
-//   * rot4 . diff_ampl = g I + h J (J = [[0,1],[-1,0]]: both factors have that form), applied
-//     to the amplitude matrix; temp_rot1 depends on phi only and is applied to the bin's sum
-//     after the beam loop (apply_temp_rot1).
+// doubles bit for bit: roots, reciprocals and quotients come from shorter sequences that equal the
+// IEEE operations (sqrt_cr, rcp_cr, div_by).  Bound by FP64 VALU issue, so what is left out counts:
+//   * the reference's ten sines and cosines per triangle need three table lookups besides bvk's:
+//     delta_j + omega1 and delta_j + omega2 are both the phase of vertex j + 1 up to rounding
+//     (~1e-14), so their values are delta_{j+1}'s moved by the exact difference (sincos_shift64),
+//     rounded as their own lookups would be.  Clamped slopes (diff_mod.f90:379-382) move the phase
+//     further: those edges look their own values up;
+//   * the two roots |x1| and |x3| = |x1| (1 + rounding) share one hardware approximation, and the
+//     reciprocals of both and of bvk follow from it.
+// The amplitude algebra around the phases is reorganised; each step there changes a result by a
+// few ulp at most:
+//   * rot4 . diff_ampl = g I + h J (J = [[0,1],[-1,0]]: both factors have that form); away from the
+//     k_y clamp and the forward fallback, hc = unit(inc x k) is normal to k, so with the Karczewski
+//     vector m both come from one reciprocal root (the closed form of beam_bin_mixed);
+//   * f (g I + h J) A summed through the projectors of J (beam_bin_mixed), which fp64_finish turns
+//     into the amplitude matrix; temp_rot1 depends on phi only and is applied there too.
 // The edge terms of contour_integral cancel one another, so they keep the reference's
 // operations as well (the divisions included), in its order.
-// acc: re/im of (1,1) (2,1) (1,2) (2,2), before temp_rot1.  tab: the exponential table (LDS).
-// incoherent: acc[0] += |amplC|_F^2 instead (temp_rot1 is orthogonal: the norm is final).
-__host__ __device__ __forceinline__ void beam_bin_fp64(const double* __restrict__ r,
-                                                       const double* __restrict__ vrecs,
-                                                       const DevGrid& g, const BinIn& bi,
-                                                       const double* __restrict__ tab, int fast_diff,
-                                                       double acc[8], bool incoherent = false)
+// The default column's diff_main (3702 beams x 64,980 bins): 630 VALU instructions and 6.5 ms of kernels
+// before, 4.0 ms now; 5 orientations x 16,290 bins batched 7.9 -> 3.3 ms.
+// acc: the projector sums S+ (0..3) and S- (4..7).  tab: the exponential table (LDS).
+// INCOH: acc[0] += |amplC|_F^2 instead (temp_rot1 is orthogonal: the norm is final).
+template <bool INCOH>
+__host__ __device__ __forceinline__ void beam_bin_fp64p(const double* __restrict__ r,
+                                                        const double* __restrict__ vrecs,
+                                                        const DevGrid& g, const BinIn& bi,
+                                                        const double* __restrict__ tab, int fast_diff,
+                                                        double acc[8])
 {
 #pragma clang fp contract(off)
     const double x1 = bi.x - r[R_COM], y1 = bi.y - r[R_COM + 1], z1 = bi.z - r[R_COM + 2];
-    const double r1 = sqrt(x1 * x1 + y1 * y1 + z1 * z1);
+    double ir1;
+    const double r1 = sqrt_cr(x1 * x1 + y1 * y1 + z1 * z1, &ir1);
     if (fast_diff) {
-        double vx = x1 / r1, vy = y1 / r1, vz = z1 / r1;
+        const double vx = div_by(x1, r1, ir1), vy = div_by(y1, r1, ir1), vz = div_by(z1, r1, ir1);
         if (vx * r[R_PROP0] + vy * r[R_PROP0 + 1] + vz * r[R_PROP0 + 2] < r[R_COSFOV]) return;
     }
     const double* R = r + R_RR;
@@ -602,46 +713,63 @@ __host__ __device__ __forceinline__ void beam_bin_fp64(const double* __restrict_
     const double Kx = r[R_PROP2], Ky = r[R_PROP2 + 1], Kz = r[R_PROP2 + 2];
     // the phase inputs of contour_integral (diff_mod.f90:357-375)
     const double w = g.waveno;
-    const double bvk = w * sqrt(x3 * x3 + y3 * y3 + z3 * z3);
-    const double ibvk = 1.0 / bvk;
+    const double bvk = w * sqrt_from(x3 * x3 + y3 * y3 + z3 * z3, ir1);
+    const double ibvk = rcp_from(bvk, ir1 * g.inv_waveno);
     const double ww = w * w;
     double kxx = Kx * w - div_by(ww * x3, bvk, ibvk);
     double kyy = Ky * w - div_by(ww * y3, bvk, ibvk);
     if (fabs(kxx) < KMIN) kxx = KMIN;
     if (fabs(kyy) < KMIN) kyy = KMIN;
-    // karczewski (diff_mod.f90:145-181): k = x3 / r1 as the reference divides, since k also
-    // decides the k_y clamp and the forward test below
-    const double ir1 = 1.0 / r1;
+    // karczewski (diff_mod.f90:145-181): k = x3 / r1 as the reference divides, since k_y also
+    // decides the clamp below
     const double k1 = div_by(x3, r1, ir1), k3 = div_by(z3, r1, ir1);
-    double k2 = div_by(y3, r1, ir1);
-    if (fabs(k2) > K2CLAMP) k2 = copysign(K2CLAMP, k2);
-    const double omk = fma(-k2, k2, 1.0);
-    const double isq = rsq64(omk);                       // 1 / sqrt(1 - k2^2)
-    const double k12 = k1 * k2;
-    const double m1 = -(k12 * isq), m2 = omk * isq, m3 = -(k2 * k3 * isq);
-    const double frac = m2 * r[R_FRAC];                  // sqrt((1 - k2^2) / (1 - Ky^2))
-    const double ifrac = isq * r[R_ISIG];                // its reciprocal
-    const double a1m = -(Kz * frac), b2m = -(k3 * ifrac);
-    const double b1m = fma(Kx * Ky, frac, -(k12 * ifrac));
-    const double d11 = 0.5 * (a1m + b2m), d12 = 0.5 * b1m;   // diff_ampl = d11 I + d12 J
-    // scattering-plane vector hc (diff_mod.f90:630-635) and rot4 = p I - qh J
-    const double i1 = r[R_INC2], i2 = r[R_INC2 + 1], i3 = r[R_INC2 + 2];
-    double kk1 = k1, kk2 = k2, kk3 = k3;
-    if (!(fabs(i1 * k1 + i2 * k2 + i3 * k3) < FWD_DOT)) {
-        const double xt1 = bi.xt - r[R_COM], yt1 = bi.yt - r[R_COM + 1], zt1 = bi.zt - r[R_COM + 2];
-        const double irt = 1.0 / sqrt(xt1 * xt1 + yt1 * yt1 + zt1 * zt1);
-        kk1 = (R[0] * xt1 + R[1] * yt1 + R[2] * zt1) * irt;
-        kk2 = (R[3] * xt1 + R[4] * yt1 + R[5] * zt1) * irt;
-        kk3 = (R[6] * xt1 + R[7] * yt1 + R[8] * zt1) * irt;
+    const double k2 = div_by(y3, r1, ir1);
+    const double* C = r + R_C64P;
+    double gg, hj;   // rot4 . diff_ampl = gg I + hj J
+    const double uz = z1 * ir1;
+    const bool kclamp = fabs(k2) > K2CLAMP, fwd = !(fabs(uz) < FWD_DOT);
+    if (!kclamp && !fwd) {
+        const double ux = x1 * ir1, uy = y1 * ir1;
+        const double omk = fma(-k2, k2, 1.0);
+        const double P0 = fma(R[3], uy, -(R[4] * ux));       // |inc x k| h_y
+        const double Q0 = fma(-uz, k2, R[5]);                // |inc x k| (hc x k)_y
+        const double rh = rsq64_3(fma(ux, ux, uy * uy) * (omk * omk));   // 1 / (|inc x k| (1 - k_y^2))
+        const double P = P0 * rh, Q = Q0 * rh;
+        const double A = fma(C[0], omk, C[1] * k3);
+        const double B = fma(C[2], omk, C[1] * (k1 * k2));
+        gg = fma(P, A, Q * B);
+        hj = fma(P, B, -(Q * A));
+    } else {
+        const double k2c = kclamp ? copysign(K2CLAMP, k2) : k2;
+        const double omk = fma(-k2c, k2c, 1.0);
+        const double isq = rsq64_3(omk);                     // 1 / sqrt(1 - k2^2)
+        const double k12 = k1 * k2c;
+        const double m1 = -(k12 * isq), m2 = omk * isq, m3 = -(k2c * k3 * isq);
+        const double frac = m2 * r[R_FRAC];                  // sqrt((1 - k2^2) / (1 - Ky^2))
+        const double ifrac = isq * r[R_ISIG];                // its reciprocal
+        const double a1m = -(Kz * frac), b2m = -(k3 * ifrac);
+        const double b1m = fma(Kx * Ky, frac, -(k12 * ifrac));
+        const double d11 = 0.5 * (a1m + b2m), d12 = 0.5 * b1m;   // diff_ampl = d11 I + d12 J
+        // scattering-plane vector hc (diff_mod.f90:630-635) and rot4 = p I - qh J
+        const double i1 = r[R_INC2], i2 = r[R_INC2 + 1], i3 = r[R_INC2 + 2];
+        double kk1 = k1, kk2 = k2c, kk3 = k3;
+        if (fwd) {
+            const double xt1 = bi.xt - r[R_COM], yt1 = bi.yt - r[R_COM + 1], zt1 = bi.zt - r[R_COM + 2];
+            const double irt = rsq64_3(xt1 * xt1 + yt1 * yt1 + zt1 * zt1);
+            kk1 = (R[0] * xt1 + R[1] * yt1 + R[2] * zt1) * irt;
+            kk2 = (R[3] * xt1 + R[4] * yt1 + R[5] * zt1) * irt;
+            kk3 = (R[6] * xt1 + R[7] * yt1 + R[8] * zt1) * irt;
+        }
+        const double h1 = fma(i2, kk3, -(i3 * kk2)), h2 = fma(i3, kk1, -(i1 * kk3)), h3 = fma(i1, kk2, -(i2 * kk1));
+        const double e1 = fma(k2c, m3, -(k3 * m2)), e2 = fma(k3, m1, -(k1 * m3)), e3 = fma(k1, m2, -(k2c * m1));
+        const double hh = fma(h1, h1, fma(h2, h2, h3 * h3));
+        const double ee = fma(e1, e1, fma(e2, e2, e3 * e3));
+        const double ihh = rsq64_3(hh);
+        const double p = fma(h1, m1, fma(h2, m2, h3 * m3)) * ihh;
+        const double qh = fma(h1, e1, fma(h2, e2, h3 * e3)) * (ihh * rsq64_3(ee));
+        gg = fma(p, d11, qh * d12);
+        hj = fma(p, d12, -(qh * d11));
     }
-    const double h1 = fma(i2, kk3, -(i3 * kk2)), h2 = fma(i3, kk1, -(i1 * kk3)), h3 = fma(i1, kk2, -(i2 * kk1));
-    const double e1 = fma(k2, m3, -(k3 * m2)), e2 = fma(k3, m1, -(k1 * m3)), e3 = fma(k1, m2, -(k2 * m1));
-    const double hh = fma(h1, h1, fma(h2, h2, h3 * h3));
-    const double ee = fma(e1, e1, fma(e2, e2, e3 * e3));
-    const double ihh = rsq64(hh);
-    const double p = fma(h1, m1, fma(h2, m2, h3 * m3)) * ihh;
-    const double qh = fma(h1, e1, fma(h2, e2, h3 * e3)) * (ihh * rsq64(ee));
-    const double gg = fma(p, d11, qh * d12), hj = fma(p, d12, -(qh * d11));   // rot4 . diff_ampl
     // contour_integral (diff_mod.f90:357-421), edge by edge as the reference sums: the edge
     // terms cancel, so their roundings are kept too
     double sb, cb;
@@ -649,62 +777,117 @@ __host__ __device__ __forceinline__ void beam_bin_fp64(const double* __restrict_
     const double lam = g.lambda, ilam = g.inv_lambda;
     const double tkx = 2 * kxx, tky = 2 * kyy;
     double ar = 0.0, ai = 0.0;
-    const auto edge = [&](double xj, double yj, double mj, double nj, double dx, double dy) {
+    // one edge from vertex j (phase d0, sine and cosine s0, c0) to the next (phase dn, v its parts)
+    const auto edge = [&](double d0, double s0, double c0, double dn, const SinCos& v, double sn, double cn,
+                          double mj, double nj, double dx, double dy) {
 #pragma clang fp contract(off)
-        const double delta = kxx * xj + kyy * yj;
         const double delta1 = kyy * mj + kxx;
         const double delta2 = kxx * nj + kyy;
         const double omega1 = dx * delta1;
         const double omega2 = dy * delta2;
-        const double alpha = 1 / (tky * delta1);
-        const double beta = 1 / (tkx * delta2);
-        double s0, c0, s1, c1, s2, c2;
-        sincos_tab64(delta, tab, &s0, &c0);
-        sincos_tab64(delta + omega1, tab, &s1, &c1);
-        sincos_tab64(delta + omega2, tab, &s2, &c2);
+        const double alpha = rcp_cr(tky * delta1);
+        const double beta = rcp_cr(tkx * delta2);
+        const double f1 = d0 + omega1, f2 = d0 + omega2;
+        const double e1 = f1 - dn, e2 = f2 - dn;
+        double s1, c1, s2, c2;
+        sincos_shift64(v, cn, sn, e1, &s1, &c1);
+        sincos_shift64(v, cn, sn, e2, &s2, &c2);
+        if (!(fmax(fabs(e1), fabs(e2)) <= SHIFT_MAX)) {
+            sincos_tab64(f1, tab, &s1, &c1);
+            sincos_tab64(f2, tab, &s2, &c2);
+        }
         const double sumim = alpha * (c0 - c1) - beta * (c0 - c2);
         const double sumre = -(alpha * (s0 - s1)) + beta * (s0 - s2);
         ar = ar + div_by(cb * sumre - sb * sumim, lam, ilam);
         ai = ai + div_by(cb * sumim + sb * sumre, lam, ilam);
     };
-    // triangles: edges inline in the record; polygons: the vertex records.  Two
-    // loops, so each reads one address space (records staged in LDS, vrecs global).
-    const int nv = (int)r[R_NV];
-    if (nv <= 3) {
-        for (int j = 0; j < nv; j++)
-            edge(r[R_EX + j], r[R_EY + j], r[R_EM + j], r[R_EN + j], r[R_EDX + j], r[R_EDY + j]);
+    // triangles: edges inline in the record; other vertex counts: a loop (polygons' vertex records)
+    const int nv = record_int(r[R_NV]);
+    if (nv == 3) {
+        double d[3], s[3], c[3];
+        SinCos v[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            d[j] = kxx * r[R_EX + j] + kyy * r[R_EY + j];
+            v[j] = sincos_parts64(d[j], tab);
+            s[j] = v[j].s();
+            c[j] = v[j].c();
+        }
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int n = j == 2 ? 0 : j + 1;
+            edge(d[j], s[j], c[j], d[n], v[n], s[n], c[n], r[R_EM + j], r[R_EN + j], r[R_EDX + j], r[R_EDY + j]);
+        }
     } else {
-        const double* vr = vrecs + (int64_t)r[R_VOFF] * VREC;
+        const double* vr = vrecs + (int64_t)record_int(r[R_VOFF]) * VREC;
+        const auto field = [&](int j, int f, int inl) { return nv > 3 ? vr[VREC * j + f] : r[inl + j]; };
+        const auto phase = [&](int j) {
+#pragma clang fp contract(off)
+            return kxx * field(j, V_X, R_EX) + kyy * field(j, V_Y, R_EY);
+        };
+        const double df = phase(0);
+        const SinCos vf = sincos_parts64(df, tab);
+        double d0 = df, s0 = vf.s(), c0 = vf.c();
         for (int j = 0; j < nv; j++) {
-            const double* v = vr + VREC * j;
-            edge(v[V_X], v[V_Y], v[V_M], v[V_N], v[V_DX], v[V_DY]);
+            const bool last = j == nv - 1;
+            double dn = df;
+            SinCos v = vf;
+            if (!last) {
+                dn = phase(j + 1);
+                v = sincos_parts64(dn, tab);
+            }
+            const double sn = v.s(), cn = v.c();
+            edge(d0, s0, c0, dn, v, sn, cn, field(j, V_M, R_EM), field(j, V_N, R_EN), field(j, V_DX, R_EDX),
+                 field(j, V_DY, R_EDY));
+            d0 = dn;
+            s0 = sn;
+            c0 = cn;
         }
     }
-    // (g I + h J) . ampl, times the aperture integral
-    const double* A = r + R_AMPL;
-    double o[8];
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-#pragma unroll
-        for (int ri = 0; ri < 2; ri++) {
-            const double a1 = A[4 * q + ri], a2 = A[4 * q + 2 + ri];   // A(1,q), A(2,q)
-            o[4 * q + ri] = fma(gg, a1, hj * a2);
-            o[4 * q + 2 + ri] = fma(gg, a2, -(hj * a1));
-        }
-    if (incoherent) {
+    if (INCOH) {
         // diagnostic: sum over beams of |amplC|_F^2 (conditioning of the coherent sum)
-        double n2 = 0.0;
+        double a2 = 0.0;
 #pragma unroll
-        for (int q = 0; q < 8; q++) n2 = fma(o[q], o[q], n2);
-        acc[0] = fma(n2, fma(ar, ar, ai * ai), acc[0]);
+        for (int q = 0; q < 8; q++) a2 = fma(r[R_AMPL + q], r[R_AMPL + q], a2);
+        acc[0] = fma(a2 * fma(gg, gg, hj * hj), fma(ar, ar, ai * ai), acc[0]);
         return;
     }
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const double br = o[2 * q], bim = o[2 * q + 1];
-        acc[2 * q] = fma(br, ar, fma(-bim, ai, acc[2 * q]));
-        acc[2 * q + 1] = fma(br, ai, fma(bim, ar, acc[2 * q + 1]));
-    }
+    // f (gg I + hj J) A = w P A + w' Q A, w = f (gg + i hj), w' = f (gg - i hj)
+    const double ta = ar * gg, tc = ar * hj;
+    const double wr = fma(-ai, hj, ta), wi = fma(ai, gg, tc);
+    const double vr_ = fma(ai, hj, ta), vi = fma(ai, gg, -tc);
+    const double* rp = r + R_RP64;
+    const double* rm = r + R_RM64;
+    acc[0] = fma(wr, rp[0], fma(-wi, rp[1], acc[0]));
+    acc[1] = fma(wr, rp[1], fma(wi, rp[0], acc[1]));
+    acc[2] = fma(wr, rp[2], fma(-wi, rp[3], acc[2]));
+    acc[3] = fma(wr, rp[3], fma(wi, rp[2], acc[3]));
+    acc[4] = fma(vr_, rm[0], fma(-vi, rm[1], acc[4]));
+    acc[5] = fma(vr_, rm[1], fma(vi, rm[0], acc[5]));
+    acc[6] = fma(vr_, rm[2], fma(-vi, rm[3], acc[6]));
+    acc[7] = fma(vr_, rm[3], fma(vi, rm[2], acc[7]));
+}
+
+// From the projector sums to the amplitude matrix X = [S+ + S-; i (S+ - S-)], in place:
+// re/im of (1,1) (2,1) (1,2) (2,2).
+__host__ __device__ __forceinline__ void projectors_to_matrix(double a[8])
+{
+    const double x[8] = {a[0] + a[4], a[1] + a[5], -(a[1] - a[5]), a[0] - a[4],
+                         a[2] + a[6], a[3] + a[7], -(a[3] - a[7]), a[2] - a[6]};
+    for (int q = 0; q < 8; q++) a[q] = x[q];
+}
+
+// One beam, one bin of the plain body, added to the amplitude matrix acc (before temp_rot1).
+__host__ __device__ __forceinline__ void beam_bin_fp64(const double* __restrict__ r,
+                                                       const double* __restrict__ vrecs,
+                                                       const DevGrid& g, const BinIn& bi,
+                                                       const double* __restrict__ tab, int fast_diff,
+                                                       double acc[8])
+{
+    double s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    beam_bin_fp64p<false>(r, vrecs, g, bi, tab, fast_diff, s);
+    projectors_to_matrix(s);
+    for (int q = 0; q < 8; q++) acc[q] += s[q];
 }
 
 // Difference form of one edge of the rotation-invariant form factor, from the full vertex
@@ -952,19 +1135,13 @@ __host__ __device__ __forceinline__ void apply_bin_phase(double acc[8], double k
 }
 
 // From the projector sums S+ = acc[0..3], S- = acc[4..7] (columns 1, 2) to the
-// amplitude matrix X = [S+ + S-; i (S+ - S-)], then temp_rot1 on the right.
+// amplitude matrix, then temp_rot1 on the right.
 __host__ __device__ __forceinline__ void apply_temp_rot1(double acc[8], double cp, double sp);
 
 __host__ __device__ __forceinline__ void mixed_finish(double acc[8], double cp, double sp)
 {
-    double x[8];
-    // layout of x: (1,1) (2,1) (1,2) (2,2), re/im
-    x[0] = acc[0] + acc[4];          x[1] = acc[1] + acc[5];           // X(1,1)
-    x[2] = -(acc[1] - acc[5]);       x[3] = acc[0] - acc[4];           // X(2,1) = i (S+1 - S-1)
-    x[4] = acc[2] + acc[6];          x[5] = acc[3] + acc[7];           // X(1,2)
-    x[6] = -(acc[3] - acc[7]);       x[7] = acc[2] - acc[6];           // X(2,2) = i (S+2 - S-2)
-    apply_temp_rot1(x, cp, sp);
-    for (int q = 0; q < 8; q++) acc[q] = x[q];
+    projectors_to_matrix(acc);
+    apply_temp_rot1(acc, cp, sp);
 }
 
 // The mixed kernel sums f_b G_b A_b over beams per bin; the phi-only rotation

@@ -203,6 +203,9 @@ __host__ __device__ inline void make_beam_record(const double* ampl, const doubl
     rec[R_C64 + 0] = -0.5 * prop2[2] * rec[R_FRAC] / krev;
     rec[R_C64 + 1] = -0.5 * isig / krev;
     rec[R_C64 + 2] = 0.5 * prop2[0] * prop2[1] * rec[R_FRAC] / krev;
+    rec[R_C64P + 0] = -0.5 * prop2[2] * rec[R_FRAC];
+    rec[R_C64P + 1] = -0.5 * isig;
+    rec[R_C64P + 2] = 0.5 * prop2[0] * prop2[1] * rec[R_FRAC];
     rec[R_ISIG] = isig;
     rg[G_C1] = (float)rec[R_C64 + 0];
     rg[G_C2] = (float)rec[R_C64 + 1];

@@ -46,7 +46,9 @@ enum : int {
     R_RM64 = 100,   // [4] r- = (A(1,:) + i A(2,:)) / 2
     R_C64 = 104,    // [3] the Karczewski coefficients G_C1, G_C2, G_C3 in FP64
     R_ISIG = 107,   // sqrt(1 - prop2_y^2)
-    REC = 108       // padded to a multiple of 4 doubles (32 bytes)
+    // Karczewski coefficients of the plain FP64 body (R_C64 without the krev scaling)
+    R_C64P = 108,   // [3]
+    REC = 112       // padded to a multiple of 4 doubles (32 bytes)
 };
 
 // float offsets inside the FP32 block of a beam record
@@ -90,6 +92,7 @@ struct DevGrid {
     double inv_krev;                        // 1/krev (restructured FP64 body)
     double tri_scale;                       // 1 / (2 pi^2 lambda) (its triangle form factor)
     double inv_lambda;                      // 1 / lambda (plain FP64 body)
+    double inv_waveno;                      // 1 / waveno
     const double* x;                        // [nbins] far-field bin positions
     const double* y;
     const double* z;
@@ -134,6 +137,7 @@ inline void devgrid_constants(DevGrid& g, double lambda)
     g.inv_krev = 1.0 / g.krev;
     g.tri_scale = 1.0 / (2.0 * 9.869604401089358 * lambda);
     g.inv_lambda = 1.0 / lambda;
+    g.inv_waveno = 1.0 / g.waveno;
 }
 
 }  // namespace abt

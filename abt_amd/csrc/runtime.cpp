@@ -161,18 +161,18 @@ int theta_i_of(int64_t nth, const double* th)
     return (int)(nth - 1);
 }
 
-// How one orientation's beam list is cut: segments of `per` beams (a multiple of 32), nseg of them.
+// How one orientation's beam list is cut: segments of `per` beams (a multiple of `q`), nseg of them.
 struct Cut {
     int64_t per = 0;
     int nseg = 1;
     size_t work(int64_t nbins) const { return nseg > 1 ? sizeof(double) * 8 * (size_t)nbins * nseg : 0; }
 };
 
-Cut cut_into(int64_t nb, int64_t c)
+Cut cut_into(int64_t nb, int64_t c, int64_t q)
 {
     c = std::max<int64_t>(1, std::min<int64_t>(c, 32));   // the workspace is 64 B per bin per segment
     Cut k;
-    k.per = std::max<int64_t>(32, ((nb + c - 1) / c + 31) / 32 * 32);
+    k.per = std::max<int64_t>(q, ((nb + c - 1) / c + q - 1) / q * q);
     k.nseg = (int)std::max<int64_t>(1, (nb + k.per - 1) / k.per);
     return k;
 }
@@ -185,18 +185,18 @@ Cut cut_long(int64_t nbins, int64_t nb, int cus)
 {
     const int64_t tiles = (nbins + 255) / 256;
     const int64_t want = ((int64_t)cus * 320 + tiles - 1) / tiles;
-    return cut_into(nb, std::min<int64_t>(want, nb / 512));
+    return cut_into(nb, std::min<int64_t>(want, nb / 512), 32);
 }
 
 // The cut where a workspace for it is at hand.  When the segments of cut_long leave the chip with
-// fewer than 8 workgroups per CU, shorter ones (down to 32 beams) fill it: the default column's
+// fewer than 8 workgroups per CU, shorter ones (down to 8 beams, the mixed body's group) fill it: the default column's
 // 2838 + 864 beams on 64,980 bins (254 tiles), plain FP64, 8.1 -> 7.6 ms a diff_main call.
 Cut cut_beams(int64_t nbins, int64_t nb, int cus)
 {
     const int64_t tiles = (nbins + 255) / 256;
     const Cut l = cut_long(nbins, nb, cus);
     const int64_t fill = ((int64_t)cus * 8 + tiles - 1) / tiles;
-    return fill > l.nseg ? cut_into(nb, std::min<int64_t>(fill, nb / 32)) : l;
+    return fill > l.nseg ? cut_into(nb, std::min<int64_t>(fill, nb / 8), 8) : l;
 }
 
 }  // namespace

@@ -18,8 +18,7 @@ __device__ __forceinline__ void finish_sum(double acc[8], const DevGrid& g, int 
 {
     const int iphi = bin % g.nphi;
     const double cp = g.cphi[iphi], sp = g.sphi[iphi];
-    if (PREC == 0) apply_temp_rot1(acc, cp, sp);
-    if (PREC == 1) mixed_finish(acc, cp, sp);
+    if (PREC == 0 || PREC == 1) mixed_finish(acc, cp, sp);
     if (PREC == 3) model_finish(acc, cp, sp, g.kr_rev[bin]);
     if (PREC == 4) fp64r_finish(acc, cp, sp, g.kr_rev[bin]);
 }
