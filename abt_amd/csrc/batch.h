@@ -24,6 +24,7 @@ struct CombineArgs {
     const int32_t* list;      // list mode: the bins recomputed in FP64, ascending
     const int32_t* list_count;
     int o0, o1, nchunks, first;   // first: the chunk sums are stored, not added to
+    int summed;               // each tree's segments are already summed, in its first
 };
 
 // A run's launches: groups of orientations whose segment sums fit the plan's buffer.

@@ -22,10 +22,14 @@ constexpr int MAX_CHUNKS = 128;
 // segments fit; a group's last round of workgroups costs about 512 / (segments x tiles) of its time
 // (0.4 % at 2 GiB).
 constexpr size_t PART_BYTES = (size_t)2 << 30;
-// Workgroups a run is cut into, per CU (4 resident): the last round is then under 1 % of a run, and
-// a few coarse orientations still fill the chip.
-constexpr int64_t UNITS_PER_CU = 256;
-constexpr int64_t MIN_SEG = 32, MAX_SEG = 4096;
+// Segment length.  The last round of workgroups idles about half a segment, 0.5 x 256 bins x len / (rate
+// / 1024 slots) seconds; the segment sums cost 128 bytes per bin and segment, total / len of them, at
+// ~3 TB/s.  The two are equal at len = sqrt(total x nbins x 4e-5) for ~1.2e11 beam.bins/s (the bodies run at
+// 0.6e11 to 2.3e11; a factor of two either way costs under 1 % of a run).
+constexpr double SEG_RULE = 4e-5;
+// Below 16 beams a segment's start-up (table, bins, first records) weighs as much as its beams: 4
+// orientations x 37 x 36 bins take 88, 87, 93 and 94 us a run with at least 8, 16, 24 and 32.
+constexpr int64_t MIN_SEG = 16, MAX_SEG = 4096;
 const int TB_CAND[3] = {8, 16, 32};
 const int BPT_CAND[2] = {1, 2};
 
@@ -107,21 +111,20 @@ int shape_for(const abt_batch_plan* p, int tb, int bpt, Shape* s)
 }
 
 // The segment length and table.  A rule of the plan's sizes only (not of the tile shape), so that
-// every shape gives the same sums; lengths are multiples of 32, so that the mixed body's FP32 beam
-// groups are those of the uncut list.
+// every shape gives the same sums; lengths are multiples of 16, so that the mixed body's FP32 beam
+// groups (of 8) are those of the uncut list.
 void make_segments(abt_batch_plan* p, std::vector<abt::SweepSeg>& segs)
 {
     const int n = p->norient;
-    const int64_t nbins = p->g->nbins, tiles = ceil_div(nbins, LANES);
-    const int64_t total = p->boff[n] + p->eoff[n];
-    const int64_t want = std::max<int64_t>(1, ceil_div(UNITS_PER_CU * p->cus, tiles));
-    int64_t len = std::min(MAX_SEG, std::max(MIN_SEG, round_up(ceil_div(total, want), 32)));
+    const int64_t nbins = p->g->nbins;
+    const double total = (double)(p->boff[n] + p->eoff[n]);
+    int64_t len = std::min(MAX_SEG, std::max(MIN_SEG, round_up((int64_t)sqrt(total * (double)nbins * SEG_RULE), 16)));
     // an orientation's segments fit the buffer and one launch
     const int64_t most = std::max<int64_t>(2, std::min<int64_t>(65535, (int64_t)(PART_BYTES / (64 * (size_t)nbins))));
     int64_t largest = 1;
     for (int o = 0; o < n; o++)
         largest = std::max(largest, p->boff[o + 1] - p->boff[o] + p->eoff[o + 1] - p->eoff[o]);
-    len = std::max(len, most > 2 ? round_up(ceil_div(largest, most - 1), 32) : round_up(largest, 32));
+    len = std::max(len, most > 2 ? round_up(ceil_div(largest, most - 1), 16) : round_up(largest, 16));
     p->seg_len = len;
     p->seg_off.assign(1, 0);
     for (int o = 0; o < n; o++)
@@ -234,8 +237,8 @@ int abt_batch_plan_create(const abt_dev_grid* g, int32_t norient, const int64_t*
     p->cus = cus;
     p->boff.assign(beam_off, beam_off + norient + 1);
     p->eoff.assign(ext_off, ext_off + norient + 1);
-    // (the restructured body's 8-beam tiles hold 4 waves per SIMD)
-    rc = shape_for(p, precision == ABT_FP64_FAST ? 8 : 16, 1, &p->shape);
+    // (the FP64 bodies' 8-beam tiles hold 4 waves per SIMD)
+    rc = shape_for(p, precision == ABT_FP64_FAST || precision == ABT_FP64 ? 8 : 16, 1, &p->shape);
     if (rc) { delete p; return rc; }
     std::vector<abt::SweepSeg> segs;
     make_segments(p, segs);
