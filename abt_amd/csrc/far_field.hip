@@ -34,9 +34,9 @@ constexpr int BLOCK = 256;
 template <int PREC>
 __device__ __forceinline__ BinIn load_bin(const DevGrid& g, int bc)
 {
+    const int bt = bc % g.nphi + g.nphi * g.theta_i;   // the theta_i bin of the same phi
     BinIn bi;
     bi.x = g.x[bc]; bi.y = g.y[bc]; bi.z = g.z[bc];
-    const int bt = bc % g.nphi + g.nphi * g.theta_i;
     bi.xt = g.x[bt]; bi.yt = g.y[bt]; bi.zt = g.z[bt];
     bi.rad = PREC >= 3 ? g.rad[bc] : 0.0;
     return bi;
@@ -55,9 +55,9 @@ void k_sweep(SweepArgs a)
     // bodies need their registers: one tile, loaded between barriers.
     constexpr bool DB = PREC == 1 && TB <= 16 && BPT == 1;
     __shared__ double tile[(DB ? 2 : 1) * TB * REC];
-    // the exponential table and the FP64r body's constants, or the table with its low parts
+    // the exponential table, or the table with its low parts
     constexpr bool TAB = PREC == 0 || PREC == 2 || PREC == 4;
-    __shared__ double etab[PREC == 4 ? ETAB_LDS : (TAB ? ETAB_GRID : 1)];
+    __shared__ double etab[PREC == 4 ? ETAB_DOUBLES : (TAB ? ETAB_GRID : 1)];
     constexpr int PF = DB ? (TB * REC + BLOCK - 1) / BLOCK : 1;   // doubles per lane per tile
     const DevGrid& g = a.g;
     const int tid = threadIdx.x;
@@ -66,13 +66,15 @@ void k_sweep(SweepArgs a)
     if ((int)blockIdx.x * (BLOCK * BPT) >= nslots) return;   // LIST: tiles past the listed bins
     if (TAB) {   // published by the barriers of the tile loop before any use
         for (int q = tid; q < (PREC == 4 ? ETAB_DOUBLES : ETAB_GRID); q += BLOCK) etab[q] = g.etab[q];
-        if (PREC == 4 && tid == 0) fp64r_constants(g, etab + ETAB_DOUBLES);
     }
     BinIn bi[BPT];
+    FarBin fb[BPT];
 #pragma unroll
     for (int j = 0; j < BPT; j++) {
         const int sc = min(slot0 + j * BLOCK, nslots - 1);
-        bi[j] = load_bin<PREC>(g, LIST ? a.list[sc] : sc);
+        const int bc = LIST ? a.list[sc] : sc;
+        bi[j] = load_bin<PREC>(g, bc);
+        if (PREC == 4) fb[j] = far_bin(bi[j]);
     }
     double acc[BPT][8], inc[BPT];
 #pragma unroll
@@ -154,7 +156,8 @@ void k_sweep(SweepArgs a)
 #pragma unroll
                 for (int j = 0; j < BPT; j++) {
                     if (PREC == 4)
-                        beam_bin_fp64r(cur + bb * REC, vrecs, g, bi[j], etab, a.fast_diff, acc[j]);
+                        beam_bin_fp64r_far(cur + bb * REC, vrecs, fb[j], bi[j].xt, bi[j].yt, etab, g.cc_far, a.fast_diff,
+                                           acc[j]);
                     else if (PREC == 3) {
                         AdjBeam B;
                         adj_beam_from_record(cur + bb * REC, B);

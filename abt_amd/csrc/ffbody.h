@@ -144,6 +144,26 @@ __host__ __device__ __forceinline__ int record_int(double x)
 #endif
 }
 
+// x == 3.0 for a value that is the same in every lane of a wave, as a scalar condition
+__host__ __device__ __forceinline__ bool record_is3(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_readfirstlane((int)(__builtin_bit_cast(uint64_t, x) >> 32)) == 0x40080000;
+#else
+    return x == 3.0;
+#endif
+}
+
+// a <= b for two values that are the same in every lane of a wave, as a scalar condition
+__host__ __device__ __forceinline__ bool record_less(double a, double b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_ballot_w64(a <= b) != 0;
+#else
+    return a <= b;
+#endif
+}
+
 constexpr float SERIES_QA2 = 2.25f;  // (|q_perp| a)^2 below which the FP64 series is used
 constexpr int SERIES_N = 16;         // truncation < 3e-12 relative at |q| a = 1.5
 
@@ -446,19 +466,6 @@ __host__ __device__ __forceinline__ double rsq64(double x)
     return fma(0.5 * y, e, y);
 }
 
-// reciprocal and reciprocal square root to ~1e-14: the FP32 hardware approximation and
-// one Newton step in FP64 (inputs within the FP32 range)
-__host__ __device__ __forceinline__ double rcp64_1(double x)
-{
-    const double y = (double)abt_rcpf((float)x);
-    return fma(y, fma(-x, y, 1.0), y);
-}
-__host__ __device__ __forceinline__ double rsq64_1(double x)
-{
-    const double y = (double)abt_rsqf((float)x);
-    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
-}
-
 // Hardware approximations in FP64 (relative error below 2^-24 and 2^-24 on gfx950, measured on 10^9
 // values); one costs as much as the FP32 one with its two conversions.
 __host__ __device__ __forceinline__ double rcp_seed(double x)
@@ -476,6 +483,18 @@ __host__ __device__ __forceinline__ double rsq_seed(double x)
 #else
     return 1.0 / sqrt(x);
 #endif
+}
+
+// reciprocal and reciprocal square root to ~5e-15: one Newton step
+__host__ __device__ __forceinline__ double rcp64_1(double x)
+{
+    const double y = rcp_seed(x);
+    return fma(y, fma(-x, y, 1.0), y);
+}
+__host__ __device__ __forceinline__ double rsq64_1(double x)
+{
+    const double y = rsq_seed(x);
+    return fma(0.5 * y, fma(-x * y, y, 1.0), y);
 }
 
 // The functions below work on normal values whose squares and reciprocals are normal too, as the
@@ -549,16 +568,8 @@ inline void fill_exp_table(double* tab)
     }
 }
 
-// The grid constants the FP64r body reads, stored after the table in its LDS block (read
-// there, they take no scalar registers across the beam loop).
-__host__ __device__ __forceinline__ void fp64r_constants(const DevGrid& g, double* c)
-{
-    c[ETAB_KREV - ETAB_DOUBLES] = g.krev;
-    c[ETAB_K2CLAMP - ETAB_DOUBLES] = g.krev_k2clamp;
-    c[ETAB_INV_KREV - ETAB_DOUBLES] = g.inv_krev;
-    c[ETAB_TRI_SCALE - ETAB_DOUBLES] = g.tri_scale;
-    c[ETAB_LAMBDA - ETAB_DOUBLES] = g.lambda;
-}
+// What a caller keeps after the table for beam_bin_fp64r: the grid's far limit.
+__host__ __device__ __forceinline__ void fp64r_constants(const DevGrid& g, double* c) { c[0] = g.cc_far; }
 
 // e^{i pi t} for an FP64 t (half revolutions): t = 2m + j / ETAB_N + r with |r| <= 1 / (2 ETAB_N)
 // (every step exact), e^{i pi t} = tab[j] e^{i pi r}, the last from its Taylor polynomials
@@ -579,24 +590,25 @@ __host__ __device__ __forceinline__ void expi_pi64(double t, const double* __res
     *s = fma(s0, cr, c0 * sr);
 }
 
-// e^{2 pi i t} for an FP64 t (revolutions, |t| < 2^20), from the same table: t = J / (2 ETAB_N) + r
-// with J = rint(2 ETAB_N t) and |r| <= 1 / (4 ETAB_N) (exact: t and J / (2 ETAB_N) are multiples of
-// the ulp of t), e^{2 pi i t} = e^{2 pi i J / (2 ETAB_N)} e^{2 pi i r}; the table holds the angle
-// 2 pi J / (2 ETAB_N) modulo 2 pi at index J mod 2 ETAB_N.  e^{2 pi i r} from its Taylor
-// polynomials in r itself, 2 pi folded into the coefficients (truncation below 2e-18).
-constexpr double EXP_S1 = 6.283185307179586;     // 2 pi
-constexpr double EXP_S3 = -41.34170224039976;    // -(2 pi)^3 / 6
-constexpr double EXP_S5 = 81.60524927607506;     // (2 pi)^5 / 120
-constexpr double EXP_C2 = -19.739208802178716;   // -(2 pi)^2 / 2
-constexpr double EXP_C4 = 64.9393940226683;      // (2 pi)^4 / 24
-__host__ __device__ __forceinline__ void expi_2pi64(double t, const double* __restrict__ tab, double* c, double* s)
+// e^{2 pi i T / (2 ETAB_N)} for an FP64 T in table steps (|T| < 2^31), from the same table: T = J + r with
+// J = rint(T) and |r| <= 1/2 (exact); the table holds the angle of J at index J mod 2 ETAB_N.  The rest
+// is |y| <= pi / 1024: cos y from its Taylor polynomial (truncation below 2e-18), sin y from the cubic
+// that is best in the largest error, y^5 / 120 replaced by its Chebyshev cubic (1.4e-16; a third
+// coefficient would cost one instruction per exponential for less than the table's own rounding).
+constexpr double EXP_H = 6.283185307179586 / (2.0 * ETAB_N);       // radians per step
+constexpr double EXP_Y = 0.5 * EXP_H;                              // largest |y|
+constexpr double EXP_S1 = EXP_H * (1.0 - EXP_Y * EXP_Y * EXP_Y * EXP_Y / 384.0);
+constexpr double EXP_S3 = EXP_H * EXP_H * EXP_H * (-1.0 / 6.0 + EXP_Y * EXP_Y / 96.0);
+constexpr double EXP_C2 = -0.5 * EXP_H * EXP_H;
+constexpr double EXP_C4 = EXP_H * EXP_H * EXP_H * EXP_H / 24.0;
+__host__ __device__ __forceinline__ void expi_step64(double T, const double* __restrict__ tab, double* c, double* s)
 {
-    const double jf = rint((double)(2 * ETAB_N) * t);
-    const double r = fma(-1.0 / (double)(2 * ETAB_N), jf, t);     // |r| <= 1 / (4 ETAB_N)
+    const double jf = rint(T);
+    const double r = T - jf;
     const int j = (int)jf & (2 * ETAB_N - 1);
     const double c0 = tab[2 * j], s0 = tab[2 * j + 1];
     const double w = r * r;
-    const double sr = r * fma(w, fma(w, EXP_S5, EXP_S3), EXP_S1);
+    const double sr = r * fma(w, EXP_S3, EXP_S1);
     const double cr = fma(w, fma(w, EXP_C4, EXP_C2), 1.0);
     *c = fma(c0, cr, -s0 * sr);
     *s = fma(s0, cr, c0 * sr);
@@ -663,6 +675,25 @@ __host__ __device__ __forceinline__ double div_by(double a, double b, double y)
     return fma(fma(-b, q, a), y, q);
 }
 
+// f (gg I + hh J) A = w P A + w' Q A, w = f (gg + i hh), w' = f (gg - i hh)
+__host__ __device__ __forceinline__ void add_projectors(const double* __restrict__ r, double FR, double FI, double gg,
+                                                        double hh, double acc[8])
+{
+    const double ta = FR * gg, tc = FR * hh;
+    const double wr = fma(-FI, hh, ta), wi = fma(FI, gg, tc);
+    const double vr = fma(FI, hh, ta), vi = fma(FI, gg, -tc);
+    const double* rp = r + R_RP64;
+    const double* rm = r + R_RM64;
+    acc[0] = fma(wr, rp[0], fma(-wi, rp[1], acc[0]));
+    acc[1] = fma(wr, rp[1], fma(wi, rp[0], acc[1]));
+    acc[2] = fma(wr, rp[2], fma(-wi, rp[3], acc[2]));
+    acc[3] = fma(wr, rp[3], fma(wi, rp[2], acc[3]));
+    acc[4] = fma(vr, rm[0], fma(-vi, rm[1], acc[4]));
+    acc[5] = fma(vr, rm[1], fma(vi, rm[0], acc[5]));
+    acc[6] = fma(vr, rm[2], fma(-vi, rm[3], acc[6]));
+    acc[7] = fma(vr, rm[3], fma(vi, rm[2], acc[7]));
+}
+
 // ---------------------------------------------------------------------------
 // FP64 plain kernel body: one beam, one bin (diffraction, diff_mod.f90:576-670; karczewski
 // :124-198; contour_integral :357-421).  Every input of a sine or cosine -- the bin offset
@@ -724,7 +755,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64p(const double* __restrict
     // decides the clamp below
     const double k1 = div_by(x3, r1, ir1), k3 = div_by(z3, r1, ir1);
     const double k2 = div_by(y3, r1, ir1);
-    const double* C = r + R_C64P;
+    const double* C = r + R_C64;
     double gg, hj;   // rot4 . diff_ampl = gg I + hj J
     const double uz = z1 * ir1;
     const bool kclamp = fabs(k2) > K2CLAMP, fwd = !(fabs(uz) < FWD_DOT);
@@ -852,20 +883,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64p(const double* __restrict
         acc[0] = fma(a2 * fma(gg, gg, hj * hj), fma(ar, ar, ai * ai), acc[0]);
         return;
     }
-    // f (gg I + hj J) A = w P A + w' Q A, w = f (gg + i hj), w' = f (gg - i hj)
-    const double ta = ar * gg, tc = ar * hj;
-    const double wr = fma(-ai, hj, ta), wi = fma(ai, gg, tc);
-    const double vr_ = fma(ai, hj, ta), vi = fma(ai, gg, -tc);
-    const double* rp = r + R_RP64;
-    const double* rm = r + R_RM64;
-    acc[0] = fma(wr, rp[0], fma(-wi, rp[1], acc[0]));
-    acc[1] = fma(wr, rp[1], fma(wi, rp[0], acc[1]));
-    acc[2] = fma(wr, rp[2], fma(-wi, rp[3], acc[2]));
-    acc[3] = fma(wr, rp[3], fma(wi, rp[2], acc[3]));
-    acc[4] = fma(vr_, rm[0], fma(-vi, rm[1], acc[4]));
-    acc[5] = fma(vr_, rm[1], fma(vi, rm[0], acc[5]));
-    acc[6] = fma(vr_, rm[2], fma(-vi, rm[3], acc[6]));
-    acc[7] = fma(vr_, rm[3], fma(vi, rm[2], acc[7]));
+    add_projectors(r, ar, ai, gg, hj, acc);
 }
 
 // From the projector sums to the amplitude matrix X = [S+ + S-; i (S+ - S-)], in place:
@@ -916,203 +934,283 @@ __host__ __device__ __forceinline__ void edge_diff64(double Wr0, double Wi0, dou
     }
 }
 
-// Restructured FP64 body: one beam, one bin; adds to the projector sums S+ (acc[0..3]) and
-// S- (acc[4..7]) that fp64r_finish turns into the amplitude matrix.  bi.rad = |x| is read.
+// What a lane keeps of its bin for the restructured FP64 body: the direction and 1 / distance.
+struct FarBin {
+    double nx, ny, nz, ir;
+};
+__host__ __device__ __forceinline__ FarBin far_bin(const BinIn& bi)
+{
+    const double ir = 1.0 / bi.rad;
+    return {bi.x * ir, bi.y * ir, bi.z * ir, ir};
+}
+
+// Restructured FP64 body: one beam, one bin, added to the projector sums S+ (acc[0..3]) and
+// S- (acc[4..7]) that fp64r_finish turns into the amplitude matrix.  Bound by FP64 VALU issue (one
+// instruction of any kind takes 4 cycles of a SIMD); the common case -- a triangle seen away from its
+// edges' nulls, its forward direction, the k_y clamp and the forward fallback -- is kept to 138 FP64
+// instructions and ~25 others (207 in all before):
+//   * the far geometry: with h = (|c|^2 / 2 - x.c) / |x|^2 small, |x - c| - |x| and 1 / |x - c| are short
+//     series in h -- no root, no reciprocal; their cut is checked per beam against the grid's limit
+//     (g.cc_far, a scalar branch), beyond which both come from the distances;
+//   * phases in table steps: the vertex coordinates carry krev and the table size, so a phase is
+//     two FMAs and its table index is its rounding;
+//   * one reciprocal root 1 / (|inc x k| (1 - k_y^2) |d0 d1 d2|) for the polarisation's normalisation
+//     and the form factor's denominator together.
+// Tried: records through scalar loads instead of LDS (fewer instructions, but a wave waits for each of
+// the ~6 scalar loads of a beam: 24 orientations x 721 x 180 bins 116 ms against 104); the other branches
+// after each tile in a pass of their own, which frees registers for a fifth wave but recomputes the
+// beam (125 ms; 112 with 4 waves).  Measured against the body before: 24 orientations x 721 x 180 bins
+// 109.1 -> 90.6 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 41.0 -> 37.2 ms.  What is left of the issue
+// rate (14 % of the cycles) is waits that 4 waves do not cover.
+struct FarGeom {
+    double ux, uy, uz;   // direction of the bin from the aperture centre
+    double kd;           // k (|x - c| - |x|) in table steps (the bin's own e^{i k |x|} follows the beam sum)
+};
+__host__ __device__ __forceinline__ FarGeom far_geometry(const double* __restrict__ r, const FarBin& fb, double cc_far)
+{
+    FarGeom o;
+    const double p = fma(fb.nx, r[R_COM], fma(fb.ny, r[R_COM + 1], fb.nz * r[R_COM + 2]));
+    if (record_less(r[R_CC], cc_far)) {
+        const double t = fma(0.5 * r[R_CC], fb.ir, -p);              // |x| h
+        const double h = t * fb.ir;
+        // |x - c| = |x| sqrt(1 + 2 h): sqrt(1 + 2 h) - 1 = h (1 - h/2 + h^2/2 - 5/8 h^3 + ..),
+        // 1 / sqrt(1 + 2 h) = 1 - h + 3/2 h^2 - 5/2 h^3 + ..
+        o.kd = (r[R_KT] * t) * fma(h, fma(h, fma(h, -0.625, 0.5), -0.5), 1.0);
+        const double gd = fma(h, fma(h, fma(h, -2.5, 1.5), -1.0), 1.0);
+        o.ux = fma(-r[R_COM], fb.ir, fb.nx) * gd;
+        o.uy = fma(-r[R_COM + 1], fb.ir, fb.ny) * gd;
+        o.uz = fma(-r[R_COM + 2], fb.ir, fb.nz) * gd;
+    } else {
+        // k (|x - c| - |x|) = k (|c|^2 - 2 x.c) / (|x - c| + |x|), formed without cancellation
+        const double rad = rcp_cr(fb.ir);
+        const double dx = fma(fb.nx, rad, -r[R_COM]), dy = fma(fb.ny, rad, -r[R_COM + 1]),
+                     dz = fma(fb.nz, rad, -r[R_COM + 2]);
+        const double s = fma(dx, dx, fma(dy, dy, dz * dz));
+        const double invd = rsq64_3(s);
+        o.ux = dx * invd;
+        o.uy = dy * invd;
+        o.uz = dz * invd;
+        o.kd = r[R_KT] * (fma(-2.0 * rad, p, r[R_CC]) * rcp_cr(fma(s, invd, rad)));
+    }
+    return o;
+}
+
+// Outside the beam's field of view (fast_diff; diff_mod.f90:593-603)
+__host__ __device__ __forceinline__ bool far_culled(const double* __restrict__ r, const FarGeom& u, int fast_diff)
+{
+    return fast_diff && u.ux * r[R_PROP0] + u.uy * r[R_PROP0 + 1] + u.uz * r[R_PROP0 + 2] < r[R_COSFOV];
+}
+
+// The vertices' phases, exponentials and phase differences, in table steps.
+struct TriPhase {
+    double Wr[3], Wi[3], d0, d1, d2;
+};
+__host__ __device__ __forceinline__ TriPhase tri_phases(const double* __restrict__ r, double q1, double q2, double kd,
+                                                        const double* __restrict__ etab)
+{
+    TriPhase o;
+    double T[3];
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+        T[l] = fma(q1, r[R_TX + l], fma(q2, r[R_TY + l], kd));
+        expi_step64(T[l], etab, &o.Wr[l], &o.Wi[l]);
+    }
+    o.d0 = T[1] - T[0];
+    o.d1 = T[2] - T[1];
+    o.d2 = T[0] - T[2];
+    return o;
+}
+
+// One denominator: the form factor of a triangle is 2 A times the second divided difference of
+// e^{i alpha} at its vertex phases alpha_l = 2 pi t_l, divided by i^2,
+//   F = 2 A (W0 d1 + W1 d2 + W2 d0) / ((2 pi)^2 d0 d1 d2),  d_j = t_{j+1} - t_j,
+// and sum_ref / lambda = -i F / lambda.  The exponentials' rounding enters the numerator as ~1.7e-16 max |d|, so
+// F / A as ~9e-18 max |d| / |d0 d1 d2|: at most 1.7e-13 under the condition below (the two smaller |d_j| times
+// each other at least 1e-4 turns^2), what the phases carry anyway (half an ulp of ~10^5 table steps is
+// 5e-14 rad a vertex).  2 % of the waves have a lane beyond it (beams of the rough column); the earlier
+// condition, every |d_j| >= 1e-3 and |q| a >= 1.5, left 13 % of them a lane in the other branch.
+__host__ __device__ __forceinline__ bool one_denominator(const TriPhase& w, double d)
+{
+    // strict: q = 0 has every d_j = 0
+    return fabs(d) > (1e-4 * (2 * ETAB_N) * (2 * ETAB_N)) * fmax(fabs(w.d0), fabs(w.d1));
+}
+
+// xt, yt: the theta_i bin of the same phi (forward fallback of hc).
+__host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __restrict__ r,
+                                                            const double* __restrict__ vrecs, const FarBin& fb,
+                                                            double xt, double yt, const double* __restrict__ etab,
+                                                            double cc_far, int fast_diff, double acc[8])
+{
+    const FarGeom u = far_geometry(r, fb, cc_far);
+    if (far_culled(r, u, fast_diff)) return;
+    const double* RR = r + R_RR;
+    const double k1 = fma(RR[0], u.ux, fma(RR[1], u.uy, RR[2] * u.uz));
+    const double k2 = fma(RR[3], u.ux, fma(RR[4], u.uy, RR[5] * u.uz));
+    const double k3 = fma(RR[6], u.ux, fma(RR[7], u.uy, RR[8] * u.uz));
+    const double q1 = r[R_PROP2] - k1, q2 = r[R_PROP2 + 1] - k2;   // q / k in the aperture plane
+    const bool nv3 = record_is3(r[R_NV]);
+    TriPhase w;
+    double d = 0.0;
+    bool one = false;
+    if (nv3) {
+        w = tri_phases(r, q1, q2, u.kd, etab);
+        d = w.d0 * w.d1 * w.d2;
+        one = one_denominator(w, d);
+    }
+    const bool kclamp = fabs(k2) > K2CLAMP, fwd = !(fabs(u.uz) < FWD_DOT);
+    const double s2 = fma(k1, k1, k3 * k3);                        // 1 - k_y^2 (unclamped)
+    // (FR, FI) = e^{i k (|x-c| - |x|)} sum_ref / lambda; gg I + hh J: karczewski + rot4 (diff_mod.f90:124-198,
+    // 630-643)
+    double FR, FI, gg, hh;
+    if (one && !kclamp && !fwd) {
+        // hc = unit(inc x khat) is normal to khat (see beam_bin_mixed)
+        const double* C = r + R_C64;
+        const double P0 = fma(RR[3], u.uy, -RR[4] * u.ux);
+        const double Q0 = fma(-u.uz, k2, RR[5]);
+        const double m = s2 * d;
+        const double ri = rsq64_1(fma(u.ux, u.ux, u.uy * u.uy) * (m * m));   // 1 / (|(ux, uy)| s2 |d|)
+        const double f = r[R_TA] * copysign(ri, d);
+        const double A = fma(C[0], s2, C[1] * k3);
+        const double B = fma(C[2], s2, C[1] * (k1 * k2));
+        FR = f * fma(w.Wi[0], w.d1, fma(w.Wi[1], w.d2, w.Wi[2] * w.d0));
+        FI = -f * fma(w.Wr[0], w.d1, fma(w.Wr[1], w.d2, w.Wr[2] * w.d0));
+        gg = fma(P0, A, Q0 * B);
+        hh = fma(P0, B, -Q0 * A);
+    } else {
+        const double qx = r[R_KREV] * q1, qy = r[R_KREV] * q2;   // revolutions per um
+        if (one) {
+            const double f = r[R_TA] * rcp64_1(d);
+            FR = f * fma(w.Wi[0], w.d1, fma(w.Wi[1], w.d2, w.Wi[2] * w.d0));
+            FI = -f * fma(w.Wr[0], w.d1, fma(w.Wr[1], w.d2, w.Wr[2] * w.d0));
+        } else if (fma(q1, q1, q2 * q2) * r[R_SA2] < (double)SERIES_QA2) {   // (|q| a)^2
+            const double tw = 6.283185307179586;
+            double sr = 0.0, si = 0.0;
+            if (nv3) {
+                const double a = tw * fma(qx, r[R_EX], qy * r[R_EY]);
+                const double b = tw * fma(qx, r[R_EX + 1], qy * r[R_EY + 1]);
+                const double c = tw * fma(qx, r[R_EX + 2], qy * r[R_EY + 2]);
+                double tr, ti;
+                tri_series(a, b, c, &tr, &ti);
+                sr = r[R_AREA] * tr;
+                si = r[R_AREA] * ti;
+            } else {
+                const int nv = record_int(r[R_NV]);
+                const double* vr = vrecs + (int64_t)record_int(r[R_VOFF]) * VREC;
+                for (int j = 0; j < nv; j++) {
+                    const int jp = (j == nv - 1) ? 0 : j + 1;
+                    const double xj = vr[VREC * j + V_X], yj = vr[VREC * j + V_Y];
+                    const double xn = vr[VREC * jp + V_X], yn = vr[VREC * jp + V_Y];
+                    const double a = tw * fma(qx, xj, qy * yj);
+                    const double b = tw * fma(qx, xn, qy * yn);
+                    const double sa = 0.5 * (xj * yn - xn * yj);
+                    double tr, ti;
+                    tri_series(0.0, a, b, &tr, &ti);
+                    sr += sa * tr;
+                    si += sa * ti;
+                }
+            }
+            // sum_ref = -i F = si - i sr
+            double cb, sb;
+            expi_step64(u.kd, etab, &cb, &sb);
+            FR = (cb * si + sb * sr) * r[R_IL];
+            FI = (sb * si - cb * sr) * r[R_IL];
+        } else {
+            constexpr double turn = 1.0 / (2 * ETAB_N);
+            double ssr = 0.0, ssi = 0.0;
+            if (nv3) {
+                edge_diff64(w.Wr[0], w.Wi[0], w.Wr[1], w.Wi[1], turn * w.d0, qx, qy, r[R_EDX], r[R_EDY], ssr, ssi);
+                edge_diff64(w.Wr[1], w.Wi[1], w.Wr[2], w.Wi[2], turn * w.d1, qx, qy, r[R_EDX + 1], r[R_EDY + 1], ssr, ssi);
+                edge_diff64(w.Wr[2], w.Wi[2], w.Wr[0], w.Wi[0], turn * w.d2, qx, qy, r[R_EDX + 2], r[R_EDY + 2], ssr, ssi);
+            } else {
+                const int nv = record_int(r[R_NV]);
+                const double* vr = vrecs + (int64_t)record_int(r[R_VOFF]) * VREC;
+                const double sx = (2 * ETAB_N) * qx, sy = (2 * ETAB_N) * qy;
+                const double T0 = fma(sx, vr[V_X], fma(sy, vr[V_Y], u.kd));
+                double Wr0, Wi0;
+                expi_step64(T0, etab, &Wr0, &Wi0);
+                double Tp = T0, Wrp = Wr0, Wip = Wi0;
+                for (int j = 0; j < nv; j++) {
+                    double Tn = T0, Wrn = Wr0, Win = Wi0;
+                    if (j < nv - 1) {
+                        Tn = fma(sx, vr[VREC * (j + 1) + V_X], fma(sy, vr[VREC * (j + 1) + V_Y], u.kd));
+                        expi_step64(Tn, etab, &Wrn, &Win);
+                    }
+                    edge_diff64(Wrp, Wip, Wrn, Win, turn * (Tn - Tp), qx, qy, vr[VREC * j + V_DX], vr[VREC * j + V_DY],
+                                ssr, ssi);
+                    Tp = Tn;
+                    Wrp = Wrn;
+                    Wip = Win;
+                }
+            }
+            const double sc = -r[R_IL] * rcp64_1(6.283185307179586 * fma(qx, qx, qy * qy));
+            FR = ssr * sc;
+            FI = ssi * sc;
+        }
+        if (!kclamp && !fwd) {
+            const double* C = r + R_C64;
+            const double P0 = fma(RR[3], u.uy, -RR[4] * u.ux);
+            const double Q0 = fma(-u.uz, k2, RR[5]);
+            const double rh = rsq64_1(fma(u.ux, u.ux, u.uy * u.uy) * (s2 * s2));   // 1 / (|(ux, uy)| s2)
+            const double P = P0 * rh, Q = Q0 * rh;
+            const double A = fma(C[0], s2, C[1] * k3);
+            const double B = fma(C[2], s2, C[1] * (k1 * k2));
+            gg = fma(P, A, Q * B);
+            hh = fma(P, B, -Q * A);
+        } else {
+            const double Kx = r[R_PROP2], Ky = r[R_PROP2 + 1], Kz = r[R_PROP2 + 2];
+            const double sig = r[R_FRAC], isig = r[R_ISIG];
+            const double k2c = kclamp ? copysign(K2CLAMP, k2) : k2;
+            const double s2c = kclamp ? (1.0 - K2CLAMP * K2CLAMP) : s2;
+            const double rs = rsq64_3(s2c);
+            const double sq = s2c * rs;
+            const double frac = sq * sig;
+            const double ifrac = rs * isig;
+            double da = -0.5 * fma(Kz, frac, k3 * ifrac);
+            double db = 0.5 * fma(Kx * Ky, frac, -k1 * k2c * ifrac);
+            {
+                // the mirror-zero form (see beam_bin_mixed)
+                const double dk3 = fma(RR[6], u.ux, fma(RR[7], u.uy, fma(RR[8], u.uz, Kz)));
+                const double u2 = -q2 * (k2 + Ky);
+                const double w2 = fma(Kx, -q2, -q1 * k2);
+                const double dan = 0.5 * rs * fma(Kz * sig, u2, -isig * dk3);
+                const double dbn = -0.5 * rs * fma(Kx * Ky * sig, u2, isig * w2);
+                const bool mir = !kclamp && s2 > 0.5;
+                da = mir ? dan : da;
+                db = mir ? dbn : db;
+            }
+            const double m1 = -k1 * k2c * rs, m2 = sq, m3 = -k2c * k3 * rs;
+            const double r13 = kclamp ? rsq64_3(s2) : rs;
+            const double ev1 = -k3 * r13, ev3 = k1 * r13;
+            double hx = u.uy, hy = -u.ux;
+            if (fwd) {
+                hx = yt - r[R_COM + 1];
+                hy = -(xt - r[R_COM]);
+            }
+            const double rh = rsq64_3(fma(hx, hx, hy * hy));
+            hx *= rh;
+            hy *= rh;
+            const double h1 = fma(RR[0], hx, RR[1] * hy);
+            const double h2 = fma(RR[3], hx, RR[4] * hy);
+            const double h3 = fma(RR[6], hx, RR[7] * hy);
+            const double pm = fma(h1, m1, fma(h2, m2, h3 * m3));
+            const double qh = fma(h1, ev1, h3 * ev3);
+            gg = fma(pm, da, qh * db);
+            hh = fma(pm, db, -qh * da);
+        }
+    }
+    add_projectors(r, FR, FI, gg, hh, acc);
+}
+
+// One beam, one bin from the bin's plain inputs (bi.rad = |x| is read); etab: the table, then
+// fp64r_constants.
 __host__ __device__ __forceinline__ void beam_bin_fp64r(const double* __restrict__ r,
                                                         const double* __restrict__ vrecs,
                                                         const DevGrid& g, const BinIn& bi,
                                                         const double* __restrict__ etab,
                                                         int fast_diff, double acc[8])
 {
-    // ---- geometry: bin direction from the aperture centre; the far-field phase relative to
-    // the bin's own, k (|x - c| - |x|) = k (|c|^2 - 2 x.c) / (|x - c| + |x|), formed without
-    // cancellation (~1e-13 rad; the per-bin e^{i k |x|} is applied after the beam sum) ----
-    const double dx = bi.x - r[R_COM], dy = bi.y - r[R_COM + 1], dz = bi.z - r[R_COM + 2];
-    const double s = fma(dx, dx, fma(dy, dy, dz * dz));
-    const double invd = rsq64_1(s);
-    const double ux = dx * invd, uy = dy * invd, uz = dz * invd;
-    if (fast_diff) {
-        if (ux * r[R_PROP0] + uy * r[R_PROP0 + 1] + uz * r[R_PROP0 + 2] < r[R_COSFOV]) return;
-    }
-    const double* K = r + R_KRR;
-    const double qx = fma(-K[0], ux, fma(-K[1], uy, fma(-K[2], uz, r[R_KP2])));
-    const double qy = fma(-K[3], ux, fma(-K[4], uy, fma(-K[5], uz, r[R_KP2 + 1])));
-    const double k1r = r[R_KP2] - qx, k2r = r[R_KP2 + 1] - qy;
-    const double rc = fma(bi.x, r[R_COM], fma(bi.y, r[R_COM + 1], bi.z * r[R_COM + 2]));
-    const double kd = etab[ETAB_KREV] * (fma(-2.0, rc, r[R_CC]) * rcp64_1(fma(s, invd, bi.rad)));   // revolutions
-    const double q2 = fma(qx, qx, qy * qy);
-    const double lam = etab[ETAB_LAMBDA];
-
-    // ---- aperture integral with the far-field phase: (FR, FI) = e^{i k|r-com|} sum_ref / lambda ----
-    double FR, FI;
-    const double* rf_ = r;   // vertex coordinates of triangles are inline
-    const bool tri = r[R_NV] == 3.0;
-    const double qa2 = (double)reinterpret_cast<const float*>(r + R_F32)[F_QA2];
-    if (q2 * qa2 < (double)SERIES_QA2) {
-        const double tw = 6.283185307179586;
-        double sr = 0.0, si = 0.0;
-        if (tri) {
-            const double a = tw * fma(qx, rf_[R_EX], qy * rf_[R_EY]);
-            const double b = tw * fma(qx, rf_[R_EX + 1], qy * rf_[R_EY + 1]);
-            const double c = tw * fma(qx, rf_[R_EX + 2], qy * rf_[R_EY + 2]);
-            double tr, ti;
-            tri_series(a, b, c, &tr, &ti);
-            sr = r[R_AREA] * tr;
-            si = r[R_AREA] * ti;
-        } else {
-            const int nv = (int)r[R_NV];
-            const double* vr = vrecs + (int64_t)r[R_VOFF] * VREC;
-            for (int j = 0; j < nv; j++) {
-                const int jp = (j == nv - 1) ? 0 : j + 1;
-                const double xj = vr[VREC * j + V_X], yj = vr[VREC * j + V_Y];
-                const double xn = vr[VREC * jp + V_X], yn = vr[VREC * jp + V_Y];
-                const double a = tw * fma(qx, xj, qy * yj);
-                const double b = tw * fma(qx, xn, qy * yn);
-                const double sa = 0.5 * (xj * yn - xn * yj);
-                double tr, ti;
-                tri_series(0.0, a, b, &tr, &ti);
-                sr += sa * tr;
-                si += sa * ti;
-            }
-        }
-        // sum_ref = -i F = si - i sr
-        double cb, sb;
-        expi_pi64(2.0 * kd, etab, &cb, &sb);
-        const double il = rcp64(lam);
-        FR = (cb * si + sb * sr) * il;
-        FI = (sb * si - cb * sr) * il;
-    } else {
-        double ssr = 0.0, ssi = 0.0;
-        bool edges = true;
-        if (tri) {
-            double t[3], Wr[3], Wi[3];
-#pragma unroll
-            for (int l = 0; l < 3; l++) {
-                t[l] = fma(qx, r[R_EX + l], fma(qy, r[R_EY + l], kd));
-                expi_2pi64(t[l], etab, &Wr[l], &Wi[l]);
-            }
-            // One denominator: the form factor of a triangle is 2 A times the second divided
-            // difference of e^{i alpha} at its vertex phases alpha_l = 2 pi t_l, divided by i^2,
-            //   F = 2 A (W0 d1 + W1 d2 + W2 d0) / ((2 pi)^2 d0 d1 d2),  d_j = t_{j+1} - t_j,
-            // and sum_ref / lambda = -i F / lambda.  Its rounding is that of the edge sum while
-            // every |d_j| >= 1e-3 (relative to the largest edge term, ~ulp / min |d_j|); below,
-            // the edge sum with its product form.
-            const double d0 = t[1] - t[0], d1 = t[2] - t[1], d2 = t[0] - t[2];
-            if (fmin(fabs(d0), fmin(fabs(d1), fabs(d2))) >= 1e-3) {
-                const double nr = fma(Wr[0], d1, fma(Wr[1], d2, Wr[2] * d0));
-                const double ni = fma(Wi[0], d1, fma(Wi[1], d2, Wi[2] * d0));
-                const double f = r[R_AREA] * etab[ETAB_TRI_SCALE] * rcp64_1(d0 * d1 * d2);
-                FR = f * ni;
-                FI = -f * nr;
-                edges = false;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 3; j++) {
-                    const int jn = j == 2 ? 0 : j + 1;
-                    edge_diff64(Wr[j], Wi[j], Wr[jn], Wi[jn], t[jn] - t[j], qx, qy, r[R_EDX + j], r[R_EDY + j],
-                                ssr, ssi);
-                }
-            }
-        } else {
-            const int nv = (int)r[R_NV];
-            const double* vr = vrecs + (int64_t)r[R_VOFF] * VREC;
-            const double t0 = fma(qx, vr[V_X], fma(qy, vr[V_Y], kd));
-            double Wr0, Wi0;
-            expi_2pi64(t0, etab, &Wr0, &Wi0);
-            double tp = t0, Wrp = Wr0, Wip = Wi0;
-            for (int j = 0; j < nv; j++) {
-                double tn = t0, Wrn = Wr0, Win = Wi0;
-                if (j < nv - 1) {
-                    tn = fma(qx, vr[VREC * (j + 1) + V_X], fma(qy, vr[VREC * (j + 1) + V_Y], kd));
-                    expi_2pi64(tn, etab, &Wrn, &Win);
-                }
-                edge_diff64(Wrp, Wip, Wrn, Win, tn - tp, qx, qy, vr[VREC * j + V_DX], vr[VREC * j + V_DY], ssr, ssi);
-                tp = tn;
-                Wrp = Wrn;
-                Wip = Win;
-            }
-        }
-        if (edges) {
-            const double sc = -rcp64_1(6.283185307179586 * lam * q2);
-            FR = ssr * sc;
-            FI = ssi * sc;
-        }
-    }
-
-    // ---- polarisation (karczewski + rot4, diff_mod.f90:124-198, 630-643) ----
-    const bool kclamp = fabs(k2r) > etab[ETAB_K2CLAMP];
-    const bool fwd = !(fabs(uz) < FWD_DOT);
-    const double ik = etab[ETAB_INV_KREV];
-    const double k1 = k1r * ik, k2 = k2r * ik;
-    const double* RR = r + R_RR;
-    const double k3 = fma(RR[6], ux, fma(RR[7], uy, RR[8] * uz));
-    const double s2 = fma(k1, k1, k3 * k3);                     // 1 - k_y^2 (unclamped)
-    const double* C = r + R_C64;
-    double gg, hh;
-    if (!kclamp && !fwd) {
-        const double P0 = fma(K[3], uy, -K[4] * ux);
-        const double Q0 = fma(-uz, k2r, K[5]);
-        const double rh = rsq64_1(fma(ux, ux, uy * uy) * (s2 * s2));   // 1 / (|(ux, uy)| s2)
-        const double P = P0 * rh, Q = Q0 * rh;
-        const double A = fma(C[0], s2, C[1] * k3);
-        const double B = fma(C[2], s2, C[1] * (k1 * k2));
-        gg = fma(P, A, Q * B);
-        hh = fma(P, B, -Q * A);
-    } else {
-        const double Kx = r[R_PROP2], Ky = r[R_PROP2 + 1], Kz = r[R_PROP2 + 2];
-        const double sig = r[R_FRAC], isig = r[R_ISIG];
-        const double k2c = kclamp ? copysign(K2CLAMP, k2) : k2;
-        const double s2c = kclamp ? (1.0 - K2CLAMP * K2CLAMP) : s2;
-        const double rs = rsq64(s2c);
-        const double sq = s2c * rs;
-        const double frac = sq * sig;
-        const double ifrac = rs * isig;
-        double da = -0.5 * fma(Kz, frac, k3 * ifrac);
-        double db = 0.5 * fma(Kx * Ky, frac, -k1 * k2c * ifrac);
-        {
-            // the mirror-zero form (see beam_bin_mixed)
-            const double dk1 = -qx * ik, dk2 = -qy * ik;
-            const double dk3 = fma(RR[6], ux, fma(RR[7], uy, fma(RR[8], uz, Kz)));
-            const double u2 = dk2 * (k2 + Ky);
-            const double w2 = fma(Kx, dk2, dk1 * k2);
-            const double dan = 0.5 * rs * fma(Kz * sig, u2, -isig * dk3);
-            const double dbn = -0.5 * rs * fma(Kx * Ky * sig, u2, isig * w2);
-            const bool mir = !kclamp && s2 > 0.5;
-            da = mir ? dan : da;
-            db = mir ? dbn : db;
-        }
-        const double m1 = -k1 * k2c * rs, m2 = sq, m3 = -k2c * k3 * rs;
-        const double r13 = kclamp ? rsq64(s2) : rs;
-        const double ev1 = -k3 * r13, ev3 = k1 * r13;
-        double hx = uy, hy = -ux;
-        if (fwd) {
-            hx = bi.yt - r[R_COM + 1];
-            hy = -(bi.xt - r[R_COM]);
-        }
-        const double rh = rsq64(fma(hx, hx, hy * hy));
-        hx *= rh;
-        hy *= rh;
-        const double h1 = fma(RR[0], hx, RR[1] * hy);
-        const double h2 = fma(RR[3], hx, RR[4] * hy);
-        const double h3 = fma(RR[6], hx, RR[7] * hy);
-        const double p = fma(h1, m1, fma(h2, m2, h3 * m3));
-        const double qh = fma(h1, ev1, h3 * ev3);
-        gg = fma(p, da, qh * db);
-        hh = fma(p, db, -qh * da);
-    }
-    // f (gg I + hh J) A = w P A + w' Q A, w = f (gg + i hh), w' = f (gg - i hh)
-    const double ta = FR * gg, tb = FI * hh, tc = FR * hh, td = FI * gg;
-    const double wr = ta - tb, wi = tc + td, vr_ = ta + tb, vi = td - tc;
-    const double* rp = r + R_RP64;
-    const double* rm = r + R_RM64;
-    acc[0] = fma(wr, rp[0], fma(-wi, rp[1], acc[0]));
-    acc[1] = fma(wr, rp[1], fma(wi, rp[0], acc[1]));
-    acc[2] = fma(wr, rp[2], fma(-wi, rp[3], acc[2]));
-    acc[3] = fma(wr, rp[3], fma(wi, rp[2], acc[3]));
-    acc[4] = fma(vr_, rm[0], fma(-vi, rm[1], acc[4]));
-    acc[5] = fma(vr_, rm[1], fma(vi, rm[0], acc[5]));
-    acc[6] = fma(vr_, rm[2], fma(-vi, rm[3], acc[6]));
-    acc[7] = fma(vr_, rm[3], fma(vi, rm[2], acc[7]));
+    (void)g;
+    beam_bin_fp64r_far(r, vrecs, far_bin(bi), bi.xt, bi.yt, etab, etab[ETAB_CC_FAR], fast_diff, acc);
 }
 
 // Beams per FP32 partial sum of the mixed kernels: every MIXED_GROUP consecutive beams

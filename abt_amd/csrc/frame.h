@@ -128,7 +128,9 @@ __host__ __device__ inline void make_beam_record(const double* ampl, const doubl
     rec[R_VOFF] = (double)voff;
     double waveno = 2.0 * PI_R4 / lambda;
     double krev = waveno / 6.283185307179586476925;
-    for (int r = 0; r < 3; r++) rec[R_KPROP + r] = prop0[r] * krev;
+    rec[R_KREV] = krev;
+    rec[R_KT] = (2.0 * ETAB_N) * krev;
+    rec[R_IL] = 1.0 / lambda;
     rec[R_CC] = com[0] * com[0] + com[1] * com[1] + com[2] * com[2];
     rec[R_KY1] = 1.0 - prop2[1] * prop2[1];
     rec[R_FRAC] = 1.0 / sqrt(rec[R_KY1]);
@@ -198,18 +200,22 @@ __host__ __device__ inline void make_beam_record(const double* ampl, const doubl
     rec[R_RP64 + 2] = 0.5 * (A[4] + A[7]); rec[R_RP64 + 3] = 0.5 * (A[5] - A[6]);
     rec[R_RM64 + 0] = 0.5 * (A[0] - A[3]); rec[R_RM64 + 1] = 0.5 * (A[1] + A[2]);
     rec[R_RM64 + 2] = 0.5 * (A[4] - A[7]); rec[R_RM64 + 3] = 0.5 * (A[5] + A[6]);
-    // Karczewski coefficients over krev (the krev-scaled polarisation of the restructured bodies)
+    // Karczewski coefficients; over krev for the krev-scaled polarisation of the mixed body
     const double isig = sqrt(rec[R_KY1]);
-    rec[R_C64 + 0] = -0.5 * prop2[2] * rec[R_FRAC] / krev;
-    rec[R_C64 + 1] = -0.5 * isig / krev;
-    rec[R_C64 + 2] = 0.5 * prop2[0] * prop2[1] * rec[R_FRAC] / krev;
-    rec[R_C64P + 0] = -0.5 * prop2[2] * rec[R_FRAC];
-    rec[R_C64P + 1] = -0.5 * isig;
-    rec[R_C64P + 2] = 0.5 * prop2[0] * prop2[1] * rec[R_FRAC];
+    rec[R_C64 + 0] = -0.5 * prop2[2] * rec[R_FRAC];
+    rec[R_C64 + 1] = -0.5 * isig;
+    rec[R_C64 + 2] = 0.5 * prop2[0] * prop2[1] * rec[R_FRAC];
     rec[R_ISIG] = isig;
-    rg[G_C1] = (float)rec[R_C64 + 0];
-    rg[G_C2] = (float)rec[R_C64 + 1];
-    rg[G_C3] = (float)rec[R_C64 + 2];
+    const double tu = 2.0 * ETAB_N;   // table steps per turn
+    rec[R_TA] = rec[R_AREA] * (tu * tu / (2.0 * 9.869604401089358 * lambda));
+    rec[R_SA2] = (waveno * amax) * (waveno * amax);
+    for (int j = 0; j < 3; j++) {
+        rec[R_TX + j] = tu * krev * rec[R_EX + j];
+        rec[R_TY + j] = tu * krev * rec[R_EY + j];
+    }
+    rg[G_C1] = (float)(rec[R_C64 + 0] / krev);
+    rg[G_C2] = (float)(rec[R_C64 + 1] / krev);
+    rg[G_C3] = (float)(rec[R_C64 + 2] / krev);
     float* rf = reinterpret_cast<float*>(rec + R_F32);
     for (int i = 0; i < 3; i++)
         for (int j = 0; j < 3; j++) rf[F_RR + 3 * i + j] = (float)rr.a[i][j];

@@ -21,7 +21,9 @@ enum : int {
     R_COSFOV = 29,  // cos(fov)
     R_NV = 30,      // number of vertices
     R_VOFF = 31,    // first vertex record of this beam (apertures with nv > 3)
-    R_KPROP = 32,   // [3] prop0 * k / (2 pi)   (revolutions per um)
+    R_KREV = 32,    // krev = k / (2 pi), revolutions per um
+    R_KT = 33,      // 2 ETAB_N krev: exponential-table steps per um
+    R_IL = 34,      // 1 / lambda
     R_CC = 35,      // |com|^2
     R_AMAX = 36,    // max_j |v20_j|, aperture radius about com
     R_AREA = 37,    // signed aperture area in the aperture frame (negative: clockwise)
@@ -44,11 +46,14 @@ enum : int {
     // FP64 copies of the mixed kernel's per-beam constants, for the restructured FP64 body
     R_RP64 = 96,    // [4] r+ = (A(1,:) - i A(2,:)) / 2: re/im of columns 1, 2
     R_RM64 = 100,   // [4] r- = (A(1,:) + i A(2,:)) / 2
-    R_C64 = 104,    // [3] the Karczewski coefficients G_C1, G_C2, G_C3 in FP64
+    R_C64 = 104,    // [3] the Karczewski coefficients -K_z / (2 S), -S / 2, K_x K_y / (2 S), S = sqrt(1 - K_y^2)
     R_ISIG = 107,   // sqrt(1 - prop2_y^2)
-    // Karczewski coefficients of the plain FP64 body (R_C64 without the krev scaling)
-    R_C64P = 108,   // [3]
-    REC = 112       // padded to a multiple of 4 doubles (32 bytes)
+    // the restructured FP64 body in units of the exponential table's steps (1 / (2 ETAB_N) turns)
+    R_TA = 108,     // signed area (2 ETAB_N)^2 / (2 pi^2 lambda)
+    R_SA2 = 109,    // (k a)^2: series branch when |prop2 - k|^2 (k a)^2 is small
+    R_TX = 110,     // [3] 2 ETAB_N krev x_j
+    R_TY = 113,     // [3] 2 ETAB_N krev y_j
+    REC = 116       // padded to a multiple of 4 doubles (32 bytes)
 };
 
 // float offsets inside the FP32 block of a beam record
@@ -89,8 +94,7 @@ struct DevGrid {
     double krev_k2clamp;                    // krev * K2CLAMP (mixed kernel's k_y clamp test)
     float inv_lambda_f;                     // 1/lambda (FP32 body of the mixed kernel)
     float inv_krev_f;                       // 1/krev
-    double inv_krev;                        // 1/krev (restructured FP64 body)
-    double tri_scale;                       // 1 / (2 pi^2 lambda) (its triangle form factor)
+    double cc_far;                          // largest |com|^2 of the far geometry (restructured FP64 body)
     double inv_lambda;                      // 1 / lambda (plain FP64 body)
     double inv_waveno;                      // 1 / waveno
     const double* x;                        // [nbins] far-field bin positions
@@ -113,9 +117,9 @@ constexpr int ETAB_N = 512;
 constexpr int ETAB_DOUBLES = 2 * (2 * ETAB_N);
 constexpr int ETAB_LO = ETAB_DOUBLES;       // offset of the low parts
 constexpr int ETAB_GRID = 2 * ETAB_DOUBLES;  // doubles of DevGrid::etab, and the plain body's LDS block
-// The FP64r body's LDS block: the table, then its grid constants (fp64r_constants).
-constexpr int ETAB_KREV = ETAB_DOUBLES, ETAB_K2CLAMP = ETAB_DOUBLES + 1, ETAB_INV_KREV = ETAB_DOUBLES + 2,
-              ETAB_TRI_SCALE = ETAB_DOUBLES + 3, ETAB_LAMBDA = ETAB_DOUBLES + 4, ETAB_LDS = ETAB_DOUBLES + 5;
+// The FP64r body's LDS block: the table's high parts, then the grid's far limit (fp64r_constants).
+constexpr int ETAB_CC_FAR = ETAB_DOUBLES, ETAB_LDS = ETAB_DOUBLES + 1;
+constexpr double BIN_RADIUS = 1e6;   // of make_far_field_bins (diff_mod.f90:846-852)
 
 // REAL*4 literals of the reference, widened to double
 constexpr double PI_R4 = 3.1415927410125732;
@@ -126,6 +130,15 @@ constexpr double ANTI_THR = 9.999999747378752e-05;
 
 // The wavelength-derived constants of a grid: waveno = 2 pi_r4 / lambda (diff_mod.f90:332,
 // with the REAL*4 pi) and the scaled forms the kernel bodies read.
+// The far geometry of the restructured FP64 body holds for centres within h = |com| / |x| of the
+// origin: its series for the distance |x - com| are cut after h^4 (phase, in turns: 7/8 krev |x| h^5 below
+// 2e-13) and h^3 (direction: 35/8 h^4 below 2e-15).
+inline double far_limit(double krev, double rad)
+{
+    const double a = __builtin_pow(2e-13 / (krev * rad), 0.2), h = a < 1.4e-4 ? a : 1.4e-4;
+    return h * rad * (h * rad);
+}
+
 inline void devgrid_constants(DevGrid& g, double lambda)
 {
     g.lambda = lambda;
@@ -134,8 +147,7 @@ inline void devgrid_constants(DevGrid& g, double lambda)
     g.krev_k2clamp = g.krev * K2CLAMP;
     g.inv_lambda_f = (float)(1.0 / lambda);
     g.inv_krev_f = (float)(1.0 / g.krev);
-    g.inv_krev = 1.0 / g.krev;
-    g.tri_scale = 1.0 / (2.0 * 9.869604401089358 * lambda);
+    g.cc_far = far_limit(g.krev, BIN_RADIUS);
     g.inv_lambda = 1.0 / lambda;
     g.inv_waveno = 1.0 / g.waveno;
 }

@@ -290,6 +290,7 @@ static int grid_build(int64_t nth, const double* th, int64_t nph, const double* 
     g->d.nbins = (int32_t)nb;
     g->d.theta_i = theta_i_of(nth, th);
     abt::devgrid_constants(g->d, lambda);
+    if (xs) g->d.cc_far = abt::far_limit(krev, *std::min_element(rad, rad + nb));   // the caller's bins
     g->d.x = d;
     g->d.y = d + nb;
     g->d.z = d + 2 * nb;
