@@ -25,8 +25,9 @@ constexpr size_t PART_BYTES = (size_t)2 << 30;
 // Segment length.  The last round of workgroups idles about half a segment, 0.5 x 256 bins x len / (rate
 // / 1024 slots) seconds; the segment sums cost 128 bytes per bin and segment, total / len of them, at
 // ~3 TB/s.  The two are equal at len = sqrt(total x nbins x 4e-5) for ~1.2e11 beam.bins/s (the bodies run at
-// 0.6e11 to 2.3e11; a factor of two either way costs under 1 % of a run).
-constexpr double SEG_RULE = 4e-5;
+// 0.7e11 to 2.3e11; a factor of two either way costs under 1 % of a run), and at sqrt(total x nbins x 1.3e-5)
+// for the accurate body's 0.4e11.
+constexpr double SEG_RULE = 4e-5, SEG_RULE_ACCURATE = 1.3e-5;
 // Below 16 beams a segment's start-up (table, bins, first records) weighs as much as its beams: 4
 // orientations x 37 x 36 bins take 88, 87, 93 and 94 us a run with at least 8, 16, 24 and 32.
 constexpr int64_t MIN_SEG = 16, MAX_SEG = 4096;
@@ -118,7 +119,8 @@ void make_segments(abt_batch_plan* p, std::vector<abt::SweepSeg>& segs)
     const int n = p->norient;
     const int64_t nbins = p->g->nbins;
     const double total = (double)(p->boff[n] + p->eoff[n]);
-    int64_t len = std::min(MAX_SEG, std::max(MIN_SEG, round_up((int64_t)sqrt(total * (double)nbins * SEG_RULE), 16)));
+    const double rule = p->prec == ABT_FP64_ACCURATE ? SEG_RULE_ACCURATE : SEG_RULE;
+    int64_t len = std::min(MAX_SEG, std::max(MIN_SEG, round_up((int64_t)sqrt(total * (double)nbins * rule), 16)));
     // an orientation's segments fit the buffer and one launch
     const int64_t most = std::max<int64_t>(2, std::min<int64_t>(65535, (int64_t)(PART_BYTES / (64 * (size_t)nbins))));
     int64_t largest = 1;
