@@ -34,6 +34,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "ffbody.h"
 #include "records.h"
 #include "trig.h"
@@ -56,6 +58,12 @@ struct AdjBeam {
     double xr[3], yr[3];        // the same over 2 pi (mixed body: phases in revolutions)
     double area;                // |N| / 2
     double qa2;                 // (aperture radius)^2: series branch when |q|^2 qa2 < SERIES_QA^2
+    // FP64 body
+    const double* r;            // the record, for what only rare bins need
+    double tA;                  // 2 area / (lambda EXP_H^2)
+    double Px, Py;              // P.e_x, P.e_y
+    double tx[3], ty[3];        // in-plane coordinates of v_l - c in table steps times 1 / k
+    double U[4], V[4];          // sigma * ampl in the eigenvectors of g I + h J: C1 + i C2, C1 - i C2 by column
     // FP32 copies for the mixed-precision body
     float fex[3], fey[3], fez[3], fP[3], fKz, fC[8];
     float fxl[3], fyl[3];
@@ -85,8 +93,23 @@ __host__ __device__ inline void adj_beam_from_record(const double* __restrict__ 
     }
     B.cc = r[R_CC];
     B.Kz = B.P[0] * B.ez[0] + B.P[1] * B.ez[1] + B.P[2] * B.ez[2];
+    B.Px = B.P[0] * B.ex[0] + B.P[1] * B.ex[1] + B.P[2] * B.ex[2];
+    B.Py = B.P[0] * B.ey[0] + B.P[1] * B.ey[1] + B.P[2] * B.ey[2];
     for (int q = 0; q < 8; q++) B.C[q] = r[R_AMPL + q];
+    for (int c = 0; c < 2; c++) {
+        const double* C = B.C + 4 * c;
+        B.U[2 * c] = C[0] - C[3];
+        B.U[2 * c + 1] = C[1] + C[2];
+        B.V[2 * c] = C[0] + C[3];
+        B.V[2 * c + 1] = C[1] - C[2];
+    }
     B.area = fabs(r[R_AREA]);
+    B.r = r;
+    B.tA = 2.0 * B.area * r[R_IL] / (EXP_H * EXP_H);
+    for (int i = 0; i < 3; i++) {
+        B.tx[i] = r[R_TX + i];
+        B.ty[i] = r[R_TY + i];
+    }
     B.qa2 = r[R_AMAX] * r[R_AMAX];
     for (int i = 0; i < 3; i++) {
         B.fex[i] = (float)B.ex[i];
@@ -144,7 +167,7 @@ __host__ __device__ inline void adj_zero(AdjAcc& a)
     }
 }
 
-// sin(x)/x and its derivative
+// sin(x)/x
 __host__ __device__ __forceinline__ double sinc64(double x)
 {
     const double z = x * x;
@@ -155,96 +178,70 @@ __host__ __device__ __forceinline__ double sinc64(double x)
     return s / x;
 }
 
-__host__ __device__ __forceinline__ double dsinc64(double x)
+// F(q) and grad_q F of the triangle (in-plane coordinates xl, yl about the centre, either
+// orientation) by the series about q = (qx, qy) = 0 (rad/um), for |q| a < SERIES_QA: complete
+// homogeneous symmetric polynomials of the vertex phases and their derivatives.
+__host__ __device__ inline void tri_series_grad(const double* __restrict__ xl, const double* __restrict__ yl,
+                                                double area, double qx, double qy, double F[2], double Gx[2],
+                                                double Gy[2])
 {
-    const double z = x * x;
-    if (fabs(x) < 0.5)
-        return x * (-1.0 / 3 + z * (1.0 / 30 + z * (-1.0 / 840 + z * (1.0 / 45360 + z * (-1.0 / 3991680 + z * (1.0 / 518918400))))));
-    double s, c;
-    sincos_f64(x, &s, &c);
-    return (c - s / x) / x;
+    double al[3];
+    for (int l = 0; l < 3; l++) al[l] = qx * xl[l] + qy * yl[l];
+    const double e1 = al[0] + al[1] + al[2];
+    const double e2 = al[0] * al[1] + al[1] * al[2] + al[2] * al[0];
+    const double e3 = al[0] * al[1] * al[2];
+    double hm3 = 0.0, hm2 = 0.0, hm1 = 1.0;          // h_{n-3}, h_{n-2}, h_{n-1} at n = 1
+    double d[3] = {0.0, 0.0, 0.0};                    // h_{n-1}(al_l, al) at n = 0
+    double f[2] = {0.5, 0.0};                         // n = 0 term: h_0 / 2!
+    double g[2][3] = {{0, 0, 0}, {0, 0, 0}};
+    double inv = 0.5, sign = 1.0;
+    // pairs (odd, even) of n: i^n has the sign + - - + by pairs on f[1], f[0]
+    for (int n = 1; n <= 23; n += 2) {
+        for (int h = 0; h < 2; h++) {
+            // d^{(l)}_{n-1} = h_{n-1} + al_l d^{(l)}_{n-2}
+            for (int l = 0; l < 3; l++) d[l] = hm1 + al[l] * d[l];
+            const double hn = e1 * hm1 - e2 * hm2 + e3 * hm3;
+            inv *= rcp_cr((double)(n + h + 2));
+            if (h == 1) sign = -sign;
+            const double t = sign * inv;
+            f[1 - h] += hn * t;
+            for (int l = 0; l < 3; l++) g[1 - h][l] += d[l] * t;
+            hm3 = hm2; hm2 = hm1; hm1 = hn;
+        }
+    }
+    const double A2 = 2.0 * area;
+    for (int c = 0; c < 2; c++) {
+        F[c] = A2 * f[c];
+        Gx[c] = A2 * (g[c][0] * xl[0] + g[c][1] * xl[1] + g[c][2] * xl[2]);
+        Gy[c] = A2 * (g[c][0] * yl[0] + g[c][1] * yl[1] + g[c][2] * yl[2]);
+    }
 }
 
-// F(q) and grad_q F of the triangle (in-plane coordinates xl, yl about the centre,
-// either orientation), q = (qx, qy) rad/um.  Series about q = 0 for |q| a < SERIES_QA
-// (complete homogeneous symmetric polynomials of the vertex phases and their
-// derivatives), else the edge form F = (i/|q|^2) sum_j c_j sinc(q.e_j/2) e^{i q.m_j}.
-__host__ __device__ inline void tri_ff_grad(const AdjBeam& B, double qx, double qy, double F[2],
-                                           double Gx[2], double Gy[2])
+// F(q): the series, or the edge form F = (i/|q|^2) sum_j c_j sinc(q.e_j/2) e^{i q.m_j}.
+__host__ __device__ inline void tri_ff(const AdjBeam& B, double qx, double qy, double F[2])
 {
     const double q2 = qx * qx + qy * qy;
     if (q2 * B.qa2 < 2.25) {
-        double al[3];
-        for (int l = 0; l < 3; l++) al[l] = qx * B.xl[l] + qy * B.yl[l];
-        const double e1 = al[0] + al[1] + al[2];
-        const double e2 = al[0] * al[1] + al[1] * al[2] + al[2] * al[0];
-        const double e3 = al[0] * al[1] * al[2];
-        double hm3 = 0.0, hm2 = 0.0, hm1 = 1.0;          // h_{n-3}, h_{n-2}, h_{n-1} at n = 1
-        double d[3] = {0.0, 0.0, 0.0};                    // h_{n-1}(al_l, al) at n = 0
-        double fr = 0.5, fi = 0.0;                        // n = 0 term: h_0 / 2!
-        double dr[3] = {0, 0, 0}, di[3] = {0, 0, 0};
-        double inv = 0.5;
-        double hprev = 1.0;                               // h_{n-1}
-        for (int n = 1; n <= 24; n++) {
-            // d^{(l)}_{n-1} = h_{n-1} + al_l d^{(l)}_{n-2}
-            for (int l = 0; l < 3; l++) d[l] = hprev + al[l] * d[l];
-            const double hn = e1 * hm1 - e2 * hm2 + e3 * hm3;
-            inv = inv / (double)(n + 2);
-            const double t = hn * inv;
-            // i^n
-            switch (n & 3) {
-                case 0: fr += t; for (int l = 0; l < 3; l++) dr[l] += d[l] * inv; break;
-                case 1: fi += t; for (int l = 0; l < 3; l++) di[l] += d[l] * inv; break;
-                case 2: fr -= t; for (int l = 0; l < 3; l++) dr[l] -= d[l] * inv; break;
-                default: fi -= t; for (int l = 0; l < 3; l++) di[l] -= d[l] * inv; break;
-            }
-            hm3 = hm2; hm2 = hm1; hm1 = hn;
-            hprev = hn;
-        }
-        const double A2 = 2.0 * B.area;
-        F[0] = A2 * fr;
-        F[1] = A2 * fi;
-        Gx[0] = Gx[1] = Gy[0] = Gy[1] = 0.0;
-        for (int l = 0; l < 3; l++) {
-            Gx[0] += A2 * dr[l] * B.xl[l];
-            Gx[1] += A2 * di[l] * B.xl[l];
-            Gy[0] += A2 * dr[l] * B.yl[l];
-            Gy[1] += A2 * di[l] * B.yl[l];
-        }
+        double Gx[2], Gy[2];
+        tri_series_grad(B.xl, B.yl, B.area, qx, qy, F, Gx, Gy);
         return;
     }
-    // orientation of (xl, yl): the edge form below is for counter-clockwise order
+    // orientation of (xl, yl): the edge form is for counter-clockwise order
     const double a2 = (B.xl[1] - B.xl[0]) * (B.yl[2] - B.yl[0]) - (B.xl[2] - B.xl[0]) * (B.yl[1] - B.yl[0]);
     const double so = a2 < 0.0 ? 1.0 : -1.0;
-    double sr = 0, si = 0, gxr = 0, gxi = 0, gyr = 0, gyi = 0;
+    double sr = 0, si = 0;
     for (int j = 0; j < 3; j++) {
         const int jn = j == 2 ? 0 : j + 1;
         const double ex = B.xl[jn] - B.xl[j], ey = B.yl[jn] - B.yl[j];
-        const double mx = 0.5 * (B.xl[j] + B.xl[jn]), my = 0.5 * (B.yl[j] + B.yl[jn]);
-        const double cj = so * (qx * ey - qy * ex);
-        const double K = qx * ex + qy * ey;
-        const double mu = qx * mx + qy * my;
-        const double S = sinc64(0.5 * K), dS = 0.5 * dsinc64(0.5 * K);
         double es, ec;
-        sincos_f64(mu, &es, &ec);
-        const double t = cj * S;
+        sincos_f64(qx * (0.5 * (B.xl[j] + B.xl[jn])) + qy * (0.5 * (B.yl[j] + B.yl[jn])), &es, &ec);
+        const double t = so * (qx * ey - qy * ex) * sinc64(0.5 * (qx * ex + qy * ey));
         sr += t * ec;
         si += t * es;
-        // d/dq of c_j S e^{i mu}: (grad c_j S + c_j dS e) e^{i mu} + i c_j S m e^{i mu}
-        const double ax = so * ey * S + cj * dS * ex, ay = -so * ex * S + cj * dS * ey;
-        gxr += ax * ec - t * mx * es;
-        gxi += ax * es + t * mx * ec;
-        gyr += ay * ec - t * my * es;
-        gyi += ay * es + t * my * ec;
     }
     const double iq2 = 1.0 / q2;
-    // F = i (sr + i si) / q2
     F[0] = -si * iq2;
     F[1] = sr * iq2;
-    Gx[0] = -gxi * iq2 - 2.0 * qx * iq2 * F[0];
-    Gx[1] = gxr * iq2 - 2.0 * qx * iq2 * F[1];
-    Gy[0] = -gyi * iq2 - 2.0 * qy * iq2 * F[0];
-    Gy[1] = gyr * iq2 - 2.0 * qy * iq2 * F[1];
 }
 
 __host__ __device__ __forceinline__ double dot3(const double* a, const double* b)
@@ -259,147 +256,408 @@ __host__ __device__ __forceinline__ void cross3(const double* a, const double* b
     o[2] = a[0] * b[1] - a[1] * b[0];
 }
 
-// One (beam, bin) of the FP64 adjoint.  lam: Lam' = Lam T_phi^T (8 doubles).
-__host__ __device__ inline void adj_bin_fp64(const AdjBeam& B, const AdjBin& bn, const double* __restrict__ lam,
-                                             double waveno, double lambda, AdjAcc& acc)
+// Per-bin inputs of the FP64 body: direction and 1 / |x|, the theta_i bin of the same phi
+// (forward fallback of hc), and k |x| in exponential-table steps, less whole turns.  x: the position.
+struct AdjFarBin {
+    FarBin f;
+    double xt, yt, kr;
+    const double* x;
+};
+
+__host__ __device__ __forceinline__ AdjFarBin adj_far_bin(const AdjBin& b)
 {
-    const double k = waveno;
-    double d[3] = {bn.x - B.c[0], bn.y - B.c[1], bn.z - B.c[2]};
-    const double rho = sqrt(dot3(d, d));
-    const double ir = 1.0 / rho;
-    double kh[3] = {d[0] * ir, d[1] * ir, d[2] * ir};
-    // phase e^{i k rho}: k (rho - |x|) without cancellation, plus k |x| from kr_rev
-    const double rc = bn.x * B.c[0] + bn.y * B.c[1] + bn.z * B.c[2];
-    const double drho = (B.cc - 2.0 * rc) / (rho + bn.rad);
-    const double ph_rev = (bn.kr_rev - rint(bn.kr_rev)) + (k / 6.283185307179586) * drho;
-    double Es, Ec;
-    sincos_f64(6.283185307179586 * (ph_rev - rint(ph_rev)), &Es, &Ec);
-    // q = k (P - khat), in-plane components
-    double q3[3] = {k * (B.P[0] - kh[0]), k * (B.P[1] - kh[1]), k * (B.P[2] - kh[2])};
-    const double qx = dot3(q3, B.ex), qy = dot3(q3, B.ey);
-    double F[2], Gx[2], Gy[2];
-    tri_ff_grad(B, qx, qy, F, Gx, Gy);
-    // polarisation
-    const double k1 = dot3(kh, B.ex), k2 = dot3(kh, B.ey), k3 = dot3(kh, B.ez);
-    const bool clamp = fabs(k2) > K2CLAMP;
-    const double k2c = clamp ? copysign(K2CLAMP, k2) : k2;
-    const double sq = sqrt(1.0 - k2c * k2c);
-    const double s13 = sqrt(1.0 - k2 * k2);
-    const bool fb = !(fabs(kh[2]) < FWD_DOT);       // |inc . khat|, inc = (0,0,-1)
-    double hv[3];
-    if (fb) {
-        hv[0] = bn.yt - B.c[1];
-        hv[1] = -(bn.xt - B.c[0]);
-    } else {
-        hv[0] = kh[1];
-        hv[1] = -kh[0];
+    const double ir = 1.0 / b.rad;
+    return {{b.x * ir, b.y * ir, b.z * ir, ir}, b.xt, b.yt, (2 * ETAB_N) * (b.kr_rev - rint(b.kr_rev)), &b.x};
+}
+
+// Sums of the FP64 body.  GU, GV: the amplitude gradient in the eigenvectors of g I + h J (below);
+// Kzb: dL/dKz, which enters e_z through K_z = P.e_z.
+struct AdjSum {
+    double GU[4], GV[4], S0, Kzb;
+    double Qx[3], Qy[3], cb[3], exb[3], eyb[3], ezb[3];
+};
+
+__host__ __device__ inline void adj_zero_sum(AdjSum& a)
+{
+    for (int q = 0; q < 4; q++) a.GU[q] = a.GV[q] = 0.0;
+    a.S0 = a.Kzb = 0.0;
+    for (int i = 0; i < 3; i++) a.Qx[i] = a.Qy[i] = a.cb[i] = a.exb[i] = a.eyb[i] = a.ezb[i] = 0.0;
+}
+
+// adds the FP64 body's sums to the accumulators that adj_finish reads
+__host__ __device__ inline void adj_add_sum(const AdjBeam& B, const AdjSum& s, AdjAcc& a)
+{
+    for (int c = 0; c < 2; c++) {
+        // G1 = GU + GV, G2 = -i (GU - GV)
+        a.GC[4 * c] += s.GU[2 * c] + s.GV[2 * c];
+        a.GC[4 * c + 1] += s.GU[2 * c + 1] + s.GV[2 * c + 1];
+        a.GC[4 * c + 2] += s.GU[2 * c + 1] - s.GV[2 * c + 1];
+        a.GC[4 * c + 3] += s.GV[2 * c] - s.GU[2 * c];
     }
-    hv[2] = 0.0;
-    const double nh = sqrt(hv[0] * hv[0] + hv[1] * hv[1]);
-    const double hc[3] = {hv[0] / nh, hv[1] / nh, 0.0};
-    double mvec[3], uu[3], evo[3];
-    for (int i = 0; i < 3; i++) mvec[i] = (B.ey[i] - k2c * kh[i]) / sq;
-    cross3(kh, B.ey, uu);
-    for (int i = 0; i < 3; i++) evo[i] = uu[i] / s13;
-    const double p = dot3(hc, mvec), qh = dot3(hc, evo);
-    const double da = -0.5 * (B.Kz * sq + k3 / sq);
-    const double db = -0.5 * k1 * k2c / sq;
-    const double g = p * da + qh * db;
-    const double h = p * db - qh * da;
-    // s = E (i / lambda) F
-    const double il = 1.0 / lambda;
-    const double EFr = Ec * F[0] - Es * F[1], EFi = Ec * F[1] + Es * F[0];
-    const double sr = -EFi * il, si = EFr * il;
-    // z1 = <Lam', C>, z2 = <Lam', J C>  (<X,Y> = sum conj(X) Y); J C rows: (C_2., -C_1.)
-    double z1r = 0, z1i = 0, z2r = 0, z2i = 0;
-    for (int cc = 0; cc < 2; cc++) {
-        const int i1 = 2 * (0 + 2 * cc), i2 = 2 * (1 + 2 * cc);   // (1,c), (2,c)
-        const double l1r = lam[i1], l1i = lam[i1 + 1], l2r = lam[i2], l2i = lam[i2 + 1];
-        const double c1r = B.C[i1], c1i = B.C[i1 + 1], c2r = B.C[i2], c2i = B.C[i2 + 1];
-        z1r += l1r * c1r + l1i * c1i + l2r * c2r + l2i * c2i;
-        z1i += l1r * c1i - l1i * c1r + l2r * c2i - l2i * c2r;
-        // (JC)(1,c) = C(2,c), (JC)(2,c) = -C(1,c)
-        z2r += l1r * c2r + l1i * c2i - (l2r * c1r + l2i * c1i);
-        z2i += l1r * c2i - l1i * c2r - (l2r * c1i - l2i * c1r);
-    }
-    // dL/dC += conj(s) (g Lam' - h J^T... ) : G_C = conj(s) (g I - h J) Lam'
-    // (g I - h J) Lam': row 1 = g L1 - h L2, row 2 = g L2 + h L1
-    for (int cc = 0; cc < 2; cc++) {
-        const int i1 = 2 * (0 + 2 * cc), i2 = 2 * (1 + 2 * cc);
-        const double r1r = g * lam[i1] - h * lam[i2], r1i = g * lam[i1 + 1] - h * lam[i2 + 1];
-        const double r2r = g * lam[i2] + h * lam[i1], r2i = g * lam[i2 + 1] + h * lam[i1 + 1];
-        acc.GC[i1] += sr * r1r + si * r1i;
-        acc.GC[i1 + 1] += sr * r1i - si * r1r;
-        acc.GC[i2] += sr * r2r + si * r2i;
-        acc.GC[i2 + 1] += sr * r2i - si * r2r;
-    }
-    const double gg = sr * z1r - si * z1i;          // Re(s z1)
-    const double gh = sr * z2r - si * z2i;          // Re(s z2)
-    // nu = (g z1 + h z2) E i / lambda
-    const double mur = g * z1r + h * z2r, mui = g * z1i + h * z2i;
-    const double mEr = mur * Ec - mui * Es, mEi = mur * Es + mui * Ec;
-    const double nur = -mEi * il, nui = mEr * il;
-    const double nFr = nur * F[0] - nui * F[1], nFi = nur * F[1] + nui * F[0];
-    const double Rx = nur * Gx[0] - nui * Gx[1];
-    const double Ry = nur * Gy[0] - nui * Gy[1];
-    acc.S0 += nFr;
+    a.S0 += s.S0;
     for (int i = 0; i < 3; i++) {
-        acc.Qx[i] += q3[i] * Rx;
-        acc.Qy[i] += q3[i] * Ry;
+        a.Qx[i] += s.Qx[i];
+        a.Qy[i] += s.Qy[i];
+        a.cb[i] += s.cb[i];
+        a.exb[i] += s.exb[i];
+        a.eyb[i] += s.eyb[i];
+        a.ezb[i] += fma(s.Kzb, B.P[i], s.ezb[i]);
     }
-    // khat adjoint: q = k (P - khat) and the polarisation
-    double kb[3];
-    for (int i = 0; i < 3; i++) kb[i] = -k * (Rx * B.ex[i] + Ry * B.ey[i]);
+}
+
+// Lam' (re/im, Fortran pair order) in the eigenvectors of g I + h J, halved:
+// (L1 + i L2) / 2 of columns 1, 2, then (L1 - i L2) / 2.
+__host__ __device__ __forceinline__ void adj_lam_split(const double* L, double* o)
+{
+    for (int c = 0; c < 2; c++) {
+        const double l1r = 0.5 * L[4 * c], l1i = 0.5 * L[4 * c + 1], l2r = 0.5 * L[4 * c + 2], l2i = 0.5 * L[4 * c + 3];
+        o[2 * c] = l1r - l2i;
+        o[2 * c + 1] = l1i + l2r;
+        o[4 + 2 * c] = l1r + l2i;
+        o[4 + 2 * c + 1] = l1i - l2r;
+    }
+}
+
+// One edge of the form factor from the full vertex exponentials W (far-field phase included) of its
+// ends: D = sinc(K/2) e^{i (alpha_0 + alpha_1)/2} = (W1 - W0) / (i K) and its derivatives by
+// alpha_0 and alpha_1, K = alpha_1 - alpha_0 in rad; series of the product form for |K| < 1.
+__host__ __device__ __forceinline__ void edge_grad64(double W0r, double W0i, double W1r, double W1i, double K,
+                                                     double D[2], double D0[2], double D1[2])
+{
+    const double x = 0.5 * K;
+    if (fabs(x) < 0.5) {
+        const double z = x * x;
+        const double S = 1.0 + z * (-1.0 / 6 + z * (1.0 / 120 + z * (-1.0 / 5040 + z * (1.0 / 362880 + z * (-1.0 / 39916800)))));
+        const double hS = 0.5 * x * (-1.0 / 3 + z * (1.0 / 30 + z * (-1.0 / 840 + z * (1.0 / 45360 + z * (-1.0 / 3991680 + z * (1.0 / 518918400))))));
+        double s, c;
+        sincos_f64(x, &s, &c);
+        const double mr = W0r * c - W0i * s, mi = W0r * s + W0i * c;   // e^{i (alpha_0 + alpha_1)/2}
+        D[0] = S * mr;
+        D[1] = S * mi;
+        D0[0] = -0.5 * D[1] - hS * mr;
+        D0[1] = 0.5 * D[0] - hS * mi;
+        D1[0] = -0.5 * D[1] + hS * mr;
+        D1[1] = 0.5 * D[0] + hS * mi;
+    } else {
+        const double iK = rcp_cr(K);
+        D[0] = (W1i - W0i) * iK;
+        D[1] = (W0r - W1r) * iK;
+        D0[0] = (D[0] - W0r) * iK;
+        D0[1] = (D[1] - W0i) * iK;
+        D1[0] = (W1r - D[0]) * iK;
+        D1[1] = (W1i - D[1]) * iK;
+    }
+}
+
+// F e^{i k |x - c|} / lambda and its derivatives by (q_x, q_y) / k, for the bins where the one
+// denominator of adj_bin_far does not hold: series about q = 0, or the edge form.
+__host__ __device__ inline void tri_ff_grad_other(const double* __restrict__ r, const TriPhase& w, double qx, double qy, double kd,
+                                                  const double* __restrict__ tab, double k, double F[2], double Gx[2],
+                                                  double Gy[2])
+{
+    const double* xl = r + R_EX;
+    const double* yl = r + R_EY;
+    const double il = r[R_IL];
+    double sc = k * il;
+    if (fma(qx, qx, qy * qy) * (r[R_AMAX] * r[R_AMAX]) < 2.25) {
+        double f[2], gx[2], gy[2], c, s;
+        tri_series_grad(xl, yl, fabs(r[R_AREA]), qx, qy, f, gx, gy);
+        expi_step64(kd, tab, &c, &s);
+        F[0] = il * (c * f[0] - s * f[1]);
+        F[1] = il * (c * f[1] + s * f[0]);
+        c *= sc;
+        s *= sc;
+        Gx[0] = c * gx[0] - s * gx[1];
+        Gx[1] = c * gx[1] + s * gx[0];
+        Gy[0] = c * gy[0] - s * gy[1];
+        Gy[1] = c * gy[1] + s * gy[0];
+        return;
+    }
+    // F = (i / |q|^2) sum_j c_j D_j for counter-clockwise order
+    const double a2 = (xl[1] - xl[0]) * (yl[2] - yl[0]) - (xl[2] - xl[0]) * (yl[1] - yl[0]);
+    const double so = a2 < 0.0 ? 1.0 : -1.0;
+    const double K[3] = {EXP_H * w.d0, EXP_H * w.d1, EXP_H * w.d2};
+    double sr = 0, si = 0, gxr = 0, gxi = 0, gyr = 0, gyi = 0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const int jn = j == 2 ? 0 : j + 1;
+        double D[2], D0[2], D1[2];
+        edge_grad64(w.Wr[j], w.Wi[j], w.Wr[jn], w.Wi[jn], K[j], D, D0, D1);
+        const double ex = so * (xl[jn] - xl[j]), ey = so * (yl[jn] - yl[j]);
+        const double cj = qx * ey - qy * ex;
+        sr += cj * D[0];
+        si += cj * D[1];
+        gxr += ey * D[0] + cj * (D0[0] * xl[j] + D1[0] * xl[jn]);
+        gxi += ey * D[1] + cj * (D0[1] * xl[j] + D1[1] * xl[jn]);
+        gyr += -ex * D[0] + cj * (D0[0] * yl[j] + D1[0] * yl[jn]);
+        gyi += -ex * D[1] + cj * (D0[1] * yl[j] + D1[1] * yl[jn]);
+    }
+    const double iq2 = rcp_cr(fma(qx, qx, qy * qy)), tx = 2.0 * qx * iq2, ty = 2.0 * qy * iq2;
+    sc *= iq2;
+    F[0] = -si * iq2 * il;
+    F[1] = sr * iq2 * il;
+    Gx[0] = -gxi * sc - k * tx * F[0];
+    Gx[1] = gxr * sc - k * tx * F[1];
+    Gy[0] = -gyi * sc - k * ty * F[0];
+    Gy[1] = gyr * sc - k * ty * F[1];
+}
+
+// The polarisation numbers g, h of one beam and bin and, for gg = dL/dg and gh = dL/dh, the adjoints
+// of what they are made of: the three k_j, K_z, e_y (less its k_2 part), khat beyond the k_j, and
+// in the forward fallback the centre.
+struct AdjPol {
+    double g, h, k1b, k2b, k3b, Kzb;
+    double eyb[3], kb[3], cb0, cb1;
+};
+
+// Away from the clamp and the forward fallback, hc = unit(inc x khat) is normal to khat, so
+// g = D (P0 A + Q0 B), h = D (P0 B - Q0 A) with D = 1 / (|inc x khat| (1 - k_2^2)), P0 = e_y . (kh_y, -kh_x, 0),
+// Q0 = e_y . ((inc.khat) khat - inc), A = -(K_z (1 - k_2^2) + k_3) / 2, B = -k_1 k_2 / 2.
+// is2 = 1 / s2, s2 = 1 - k_2^2.  The radial part of kb is left out where it is free: only the part of kb
+// normal to khat is used.
+__host__ __device__ __forceinline__ AdjPol adj_pol_fast(const AdjBeam& B, const FarGeom& u, double k1, double k2,
+                                                        double k3, double s2, double is2, double gg, double gh)
+{
+    AdjPol o;
+    const double P0 = fma(B.ey[0], u.uy, -B.ey[1] * u.ux);
+    const double Q0 = fma(-u.uz, k2, B.ey[2]);
+    const double rh = rsq64_3(fma(u.ux, u.ux, u.uy * u.uy));
+    const double D = rh * is2;
+    const double A = -0.5 * fma(B.Kz, s2, k3), Bq = -0.5 * k1 * k2;
+    const double DA = D * A, DB = D * Bq;
+    o.g = fma(P0, DA, Q0 * DB);
+    o.h = fma(P0, DB, -Q0 * DA);
+    const double Pb = fma(gg, DA, gh * DB), Qb = fma(gg, DB, -gh * DA);
+    const double hD = -0.5 * D;
+    const double Ab = hD * fma(gg, P0, -gh * Q0);          // -dL/dA / 2
+    const double Bb = hD * fma(gg, Q0, gh * P0);           // -dL/dB / 2
+    const double w = fma(gg, o.g, gh * o.h);               // D dL/dD
+    const double rw = w * (rh * rh);
+    o.Kzb = s2 * Ab;
+    o.k3b = Ab;
+    o.k1b = k2 * Bb;
+    o.k2b = fma(k2, 2.0 * fma(w, is2, -B.Kz * Ab), fma(k1, Bb, -u.uz * Qb));
+    o.kb[0] = fma(-rw, u.ux, -B.ey[1] * Pb);
+    o.kb[1] = fma(-rw, u.uy, B.ey[0] * Pb);
+    o.kb[2] = -k2 * Qb;
+    o.eyb[0] = u.uy * Pb;
+    o.eyb[1] = -u.ux * Pb;
+    o.eyb[2] = Qb;
+    o.cb0 = o.cb1 = 0.0;
+    return o;
+}
+
+// Within the clamp 1 - k_2^2 is 2e-6 and less, so its rounding (1e-16) shows in p and qh; there it is formed
+// from the position in the plain manner, as the forward model forms it.
+__host__ __device__ inline AdjPol adj_pol_other(const AdjBeam& B, const FarGeom& u, const AdjFarBin& bn, double k1,
+                                                double k2, double k3, bool clamp, bool fb, double gg, double gh)
+{
+    AdjPol o;
+    const double kh[3] = {u.ux, u.uy, u.uz};
+    const double k2c = clamp ? copysign(K2CLAMP, k2) : k2;
+    const double sq = sqrt(1.0 - k2c * k2c), isq = 1.0 / sq;
+    double s13q = fma(k1, k1, k3 * k3);                // 1 - k_2^2
+    if (clamp) {
+        const double d[3] = {bn.x[0] - B.c[0], bn.x[1] - B.c[1], bn.x[2] - B.c[2]};
+        const double ir = 1.0 / sqrt(dot3(d, d));
+        const double w[3] = {d[0] * ir, d[1] * ir, d[2] * ir};
+        const double w2 = dot3(w, B.ey);
+        s13q = 1.0 - w2 * w2;
+    }
+    const double is13 = 1.0 / sqrt(s13q);
+    const double hx = fb ? bn.yt - B.c[1] : kh[1], hy = fb ? B.c[0] - bn.xt : -kh[0];
+    const double inh = 1.0 / sqrt(hx * hx + hy * hy);
+    const double hc[3] = {hx * inh, hy * inh, 0.0};
+    double m[3], e[3], t[3];
+    cross3(kh, B.ey, e);
+    for (int i = 0; i < 3; i++) {
+        m[i] = (B.ey[i] - k2c * kh[i]) * isq;
+        e[i] *= is13;
+    }
+    const double p = dot3(hc, m), qh = dot3(hc, e);
+    const double da = -0.5 * (B.Kz * sq + k3 * isq), db = -0.5 * k1 * k2c * isq;
+    o.g = p * da + qh * db;
+    o.h = p * db - qh * da;
     const double pb = gg * da + gh * db, qb = gg * db - gh * da;
     const double dab = gg * p - gh * qh, dbb = gg * qh + gh * p;
-    const double Kzb = -0.5 * sq * dab;
-    double sqb = -0.5 * (B.Kz - k3 / (sq * sq)) * dab + 0.5 * k1 * k2c / (sq * sq) * dbb;
-    const double k3b = -0.5 * dab / sq;
-    const double k1b = -0.5 * k2c / sq * dbb;
-    double k2cb = -0.5 * k1 / sq * dbb;
-    double hcb[3], mb[3];
-    for (int i = 0; i < 3; i++) {
-        hcb[i] = pb * mvec[i] + qb * evo[i];
-        mb[i] = pb * hc[i];
-    }
-    k2cb += -dot3(mb, kh) / sq;
-    sqb += -dot3(mb, mvec) / sq;
-    double ub[3];
-    for (int i = 0; i < 3; i++) {
-        acc.eyb[i] += mb[i] / sq;
-        kb[i] += -k2c / sq * mb[i];
-        ub[i] = qb * hc[i] / s13;
-    }
-    const double s13b = -qb * dot3(hc, evo) / s13;
-    double t3[3];
-    cross3(B.ey, ub, t3);
-    for (int i = 0; i < 3; i++) kb[i] += t3[i];
-    cross3(ub, kh, t3);
-    for (int i = 0; i < 3; i++) acc.eyb[i] += t3[i];
-    double k2b = -k2 / s13 * s13b;
-    k2cb += -k2c / sq * sqb;
-    if (!clamp) k2b += k2cb;
-    for (int i = 0; i < 3; i++) {
-        kb[i] += k1b * B.ex[i] + k2b * B.ey[i] + k3b * B.ez[i];
-        acc.exb[i] += k1b * kh[i];
-        acc.eyb[i] += k2b * kh[i];
-        acc.ezb[i] += k3b * kh[i] + Kzb * B.P[i];
-    }
+    o.Kzb = -0.5 * sq * dab;
+    o.k3b = -0.5 * dab * isq;
+    o.k1b = -0.5 * k2c * isq * dbb;
+    const double mb[3] = {pb * hc[0], pb * hc[1], 0.0};
+    const double ub[3] = {qb * hc[0] * is13, qb * hc[1] * is13, 0.0};
+    const double sqb = -0.5 * (B.Kz - k3 * isq * isq) * dab + 0.5 * k1 * k2c * isq * isq * dbb - dot3(mb, m) * isq;
+    const double k2cb = -0.5 * k1 * isq * dbb - dot3(mb, kh) * isq - k2c * isq * sqb;
+    o.k2b = k2 * is13 * is13 * qb * qh;
+    if (!clamp) o.k2b += k2cb;
+    cross3(ub, kh, t);
+    for (int i = 0; i < 3; i++) o.eyb[i] = mb[i] * isq + t[i];
+    cross3(B.ey, ub, t);
+    for (int i = 0; i < 3; i++) o.kb[i] = t[i] - k2c * isq * mb[i];
     // hc = hv / |hv|, hv = inc x khat (or inc x (x_t - c)); d/dy (inc x y).hvb = y.(hvb x inc)
-    const double hdot = hcb[0] * hc[0] + hcb[1] * hc[1];
-    const double hvbx = (hcb[0] - hdot * hc[0]) / nh, hvby = (hcb[1] - hdot * hc[1]) / nh;
-    const double tx = -hvby, ty = hvbx;               // hvb x (0,0,-1)
-    if (fb) {
-        acc.cb[0] -= tx;
-        acc.cb[1] -= ty;
+    const double hcb0 = pb * m[0] + qb * e[0], hcb1 = pb * m[1] + qb * e[1];
+    const double hdot = hcb0 * hc[0] + hcb1 * hc[1];
+    const double tx = -(hcb1 - hdot * hc[1]) * inh, ty = (hcb0 - hdot * hc[0]) * inh;   // hvb x (0,0,-1)
+    o.cb0 = fb ? -tx : 0.0;
+    o.cb1 = fb ? -ty : 0.0;
+    o.kb[0] += fb ? 0.0 : tx;
+    o.kb[1] += fb ? 0.0 : ty;
+    return o;
+}
+
+// One denominator for F and its gradient (adj_bin_far), d = d0 d1 d2 in table steps.  The exponentials'
+// rounding (1.7e-16) enters dF / (2 A dalpha) as ~1.7e-16 max |K| / (|K0 K1 K2| min |K|), K_j = EXP_H d_j: at most
+// 1.7e-13 of the 1/6 it has at q = 0 under the condition (min |K| of an edge seen at 100 rad across: 3e-3 rad).
+__host__ __device__ __forceinline__ bool one_denominator_grad(const TriPhase& w, double d)
+{
+    const double a = fabs(w.d0), b = fabs(w.d1), c = fabs(w.d2);
+    // strict: q = 0 has every d_j = 0.  The largest is half the sum, d0 + d1 + d2 = 0.
+    return fabs(d) * fmin(a, fmin(b, c)) > (0.5e-3 / (EXP_H * EXP_H * EXP_H)) * (a + b + c);
+}
+
+// One (beam, bin) of the FP64 adjoint.  lam: Lam' = Lam T_phi^T from adj_lam_split; far: the beam's centre is
+// within the far geometry's limit; tab: the exponential table; kt: its steps per um.
+//
+// Bound by FP64 VALU issue, as the forward body (ffbody.h), whose means it uses: the far geometry in
+// series, phases in table steps, three vertex exponentials W_l = e^{i (alpha_l + k |x - c|)} in place of
+// twelve trigonometric pairs, and, away from the edges' nulls and the clamp,
+//   F = 2 A N / (K0 K1 K2), N = W0 K1 + W1 K2 + W2 K0, K_j = alpha_{j+1} - alpha_j,
+// whose derivatives are taken as real numbers, rho_l = Re(nu dF/dalpha_l): with u + i v = nu f W (f N = F)
+//   rho_0 = u_1 - u_2 - K_1 v_0 - Re(nu F) (1/K_2 - 1/K_0), and cyclic,
+// from which q_x and q_y gather sum_l rho_l x_l, rho_l y_l.  The amplitude side works in the
+// eigenvectors of g I + h J, U = C1 + i C2 (eigenvalue g - i h) and V = C1 - i C2 (g + i h): half the products.
+// 376 instructions a beam and bin where six edge terms, each with its own trigonometry, took 1634: 5 orientations
+// of the rough column (209 blocks of 64 beams) x 16,290 bins 15.2 -> 5.2 ms, 3.3 ms with finer chunks of bins;
+// the issue rate alone is 2.4 ms, the rest the last round of waves and waits that two waves per SIMD leave open.
+__host__ __device__ __forceinline__ void adj_bin_far(const AdjBeam& B, const AdjFarBin& bn,
+                                                     const double* __restrict__ lam, bool far,
+                                                     const double* __restrict__ tab, double k, double kt,
+                                                     AdjSum& acc)
+{
+    const FarGeom u = far_geometry_of(B.c, B.cc, kt, bn.f, far);
+    const double kd = u.kd + bn.kr;
+    const double k1 = fma(u.ux, B.ex[0], fma(u.uy, B.ex[1], u.uz * B.ex[2]));
+    const double k2 = fma(u.ux, B.ey[0], fma(u.uy, B.ey[1], u.uz * B.ey[2]));
+    const double k3 = fma(u.ux, B.ez[0], fma(u.uy, B.ez[1], u.uz * B.ez[2]));
+    const double q1 = B.Px - k1, q2 = B.Py - k2;              // q / k in the aperture plane
+    const TriPhase w = tri_phases_of(B.tx, B.ty, q1, q2, kd, tab);
+    const double d12 = w.d1 * w.d2, d = w.d0 * d12;
+    const bool one = one_denominator_grad(w, d);
+    const bool clamp = fabs(k2) > K2CLAMP, fb = !(fabs(u.uz) < FWD_DOT);
+    const bool fast = !clamp && !fb;
+    const double s2 = fma(k1, k1, k3 * k3);                   // 1 - k_2^2
+    double id, is2;
+    if (one && fast) {
+        const double r = rcp_cr(s2 * d);
+        id = r * s2;
+        is2 = r * d;
     } else {
-        kb[0] += tx;
-        kb[1] += ty;
+        id = rcp_cr(d);
+        is2 = rcp_cr(s2);
+    }
+    // F e^{i k |x - c|} / lambda
+    double F[2], Gx[2], Gy[2];
+    const double f = B.tA * id;
+    if (one) {
+        F[0] = f * fma(w.Wr[0], w.d1, fma(w.Wr[1], w.d2, w.Wr[2] * w.d0));
+        F[1] = f * fma(w.Wi[0], w.d1, fma(w.Wi[1], w.d2, w.Wi[2] * w.d0));
+        Gx[0] = Gx[1] = Gy[0] = Gy[1] = 0.0;
+    } else {
+        tri_ff_grad_other(B.r, w, k * q1, k * q2, kd, tab, k, F, Gx, Gy);
+    }
+    const double sr = -F[1], si = F[0];                       // s = i F
+    // <Lam', U> and <Lam', V> over the columns; z1 = <Lam', C> = zu + zv, z2 = <Lam', J C> = -i (zu - zv)
+    double zur = 0, zui = 0, zvr = 0, zvi = 0;
+#pragma unroll
+    for (int c = 0; c < 4; c += 2) {
+        zur = fma(lam[c], B.U[c], fma(lam[c + 1], B.U[c + 1], zur));
+        zui = fma(lam[c], B.U[c + 1], fma(-lam[c + 1], B.U[c], zui));
+        zvr = fma(lam[4 + c], B.V[c], fma(lam[5 + c], B.V[c + 1], zvr));
+        zvi = fma(lam[4 + c], B.V[c + 1], fma(-lam[5 + c], B.V[c], zvi));
+    }
+    const double z1r = zur + zvr, z1i = zui + zvi, z2r = zui - zvi, z2i = zvr - zur;
+    const double gg = fma(sr, z1r, -si * z1i), gh = fma(sr, z2r, -si * z2i);
+    const AdjPol o = fast ? adj_pol_fast(B, u, k1, k2, k3, s2, is2, gg, gh)
+                          : adj_pol_other(B, u, bn, k1, k2, k3, clamp, fb, gg, gh);
+    // dL/dC = conj(s) (g I - h J) Lam'
+    {
+        const double ur = fma(sr, o.g, si * o.h), ui = fma(si, o.g, -sr * o.h);   // s (g - i h)
+        const double vr = fma(sr, o.g, -si * o.h), vi = fma(si, o.g, sr * o.h);   // s (g + i h)
+#pragma unroll
+        for (int c = 0; c < 4; c += 2) {
+            acc.GU[c] = fma(ur, lam[c], fma(ui, lam[c + 1], acc.GU[c]));
+            acc.GU[c + 1] = fma(ur, lam[c + 1], fma(-ui, lam[c], acc.GU[c + 1]));
+            acc.GV[c] = fma(vr, lam[4 + c], fma(vi, lam[5 + c], acc.GV[c]));
+            acc.GV[c + 1] = fma(vr, lam[5 + c], fma(-vi, lam[4 + c], acc.GV[c + 1]));
+        }
+    }
+    // nu = i (g z1 + h z2): nu F = its part of dL;  Rx = Re(nu dF/d(q_x / k)) = k Re(nu dF/dq_x)
+    const double nur = -fma(o.g, z1i, o.h * z2i), nui = fma(o.g, z1r, o.h * z2r);
+    double S, ph, Rx, Ry;
+    if (one) {
+        const double ar = nur * f, ai = nui * f, br = EXP_H * ar, bi = EXP_H * ai;
+        double U[3], V[3];
+#pragma unroll
+        for (int l = 0; l < 3; l++) {
+            U[l] = fma(ar, w.Wr[l], -ai * w.Wi[l]);
+            V[l] = fma(br, w.Wi[l], bi * w.Wr[l]);
+        }
+        const double V0 = w.d1 * V[0], V1 = w.d2 * V[1], V2 = w.d0 * V[2];
+        S = fma(U[0], w.d1, fma(U[1], w.d2, U[2] * w.d0));
+        ph = (k / EXP_H) * (V0 + V1 + V2);
+        const double Si = S * id;
+        const double S0 = Si * d12, S1 = Si * (w.d2 * w.d0), S2 = Si * (w.d0 * w.d1);   // S / d_j
+        const double r0 = (U[1] - U[2]) - V0 + (S0 - S2);
+        const double r1 = (U[2] - U[0]) - V1 + (S1 - S0);
+        const double r2 = (U[0] - U[1]) - V2 + (S2 - S1);
+        Rx = fma(r0, B.tx[0], fma(r1, B.tx[1], r2 * B.tx[2]));
+        Ry = fma(r0, B.ty[0], fma(r1, B.ty[1], r2 * B.ty[2]));
+    } else {
+        S = fma(nur, F[0], -nui * F[1]);
+        ph = k * fma(nur, F[1], nui * F[0]);
+        Rx = fma(nur, Gx[0], -nui * Gx[1]);
+        Ry = fma(nur, Gy[0], -nui * Gy[1]);
+    }
+    acc.S0 += S;
+    acc.Kzb += o.Kzb;
+    const double kh[3] = {u.ux, u.uy, u.uz};
+    const double b1 = o.k1b - Rx, b2 = o.k2b - Ry;            // q = k (P - khat) and the polarisation
+    double kb[3];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const double qk = B.P[i] - kh[i];
+        acc.Qx[i] = fma(qk, Rx, acc.Qx[i]);
+        acc.Qy[i] = fma(qk, Ry, acc.Qy[i]);
+        kb[i] = fma(b1, B.ex[i], fma(b2, B.ey[i], fma(o.k3b, B.ez[i], o.kb[i])));
+        acc.exb[i] = fma(o.k1b, kh[i], acc.exb[i]);
+        acc.eyb[i] = fma(o.k2b, kh[i], acc.eyb[i] + o.eyb[i]);
+        acc.ezb[i] = fma(o.k3b, kh[i], acc.ezb[i]);
     }
     // khat = d / rho, d = x - c:  dc = -(I - khat khat^T) kb / rho;  phase: k Im(nu F) khat
-    const double kk = dot3(kb, kh);
-    const double ph = k * nFi;
-    for (int i = 0; i < 3; i++) acc.cb[i] += -(kb[i] - kk * kh[i]) * ir + ph * kh[i];
+    const double kk = fma(kb[0], kh[0], fma(kb[1], kh[1], kb[2] * kh[2]));
+    const double t = fma(kk, u.id, ph);
+#pragma unroll
+    for (int i = 0; i < 3; i++) acc.cb[i] = fma(t, kh[i], fma(-kb[i], u.id, acc.cb[i]));
+    acc.cb[0] += o.cb0;
+    acc.cb[1] += o.cb1;
+}
+
+// One (beam, bin) from plain inputs, on the host.  lam: Lam' = Lam T_phi^T (8 doubles).
+inline void adj_bin_fp64(const AdjBeam& B, const AdjBin& bn, const double* __restrict__ lam, double waveno,
+                         double lambda, AdjAcc& acc)
+{
+    static const std::vector<double> tab = [] {
+        std::vector<double> t(ETAB_GRID);
+        fill_exp_table(t.data());
+        return t;
+    }();
+    (void)lambda;
+    double ls[8];
+    adj_lam_split(lam, ls);
+    AdjSum s;
+    adj_zero_sum(s);
+    adj_bin_far(B, adj_far_bin(bn), ls, B.cc <= far_limit(waveno / 6.283185307179586, bn.rad), tab.data(), waveno,
+                B.r[R_KT], s);
+    adj_add_sum(B, s, acc);
 }
 
 // sin(x)/x and its derivative for |x| < 0.5 (FP32 series)
@@ -433,8 +691,8 @@ __host__ __device__ inline void model_bin_fp64(const AdjBeam& B, double x, doubl
     double Es, Ec;
     sincos_f64(k * drho, &Es, &Ec);
     const double q3[3] = {k * (B.P[0] - kh[0]), k * (B.P[1] - kh[1]), k * (B.P[2] - kh[2])};
-    double F[2], Gx[2], Gy[2];
-    tri_ff_grad(B, dot3(q3, B.ex), dot3(q3, B.ey), F, Gx, Gy);
+    double F[2];
+    tri_ff(B, dot3(q3, B.ex), dot3(q3, B.ey), F);
     const double k1 = dot3(kh, B.ex), k2 = dot3(kh, B.ey), k3 = dot3(kh, B.ez);
     const double k2c = fabs(k2) > K2CLAMP ? copysign(K2CLAMP, k2) : k2;
     const double sq = sqrt(1.0 - k2c * k2c), s13 = sqrt(1.0 - k2 * k2);

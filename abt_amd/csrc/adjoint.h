@@ -8,7 +8,9 @@
 
 namespace abt {
 
-// One workgroup's work: up to 64 beams of one tree of one orientation, on one bin chunk.
+constexpr int ADJ_BIN = 12;   // doubles of a bin's row of inputs
+
+// One wavefront's work: up to 64 beams of one tree of one orientation, on one bin chunk.
 struct AdjUnit {
     int64_t start;    // first beam (index into the tree's records)
     int32_t o;        // orientation
@@ -20,18 +22,21 @@ struct AdjUnit {
 struct AdjArgs {
     const double* recs_b;     // prepared records, beam trees of all orientations
     const double* recs_e;     // prepared records, ext trees
-    const double* bins;       // [nbins][8]
+    const double* bins;       // [nbins][ADJ_BIN] AdjFarBin (FP64) or AdjBin (mixed)
+    const double* etab;       // the grid's exponential table
     double* lam;              // [norient][nbins][8]  Lam' = k dL/dX T_phi^T
     const AdjUnit* units;
     double* part;             // [nchunks][nb_total][17] per-beam gradients (vertices 9, ampl 8)
     int64_t nb_beam, nb_total;
     int nbins, nchunks;
     double waveno, lambda;
+    double kt;                // exponential-table steps per um
+    double cc_far;            // the grid's limit of the far geometry
 };
 
 }  // namespace abt
 
-extern "C" int abt_launch_adj_bins(const abt::DevGrid* g, double* bins, hipStream_t st);
+extern "C" int abt_launch_adj_bins(const abt::DevGrid* g, int prec, double* bins, hipStream_t st);
 // Lam' from G = dL/dX (batched-forward amplitude layout), the adjoint kernel (prec 0: FP64,
 // 1: mixed) over nunits units, and the chunk reduction into the four outputs (any may be null).
 extern "C" int abt_launch_adjoint(const abt::AdjArgs* a, int prec, int nunits, const double* G,

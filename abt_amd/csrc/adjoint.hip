@@ -6,8 +6,8 @@
 // orientation o (both trees) then has dL/dA_b = k G_o, and its gradients are sums over
 // bins of per-(beam, bin) terms (adjbody.h).
 //
-// Work decomposition: one lane per beam, 64 lanes per workgroup, all lanes of a
-// workgroup from one orientation and tree, so every lane reads the same bin at the same
+// Work decomposition: one lane per beam, 64 lanes per unit, all lanes of a
+// unit from one orientation and tree, so every lane reads the same bin at the same
 // time: the bin's position and Lam' come through scalar loads and stay in scalar
 // registers, the beam's constants and its 27 accumulators stay in vector registers, and
 // no reduction across lanes is needed.  A unit may cover a chunk of the bins only (when
@@ -22,10 +22,12 @@
 
 namespace abt {
 
-constexpr int AL = 64;   // lanes per workgroup (one wavefront)
+constexpr int AL = 64;   // lanes of a unit (one wavefront)
+constexpr int AW = 4;    // units of a workgroup of the FP64 kernel: they share the exponential table in LDS
 
-// Lam' = k G T_phi^T per (orientation, bin), [o][bin][8] (FP64, or FP32 for the mixed
-// kernel); G in the batched forward's amplitude layout [o][8][nbins].
+// Lam' = k G T_phi^T per (orientation, bin), [o][bin][8]: FP64 in the eigenvectors of g I + h J
+// (adj_lam_split), or FP32 plain for the mixed kernel; G in the batched forward's amplitude layout
+// [o][8][nbins].
 // T_phi = [[-s, -c], [c, -s]] (diff_mod.f90:646-650).
 template <typename T>
 __global__ __launch_bounds__(256) void k_adj_lam(const double* __restrict__ G, const double* __restrict__ cphi,
@@ -42,85 +44,134 @@ __global__ __launch_bounds__(256) void k_adj_lam(const double* __restrict__ G, c
 #pragma unroll
     for (int q = 0; q < 8; q++) L[q] = k * g[(int64_t)q * nbins];
     T* out = lam + i * 8;
+    double P[8];
     // pair (r, col): index 2 (r + 2 col)
 #pragma unroll
     for (int r = 0; r < 2; r++)
 #pragma unroll
         for (int ri = 0; ri < 2; ri++) {
             const double l1 = L[2 * r + ri], l2 = L[2 * (r + 2) + ri];
-            out[2 * r + ri] = (T)(-s * l1 - c * l2);            // Lam'(r,1)
-            out[2 * (r + 2) + ri] = (T)(c * l1 - s * l2);       // Lam'(r,2)
+            P[2 * r + ri] = -s * l1 - c * l2;            // Lam'(r,1)
+            P[2 * (r + 2) + ri] = c * l1 - s * l2;       // Lam'(r,2)
         }
+    if (sizeof(T) == sizeof(double)) adj_lam_split(P, L);
+#pragma unroll
+    for (int q = 0; q < 8; q++) out[q] = sizeof(T) == sizeof(double) ? (T)L[q] : (T)P[q];
 }
 
-// per-bin inputs: x, y, z, x_t, y_t (theta_i bin of the same phi), |x|, k|x|/2pi, 0
+// Per-bin inputs, ADJ_BIN doubles.  Mixed: AdjBin; FP64: AdjFarBin's values, then the position at 8.
+template <int PREC>
 __global__ __launch_bounds__(256) void k_adj_bins(DevGrid g, double* __restrict__ bins)
 {
     const int bin = blockIdx.x * 256 + threadIdx.x;
     if (bin >= g.nbins) return;
     const int bt = bin % g.nphi + g.nphi * g.theta_i;
-    double* o = bins + (int64_t)bin * 8;
-    o[0] = g.x[bin]; o[1] = g.y[bin]; o[2] = g.z[bin];
-    o[3] = g.x[bt]; o[4] = g.y[bt];
-    o[5] = g.rad[bin]; o[6] = g.kr_rev[bin]; o[7] = 0.0;
+    const AdjBin b{g.x[bin], g.y[bin], g.z[bin], g.x[bt], g.y[bt], g.rad[bin], g.kr_rev[bin]};
+    double* o = bins + (int64_t)bin * ADJ_BIN;
+    if (PREC == 0) {
+        const AdjFarBin f = adj_far_bin(b);
+        o[0] = f.f.nx; o[1] = f.f.ny; o[2] = f.f.nz; o[3] = f.f.ir;
+        o[4] = f.xt; o[5] = f.yt; o[6] = f.kr;
+        o[8] = b.x; o[9] = b.y; o[10] = b.z;
+    } else {
+        o[0] = b.x; o[1] = b.y; o[2] = b.z;
+        o[3] = b.xt; o[4] = b.yt;
+        o[5] = b.rad; o[6] = b.kr_rev;
+    }
 }
 
-// two waves per SIMD: the beam's constants and 27 FP64 accumulators live in registers
-template <int PREC>
-__global__ __launch_bounds__(AL, 2) void k_adjoint(AdjArgs a)
+// Bins of a unit's chunk
+__device__ __forceinline__ void chunk_bins(const AdjArgs& a, const AdjUnit& U, int* b0, int* b1)
 {
-    const AdjUnit U = a.units[blockIdx.x];
-    const int lane = threadIdx.x;
-    const bool act = lane < U.count;
-    const int64_t beam = U.start + (act ? lane : 0);
-    const double* recs = U.tree ? a.recs_e : a.recs_b;
-    const double* r = recs + beam * REC;
-    AdjBeam B;
-    adj_beam_from_record(r, B);
-    const bool tri = r[R_NV] == 3.0;
-    AdjAcc acc;
-    adj_zero(acc);
-    const int chunk_bins = (a.nbins + a.nchunks - 1) / a.nchunks;
-    const int b0 = U.chunk * chunk_bins;
-    const int b1 = min(a.nbins, b0 + chunk_bins);
-    if (PREC == 0) {
-        const double* lam = a.lam + (int64_t)U.o * a.nbins * 8;
-        for (int i = b0; i < b1; i++) {
-            const double* bb = a.bins + (int64_t)i * 8;
-            const AdjBin bn{bb[0], bb[1], bb[2], bb[3], bb[4], bb[5], bb[6]};
-            adj_bin_fp64(B, bn, lam + (int64_t)i * 8, a.waveno, a.lambda, acc);
-        }
-    } else {
-        // FP32 partial sums over groups of ADJ_GROUP bins, added into FP64
-        const float* lam = reinterpret_cast<const float*>(a.lam) + (int64_t)U.o * a.nbins * 8;
-        for (int i0 = b0; i0 < b1; i0 += ADJ_GROUP) {
-            AdjAccF af;
-            adj_zero_f(af);
-            const int i1 = min(b1, i0 + ADJ_GROUP);
-            for (int i = i0; i < i1; i++) {
-                const double* bb = a.bins + (int64_t)i * 8;
-                const AdjBin bn{bb[0], bb[1], bb[2], bb[3], bb[4], bb[5], bb[6]};
-                adj_bin_mixed(B, bn, lam + (int64_t)i * 8, a.waveno, a.lambda, af);
-            }
-            adj_add(acc, af);
-        }
-    }
-    if (!act) return;
+    const int n = (a.nbins + a.nchunks - 1) / a.nchunks;
+    *b0 = U.chunk * n;
+    *b1 = min(a.nbins, *b0 + n);
+}
+
+// Per-beam gradients of one lane's sums to its row of the partials, [chunk][tree offset + beam][17].
+__device__ __forceinline__ void store_beam(const AdjArgs& a, const AdjUnit& U, int64_t beam,
+                                           const double* __restrict__ r, const AdjBeam& B, const AdjAcc& acc)
+{
     double gv[9], ga[8];
     adj_finish(B, r + R_V20, r[R_SIGMA], acc, gv, ga);
-    if (!tri) {   // the adjoint covers triangular apertures only
+    if (r[R_NV] != 3.0) {   // the adjoint covers triangular apertures only
 #pragma unroll
         for (int q = 0; q < 9; q++) gv[q] = __builtin_nan("");
 #pragma unroll
         for (int q = 0; q < 8; q++) ga[q] = __builtin_nan("");
     }
-    // [chunk][tree offset + beam][17]
     const int64_t row = (U.tree ? a.nb_beam : 0) + beam;
     double* o = a.part + ((int64_t)U.chunk * a.nb_total + row) * 17;
 #pragma unroll
     for (int q = 0; q < 9; q++) o[q] = gv[q];
 #pragma unroll
     for (int q = 0; q < 8; q++) o[9 + q] = ga[q];
+}
+
+// FP64: AW units per workgroup, one per wave; two waves per SIMD, the beam's constants and sums
+// in registers.
+__global__ __launch_bounds__(AL * AW, 2) void k_adjoint64(AdjArgs a, int nunits)
+{
+    __shared__ double2 tab[ETAB_DOUBLES / 2];
+    for (int i = threadIdx.x; i < ETAB_DOUBLES / 2; i += AL * AW)
+        tab[i] = reinterpret_cast<const double2*>(a.etab)[i];
+    __syncthreads();
+    const int unit = blockIdx.x * AW + __builtin_amdgcn_readfirstlane(threadIdx.x / AL);
+    if (unit >= nunits) return;
+    const AdjUnit U = a.units[unit];
+    const int lane = threadIdx.x % AL;
+    const bool act = lane < U.count;
+    const int64_t beam = U.start + (act ? lane : 0);
+    const double* r = (U.tree ? a.recs_e : a.recs_b) + beam * REC;
+    AdjBeam B;
+    adj_beam_from_record(r, B);
+    const bool far = B.cc <= a.cc_far;
+    AdjSum sum;
+    adj_zero_sum(sum);
+    int b0, b1;
+    chunk_bins(a, U, &b0, &b1);
+    const double* lam = a.lam + (int64_t)U.o * a.nbins * 8;
+    for (int i = b0; i < b1; i++) {
+        const double* bb = a.bins + (int64_t)i * ADJ_BIN;
+        const AdjFarBin bn{{bb[0], bb[1], bb[2], bb[3]}, bb[4], bb[5], bb[6], bb + 8};
+        adj_bin_far(B, bn, lam + (int64_t)i * 8, far, reinterpret_cast<const double*>(tab), a.waveno, a.kt,
+                    sum);
+    }
+    if (!act) return;
+    AdjAcc acc;
+    adj_zero(acc);
+    adj_add_sum(B, sum, acc);
+    store_beam(a, U, beam, r, B, acc);
+}
+
+// Mixed: one unit per workgroup.
+__global__ __launch_bounds__(AL, 2) void k_adjoint_mixed(AdjArgs a)
+{
+    const AdjUnit U = a.units[blockIdx.x];
+    const int lane = threadIdx.x;
+    const bool act = lane < U.count;
+    const int64_t beam = U.start + (act ? lane : 0);
+    const double* r = (U.tree ? a.recs_e : a.recs_b) + beam * REC;
+    AdjBeam B;
+    adj_beam_from_record(r, B);
+    AdjAcc acc;
+    adj_zero(acc);
+    int b0, b1;
+    chunk_bins(a, U, &b0, &b1);
+    // FP32 partial sums over groups of ADJ_GROUP bins, added into FP64
+    const float* lam = reinterpret_cast<const float*>(a.lam) + (int64_t)U.o * a.nbins * 8;
+    for (int i0 = b0; i0 < b1; i0 += ADJ_GROUP) {
+        AdjAccF af;
+        adj_zero_f(af);
+        const int i1 = min(b1, i0 + ADJ_GROUP);
+        for (int i = i0; i < i1; i++) {
+            const double* bb = a.bins + (int64_t)i * ADJ_BIN;
+            const AdjBin bn{bb[0], bb[1], bb[2], bb[3], bb[4], bb[5], bb[6]};
+            adj_bin_mixed(B, bn, lam + (int64_t)i * 8, a.waveno, a.lambda, af);
+        }
+        adj_add(acc, af);
+    }
+    if (act) store_beam(a, U, beam, r, B, acc);
 }
 
 // sum the chunk partials in chunk order and split them into the four outputs
@@ -149,9 +200,13 @@ __global__ __launch_bounds__(256) void k_adj_reduce(const double* __restrict__ p
 
 using namespace abt;
 
-extern "C" int abt_launch_adj_bins(const DevGrid* g, double* bins, hipStream_t st)
+extern "C" int abt_launch_adj_bins(const DevGrid* g, int prec, double* bins, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_adj_bins, dim3((unsigned)((g->nbins + 255) / 256)), dim3(256), 0, st, *g, bins);
+    const dim3 nb((unsigned)((g->nbins + 255) / 256));
+    if (prec == 0)
+        hipLaunchKernelGGL(k_adj_bins<0>, nb, dim3(256), 0, st, *g, bins);
+    else
+        hipLaunchKernelGGL(k_adj_bins<1>, nb, dim3(256), 0, st, *g, bins);
     return (int)hipGetLastError();
 }
 
@@ -168,9 +223,9 @@ extern "C" int abt_launch_adjoint(const AdjArgs* a, int prec, int nunits, const 
                            g->sphi, g->nphi, g->nbins, norient, g->waveno, reinterpret_cast<float*>(a->lam));
     if (nunits > 0) {
         if (prec == 0)
-            hipLaunchKernelGGL(k_adjoint<0>, dim3(nunits), dim3(AL), 0, st, *a);
+            hipLaunchKernelGGL(k_adjoint64, dim3((nunits + AW - 1) / AW), dim3(AL * AW), 0, st, *a, nunits);
         else
-            hipLaunchKernelGGL(k_adjoint<1>, dim3(nunits), dim3(AL), 0, st, *a);
+            hipLaunchKernelGGL(k_adjoint_mixed, dim3(nunits), dim3(AL), 0, st, *a);
     }
     const int64_t n = a->nb_total * 17;
     if (n > 0)

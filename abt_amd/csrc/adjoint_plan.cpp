@@ -13,7 +13,10 @@
 
 namespace {
 constexpr int LANES = 64;
-constexpr int MAX_BIN_CHUNKS = 16;
+// Bin chunks at most.  FP64: 5 orientations of the rough column (209 blocks, 16,290 bins; the whole gradient
+// step) take 9.1, 7.9, 8.7, 7.9 and 7.5 ms with 16, 24, 32, 48 and 63 chunks: what counts is how full the
+// last of 1.6 to 6.4 rounds is.  Mixed: the FP32 groups of bins start with a chunk, and 16 already fill it.
+constexpr int MAX_BIN_CHUNKS64 = 64, MAX_BIN_CHUNKS = 16;
 }  // namespace
 
 struct abt_adjoint_plan {
@@ -57,9 +60,9 @@ int abt_adjoint_plan_create(const abt_dev_grid* g, int32_t norient, const int64_
     int64_t nblocks = 0;
     for (int o = 0; o < norient; o++)
         nblocks += (beam_off[o + 1] - beam_off[o] + LANES - 1) / LANES + (ext_off[o + 1] - ext_off[o] + LANES - 1) / LANES;
-    const int64_t want = (int64_t)cus * 4 * 16;
+    const int64_t want = (int64_t)cus * 4 * 16, most = precision == ABT_MIXED ? MAX_BIN_CHUNKS : MAX_BIN_CHUNKS64;
     int64_t nch = nblocks > 0 ? (want + nblocks - 1) / nblocks : 1;
-    nch = std::max<int64_t>(1, std::min<int64_t>(nch, std::min<int64_t>(MAX_BIN_CHUNKS, std::max<int64_t>(1, g->nbins / 256))));
+    nch = std::max<int64_t>(1, std::min<int64_t>(nch, std::min<int64_t>(most, std::max<int64_t>(1, g->nbins / 256))));
     p->nchunks = (int)nch;
     std::vector<abt::AdjUnit> units;
     units.reserve((size_t)(nblocks * nch));
@@ -81,7 +84,7 @@ int abt_adjoint_plan_create(const abt_dev_grid* g, int32_t norient, const int64_
     const int64_t nbins = g->nbins, nbt = p->nb_beam + p->nb_ext;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
-    const size_t o_bins = take(sizeof(double) * 8 * nbins);
+    const size_t o_bins = take(sizeof(double) * abt::ADJ_BIN * nbins);
     const size_t o_lam = take(sizeof(double) * 8 * nbins * (size_t)norient);
     const size_t o_part = take(sizeof(double) * 17 * (size_t)nbt * p->nchunks);
     const size_t o_units = take(sizeof(abt::AdjUnit) * std::max<size_t>(1, units.size()));
@@ -98,7 +101,7 @@ int abt_adjoint_plan_create(const abt_dev_grid* g, int32_t norient, const int64_
     if (!units.empty())
         e = hipMemcpy(p->units, units.data(), sizeof(abt::AdjUnit) * units.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        int le = abt_launch_adj_bins(&g->d, p->bins, nullptr);
+        int le = abt_launch_adj_bins(&g->d, precision == ABT_MIXED ? 1 : 0, p->bins, nullptr);
         if (le) e = (hipError_t)le;
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
@@ -132,6 +135,9 @@ int abt_adjoint_run(const abt_adjoint_plan* p, const double* dev_recs_beam, cons
     a.recs_b = dev_recs_beam;
     a.recs_e = dev_recs_ext;
     a.bins = p->bins;
+    a.etab = p->g->d.etab;
+    a.kt = 2 * abt::ETAB_N * p->g->d.krev;
+    a.cc_far = p->g->d.cc_far;
     a.lam = p->lam;
     a.units = p->units;
     a.part = p->part;

@@ -965,34 +965,41 @@ __host__ __device__ __forceinline__ FarBin far_bin(const BinIn& bi)
 struct FarGeom {
     double ux, uy, uz;   // direction of the bin from the aperture centre
     double kd;           // k (|x - c| - |x|) in table steps (the bin's own e^{i k |x|} follows the beam sum)
+    double id;           // 1 / |x - c|
 };
-__host__ __device__ __forceinline__ FarGeom far_geometry(const double* __restrict__ r, const FarBin& fb, double cc_far)
+// c: the centre, cc = |c|^2, kt: table steps per um; far: cc is within the far geometry's limit
+__host__ __device__ __forceinline__ FarGeom far_geometry_of(const double* __restrict__ c, double cc, double kt,
+                                                            const FarBin& fb, bool far)
 {
     FarGeom o;
-    const double p = fma(fb.nx, r[R_COM], fma(fb.ny, r[R_COM + 1], fb.nz * r[R_COM + 2]));
-    if (record_less(r[R_CC], cc_far)) {
-        const double t = fma(0.5 * r[R_CC], fb.ir, -p);              // |x| h
+    const double p = fma(fb.nx, c[0], fma(fb.ny, c[1], fb.nz * c[2]));
+    if (far) {
+        const double t = fma(0.5 * cc, fb.ir, -p);                   // |x| h
         const double h = t * fb.ir;
         // |x - c| = |x| sqrt(1 + 2 h): sqrt(1 + 2 h) - 1 = h (1 - h/2 + h^2/2 - 5/8 h^3 + ..),
         // 1 / sqrt(1 + 2 h) = 1 - h + 3/2 h^2 - 5/2 h^3 + ..
-        o.kd = (r[R_KT] * t) * fma(h, fma(h, fma(h, -0.625, 0.5), -0.5), 1.0);
+        o.kd = (kt * t) * fma(h, fma(h, fma(h, -0.625, 0.5), -0.5), 1.0);
         const double gd = fma(h, fma(h, fma(h, -2.5, 1.5), -1.0), 1.0);
-        o.ux = fma(-r[R_COM], fb.ir, fb.nx) * gd;
-        o.uy = fma(-r[R_COM + 1], fb.ir, fb.ny) * gd;
-        o.uz = fma(-r[R_COM + 2], fb.ir, fb.nz) * gd;
+        o.ux = fma(-c[0], fb.ir, fb.nx) * gd;
+        o.uy = fma(-c[1], fb.ir, fb.ny) * gd;
+        o.uz = fma(-c[2], fb.ir, fb.nz) * gd;
+        o.id = fb.ir * gd;
     } else {
         // k (|x - c| - |x|) = k (|c|^2 - 2 x.c) / (|x - c| + |x|), formed without cancellation
         const double rad = rcp_cr(fb.ir);
-        const double dx = fma(fb.nx, rad, -r[R_COM]), dy = fma(fb.ny, rad, -r[R_COM + 1]),
-                     dz = fma(fb.nz, rad, -r[R_COM + 2]);
+        const double dx = fma(fb.nx, rad, -c[0]), dy = fma(fb.ny, rad, -c[1]), dz = fma(fb.nz, rad, -c[2]);
         const double s = fma(dx, dx, fma(dy, dy, dz * dz));
-        const double invd = rsq64_3(s);
-        o.ux = dx * invd;
-        o.uy = dy * invd;
-        o.uz = dz * invd;
-        o.kd = r[R_KT] * (fma(-2.0 * rad, p, r[R_CC]) * rcp_cr(fma(s, invd, rad)));
+        o.id = rsq64_3(s);
+        o.ux = dx * o.id;
+        o.uy = dy * o.id;
+        o.uz = dz * o.id;
+        o.kd = kt * (fma(-2.0 * rad, p, cc) * rcp_cr(fma(s, o.id, rad)));
     }
     return o;
+}
+__host__ __device__ __forceinline__ FarGeom far_geometry(const double* __restrict__ r, const FarBin& fb, double cc_far)
+{
+    return far_geometry_of(r + R_COM, r[R_CC], r[R_KT], fb, record_less(r[R_CC], cc_far));
 }
 
 // Outside the beam's field of view (fast_diff; diff_mod.f90:593-603)
@@ -1005,20 +1012,26 @@ __host__ __device__ __forceinline__ bool far_culled(const double* __restrict__ r
 struct TriPhase {
     double Wr[3], Wi[3], d0, d1, d2;
 };
-__host__ __device__ __forceinline__ TriPhase tri_phases(const double* __restrict__ r, double q1, double q2, double kd,
-                                                        const double* __restrict__ etab)
+__host__ __device__ __forceinline__ TriPhase tri_phases_of(const double* __restrict__ tx, const double* __restrict__ ty,
+                                                           double q1, double q2, double kd,
+                                                           const double* __restrict__ etab)
 {
     TriPhase o;
     double T[3];
 #pragma unroll
     for (int l = 0; l < 3; l++) {
-        T[l] = fma(q1, r[R_TX + l], fma(q2, r[R_TY + l], kd));
+        T[l] = fma(q1, tx[l], fma(q2, ty[l], kd));
         expi_step64(T[l], etab, &o.Wr[l], &o.Wi[l]);
     }
     o.d0 = T[1] - T[0];
     o.d1 = T[2] - T[1];
     o.d2 = T[0] - T[2];
     return o;
+}
+__host__ __device__ __forceinline__ TriPhase tri_phases(const double* __restrict__ r, double q1, double q2, double kd,
+                                                        const double* __restrict__ etab)
+{
+    return tri_phases_of(r + R_TX, r + R_TY, q1, q2, kd, etab);
 }
 
 // One denominator: the form factor of a triangle is 2 A times the second divided difference of
