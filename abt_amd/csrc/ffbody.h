@@ -444,28 +444,6 @@ __host__ __device__ __forceinline__ void beam_bin_mixed(const double* __restrict
 
 constexpr double PI64 = 3.141592653589793;
 
-// reciprocal and reciprocal square root: hardware approximations refined by Newton steps
-__host__ __device__ __forceinline__ double rcp64(double x)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    double y = __builtin_amdgcn_rcp(x);
-    double e = fma(-x, y, 1.0);
-    y = fma(y, e, y);
-    e = fma(-x, y, 1.0);
-    return fma(y, e, y);
-#else
-    return 1.0 / x;
-#endif
-}
-__host__ __device__ __forceinline__ double rsq64(double x)
-{
-    double y = (double)abt_rsqf((float)x);
-    double e = fma(-x * y, y, 1.0);
-    y = fma(0.5 * y, e, y);
-    e = fma(-x * y, y, 1.0);
-    return fma(0.5 * y, e, y);
-}
-
 // Hardware approximations in FP64 (relative error below 2^-24 and 2^-24 on gfx950, measured on 10^9
 // values); one costs as much as the FP32 one with its two conversions.
 __host__ __device__ __forceinline__ double rcp_seed(double x)
@@ -571,26 +549,7 @@ inline void fill_exp_table(double* tab)
 // What a caller keeps after the table for beam_bin_fp64r: the grid's far limit.
 __host__ __device__ __forceinline__ void fp64r_constants(const DevGrid& g, double* c) { c[0] = g.cc_far; }
 
-// e^{i pi t} for an FP64 t (half revolutions): t = 2m + j / ETAB_N + r with |r| <= 1 / (2 ETAB_N)
-// (every step exact), e^{i pi t} = tab[j] e^{i pi r}, the last from its Taylor polynomials
-// (|pi r| <= 3.1e-3: truncation below 2e-18).  tab: the exponential table (in LDS on the device).
-__host__ __device__ __forceinline__ void expi_pi64(double t, const double* __restrict__ tab, double* c, double* s)
-{
-    const double m = rint(0.5 * t);
-    const double u = fma(-2.0, m, t);                       // [-1, 1]
-    const double jf = rint((double)ETAB_N * u);
-    const double r = fma(-1.0 / (double)ETAB_N, jf, u);     // |r| <= 1 / (2 ETAB_N)
-    const int j = (int)jf & (2 * ETAB_N - 1);
-    const double c0 = tab[2 * j], s0 = tab[2 * j + 1];
-    const double y = PI64 * r;
-    const double z = y * y;
-    const double sr = fma(y * z, fma(z, 1.0 / 120.0, -1.0 / 6.0), y);
-    const double cr = fma(z, fma(z, 1.0 / 24.0, -0.5), 1.0);
-    *c = fma(c0, cr, -s0 * sr);
-    *s = fma(s0, cr, c0 * sr);
-}
-
-// e^{2 pi i T / (2 ETAB_N)} for an FP64 T in table steps (|T| < 2^31), from the same table: T = J + r with
+// e^{2 pi i T / (2 ETAB_N)} for an FP64 T in table steps (|T| < 2^31), from the table (in LDS on the device): T = J + r with
 // J = rint(T) and |r| <= 1/2 (exact); the table holds the angle of J at index J mod 2 ETAB_N.  The rest
 // is |y| <= pi / 1024: cos y from its Taylor polynomial (truncation below 2e-18), sin y from the cubic
 // that is best in the largest error, y^5 / 120 replaced by its Chebyshev cubic (1.4e-16; a third

@@ -4,16 +4,12 @@
 // 3.16), phi integration by simpne (get_1d_mueller, outputs_mod.f90:280-329;
 // simpne misc_submod.f90:2392-2531), theta integrals (scattering cross
 // sections, asymmetry parameters, back-scattering) and the optional energy
-// scaling (outputs_mod.f90:146-184).  FP64 throughout, contraction off so the
-// epilogue rounds like the reference.
-//
-// Also the incoherent orientation sum (summation, outputs_mod.f90:407-471):
-// mueller_total += mueller in a fixed order.
+// scaling (outputs_mod.f90:146-184).  FP64 throughout; amplitudes and matrices
+// with contraction off, so that they round like the reference, the integrals as
+// weighted sums in a fixed order.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
-
-#include <mutex>
 
 #include "../../include/abt_diff.h"
 #include "mueller.h"
@@ -25,218 +21,205 @@ namespace abt {
 
 constexpr int MB = 256;
 
-__global__ __launch_bounds__(MB) void k_scale_sum(double* __restrict__ ab, double* __restrict__ ae,
-                                                  double* __restrict__ tot, double fb, double fe,
-                                                  const double* __restrict__ dev_f, int64_t n)
+// a complex amplitude; a caller's array need not be aligned beyond its doubles
+typedef double Pair __attribute__((ext_vector_type(2), aligned(8)));
+
+// One bin's amplitudes: k ampl, divided by the energy scaling factor where there is one (the
+// reference's two steps).
+__device__ __forceinline__ void load_ampl(const Pair* __restrict__ A, int64_t b, int64_t nb, double k,
+                                          const double* __restrict__ f, double s[8])
 {
 #pragma clang fp contract(off)
-    const int64_t i = (int64_t)blockIdx.x * MB + threadIdx.x;
-    if (i >= n) return;
-    double b = ab[i], e = ae[i];
-    if (dev_f) {   // energy scaling: divide by the factors computed on the device
-        b = b / dev_f[0];
-        e = e / dev_f[1];
-    } else {
-        b = b * fb;
-        e = e * fe;
-    }
-    ab[i] = b;
-    ae[i] = e;
-    tot[i] = b + e;
-}
-
-__device__ __forceinline__ void mueller_bin(const double* __restrict__ a, int64_t b, int64_t nb,
-                                            double* __restrict__ M)
-{
-    double s[8], m[16];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        s[2 * q] = a[2 * (b + nb * q)];
-        s[2 * q + 1] = a[2 * (b + nb * q) + 1];
+        const Pair v = A[b + nb * q];
+        s[2 * q] = v.x * k;
+        s[2 * q + 1] = v.y * k;
     }
-    mueller16(s, m);
+    if (f) {
+        const double d = *f;
 #pragma unroll
-    for (int e = 0; e < 16; e++) M[b + nb * e] = m[e];
+        for (int q = 0; q < 8; q++) s[q] = s[q] / d;
+    }
 }
 
-// three amplitude arrays -> three Mueller arrays (any output may be null)
-__global__ __launch_bounds__(MB) void k_mueller3(const double* __restrict__ a0,
-                                                 const double* __restrict__ a1,
-                                                 const double* __restrict__ a2, double* M0,
-                                                 double* M1, double* M2, int64_t nb)
+__device__ __forceinline__ void store_ampl(Pair* __restrict__ A, int64_t b, int64_t nb, const double s[8])
 {
-    const int64_t b = (int64_t)blockIdx.x * MB + threadIdx.x;
-    if (b >= nb) return;
-    if (M0) mueller_bin(a0, b, nb, M0);
-    if (M1) mueller_bin(a1, b, nb, M1);
-    if (M2) mueller_bin(a2, b, nb, M2);
+#pragma unroll
+    for (int q = 0; q < 4; q++) A[b + nb * q] = Pair{s[2 * q], s[2 * q + 1]};
 }
 
-__device__ __forceinline__ double simpne_dev(int n, const double* __restrict__ x,
-                                             const double* __restrict__ y, int64_t stride)
+// Adds N values over a wave by halving: lanes a bit apart keep one half of the values each and pass the
+// other, so 48 values take 24 + 12 + 6 + 3 exchanges and two rounds of 3 instead of six rounds of
+// 48.  v[0 .. N/16) holds the sums of the values at N/2 b0 + N/4 b1 + N/8 b2 + N/16 b3, b the lane's bits.
+template <int N, int BIT>
+__device__ __forceinline__ void wave_sums(double* v, int lane)
 {
-    return simpne_eval(n, x, y, stride);
+    if constexpr (BIT < 4) {
+        const bool up = (lane >> BIT) & 1;
+#pragma unroll
+        for (int i = 0; i < N / 2; i++) {
+            const double keep = up ? v[i + N / 2] : v[i], give = up ? v[i] : v[i + N / 2];
+            v[i] = keep + __shfl_xor(give, 1 << BIT);
+        }
+        wave_sums<N / 2, BIT + 1>(v, lane);
+    } else if constexpr (BIT < 6) {
+#pragma unroll
+        for (int i = 0; i < N; i++) v[i] += __shfl_xor(v[i], 1 << BIT);
+        wave_sums<N, BIT + 1>(v, lane);
+    }
 }
 
-// mueller_1d(theta, e) of up to three matrices: one lane per (matrix, element, theta)
-__global__ __launch_bounds__(MB) void k_phi_integrate(const double* M0, const double* M1,
-                                                      const double* M2, const double* __restrict__ phi,
-                                                      int nphi, int ntheta, double* o0, double* o1,
-                                                      double* o2)
-{
-    const int64_t t = (int64_t)blockIdx.x * MB + threadIdx.x;
-    if (t >= (int64_t)3 * 16 * ntheta) return;
-    const int mat = (int)(t / (16 * ntheta));
-    const int rem = (int)(t - (int64_t)mat * 16 * ntheta);
-    const int e = rem / ntheta, j = rem - e * ntheta;
-    const double* M = mat == 0 ? M0 : (mat == 1 ? M1 : M2);
-    double* o = mat == 0 ? o0 : (mat == 1 ? o1 : o2);
-    if (!M || !o) return;
-    const int64_t nb = (int64_t)nphi * ntheta;
-    o[j + (int64_t)ntheta * e] = simpne_dev(nphi, phi, M + nb * e + (int64_t)nphi * j, 1);
-}
-
-// theta integrals (outputs_mod.f90:133-135, 198-205): the integrands of the three
-// matrices in parallel (one workgroup), then one lane per matrix runs simpne in the
-// reference's order.
-// params: scatt, scatt_beam, scatt_ext, g, g_beam, g_ext, back_scatt, f_beam, f_ext;
-// tmp: 3*ntheta scratch.  pass 0 with scaling: computes the energy scaling
-// factors f = sqrt(scatt_x / energy_x) into params[7..8].
-__global__ __launch_bounds__(MB) void k_theta_params(const double* __restrict__ m0, const double* __restrict__ m1,
-                                                     const double* __restrict__ m2, const double* __restrict__ M0,
-                                                     const double* __restrict__ theta, int ntheta, int nphi,
-                                                     double waveno, int scaling_pass, double ebeam, double eext,
-                                                     double* __restrict__ tmp, double* __restrict__ params)
+// The epilogue of one theta per workgroup, a lane per phi: the scaled amplitudes, the three Mueller
+// matrices (total, beam, ext) and their phi integrals (simpne as weights) in one pass over the bins.
+// Bound by its writes, 512 of 640 bytes a bin.  FULL = false: the phi integrals of S11 of beam and
+// ext alone, for the energy scaling factors; nothing else is written.
+// 721 theta x 180 phi with energy scaling, all kernels of the epilogue: 420 -> 31 us.  Before, eight kernels:
+// amplitudes, matrices and integrals apart (the integrals a lane per theta and element, uncoalesced,
+// 34 us a pass), and the theta integrals as three serial chains of 721 (146 us a pass).
+template <bool FULL>
+__global__ __launch_bounds__(MB) void k_epilogue(DevGrid g, double* __restrict__ ab, double* __restrict__ ae,
+                                                 const double* __restrict__ f, double* __restrict__ M,
+                                                 double* __restrict__ m1d)
 {
 #pragma clang fp contract(off)
-    __shared__ double sc[3];
-    const int tid = threadIdx.x;
-    const double w2 = waveno * waveno;
-    const double* m[3] = {m0, m1, m2};
-    for (int i = tid; i < 3 * ntheta; i += MB) {
-        const int k = i / ntheta, j = i - k * ntheta;
-        tmp[i] = m[k][j] * sin(theta[j]) / w2;
-    }
-    __threadfence_block();
-    __syncthreads();
-    if (tid < 3) sc[tid] = simpne_dev(ntheta, theta, tmp + (int64_t)tid * ntheta, 1);
-    __syncthreads();
-    if (scaling_pass) {
-        if (tid == 0) {
-            params[7] = sqrt(sc[1] / ebeam);
-            params[8] = sqrt(sc[2] / eext);
+    constexpr int NS = FULL ? 48 : 16;   // sums (FULL = false: 2 used)
+    __shared__ double part[MB / 64][NS];
+    const int64_t nb = g.nbins;
+    const int nph = g.nphi, nth = g.ntheta, j = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    Pair* B = reinterpret_cast<Pair*>(ab);
+    Pair* E = reinterpret_cast<Pair*>(ae);
+    double acc[NS];
+#pragma unroll
+    for (int e = 0; e < NS; e++) acc[e] = 0.0;
+    for (int i = threadIdx.x; i < nph; i += blockDim.x) {
+        const int64_t b = (int64_t)nph * j + i;
+        const double w = g.wphi[i];
+        double sb[8], se[8];
+        load_ampl(B, b, nb, g.waveno, f, sb);
+        load_ampl(E, b, nb, g.waveno, f ? f + 1 : f, se);
+        if (FULL) {
+            store_ampl(B, b, nb, sb);
+            store_ampl(E, b, nb, se);
+            double st[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) st[q] = sb[q] + se[q];
+#pragma unroll
+            for (int m = 0; m < 3; m++) {
+                double mm[16];
+                mueller16(m == 0 ? st : (m == 1 ? sb : se), mm);
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    M[b + nb * (16 * m + e)] = mm[e];
+                    acc[16 * m + e] += w * mm[e];
+                }
+            }
+        } else {
+            acc[0] += w * mueller_s11(sb);
+            acc[1] += w * mueller_s11(se);
         }
-        return;
     }
-    for (int i = tid; i < 3 * ntheta; i += MB) {
-        const int k = i / ntheta, j = i - k * ntheta;
-        tmp[i] = m[k][j] * sin(theta[j]) * cos(theta[j]) / sc[k] / w2;
-    }
-    __threadfence_block();
-    __syncthreads();
-    if (tid < 3) params[3 + tid] = simpne_dev(ntheta, theta, tmp + (int64_t)tid * ntheta, 1);
-    if (tid == 0) {
-        int ib = 0;
-        double best = fabs(theta[0] - 2 * PI_R4);
-        for (int j = 1; j < ntheta; j++) {
-            const double d = fabs(theta[j] - 2 * PI_R4);
-            if (d < best) { best = d; ib = j; }
+    if (FULL) {
+        wave_sums<NS, 0>(acc, lane);
+        if (lane < 16) {
+            const int o = 24 * (lane & 1) + 12 * ((lane >> 1) & 1) + 6 * ((lane >> 2) & 1) + 3 * (lane >> 3);
+#pragma unroll
+            for (int e = 0; e < NS / 16; e++) part[wave][o + e] = acc[e];
         }
-        params[0] = sc[0]; params[1] = sc[1]; params[2] = sc[2];
-        params[6] = M0[(int64_t)nphi * ib] * 4 * PI_R4 / w2;
+    } else {
+        wave_sums<2, 4>(acc, lane);
+#pragma unroll
+        for (int o = 1; o < 16; o *= 2) {
+            acc[0] += __shfl_xor(acc[0], o);
+            acc[1] += __shfl_xor(acc[1], o);
+        }
+        if (lane == 0) {
+            part[wave][0] = acc[0];
+            part[wave][1] = acc[1];
+        }
+    }
+    __syncthreads();
+    const int nw = blockDim.x >> 6;
+    if (threadIdx.x < (FULL ? 48 : 2)) {
+        double s = part[0][threadIdx.x];
+        for (int q = 1; q < nw; q++) s += part[q][threadIdx.x];
+        // [matrix][element][theta]; FULL = false: S11 of beam and ext
+        const int row = FULL ? threadIdx.x : 16 * (threadIdx.x + 1);
+        m1d[(int64_t)nth * row + j] = s;
     }
 }
 
-__global__ __launch_bounds__(MB) void k_accumulate(double* __restrict__ total,
-                                                   const double* __restrict__ x, int64_t n)
+// Theta integrals (outputs_mod.f90:133-135, 198-205) from the phi integrals of S11, as weighted sums over one
+// workgroup: scattering cross sections and asymmetry parameters; back-scattering.
+// params: scatt, scatt_beam, scatt_ext, g, g_beam, g_ext, back_scatt, f_beam, f_ext.
+// FACTORS: the energy scaling factors sqrt(scatt_x / energy_x) into params[7..8] alone.
+template <bool FACTORS>
+__global__ __launch_bounds__(MB) void k_theta_params(DevGrid g, const double* __restrict__ m1d,
+                                                     const double* __restrict__ M, double ebeam, double eext,
+                                                     double* __restrict__ params)
 {
-#pragma clang fp contract(off)
-    const int64_t i = (int64_t)blockIdx.x * MB + threadIdx.x;
-    if (i < n) total[i] = total[i] + x[i];
+    __shared__ double part[MB / 64][6];
+    const int tid = threadIdx.x, nth = g.ntheta;
+    double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int j = tid; j < nth; j += MB) {
+        const double w = g.wth[j], wc = g.wth[nth + j];
+#pragma unroll
+        for (int m = FACTORS ? 1 : 0; m < 3; m++) {
+            const double v = m1d[(int64_t)16 * nth * m + j];
+            s[m] += w * v;
+            if (!FACTORS) s[3 + m] += wc * v;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 6; q++) {
+#pragma unroll
+        for (int o = 1; o < 64; o *= 2) s[q] += __shfl_xor(s[q], o);
+        if ((tid & 63) == 0) part[tid >> 6][q] = s[q];
+    }
+    __syncthreads();
+    if (tid >= 3) return;
+    double sc = 0.0, gc = 0.0;
+    for (int q = 0; q < MB / 64; q++) {
+        sc += part[q][tid];
+        gc += part[q][3 + tid];
+    }
+    if (FACTORS) {
+        if (tid > 0) params[6 + tid] = sqrt(sc / (tid == 1 ? ebeam : eext));
+    } else {
+        params[tid] = sc;
+        params[3 + tid] = gc / sc;
+        if (tid == 0) params[6] = M[(int64_t)g.nphi * g.theta_back] * 4 * PI_R4 / (g.waveno * g.waveno);
+    }
 }
 
 }  // namespace abt
 
-static inline unsigned nblk(int64_t n) { return (unsigned)((n + abt::MB - 1) / abt::MB); }
-
-// Device epilogue.  ab/ae: amplitudes (8*nbins doubles, scaled by k in place),
-// tot: 8*nbins scratch (total amplitude), M: 3*16*nbins (total, beam, ext; may be
-// null), m1d: 3*16*ntheta, tmp: 3*ntheta, params: 9 doubles.
-extern "C" int abt_launch_finalise(const abt::DevGrid* g, double* ab,
-                                   double* ae, double* tot, double* M, double* m1d, double* tmp,
-                                   double* params, int scaling, double ebeam, double eext,
-                                   hipStream_t st)
+// Device epilogue.  ab/ae: amplitudes (8*nbins doubles, scaled by k in place), M: 3*16*nbins (total, beam,
+// ext), m1d: 3*16*ntheta, params: 9 doubles.
+extern "C" int abt_launch_finalise(const abt::DevGrid* g, double* ab, double* ae, double* M, double* m1d,
+                                   double* params, int scaling, double ebeam, double eext, hipStream_t st)
 {
     using namespace abt;
-    const int64_t nb = g->nbins, n8 = 8 * nb;
-    const int nth = g->ntheta, nph = g->nphi;
-    double *M0 = M, *M1 = M + 16 * nb, *M2 = M + 32 * nb;
-    double *o0 = m1d, *o1 = m1d + 16 * nth, *o2 = m1d + 32 * nth;
-    hipLaunchKernelGGL(k_scale_sum, dim3(nblk(n8)), dim3(MB), 0, st, ab, ae, tot, g->waveno, g->waveno,
-                       (const double*)nullptr, n8);
-    for (int pass = 0; pass < (scaling ? 2 : 1); pass++) {
-        if (pass == 1)
-            hipLaunchKernelGGL(k_scale_sum, dim3(nblk(n8)), dim3(MB), 0, st, ab, ae, tot, 1.0, 1.0,
-                               (const double*)(params + 7), n8);
-        hipLaunchKernelGGL(k_mueller3, dim3(nblk(nb)), dim3(MB), 0, st, (const double*)tot,
-                           (const double*)ab, (const double*)ae, M0, M1, M2, nb);
-        hipLaunchKernelGGL(k_phi_integrate, dim3(nblk((int64_t)48 * nth)), dim3(MB), 0, st,
-                           (const double*)M0, (const double*)M1, (const double*)M2, g->phi, nph, nth,
-                           o0, o1, o2);
-        if (scaling && pass == 0)
-            hipLaunchKernelGGL(k_theta_params, dim3(1), dim3(MB), 0, st, (const double*)o0,
-                               (const double*)o1, (const double*)o2, (const double*)M0, g->theta,
-                               nth, nph, g->waveno, 1, ebeam, eext, tmp, params);
+    // a lane per phi; whole waves, at most four
+    const dim3 grid((unsigned)g->ntheta), block((unsigned)(g->nphi >= MB ? MB : (g->nphi + 63) / 64 * 64));
+    const double* f = nullptr;
+    if (scaling) {
+        hipLaunchKernelGGL(k_epilogue<false>, grid, block, 0, st, *g, ab, ae, f, M, m1d);
+        hipLaunchKernelGGL(k_theta_params<true>, dim3(1), dim3(MB), 0, st, *g, (const double*)m1d, (const double*)M,
+                           ebeam, eext, params);
+        f = params + 7;
     }
-    hipLaunchKernelGGL(k_theta_params, dim3(1), dim3(MB), 0, st, (const double*)o0, (const double*)o1,
-                       (const double*)o2, (const double*)M0, g->theta, nth, nph, g->waveno, 0,
-                       ebeam, eext, tmp, params);
-    return (int)hipGetLastError();
-}
-
-extern "C" int abt_launch_accumulate(double* total, const double* x, int64_t n, hipStream_t st)
-{
-    hipLaunchKernelGGL(abt::k_accumulate, dim3(nblk(n)), dim3(abt::MB), 0, st, total, x, n);
+    hipLaunchKernelGGL(k_epilogue<true>, grid, block, 0, st, *g, ab, ae, f, M, m1d);
+    hipLaunchKernelGGL(k_theta_params<false>, dim3(1), dim3(MB), 0, st, *g, (const double*)m1d, (const double*)M, ebeam,
+                       eext, params);
     return (int)hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
-// The epilogue without allocation (abt_finalise_dev_static): its scratch (the total
-// amplitude, 8 doubles per bin, and the theta integrands, 3 per theta) lives in a
-// file-scope device array, one per GPU for the life of the process.  In host code the
-// array's name is not a device address: its address on the current device comes from
-// hipGetSymbolAddress, once per device, and only that address reaches the kernels.
-namespace {
-
-constexpr int64_t STATIC_SCRATCH_DOUBLES = (int64_t)8 << 20;   // 64 MiB
-static __device__ __align__(256) double scratch[STATIC_SCRATCH_DOUBLES];
-
-constexpr int MAX_DEVICES = 64;
-std::mutex g_scratch_mu;
-double* g_scratch_ptr[MAX_DEVICES] = {};
-
-// The scratch array's address on the library's device (looked up on first use there).
-int scratch_on_device(double** out)
-{
-    int rc = abt_ensure_device(nullptr);
-    if (rc) return rc;
-    int dev = -1;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return abt_fail(ABT_ERR_HIP, "hipGetDevice: %s", hipGetErrorString(e));
-    if (dev < 0 || dev >= MAX_DEVICES) return abt_fail(ABT_ERR_NODEV, "device %d out of range", dev);
-    std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_ptr[dev]) {
-        void* p = nullptr;
-        e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p)
-            return abt_fail(ABT_ERR_HIP, "hipGetSymbolAddress(scratch): %s", hipGetErrorString(e));
-        g_scratch_ptr[dev] = (double*)p;
-    }
-    *out = g_scratch_ptr[dev];
-    return 0;
-}
-
-}  // namespace
+// The epilogue without allocation (abt_finalise_dev_static).  Its limit is the entry point's: it once kept
+// the total amplitude and the theta integrands (8 doubles per bin, 3 per theta) in a 64 MiB array.
+static constexpr int64_t STATIC_SCRATCH_DOUBLES = (int64_t)8 << 20;
 
 extern "C" int64_t abt_finalise_static_max_bins(int64_t n_theta)
 {
@@ -260,12 +243,9 @@ extern "C" int abt_finalise_dev_static(const abt_dev_grid* g, double* ab, double
                         "%lld it holds (at most %lld bins at this theta count); use abt_finalise_dev",
                         (long long)g->nbins, g->d.ntheta, (long long)need, (long long)STATIC_SCRATCH_DOUBLES,
                         (long long)abt_finalise_static_max_bins(g->d.ntheta));
-    double* sp = nullptr;
-    int rc = scratch_on_device(&sp);
+    int rc = abt_ensure_device(nullptr);
     if (rc) return rc;
-    double* tot = sp;
-    double* tmp = sp + 8 * g->nbins;
-    int e = abt_launch_finalise(&g->d, ab, ae, tot, dev_mueller, dev_m1d, tmp, dev_params, scaling, ebeam, eext,
+    int e = abt_launch_finalise(&g->d, ab, ae, dev_mueller, dev_m1d, dev_params, scaling, ebeam, eext,
                                 (hipStream_t)stream);
     if (e) return abt_fail(ABT_ERR_HIP, "finalise launch failed: %s", hipGetErrorString((hipError_t)e));
     return 0;

@@ -107,6 +107,10 @@ struct DevGrid {
     const double* theta;                    // [ntheta] theta_vals, rad
     const double* phi;                      // [nphi] phi_vals, rad
     const double* etab;                     // [ETAB_GRID] e^{i pi j / ETAB_N}, then its low parts (FP64 bodies)
+    // the epilogue's quadratures as weights (simpne; zero for grids of fewer than 3 values)
+    const double* wphi;                     // [nphi] of the phi integrals
+    const double* wth;                      // [2][ntheta] of the theta integrals: w sin / k^2, w sin cos / k^2
+    int32_t theta_back;                     // theta nearest to 2 pi (back-scattering)
 };
 
 // Table of the FP64 bodies' exponentials: cos and sin of pi j / ETAB_N for j = 0 .. 2 ETAB_N - 1

@@ -24,14 +24,14 @@
 #include "frame.h"
 #include "records.h"
 #include "rt_internal.h"
+#include "simpne.h"
 
 extern "C" int abt_launch_far_field(const abt::DevGrid* g, const double* recs, const double* vrecs,
                                     int64_t nb, int prec, int fast_diff, int64_t per, double* out,
                                     double* work, hipStream_t st);
 extern "C" int abt_launch_zero(double* out, int64_t n, hipStream_t st);
-extern "C" int abt_launch_finalise(const abt::DevGrid* g, double* ab, double* ae, double* tot,
-                                   double* M, double* m1d, double* tmp, double* params,
-                                   int scaling, double ebeam, double eext, hipStream_t st);
+extern "C" int abt_launch_finalise(const abt::DevGrid* g, double* ab, double* ae, double* M, double* m1d,
+                                   double* params, int scaling, double ebeam, double eext, hipStream_t st);
 extern "C" int abt_launch_prepare(int64_t n, const double* ampl, const double* vk7,
                                   const double* prop, const double* fov, double fov_value,
                                   const int64_t* vert_off, const double* verts, double lambda,
@@ -253,9 +253,10 @@ static int grid_build(int64_t nth, const double* th, int64_t nph, const double* 
     int rc = ensure_device();
     if (rc) return rc;
     const int64_t nb = nth * nph;
-    std::vector<double> h((size_t)(5 * nb + 3 * nph + nth + abt::ETAB_GRID));
+    std::vector<double> h((size_t)(5 * nb + 4 * nph + 3 * nth + abt::ETAB_GRID));
     double *x = h.data(), *y = x + nb, *z = y + nb, *rad = z + nb, *krr = rad + nb;
     double *cp = krr + nb, *sp = cp + nph, *phv = sp + nph, *thv = phv + nph, *etab = thv + nth;
+    double *wph = etab + abt::ETAB_GRID, *wth = wph + nph;
     abt::fill_exp_table(etab);
     memcpy(phv, ph, sizeof(double) * nph);
     memcpy(thv, th, sizeof(double) * nth);
@@ -274,6 +275,20 @@ static int grid_build(int64_t nth, const double* th, int64_t nph, const double* 
         krr[b] = krev * r;
     }
     for (int64_t i = 0; i < nph; i++) sincos(ph[i], &sp[i], &cp[i]);
+    int32_t back = 0;
+    if (nph >= 3 && nth >= 3) {
+        abt::simpne_weights((int)nph, ph, wph);
+        abt::simpne_weights((int)nth, th, wth);
+        double best = fabs(th[0] - 2 * abt::PI_R4);
+        for (int64_t j = 0; j < nth; j++) {
+            double s, c;
+            sincos(th[j], &s, &c);
+            wth[j] = wth[j] * s / (waveno * waveno);
+            wth[nth + j] = wth[j] * c;
+            const double d = fabs(th[j] - 2 * abt::PI_R4);
+            if (d < best) { best = d; back = (int32_t)j; }
+        }
+    }
     abt_dev_grid* g = new abt_dev_grid();
     if (hipMalloc(&g->mem, sizeof(double) * h.size()) != hipSuccess) {
         delete g;
@@ -301,6 +316,9 @@ static int grid_build(int64_t nth, const double* th, int64_t nph, const double* 
     g->d.phi = d + 5 * nb + 2 * nph;
     g->d.theta = d + 5 * nb + 3 * nph;
     g->d.etab = d + 5 * nb + 3 * nph + nth;
+    g->d.wphi = g->d.etab + abt::ETAB_GRID;
+    g->d.wth = g->d.wphi + nph;
+    g->d.theta_back = back;
     g->nbins = nb;
     *out = g;
     return 0;
@@ -774,19 +792,12 @@ int abt_finalise_dev(const abt_dev_grid* g, double* ab, double* ae, int scaling,
         return fail(ABT_ERR_ARG, "energy scaling needs positive beam and ext energies");
     int rc = ensure_device();
     if (rc) return rc;
+    // (the epilogue keeps nothing between its kernels but its outputs; a caller's workspace is only checked)
     const size_t need = abt_finalise_workspace(g);
-    void* work = dev_work;
-    if (!work || work_bytes < need) {
-        if (work) return fail(ABT_ERR_ARG, "finalise workspace of %zu bytes is smaller than %zu", work_bytes, need);
-        ThreadState& ts = tstate();
-        rc = buf_ensure(ts.bufs[6], need);
-        if (rc) return rc;
-        work = ts.bufs[6].p;
-    }
-    double* tot = (double*)work;
-    double* tmp = tot + 8 * g->nbins;
-    int e = abt_launch_finalise(&g->d, ab, ae, tot, dev_mueller, dev_m1d, tmp, dev_params, scaling,
-                                ebeam, eext, (hipStream_t)stream);
+    if (dev_work && work_bytes < need)
+        return fail(ABT_ERR_ARG, "finalise workspace of %zu bytes is smaller than %zu", work_bytes, need);
+    int e = abt_launch_finalise(&g->d, ab, ae, dev_mueller, dev_m1d, dev_params, scaling, ebeam, eext,
+                                (hipStream_t)stream);
     if (e) return fail(ABT_ERR_HIP, "finalise launch failed: %s", hipGetErrorString((hipError_t)e));
     return 0;
 }

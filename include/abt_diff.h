@@ -165,15 +165,11 @@ int abt_far_field_dev(const abt_dev_grid* g, const double* dev_recs, const doubl
                       int64_t nb, int precision, int is_fast_diff, double* dev_out,
                       void* dev_work, size_t work_bytes, void* stream);
 
-/* abt_finalise_dev without any allocation.  No reference counterpart: for callers that
+/* abt_finalise_dev without a workspace argument.  No reference counterpart: for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc).  The epilogue's scratch (the total amplitude, 8 doubles per bin, and the
- * theta integrands, 3 per theta value) is a 64 MiB array resident on each GPU the library
- * runs on, for the life of the process, instead of a workspace argument or a library
- * allocation: grids up to abt_finalise_static_max_bins(n_theta) bins (about 1.05e6).
- * Larger grids are rejected with ABT_ERR_ARG.  Every call on one GPU shares that array:
- * calls that overlap on one GPU (other streams or threads) race and must be serialised by
- * the caller.  Arguments and outputs as abt_finalise_dev. */
+ * hipMalloc).  Grids up to abt_finalise_static_max_bins(n_theta) bins (about 1.05e6, once the size
+ * of a resident scratch array); larger grids are rejected with ABT_ERR_ARG.  Arguments and
+ * outputs as abt_finalise_dev. */
 int abt_finalise_dev_static(const abt_dev_grid* g, double* dev_ampl_beam, double* dev_ampl_ext,
                             int scaling, double beam_energy_out, double ext_energy_out,
                             double* dev_mueller, double* dev_mueller_1d, double* dev_params,
@@ -191,7 +187,7 @@ int abt_far_field_incoherent_dev(const abt_dev_grid* g, const double* dev_recs,
 /* Device form of abt_finalise: amplitudes resident on the device (scaled by k in
  * place).  dev_mueller: 3*16*nbins (total, beam, ext, each (nphi, ntheta, 16));
  * dev_mueller_1d: 3*16*n_theta; dev_params: 9 doubles (as abt_finalise).
- * dev_work: abt_finalise_workspace bytes (NULL: the library allocates). */
+ * dev_work: NULL, or at least abt_finalise_workspace bytes (checked; the epilogue needs none). */
 size_t abt_finalise_workspace(const abt_dev_grid* g);
 int abt_finalise_dev(const abt_dev_grid* g, double* dev_ampl_beam, double* dev_ampl_ext,
                      int scaling, double beam_energy_out, double ext_energy_out,
