@@ -11,26 +11,24 @@
 // projection (edge checks); the first non-beam blocker of another aperture
 // ends the scan, beam facets record the nearest one (id_beam, dist_beam).
 //
-// Here, for many beams at once (beam = blockIdx.y):
-//   k_vis_boxes   one workgroup per beam: x-y extents (block min/max), box
-//                 midpoints, the illuminating facets' extent;
-//   k_vis_facets  one lane per facet: box, candidate mask, cull and shadow
-//                 flags, initial outputs;
-//   k_vis_map     field_in -> mapping (last position wins, as the reference's
-//                 sequential store);
-//   k_vis_lists   one workgroup per beam: per box, the ascending candidate
-//                 list and the ascending list of tested facets (block-wide
-//                 ballot scans, so list order is facet order);
+// Here, for many beams at once:
+//   k_vis_setup   one workgroup per beam: x-y extents (block min/max), the boxes, then per facet its box,
+//                 candidate mask, cull and shadow flags and initial outputs; field_in -> mapping
+//                 (last position wins, as the reference's sequential store); per box the ascending
+//                 candidate list and the ascending list of tested facets (each wave owns a run of facets
+//                 and writes after the waves before it, so list order is facet order);
 //   k_vis_main    one wave per 64 tested facets of one box: every lane of the
-//                 wave scans the same candidate list in facet order; tiles of
-//                 candidates (depth, aperture, projected vertices) are gathered
-//                 into LDS by parallel loads and read back as broadcasts; a lane
+//                 wave scans the same candidate list in facet order, so a candidate is wave-uniform: its
+//                 list entry comes through scalar loads and its projected vertices as broadcasts
+//                 from LDS, where the workgroup keeps its beam's vertices; a lane
 //                 stops at its blocker, the wave when all lanes have stopped.
+// Triangles seen from the side on which no midpoint can pass their edge checks are left out (see faces_away).
 // All arithmetic is the reference's FP64 operations with contraction off and
 // comparisons in the same sense; min/max reductions are exact, so results do
 // not depend on the decomposition.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <limits.h>
 #include <math.h>
 #include <stdint.h>
 #include <string.h>
@@ -43,72 +41,112 @@ namespace vis {
 
 constexpr int NB = 16;                                // 4 x 4 boxes
 constexpr int BLK = 256;
+constexpr int SETUP = 256, SETUP_FEW = 1024;          // threads of k_vis_setup: many beams, few
 constexpr int WAVE = 64;
+constexpr int XCDS = 8;                               // dies, which workgroups go round
+constexpr int MW = 4;                                 // waves of a k_vis_main workgroup
 constexpr int OFFS = 2 * (NB + 1) + 2;                // per-beam list offsets (padded)
-constexpr int TC = 32;                                // candidates per LDS tile of the scan
 constexpr int UNR = 4;                                // candidates evaluated together in the scan
-constexpr int NVS = 8;                                // vertices per candidate staged in LDS
-constexpr int SLOT = 4 + 2 * NVS;                     // doubles per staged candidate
+constexpr int64_t STAGE_NV = 3584;                    // vertices of a beam kept in LDS, at most (56 KB of 64)
 constexpr int64_t BEAM_CHUNK = 65535;                 // beams per launch (grid.y)
 constexpr double FAC = 1.100000023841858;             // fac = 1.1, a REAL*4 literal (:2679)
 constexpr double C001 = 0.009999999776482582;         // 0.01, a REAL*4 literal
 
-struct BeamBox {
-    double bx[NB], by[NB];
-    double xmin, xmax, ymin, ymax;   // x-y extent of the illuminating facets (int / ext)
-    double pad[4];
+// One entry of a candidate list.
+struct __align__(32) Cand {
+    double z;        // depth of the facet's midpoint
+    int j;           // facet
+    int v[3];        // its first vertices; v[0] < 0: not a triangle; v[1] < 0: faces away (only counted)
+    int ap, map;     // aperture, position in field_in (0: not a beam facet)
 };
 
+// A wave-uniform entry through scalar loads: the lists are not written while a scan runs, which the constant
+// address space says (the scan's own stores of its results would otherwise rule it out).
+__device__ __forceinline__ Cand load_scalar(const Cand* p)
+{
+    typedef int Words __attribute__((ext_vector_type(8)));
+    static_assert(sizeof(Words) == sizeof(Cand), "an entry is 32 bytes");
+    return __builtin_bit_cast(Cand, *(const __attribute__((address_space(4))) Words*)(uintptr_t)p);
+}
+
 struct Work {
-    BeamBox* boxes;     // [nbeam]
-    int32_t* fbox;      // [nbeam][nf] box of a tested facet's midpoint, -1: not tested
-    int32_t* fmask;     // [nbeam][nf] bit k: candidate blocker in box k
+    uint32_t* fbits;    // [nbeam][nf] bits 0-15: candidate blocker in box k; F_BOX, F_TESTED, F_AWAY
     int32_t* mapping;   // [nbeam][nf] 1-based position in field_in (the last), 0: not a beam facet
     int32_t* offs;      // [nbeam][OFFS] candidate-list offsets [0..NB], tested-list offsets [NB+1..2NB+1]
-    int2* cand;         // [nbeam][3 nf] (blocker facet, f_off of it)
+    Cand* cand;         // [nbeam][3 nf]
     int32_t* mlist;     // [nbeam][nf]
     int64_t nvref;      // f_off[nf]
     int64_t b0;         // first beam of this launch
+    int nb, parts;      // beams of this launch; workgroups of k_vis_main per beam
+    int keep_all;       // lists for a counted scan: the facets that face away too
 };
+constexpr uint32_t F_BOX = 16, F_TESTED = 1u << 20, F_AWAY = 1u << 21;   // F_BOX: shift of the tested facet's box
 
 __device__ __forceinline__ int64_t clampi(int64_t i, int64_t n) { return i < 0 ? 0 : (i >= n ? n - 1 : i); }
 
 // minloc over the box midpoints of sqrt((bx - px)**2 + (by - py)**2), first minimum
-// (beam_loop_mod.f90:2087-2093)
+// (beam_loop_mod.f90:2087-2093), box k = 4 i + j at (bx[i], by[j]).
 // The square root is monotonic, so the smallest distance is the root of the smallest
-// squared distance d2[k0] (k0 its first index); an earlier box ties with it only if its
-// squared distance rounds to the same root, which needs d2[k] <= d2[k0] (1 + 2^-51): those
-// few are decided by the roots themselves, as the reference does.  bx, by: the box
-// midpoints in registers; gbx, gby: the same in memory.
-__device__ __forceinline__ int nearest_box(const double* bx, const double* by, const double* gbx,
-                                           const double* gby, double px, double py)
+// squared distance; a box before it ties with it only if its squared distance rounds to the same
+// root, which needs d2 <= dmin (1 + 2^-51).  Rounded sums are monotonic too: the smallest d2 is that of
+// the smallest dx^2 and dy^2, and if neither the second smallest of each with the smallest of the
+// other comes within the limit, no other box does.  The rest (ties, points that are not finite) scan all
+// boxes as the reference does; finite: the boxes are.
+// lx, ly: bx, by in memory, for the rare path's rolled loop.
+__device__ __forceinline__ int nearest_box(const double* bx, const double* by, const double* lx, const double* ly,
+                                           bool finite, double px, double py)
 {
 #pragma clang fp contract(off)
-    double d2[NB];
-    double dmin = 0.0;
-    int k0 = 0;
+    double m[2], n[2];   // smallest and second smallest squared offset in x, y
+    int k[2];
 #pragma unroll
-    for (int k = 0; k < NB; k++) {
-        const double dx = bx[k] - px, dy = by[k] - py;
-        d2[k] = dx * dx + dy * dy;
-        if (k == 0 || d2[k] < dmin) {
-            dmin = d2[k];
-            k0 = k;
+    for (int c = 0; c < 2; c++) {
+        double d[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const double o = (c ? by[i] : bx[i]) - (c ? py : px);
+            d[i] = o * o;
+        }
+        k[c] = d[1] < d[0] ? 1 : 0;
+        m[c] = fmin(d[0], d[1]);
+        n[c] = fmax(d[0], d[1]);
+#pragma unroll
+        for (int i = 2; i < 4; i++) {
+            k[c] = d[i] < m[c] ? i : k[c];
+            n[c] = fmin(n[c], fmax(m[c], d[i]));
+            m[c] = fmin(m[c], d[i]);
         }
     }
-    const double lim = dmin + ldexp(dmin, -49);
-    bool near = false;
-#pragma unroll
-    for (int k = 0; k < NB; k++) near |= k < k0 && d2[k] <= lim;
-    if (!near) return k0;
-    // rare: recompute from the boxes in memory (a rolled loop, no register indexing)
-    const double s0 = sqrt(dmin);
-    for (int k = 0; k < k0; k++) {
-        const double dx = gbx[k] - px, dy = gby[k] - py;
-        const double d = dx * dx + dy * dy;
-        if (d <= lim && sqrt(d) == s0) return k;
+    const double dmin = m[0] + m[1], lim = dmin + ldexp(dmin, -49);
+    if (finite && n[0] + m[1] > lim && m[0] + n[1] > lim) return 4 * k[0] + k[1];
+    double best = 0.0;
+    int kb = 0;
+#pragma unroll 1
+    for (int q = 0; q < NB; q++) {
+        const double dx = lx[q >> 2] - px, dy = ly[q & 3] - py;
+        const double d = sqrt(dx * dx + dy * dy);
+        if (q == 0 || d < best) {
+            best = d;
+            kb = q;
+        }
     }
-    return k0;
+    return kb;
+}
+
+// Whether no midpoint can pass the edge checks of this triangle, rounding included.  The exact checks of the
+// three edges, C_e = (m - x_e) x (x_e+1 - x_e), add up to minus twice the signed area whatever m is, so one of them
+// is at least a third of it when the area is negative (positive for find_vis_ext, whose checks have
+// the other sign): outside that edge.  A computed check is within 4 u (|m_x - x_e| |e_y| + |m_y - y_e| |e_x|)
+// of C_e, u = 1.1e-16, as is the computed area of its own; the extents of vertices and midpoints together, ex
+// and ey, bound the offsets.  64 u covers the factors 3, 4 and their sum four times over.
+__device__ __forceinline__ bool faces_away(int mode, double x0, double y0, double x1, double y1, double x2, double y2,
+                                           double ex, double ey)
+{
+    const double ax = x1 - x0, ay = y1 - y0, bx = x2 - x0, by = y2 - y0;
+    const double area2 = ax * by - ay * bx;
+    const double lx = fmax(fabs(ax), fmax(fabs(bx), fabs(x2 - x1))), ly = fmax(fabs(ay), fmax(fabs(by), fabs(y2 - y1)));
+    const double tol = 7.2e-15 * (ex * ly + ey * lx);
+    return mode == ABT_VIS_EXT ? area2 > tol : area2 < -tol;
 }
 
 __device__ __forceinline__ double wave_min(double v)
@@ -130,384 +168,417 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(BLK) void k_vis_boxes(abt_vis_batch a, Work w)
-{
-#pragma clang fp contract(off)
-    __shared__ double red[BLK / WAVE][8];
-    const int64_t b = w.b0 + blockIdx.x;
-    const int tid = threadIdx.x;
-    const double* x = a.v + 3 * a.nv * b;
-    const double* y = x + a.nv;
-    double r[8];
-#pragma unroll
-    for (int q = 0; q < 8; q += 2) {
-        r[q] = INFINITY;
-        r[q + 1] = -INFINITY;
-    }
-    for (int64_t i = tid; i < a.nv; i += BLK) {
-        const double xi = x[i], yi = y[i];
-        r[0] = xi < r[0] ? xi : r[0];
-        r[1] = xi > r[1] ? xi : r[1];
-        r[2] = yi < r[2] ? yi : r[2];
-        r[3] = yi > r[3] ? yi : r[3];
-    }
-    if (a.mode != ABT_VIS_INC) {
-        const int64_t e0 = a.in_off[b], e1 = a.in_off[b + 1];
-        for (int64_t e = e0 + tid; e < e1; e += BLK) {
-            const int64_t fi = clampi(a.field_in[e] - 1, a.nf);
-            for (int64_t k = a.f_off[fi]; k < a.f_off[fi + 1]; k++) {
-                const int64_t vk = clampi(a.f_vi[k] - 1, a.nv);
-                const double xk = x[vk], yk = y[vk];
-                r[4] = xk < r[4] ? xk : r[4];
-                r[5] = xk > r[5] ? xk : r[5];
-                r[6] = yk < r[6] ? yk : r[6];
-                r[7] = yk > r[7] ? yk : r[7];
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < 8; q++) r[q] = (q & 1) ? wave_max(r[q]) : wave_min(r[q]);
-    if ((tid & (WAVE - 1)) == 0) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) red[tid / WAVE][q] = r[q];
-    }
-    __syncthreads();
-    if (tid != 0) return;
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        double v = red[0][q];
-        for (int s = 1; s < BLK / WAVE; s++) {
-            const double u = red[s][q];
-            v = (q & 1) ? (u > v ? u : v) : (u < v ? u : v);
-        }
-        r[q] = v;
-    }
-    // box corners fac * (min + (max - min) / 4 * (i - 1)) (:2711-2720), box k = 4 (i-1) + (j-1)
-    // with corners (i, j), (i, j+1), (i+1, j+1), (i+1, j) summed in that order, / 4 (:2732-2740,
-    // compute_geometry_midpoints misc_submod.f90:199-209)
-    const double min_x = r[0], max_x = r[1], min_y = r[2], max_y = r[3];
-    BeamBox* B = w.boxes + b;
-    for (int i = 1; i <= 4; i++) {
-        const double x0 = FAC * (min_x + (max_x - min_x) / 4.0 * (double)(i - 1));
-        const double x1 = FAC * (min_x + (max_x - min_x) / 4.0 * (double)i);
-        for (int j = 1; j <= 4; j++) {
-            const double y0 = FAC * (min_y + (max_y - min_y) / 4.0 * (double)(j - 1));
-            const double y1 = FAC * (min_y + (max_y - min_y) / 4.0 * (double)j);
-            const int k = 4 * (i - 1) + (j - 1);
-            B->bx[k] = (((0.0 + x0) + x0) + x1) + x1;
-            B->bx[k] = B->bx[k] / 4.0;
-            B->by[k] = (((0.0 + y0) + y1) + y1) + y0;
-            B->by[k] = B->by[k] / 4.0;
-        }
-    }
-    B->xmin = r[4];
-    B->xmax = r[5];
-    B->ymin = r[6];
-    B->ymax = r[7];
-}
-
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(BLK) void k_vis_facets(abt_vis_batch a, Work w)
-{
-#pragma clang fp contract(off)
-    const int64_t b = w.b0 + blockIdx.y;
-    const int64_t i = (int64_t)blockIdx.x * BLK + threadIdx.x;
-    if (i >= a.nf) return;
-    const int64_t nf = a.nf;
-    const BeamBox& B = w.boxes[b];
-    double bx[NB], by[NB];
-#pragma unroll
-    for (int k = 0; k < NB; k++) {
-        bx[k] = B.bx[k];
-        by[k] = B.by[k];
-    }
-    const double* x = a.v + 3 * a.nv * b;
-    const double* y = x + a.nv;
-    const double* mid = a.f_mid + 3 * nf * b + 3 * i;
-    const double mx = mid[0], my = mid[1];
-    const int f3 = nearest_box(bx, by, B.bx, B.by, mx, my);
-    const int64_t o0 = a.f_off[i];
-    int mask = 0;
-    for (int q = 0; q < 3; q++) {
-        const int64_t vq = clampi(a.f_vi[min(o0 + q, w.nvref - 1)] - 1, a.nv);
-        mask |= 1 << nearest_box(bx, by, B.bx, B.by, x[vq], y[vq]);
-    }
-    const double nz = a.f_nz[nf * b + i];
-    const int64_t api = a.f_ap[i];
-    const double apn = a.ap_nz[a.na * b + clampi(api - 1, a.na)];
-    bool vis = true;
-    if (a.mode != ABT_VIS_INC) {   // midpoint outside the beam's extent (:2145-2155)
-        if (mx < B.xmin) vis = false;
-        else if (mx > B.xmax) vis = false;
-        else if (my < B.ymin) vis = false;
-        else if (my > B.ymax) vis = false;
-    }
-    const bool shad = a.mode == ABT_VIS_INT ? nz >= 0 : nz <= 0;                 // :2158, :2370, :2543
-    const bool down = a.mode == ABT_VIS_INT ? apn > -C001 : apn < C001;          // :2165, :2377, :2547
-    const bool tested = vis && !down;
-    const int64_t o = nf * b + i;
-    a.in_beam[o] = (a.mode == ABT_VIS_INC && !down) ? 1 : 0;
-    if (a.is_vis) a.is_vis[o] = tested ? 1 : 0;
-    a.dist_beam[o] = 0.0;
-    a.id_beam[o] = 0;
-    a.is_shad[o] = shad ? 1 : 0;
-    w.fbox[o] = tested ? f3 : -1;
-    // the incident beam's blockers face up (:2553)
-    w.fmask[o] = (a.mode == ABT_VIS_INC && nz < C001) ? 0 : mask;
-    w.mapping[o] = 0;
-}
-
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(BLK) void k_vis_map(abt_vis_batch a, Work w)
-{
-    const int64_t b = w.b0 + blockIdx.x;
-    const int64_t e0 = a.in_off[b], e1 = a.in_off[b + 1];
-    for (int64_t e = e0 + threadIdx.x; e < e1; e += BLK) {
-        const int64_t fi = a.field_in[e] - 1;
-        if (fi < 0 || fi >= a.nf) continue;
-        atomicMax(w.mapping + a.nf * b + fi, (int)(e - e0 + 1));
-    }
-}
-
-// ---------------------------------------------------------------------------
 __device__ __forceinline__ int lanes_below(unsigned long long m)
 {
     return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
-__global__ __launch_bounds__(BLK) void k_vis_lists(abt_vis_batch a, Work w)
+// ---------------------------------------------------------------------------
+// Everything before the scan, one workgroup per beam.  Bound by memory where there are many beams (31 bytes a
+// facet of initial outputs, 32 a list entry, 64 read), by the latency of its steps for one beam.  As four
+// kernels (boxes, facets, map, lists) with each facet's box and mask in memory between them, sixteen
+// distances a search and four barriers a block of 256 facets in the list building, 2048 beams x 2112
+// facets took 256 us; here 204.  One beam: 49 us and two more launches; here 34.
+// STAGE: the beam's projected vertices are kept in LDS (nv <= STAGE_NV): their gathers, 64 lines each,
+// otherwise fill the CU's address unit.
+template <bool STAGE>
+__global__ __launch_bounds__(SETUP_FEW) void k_vis_setup(abt_vis_batch a, Work w)
 {
+#pragma clang fp contract(off)
     constexpr int NQ = 2 * NB;   // q < NB: candidate list of box q; q >= NB: tested list of box q - NB
-    constexpr int NW = BLK / WAVE;
-    __shared__ int s_run[NQ];
-    __shared__ int s_wt[NW][NQ];
+    constexpr int NWMAX = SETUP_FEW / WAVE;
+    extern __shared__ double2 sxy[];
+    __shared__ double red[NWMAX][12];
+    __shared__ double sbx[4], sby[4], sext[6];
+    __shared__ int s_cnt[NWMAX][NQ];
     const int64_t b = w.b0 + blockIdx.x;
-    const int tid = threadIdx.x, wv = tid / WAVE;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wv = tid / WAVE, nt = blockDim.x, nw = nt / WAVE;
     const int64_t nf = a.nf;
-    const int32_t* fmask = w.fmask + nf * b;
-    const int32_t* fbox = w.fbox + nf * b;
-    if (tid < NQ) s_run[tid] = 0;
-    __syncthreads();
-    for (int64_t i = tid; i < nf; i += BLK) {
-        const int m = fmask[i], f = fbox[i];
-        for (int q = 0; q < NB; q++)
-            if ((m >> q) & 1) atomicAdd(&s_run[q], 1);
-        if (f >= 0) atomicAdd(&s_run[NB + f], 1);
-    }
-    __syncthreads();
-    int32_t* offs = w.offs + (int64_t)OFFS * b;
-    if (tid == 0) {
-        int c = 0, t = 0;
-        for (int q = 0; q < NB; q++) {
-            const int nc = s_run[q], nt = s_run[NB + q];
-            offs[q] = c;
-            offs[NB + 1 + q] = t;
-            s_run[q] = c;
-            s_run[NB + q] = t;
-            c += nc;
-            t += nt;
-        }
-        offs[NB] = c;
-        offs[2 * NB + 1] = t;
-    }
-    __syncthreads();
-    int2* cand = w.cand + 3 * nf * b;
-    int32_t* mlist = w.mlist + nf * b;
-    const int64_t* f_off = a.f_off;
-    for (int64_t base = 0; base < nf; base += BLK) {
-        const int64_t i = base + tid;
-        const bool ok = i < nf;
-        const unsigned bits = ok ? ((unsigned)fmask[i] & 0xffffu) | (fbox[i] >= 0 ? 1u << (NB + fbox[i]) : 0u) : 0u;
-        int pre[NQ];
+    const double* x = a.v + 3 * a.nv * b;
+    const double* y = x + a.nv;
+    const double* fmid = a.f_mid + 3 * nf * b;
+    {
+        // extents: the vertices', the illuminating facets', the midpoints'
+        double r[12];
 #pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            const unsigned long long bal = __ballot((bits >> q) & 1u);
-            pre[q] = lanes_below(bal);
-            if ((tid & (WAVE - 1)) == 0) s_wt[wv][q] = __popcll(bal);
+        for (int q = 0; q < 12; q += 2) {
+            r[q] = INFINITY;
+            r[q + 1] = -INFINITY;
         }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < NQ; q++) {
-            if ((bits >> q) & 1u) {
-                int pos = s_run[q] + pre[q];
-                for (int s = 0; s < wv; s++) pos += s_wt[s][q];
-                if (q < NB) cand[pos] = make_int2((int)i, (int)f_off[i]);
-                else mlist[pos] = (int32_t)i;
+        const auto grow = [&](int q, double px, double py) {
+            r[q] = px < r[q] ? px : r[q];
+            r[q + 1] = px > r[q + 1] ? px : r[q + 1];
+            r[q + 2] = py < r[q + 2] ? py : r[q + 2];
+            r[q + 3] = py > r[q + 3] ? py : r[q + 3];
+        };
+        for (int64_t i = tid; i < a.nv; i += nt) {
+            const double px = x[i], py = y[i];
+            if (STAGE) sxy[i] = make_double2(px, py);
+            grow(0, px, py);
+        }
+        if (a.mode != ABT_VIS_INC) {
+            const int64_t e0 = a.in_off[b], e1 = a.in_off[b + 1];
+            for (int64_t e = e0 + tid; e < e1; e += nt) {
+                const int64_t fi = clampi(a.field_in[e] - 1, nf);
+                for (int64_t k = a.f_off[fi]; k < a.f_off[fi + 1]; k++) {
+                    const int64_t vk = clampi(a.f_vi[k] - 1, a.nv);
+                    grow(4, x[vk], y[vk]);
+                }
             }
         }
-        __syncthreads();
-        if (tid < NQ) {
-            int t = 0;
-            for (int s = 0; s < NW; s++) t += s_wt[s][tid];
-            s_run[tid] += t;
+        for (int64_t i = tid; i < nf; i += nt) grow(8, fmid[3 * i], fmid[3 * i + 1]);
+#pragma unroll
+        for (int q = 0; q < 12; q++) r[q] = (q & 1) ? wave_max(r[q]) : wave_min(r[q]);
+        if (lane == 0) {
+#pragma unroll
+            for (int q = 0; q < 12; q++) red[wv][q] = r[q];
         }
         __syncthreads();
+        if (tid < 12) {
+            double v = red[0][tid];
+            for (int k = 1; k < nw; k++) {
+                const double u = red[k][tid];
+                v = (tid & 1) ? (u > v ? u : v) : (u < v ? u : v);
+            }
+            red[0][tid] = v;
+        }
+        __syncthreads();
+        if (tid < 8) {
+            // box corners fac * (min + (max - min) / 4 * (i - 1)) (:2711-2720), box k = 4 (i-1) + (j-1)
+            // with corners (i, j), (i, j+1), (i+1, j+1), (i+1, j) summed in that order, / 4 (:2732-2740,
+            // compute_geometry_midpoints misc_submod.f90:199-209)
+            const int c = tid >> 2, i = (tid & 3) + 1;
+            const double lo = red[0][2 * c], hi = red[0][2 * c + 1];
+            const double p0 = FAC * (lo + (hi - lo) / 4.0 * (double)(i - 1));
+            const double p1 = FAC * (lo + (hi - lo) / 4.0 * (double)i);
+            if (c == 0)
+                sbx[i - 1] = ((((0.0 + p0) + p0) + p1) + p1) / 4.0;
+            else
+                sby[i - 1] = ((((0.0 + p0) + p1) + p1) + p0) / 4.0;
+        } else if (tid < 14) {
+            const int q = tid - 8;   // the illuminating facets' extents, then the widths of vertices and midpoints
+            const double* e = red[0];
+            sext[q] = q < 4 ? e[4 + q] : fmax(e[2 * q - 7], e[2 * q + 1]) - fmin(e[2 * q - 8], e[2 * q]);
+        }
+        __syncthreads();
+    }
+    double bx[4], by[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        bx[k] = sbx[k];
+        by[k] = sby[k];
+    }
+    bool finite = true;
+#pragma unroll
+    for (int k = 0; k < 4; k++) finite = finite && isfinite(bx[k]) && isfinite(by[k]);
+    const double ex = sext[4], ey = sext[5];
+    const auto vertex = [&](int64_t q) { return clampi(a.f_vi[q < w.nvref ? q : w.nvref - 1] - 1, a.nv); };
+    // facets: each wave a run of whole 64s, in wave order
+    const int64_t run = ((nf + WAVE - 1) / WAVE + nw - 1) / nw * WAVE;
+    const int64_t i0 = run * wv, i1 = i0 + run < nf ? i0 + run : nf;
+    uint32_t* fbits = w.fbits + nf * b;
+    int cnt = 0;   // lane q: entries of list q
+    for (int64_t base = i0; base < i1; base += WAVE) {
+        const int64_t i = base + lane;
+        uint32_t bits = 0;
+        if (i < i1) {
+            const double mx = fmid[3 * i], my = fmid[3 * i + 1];
+            const uint32_t f3 = nearest_box(bx, by, sbx, sby, finite, mx, my);
+            const int64_t o0 = a.f_off[i];
+            double px[3], py[3];
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                const int64_t vq = vertex(o0 + q);
+                if (STAGE) {
+                    const double2 p = sxy[vq];
+                    px[q] = p.x;
+                    py[q] = p.y;
+                } else {
+                    px[q] = x[vq];
+                    py[q] = y[vq];
+                }
+                bits |= 1u << nearest_box(bx, by, sbx, sby, finite, px[q], py[q]);
+            }
+            const double nz = a.f_nz[nf * b + i];
+            const int64_t api = a.f_ap[i];
+            const double apn = a.ap_nz[a.na * b + clampi(api - 1, a.na)];
+            bool vis = true;
+            if (a.mode != ABT_VIS_INC) {   // midpoint outside the beam's extent (:2145-2155)
+                if (mx < sext[0]) vis = false;
+                else if (mx > sext[1]) vis = false;
+                else if (my < sext[2]) vis = false;
+                else if (my > sext[3]) vis = false;
+            }
+            const bool shad = a.mode == ABT_VIS_INT ? nz >= 0 : nz <= 0;                 // :2158, :2370, :2543
+            const bool down = a.mode == ABT_VIS_INT ? apn > -C001 : apn < C001;          // :2165, :2377, :2547
+            const bool tested = vis && !down;
+            const int64_t o = nf * b + i;
+            a.in_beam[o] = (a.mode == ABT_VIS_INC && !down) ? 1 : 0;
+            if (a.is_vis) a.is_vis[o] = tested ? 1 : 0;
+            a.dist_beam[o] = 0.0;
+            a.id_beam[o] = 0;
+            a.is_shad[o] = shad ? 1 : 0;
+            w.mapping[o] = 0;
+            // the incident beam's blockers face up (:2553)
+            if (a.mode == ABT_VIS_INC && nz < C001) bits = 0;
+            if (a.f_off[i + 1] - o0 == 3 && faces_away(a.mode, px[0], py[0], px[1], py[1], px[2], py[2], ex, ey))
+                bits = w.keep_all ? bits | F_AWAY : 0;
+            if (tested) bits |= F_TESTED | (f3 << F_BOX);
+            fbits[i] = bits;
+        }
+        const uint32_t box = bits & F_TESTED ? (bits >> F_BOX) & (NB - 1) : NB;
+#pragma unroll 4
+        for (int q = 0; q < NB; q++) {
+            const int n = __popcll(__ballot((bits >> q) & 1u)), t = __popcll(__ballot(box == (uint32_t)q));
+            cnt += lane == q ? n : (lane == NB + q ? t : 0);
+        }
+    }
+    if (lane < NQ) s_cnt[wv][lane] = cnt;
+    __syncthreads();   // (orders the zeroed mapping before the atomics too)
+    int32_t* mapping = w.mapping + nf * b;
+    if (a.mode != ABT_VIS_INC) {
+        const int64_t e0 = a.in_off[b], e1 = a.in_off[b + 1];
+        for (int64_t e = e0 + tid; e < e1; e += nt) {
+            const int64_t fi = a.field_in[e] - 1;
+            if (fi < 0 || fi >= nf) continue;
+            atomicMax(mapping + fi, (int)(e - e0 + 1));
+        }
+    }
+    // where list q of this wave's run starts (lane q): the lists before it, the waves before this one
+    int pos = 0;
+    {
+        int tot = 0, before = 0;
+        if (lane < NQ)
+            for (int k = 0; k < nw; k++) {
+                const int n = s_cnt[k][lane];
+                before += k < wv ? n : 0;
+                tot += n;
+            }
+        int end = tot;   // inclusive prefix within each 16 lists
+#pragma unroll
+        for (int o = 1; o < NB; o <<= 1) {
+            const int u = __shfl_up(end, o, NB);
+            end += (lane & (NB - 1)) >= o ? u : 0;
+        }
+        pos = end - tot + before;
+        if (wv == 0 && lane < NQ) {
+            int32_t* offs = w.offs + (int64_t)OFFS * b + (lane / NB) * (NB + 1);
+            offs[lane & (NB - 1)] = end - tot;
+            if ((lane & (NB - 1)) == NB - 1) offs[NB] = end;
+        }
+    }
+    __syncthreads();   // the mapping is complete
+    Cand* cand = w.cand + 3 * nf * b;
+    int32_t* mlist = w.mlist + nf * b;
+    for (int64_t base = i0; base < i1; base += WAVE) {
+        const int64_t i = base + lane;
+        const uint32_t bits = i < i1 ? fbits[i] : 0u;
+        const uint32_t box = bits & F_TESTED ? (bits >> F_BOX) & (NB - 1) : NB;
+        Cand c;
+        if (bits & 0xffffu) {
+            const int64_t o0 = a.f_off[i];
+            c.z = fmid[3 * i + 2];
+            c.j = (int)i;
+#pragma unroll
+            for (int q = 0; q < 3; q++) c.v[q] = (int)vertex(o0 + q);
+            if (a.f_off[i + 1] - o0 != 3) c.v[0] |= INT_MIN;
+            if (bits & F_AWAY) c.v[1] |= INT_MIN;
+            c.ap = (int)a.f_ap[i];
+            // written by atomics in L2, past this CU's cache
+            c.map = __hip_atomic_load(mapping + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        for (int q = 0; q < NQ; q++) {
+            const bool in = q < NB ? (bits >> q) & 1u : box == (uint32_t)(q - NB);
+            const unsigned long long bal = __ballot(in);
+            if (!bal) continue;
+            const int p = __builtin_amdgcn_readlane(pos, q) + lanes_below(bal);
+            if (in) {
+                if (q < NB) cand[p] = c;
+                else mlist[p] = (int32_t)i;
+            }
+            pos += lane == q ? __popcll(bal) : 0;
+        }
     }
 }
 
 // ---------------------------------------------------------------------------
-template <int MODE, bool COUNT>
-__global__ __launch_bounds__(WAVE) void k_vis_main(abt_vis_batch a, Work w)
+// The scan.  int, ext: each wave one unit (box, 64-facet slice of the box's tested list).  inc: the candidates'
+// effects are ORs and ANDs, in any order, so the workgroup's waves share one unit and take a part of its
+// candidates each, which a single incident beam (48 units on the whole chip) needs.
+// Bound by VALU issue and by the length of a beam's last units.  Nothing is gathered per lane: a tile of
+// candidates gathered lane by lane (13 loads of 64 lines each: entry, facet, vertices) kept the CU's
+// address unit busy for as long as the scan of the tile took, and waited for three loads in a row.  The
+// workgroup's waves take its units as they come free; a workgroup per few units, each wave with one,
+// left half the waves without work.  2048 beams x 2112 facets: 536 -> 324 us (half of the scan from leaving out
+// the candidates that face away); one incident beam 45 -> 10 us.  STAGE: vertices in LDS; beyond STAGE_NV
+// from memory.
+template <int MODE, bool COUNT, bool STAGE>
+__global__ __launch_bounds__(MW * WAVE, COUNT ? 4 : 8) void k_vis_main(abt_vis_batch a, Work w)
 {
 #pragma clang fp contract(off)
-    const int64_t b = w.b0 + blockIdx.y;
-    const int u = blockIdx.x;
-    const int lane = threadIdx.x;
+    constexpr bool SHARE = MODE == ABT_VIS_INC;
+    extern __shared__ double2 sxy[];
+    __shared__ int s_res[SHARE ? MW : 1][WAVE];
+    __shared__ int s_next;
+    // workgroups go round the XCDs: all of a beam's on one, next to each other, the one its set-up ran on
+    const int k8 = blockIdx.x / XCDS, bi = k8 / w.parts * XCDS + blockIdx.x % XCDS, part = k8 % w.parts;
+    if (bi >= w.nb) return;
+    const int64_t b = w.b0 + bi;
+    const int lane = threadIdx.x & (WAVE - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int64_t nf = a.nf;
     const int32_t* offs = w.offs + (int64_t)OFFS * b;
-    // unit u -> (box, 64-facet slice of that box's tested list)
-    int bb = -1, t = 0, acc = 0;
-    for (int k = 0; k < NB; k++) {
-        const int n = offs[NB + 2 + k] - offs[NB + 1 + k];
-        const int nu = (n + WAVE - 1) / WAVE;
-        if (bb < 0 && u < acc + nu) {
-            bb = k;
-            t = u - acc;
-        }
-        acc += nu;
+    // lane k: the end of box k's units (64-facet slices of its tested list) among the beam's
+    int ends = 0;
+    if (lane < NB) ends = (offs[NB + 2 + lane] - offs[NB + 1 + lane] + WAVE - 1) / WAVE;
+#pragma unroll
+    for (int o = 1; o < NB; o <<= 1) {
+        const int e = __shfl_up(ends, o, NB);
+        ends += lane >= o ? e : 0;
     }
-    if (bb < 0) return;   // uniform: no work for this unit
-    const int mi = offs[NB + 1 + bb] + t * WAVE + lane;
-    const bool has = mi < offs[NB + 2 + bb];
-    const int64_t m = has ? w.mlist[nf * b + mi] : 0;
-    const double* mid = a.f_mid + 3 * nf * b + 3 * m;
-    const double mx = mid[0], my = mid[1], mz = mid[2];
-    const int apm = (int)a.f_ap[m];
-    const int2* cand = w.cand + 3 * nf * b;
-    const int32_t* mapping = w.mapping + nf * b;
-    bool done = !has;
-    bool vis = true, inb = MODE == ABT_VIS_INC, shad = false;
-    int32_t idb = 0;
-    double dist = 0.0, zbest = 0.0;
-    uint64_t npair = 0, nedge = 0;
-    // Candidates are staged TC at a time: lane c < TC gathers candidate c's depth, aperture,
-    // vertex count, mapping and first NVS projected vertices into LDS with independent loads;
-    // then every lane walks the tile in order, reading each slot at one LDS address (a
-    // broadcast) and forming the edge normals per pair as the reference does.
-    __shared__ double tile[TC * SLOT];
+    const int total = __builtin_amdgcn_readlane(ends, NB - 1);
+    if (part >= total) return;   // no unit for the workgroup
     const double* vx = a.v + 3 * a.nv * b;
     const double* vy = vx + a.nv;
-    const double* zmid = a.f_mid + 3 * nf * b + 2;
-    const int64_t* fvi = a.f_vi;
-    const int k0 = offs[bb], k1 = offs[bb + 1];
-    for (int kt = k0; kt < k1; kt += TC) {
-        if (__all(done)) break;
-        const int nt = min(TC, k1 - kt);
-        if (lane < nt) {
-            const int2 cj = cand[kt + lane];
-            const int64_t j = cj.x, o0 = cj.y;
-            const int nvj = (int)(a.f_off[j + 1] - o0);
-            double* sl = tile + lane * SLOT;
-            sl[0] = zmid[3 * j];
-            sl[1] = __builtin_bit_cast(double, make_int2((int)a.f_ap[j], nvj));
-            sl[2] = __builtin_bit_cast(double, make_int2((int)j, mapping[j]));
-            sl[3] = __builtin_bit_cast(double, make_int2((int)o0, 0));
-            const int ns = min(nvj, NVS);
-            for (int e = 0; e < ns; e++) {
-                const int64_t vi = clampi(fvi[min(o0 + e, w.nvref - 1)] - 1, a.nv);
-                sl[4 + 2 * e] = vx[vi];
-                sl[5 + 2 * e] = vy[vi];
-            }
+    if (STAGE) {
+        for (int i = threadIdx.x; i < (int)a.nv; i += MW * WAVE) sxy[i] = make_double2(vx[i], vy[i]);
+    }
+    if (threadIdx.x == 0) s_next = 0;
+    __syncthreads();
+    const auto at = [&](int v) { return STAGE ? sxy[v] : make_double2(vx[v], vy[v]); };
+    // units part, part + parts, ...: taken by the waves as they come free, or (SHARE) by all waves together
+    uint64_t npair = 0, nedge = 0;
+    for (int n = 0;; n++) {
+        if (!SHARE) {
+            int t = 0;
+            if (lane == 0) t = atomicAdd(&s_next, 1);
+            n = __builtin_amdgcn_readfirstlane(t);
         }
-        __syncthreads();
+        const int u = part + n * w.parts;
+        if (u >= total) break;
+        const int bb = __popcll(__ballot(lane < NB && ends <= u));
+        const int t = u - (bb > 0 ? __builtin_amdgcn_readlane(ends, bb - 1) : 0);
+        const int mi = offs[NB + 1 + bb] + t * WAVE + lane;
+        const bool has = mi < offs[NB + 2 + bb];
+        const int m = has ? w.mlist[nf * b + mi] : 0;
+        const double* mid = a.f_mid + 3 * nf * b + 3 * (int64_t)m;
+        const double mx = mid[0], my = mid[1], mz = mid[2];
+        const int apm = (int)a.f_ap[m];
+        const Cand* cand = w.cand + 3 * nf * b;
+        bool done = !has;
+        bool vis = true, inb = MODE == ABT_VIS_INC, shad = false;
+        int32_t idb = 0;
+        double dist = 0.0, zbest = 0.0;
+        // edge k from vertex k to k+1 (the last back to the first): edge_norm1 = y_{k+1} - y_k,
+        // edge_norm2 = -x_{k+1} + x_k, offset (mx - x_k, my - y_k) (:2149-2162)
+        const auto outside = [&](double2 p, double2 q) {
+#pragma clang fp contract(off)
+            const double en2 = -q.x + p.x, en1 = q.y - p.y;
+            const double vb1 = mx - p.x, vb2 = my - p.y;
+            const double chk = MODE == ABT_VIS_EXT ? -vb1 * en1 - vb2 * en2 : vb1 * en1 + vb2 * en2;
+            return chk > 0;
+        };
+        int c0 = offs[bb], c1 = offs[bb + 1];
+        if (SHARE) {
+            const int n = c1 - c0;
+            c1 = c0 + (int)((int64_t)n * (wv + 1) / MW);
+            c0 = c0 + (int)((int64_t)n * wv / MW);
+        }
         // UNR candidates at a time: their depth and edge tests are independent of the scan state,
-        // so they are evaluated together (their LDS reads and FP64 chains overlap); the
+        // so they are evaluated together (their loads and FP64 chains overlap); the
         // reference's order-dependent rules are then applied to them in candidate order.
-        for (int c = 0; c < nt; c += UNR) {
+        for (int c = c0; c < c1; c += UNR) {
             if (__all(done)) break;
             bool pr[UNR], fr[UNR], hit[UNR];
-            double qz[UNR];
-            int qap[UNR], qmap[UNR], qnv[UNR];
+            Cand e[UNR];
+#pragma unroll
+            for (int q = 0; q < UNR; q++) e[q] = load_scalar(cand + min(c + q, c1 - 1));
+            bool poly = false;
 #pragma unroll
             for (int q = 0; q < UNR; q++) {
-                const bool valid = c + q < nt;
-                const double* sl = tile + (valid ? c + q : 0) * SLOT;
-                const int2 jm = __builtin_bit_cast(int2, sl[2]);
-                const int2 an = __builtin_bit_cast(int2, sl[1]);
-                qz[q] = sl[0];
-                qap[q] = an.x;
-                qnv[q] = an.y;
-                qmap[q] = jm.y;
-                pr[q] = valid && jm.x != m;
-                fr[q] = pr[q] && !(mz > qz[q]);                         // blocker not behind m
-                // edge k from vertex k to k+1 (the last back to the first): edge_norm1 =
-                // y_{k+1} - y_k, edge_norm2 = -x_{k+1} + x_k, offset (mx - x_k, my - y_k)
-                // (:2149-2162)
-                auto outside = [&](double xa, double ya, double xb, double yb) {
-                    const double en2 = -xb + xa, en1 = yb - ya;
-                    const double vb1 = mx - xa, vb2 = my - ya;
-                    const double chk = MODE == ABT_VIS_EXT ? -vb1 * en1 - vb2 * en2 : vb1 * en1 + vb2 * en2;
-                    return chk > 0;
-                };
-                const double x0 = sl[4], y0 = sl[5];
-                bool within;
-                if (an.y == 3) {
-                    const double x1 = sl[6], y1 = sl[7], x2 = sl[8], y2 = sl[9];
-                    const bool o0 = outside(x0, y0, x1, y1), o1 = outside(x1, y1, x2, y2),
-                               o2 = outside(x2, y2, x0, y0);
-                    within = !(o0 || o1 || o2);
-                } else {
-                    within = true;
-                    const int64_t o0 = __builtin_bit_cast(int2, sl[3]).x;
-                    double xa = x0, ya = y0;
-                    for (int e = 0; e < an.y; e++) {
-                        const int en = e + 1 == an.y ? 0 : e + 1;
-                        double xb, yb;
-                        if (en < NVS) {
-                            xb = sl[4 + 2 * en];
-                            yb = sl[5 + 2 * en];
-                        } else {
-                            const int64_t vi = clampi(fvi[min(o0 + en, w.nvref - 1)] - 1, a.nv);
-                            xb = vx[vi];
-                            yb = vy[vi];
-                            // keeps the two branches' loads apart: merged, they would become one
-                            // load through a generic pointer
-                            asm volatile("" : "+v"(xb), "+v"(yb));
-                        }
-                        if (outside(xa, ya, xb, yb)) {
-                            within = false;
-                            break;
-                        }
-                        xa = xb;
-                        ya = yb;
+                // (past the end the last candidate comes again, which changes nothing but the counts)
+                pr[q] = (!COUNT || c + q < c1) && e[q].j != m;
+                fr[q] = pr[q] && !(mz > e[q].z);                         // blocker not behind m
+                const double2 p0 = at(e[q].v[0] & INT_MAX), p1 = at(e[q].v[1] & INT_MAX), p2 = at(e[q].v[2]);
+                const bool o0 = outside(p0, p1), o1 = outside(p1, p2), o2 = outside(p2, p0);
+                hit[q] = fr[q] && !(o0 || o1 || o2);
+                poly = poly || e[q].v[0] < 0;
+            }
+            if (poly) {   // uniform
+#pragma unroll
+                for (int q = 0; q < UNR; q++) {
+                    if (e[q].v[0] >= 0) continue;
+                    const int64_t o0 = a.f_off[e[q].j];
+                    const int nv = (int)(a.f_off[e[q].j + 1] - o0);
+                    const double2 p0 = at(e[q].v[0] & INT_MAX);
+                    double2 p = p0;
+                    bool within = true;
+                    for (int k = 1; k <= nv; k++) {
+                        const int64_t o = o0 + k < w.nvref ? o0 + k : w.nvref - 1;
+                        const double2 n = k == nv ? p0 : at((int)clampi(a.f_vi[o] - 1, a.nv));
+                        within = within && !outside(p, n);
+                        p = n;
                     }
+                    hit[q] = fr[q] && within;
                 }
-                hit[q] = fr[q] && within;
             }
 #pragma unroll
             for (int q = 0; q < UNR; q++) {
+                if (!COUNT && !__any(hit[q] && !done)) continue;
                 if (done) break;
                 if (COUNT) {
                     npair += pr[q] ? 1 : 0;
-                    nedge += fr[q] ? (uint64_t)qnv[q] : 0;
+                    nedge += fr[q] ? (uint64_t)(e[q].v[0] >= 0 ? 3 : a.f_off[e[q].j + 1] - a.f_off[e[q].j]) : 0;
                 }
                 if (!hit[q]) continue;
                 if (MODE == ABT_VIS_INC) {                                // :2573-2580
-                    if (apm == qap[q]) shad = true;
+                    if (apm == e[q].ap) shad = true;
                     else {
                         vis = false;
                         inb = false;
                     }
                     continue;
                 }
-                if (qmap[q] > 0) {                                        // a beam facet: keep the nearest (:2166-2180)
-                    if (!inb || qz[q] < zbest) {
+                if (e[q].map > 0) {                                       // a beam facet: keep the nearest (:2166-2180)
+                    if (!inb || e[q].z < zbest) {
                         inb = true;
-                        idb = qmap[q];
-                        dist = qz[q] - mz;
-                        zbest = qz[q];
+                        idb = e[q].map;
+                        dist = e[q].z - mz;
+                        zbest = e[q].z;
                     }
                 } else {                                                  // a blocker (:2181-2197)
-                    if (apm == qap[q]) continue;
-                    if (inb && qz[q] > zbest) continue;
+                    if (apm == e[q].ap) continue;
+                    if (inb && e[q].z > zbest) continue;
                     vis = false;
                     inb = false;
                     done = true;
                 }
             }
         }
-        __syncthreads();
+        if (SHARE) {   // blocked (2) and shadowed (1) by any of the waves' candidates
+            s_res[wv][lane] = (inb ? 0 : 2) | (shad ? 1 : 0);
+            __syncthreads();
+            int r = 0;
+#pragma unroll
+            for (int k = 0; k < MW; k++) r |= s_res[k][lane];
+            __syncthreads();
+            inb = vis = !(r & 2);
+            shad = r & 1;
+        }
+        if (has && (!SHARE || wv == 0)) {
+            const int64_t o = nf * b + m;
+            a.in_beam[o] = inb ? 1 : 0;
+            if (a.is_vis) a.is_vis[o] = vis ? 1 : 0;
+            if (MODE == ABT_VIS_INC) {                                    // :2597-2602
+                if (shad) a.is_shad[o] = 1;
+                if (inb) {
+                    a.dist_beam[o] = a.beam_mid_z[b] - mz;
+                    a.id_beam[o] = 1;
+                }
+            } else {
+                a.dist_beam[o] = dist;
+                a.id_beam[o] = idb;
+            }
+        }
     }
     if (COUNT) {
 #pragma unroll
@@ -519,20 +590,6 @@ __global__ __launch_bounds__(WAVE) void k_vis_main(abt_vis_batch a, Work w)
             atomicAdd(a.counts, (unsigned long long)npair);
             atomicAdd(a.counts + 1, (unsigned long long)nedge);
         }
-    }
-    if (!has) return;
-    const int64_t o = nf * b + m;
-    a.in_beam[o] = inb ? 1 : 0;
-    if (a.is_vis) a.is_vis[o] = vis ? 1 : 0;
-    if (MODE == ABT_VIS_INC) {                                    // :2597-2602
-        if (shad) a.is_shad[o] = 1;
-        if (inb) {
-            a.dist_beam[o] = a.beam_mid_z[b] - mz;
-            a.id_beam[o] = 1;
-        }
-    } else {
-        a.dist_beam[o] = dist;
-        a.id_beam[o] = idb;
     }
 }
 
@@ -596,7 +653,7 @@ constexpr size_t ALIGN = 256;
 size_t up(size_t n) { return (n + ALIGN - 1) / ALIGN * ALIGN; }
 
 struct Layout {
-    size_t boxes, fbox, fmask, mapping, offs, cand, mlist, total;
+    size_t fbits, mapping, offs, cand, mlist, total;
 };
 
 Layout layout(int64_t nbeam, int64_t nf, int64_t nvref)
@@ -604,48 +661,55 @@ Layout layout(int64_t nbeam, int64_t nf, int64_t nvref)
     Layout L;
     size_t o = 0;
     const size_t nb = (size_t)nbeam, f = (size_t)nf;
-    L.boxes = o;   o += up(nb * sizeof(abt::vis::BeamBox));
-    L.fbox = o;    o += up(nb * f * 4);
-    L.fmask = o;   o += up(nb * f * 4);
+    L.fbits = o;   o += up(nb * f * 4);
     L.mapping = o; o += up(nb * f * 4);
     L.offs = o;    o += up(nb * abt::vis::OFFS * 4);
-    L.cand = o;    o += up(nb * 3 * f * 8);
+    L.cand = o;    o += up(nb * 3 * f * sizeof(abt::vis::Cand));
     L.mlist = o;   o += up(nb * f * 4);
     L.total = o;
     return L;
 }
 
-int launch_all(const abt_vis_batch& a, int64_t nvref, char* ws, hipStream_t st)
+int launch_all(const abt_vis_batch& a, int64_t nvref, char* ws, int cus, hipStream_t st)
 {
     using namespace abt::vis;
     const Layout L = layout(a.nbeam, a.nf, nvref);
     Work w;
-    w.boxes = (BeamBox*)(ws + L.boxes);
-    w.fbox = (int32_t*)(ws + L.fbox);
-    w.fmask = (int32_t*)(ws + L.fmask);
+    w.fbits = (uint32_t*)(ws + L.fbits);
     w.mapping = (int32_t*)(ws + L.mapping);
     w.offs = (int32_t*)(ws + L.offs);
-    w.cand = (int2*)(ws + L.cand);
+    w.cand = (Cand*)(ws + L.cand);
     w.mlist = (int32_t*)(ws + L.mlist);
     w.nvref = nvref;
-    const unsigned ftiles = (unsigned)((a.nf + BLK - 1) / BLK);
-    const unsigned units = (unsigned)((a.nf + WAVE - 1) / WAVE + NB);
+    // a scan alone may count what an earlier set-up listed
+    w.keep_all = a.counts || a.phases != 0;
+    const bool stage = a.nv <= STAGE_NV;
+    const size_t lds = stage ? sizeof(double2) * (size_t)a.nv : 0;
+    // 64-facet slices of the tested lists, at most
+    const int64_t slices = (a.nf + WAVE - 1) / WAVE + NB;
     const bool setup = a.phases != 2, scan = a.phases != 1;
     for (int64_t b0 = 0; b0 < a.nbeam; b0 += BEAM_CHUNK) {
         const unsigned nb = (unsigned)std::min<int64_t>(BEAM_CHUNK, a.nbeam - b0);
         w.b0 = b0;
         if (setup) {
-            hipLaunchKernelGGL(k_vis_boxes, dim3(nb), dim3(BLK), 0, st, a, w);
-            hipLaunchKernelGGL(k_vis_facets, dim3(ftiles, nb), dim3(BLK), 0, st, a, w);
-            if (a.mode != ABT_VIS_INC) hipLaunchKernelGGL(k_vis_map, dim3(nb), dim3(BLK), 0, st, a, w);
-            hipLaunchKernelGGL(k_vis_lists, dim3(nb), dim3(BLK), 0, st, a, w);
+            // with fewer beams than CUs a workgroup may as well be large
+            const unsigned nt = nb < 256 && a.nf > SETUP ? SETUP_FEW : SETUP;
+            if (stage) hipLaunchKernelGGL(k_vis_setup<true>, dim3(nb), dim3(nt), lds, st, a, w);
+            else hipLaunchKernelGGL(k_vis_setup<false>, dim3(nb), dim3(nt), 0, st, a, w);
         }
         if (!scan) continue;
-        const dim3 g(units, nb);
-#define VM(M)                                                                           \
-    do {                                                                                \
-        if (a.counts) hipLaunchKernelGGL((k_vis_main<M, true>), g, dim3(WAVE), 0, st, a, w);  \
-        else hipLaunchKernelGGL((k_vis_main<M, false>), g, dim3(WAVE), 0, st, a, w);          \
+        // As many workgroups a beam as there are units for, up to twice the chip's (8 per CU at 8 waves per SIMD): a
+        // beam's last unit then holds fewer waves up (2048 beams: 0.63, 0.57, 0.57 ms a batch with 1, 2, 4).
+        const int64_t most = a.mode == ABT_VIS_INC ? slices : (slices + MW - 1) / MW;
+        w.nb = (int)nb;
+        w.parts = (int)std::max<int64_t>(1, std::min<int64_t>(most, (16 * cus + nb - 1) / nb));
+        const dim3 g((nb + XCDS - 1) / XCDS * XCDS * (unsigned)w.parts), wg(MW * WAVE);
+#define VM(M)                                                                                            \
+    do {                                                                                                 \
+        if (a.counts && stage) hipLaunchKernelGGL((k_vis_main<M, true, true>), g, wg, lds, st, a, w);    \
+        else if (a.counts) hipLaunchKernelGGL((k_vis_main<M, true, false>), g, wg, 0, st, a, w);         \
+        else if (stage) hipLaunchKernelGGL((k_vis_main<M, false, true>), g, wg, lds, st, a, w);          \
+        else hipLaunchKernelGGL((k_vis_main<M, false, false>), g, wg, 0, st, a, w);                      \
     } while (0)
         if (a.mode == ABT_VIS_INT) VM(ABT_VIS_INT);
         else if (a.mode == ABT_VIS_EXT) VM(ABT_VIS_EXT);
@@ -665,6 +729,7 @@ int check_batch(const abt_vis_batch* a)
     if (a->nbeam < 0 || a->nf < 1 || a->nv < 1 || a->na < 1)
         return abt_fail(ABT_ERR_ARG, "visibility: need nbeam >= 0, nf, nv, na >= 1");
     if (a->nf >= (1LL << 31) / 3) return abt_fail(ABT_ERR_ARG, "visibility: too many facets (%lld)", (long long)a->nf);
+    if (a->nv >= (1LL << 31)) return abt_fail(ABT_ERR_ARG, "visibility: too many vertices (%lld)", (long long)a->nv);
     if (!a->f_off || !a->f_vi || !a->f_ap || !a->v || !a->f_mid || !a->f_nz || !a->ap_nz || !a->in_off ||
         !a->in_beam || !a->dist_beam || !a->id_beam || !a->is_shad)
         return abt_fail(ABT_ERR_ARG, "visibility: null array");
@@ -694,9 +759,10 @@ extern "C" int abt_find_vis_dev(const abt_vis_batch* a, int64_t nvref, void* wor
     if (!workspace || bytes < need)
         return abt_fail(ABT_ERR_ARG, "visibility workspace of %zu bytes is smaller than %zu", bytes, need);
     if ((uintptr_t)workspace % ALIGN) return abt_fail(ABT_ERR_ARG, "visibility workspace is not 256-byte aligned");
-    rc = abt_ensure_device(nullptr);
+    int cus = 0;
+    rc = abt_ensure_device(&cus);
     if (rc) return rc;
-    return launch_all(*a, nvref, (char*)workspace, (hipStream_t)stream);
+    return launch_all(*a, nvref, (char*)workspace, cus, (hipStream_t)stream);
 }
 
 extern "C" int abt_find_vis(int mode, const abt_vis_geometry* geo, int64_t nf_in, const int64_t* field_in,
@@ -712,6 +778,7 @@ extern "C" int abt_find_vis(int mode, const abt_vis_geometry* geo, int64_t nf_in
         !in_beam || !dist_beam || !id_beam || !is_shad)
         return abt_fail(ABT_ERR_ARG, "abt_find_vis: null array");
     if (nf >= (1LL << 31) / 3) return abt_fail(ABT_ERR_ARG, "abt_find_vis: too many facets (%lld)", (long long)nf);
+    if (nv >= (1LL << 31)) return abt_fail(ABT_ERR_ARG, "abt_find_vis: too many vertices (%lld)", (long long)nv);
     if (geo->f_off[0] != 0) return abt_fail(ABT_ERR_ARG, "abt_find_vis: f_off[0] must be 0");
     for (int64_t i = 0; i < nf; i++) {
         if (geo->f_off[i + 1] - geo->f_off[i] < 3)
@@ -785,7 +852,9 @@ extern "C" int abt_find_vis(int mode, const abt_vis_geometry* geo, int64_t nf_in
     a.is_shad = (uint8_t*)(d + o_shad);
     a.counts = nullptr;
     a.phases = 0;
-    rc = launch_all(a, nvref, d + o_ws, st);
+    int cus = 0;
+    rc = abt_ensure_device(&cus);
+    if (!rc) rc = launch_all(a, nvref, d + o_ws, cus, st);
     if (rc) return rc;
     HIPCHK(hipMemcpyAsync(in_beam, d + o_inb, nf, hipMemcpyDeviceToHost, st));
     if (is_vis) HIPCHK(hipMemcpyAsync(is_vis, d + o_vis, nf, hipMemcpyDeviceToHost, st));
