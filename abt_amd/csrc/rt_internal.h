@@ -14,6 +14,8 @@ int abt_ensure_device(int* cus);
 // The calling thread's stream and its grow-only device buffer `slot` (at least `bytes`
 // long; slot 8 belongs to the visibility entry points).
 int abt_thread_staging(int slot, size_t bytes, hipStream_t* st, void** p);
+// `bytes` of the calling thread's pinned host memory, for the call that asks; null: too many, or none to pin.
+char* abt_thread_pinned(size_t bytes);
 
 #define HIPCHK(expr)                                                                      \
     do {                                                                                  \

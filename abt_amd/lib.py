@@ -152,8 +152,12 @@ def grid_struct(theta, phi):
 
 def raw_to_complex(raw, nphi, nth):
     """Fortran-layout (phi, theta, 2, 2) doubles -> complex [r, c, theta, phi]."""
-    a = np.asarray(raw).reshape(2, 2, nth, nphi, 2)
-    return (a[..., 0] + 1j * a[..., 1]).transpose(1, 0, 2, 3)
+    return _complex_view(np.array(raw, dtype=np.float64), nphi, nth)
+
+
+def _complex_view(raw, nphi, nth):
+    """raw_to_complex over the buffer itself."""
+    return raw.reshape(-1).view(np.complex128).reshape(2, 2, nth, nphi).transpose(1, 0, 2, 3)
 
 
 # ---------------------------------------------------------------------------
@@ -183,7 +187,7 @@ def diff_main(theta, phi, lam, beams: BeamSet, ext: BeamSet, precision="fp64", f
                                 _ptr(oe) if oe is not None else None))
     if raw:
         return ob, oe
-    conv = lambda o: None if o is None else raw_to_complex(o, len(phi), len(theta))
+    conv = lambda o: None if o is None else _complex_view(o, len(phi), len(theta))
     return conv(ob), conv(oe)
 
 
@@ -198,7 +202,7 @@ def diffraction(theta, phi, x, y, z, lam, beams: BeamSet, b, precision="fp64", f
                                   _ptr(_f64(beams.vk7[b])), _ptr(_f64(beams.prop[b])),
                                   float(beams.fov[b]), int(o1 - o0), _ptr(verts),
                                   PRECISIONS[precision], _ptr(out)))
-    return raw_to_complex(out, len(phi), len(theta))
+    return _complex_view(out, len(phi), len(theta))
 
 
 def prepare_beams_host(beams: BeamSet, lam, fov_value=None):

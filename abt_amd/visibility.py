@@ -145,8 +145,8 @@ def find_vis(mode, geom: VisGeometry, field_in=None, beam_mid_z=0.0):
     lib._check(L.abt_find_vis(int(mode), ctypes.byref(g), len(fin), fin.ctypes.data if len(fin) else None,
                               float(beam_mid_z), inb.ctypes.data, vis.ctypes.data, dist.ctypes.data,
                               idb.ctypes.data, shad.ctypes.data))
-    return dict(in_beam=inb.astype(bool), is_vis=vis.astype(bool), dist_beam=dist, id_beam=idb,
-                is_shad=shad.astype(bool))
+    return dict(in_beam=inb.view(bool), is_vis=vis.view(bool), dist_beam=dist, id_beam=idb,
+                is_shad=shad.view(bool))
 
 
 def find_vis_int(field_in, rot_geometry: VisGeometry):
