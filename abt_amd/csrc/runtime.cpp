@@ -256,15 +256,19 @@ Cut cut_long(int64_t nbins, int64_t nb, int cus)
     return cut_into(nb, std::min<int64_t>(want, nb / 512), 32);
 }
 
-// The cut where a workspace for it is at hand.  When the segments of cut_long leave the chip with
-// fewer than 8 workgroups per CU, shorter ones (down to 8 beams, the mixed body's group) fill it: the default column's
-// 2838 + 864 beams on 64,980 bins (254 tiles), plain FP64, 8.1 -> 7.6 ms a diff_main call.
+// The cut where a workspace for it is at hand, when the segments of cut_long leave the chip with few
+// workgroups.  Their times differ (forward rows, branches), so the last round shrinks with their size until the
+// start of a workgroup (its table, its first records) and the segment sums weigh: 24 workgroups per CU of at
+// least 40 beams, and below that 8 per CU of at least 8 beams (the mixed body's group).  Measured, us, with the
+// segments per list named: 3252 beams on 254 tiles of bins, plain FP64 2744 (9), 2605 (16), 2609 (24), 2583 (32),
+// restructured 1412, 1283, 1238, 1230; 648 beams on them 559 (9), 538 (16), 551 (24), restructured 323, 289, 297.
 Cut cut_beams(int64_t nbins, int64_t nb, int cus)
 {
     const int64_t tiles = (nbins + 255) / 256;
     const Cut l = cut_long(nbins, nb, cus);
-    const int64_t fill = ((int64_t)cus * 8 + tiles - 1) / tiles;
-    return fill > l.nseg ? cut_into(nb, std::min<int64_t>(fill, nb / 8), 8) : l;
+    const auto fill = [&](int64_t per_cu) { return ((int64_t)cus * per_cu + tiles - 1) / tiles; };
+    const int64_t n = std::max(std::min(fill(8), nb / 8), std::min(fill(24), nb / 40));
+    return n > l.nseg ? cut_into(nb, n, 8) : l;
 }
 
 }  // namespace
