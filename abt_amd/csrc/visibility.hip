@@ -178,7 +178,7 @@ __device__ __forceinline__ int lanes_below(unsigned long long m)
 // facet of initial outputs, 32 a list entry, 64 read), by the latency of its steps for one beam.  As four
 // kernels (boxes, facets, map, lists) with each facet's box and mask in memory between them, sixteen
 // distances a search and four barriers a block of 256 facets in the list building, 2048 beams x 2112
-// facets took 256 us; here 204.  One beam: 49 us and two more launches; here 34.
+// facets took 256 us; here 184.  One beam: 49 us and two more launches; here 30.
 // STAGE: the beam's projected vertices are kept in LDS (nv <= STAGE_NV): their gathers, 64 lines each,
 // otherwise fill the CU's address unit.
 template <bool STAGE>
@@ -273,6 +273,7 @@ __global__ __launch_bounds__(SETUP_FEW) void k_vis_setup(abt_vis_batch a, Work w
     for (int k = 0; k < 4; k++) finite = finite && isfinite(bx[k]) && isfinite(by[k]);
     const double ex = sext[4], ey = sext[5];
     const auto vertex = [&](int64_t q) { return clampi(a.f_vi[q < w.nvref ? q : w.nvref - 1] - 1, a.nv); };
+    const auto at = [&](int v) { return STAGE ? sxy[v] : make_double2(x[v], y[v]); };
     // facets: each wave a run of whole 64s, in wave order
     const int64_t run = ((nf + WAVE - 1) / WAVE + nw - 1) / nw * WAVE;
     const int64_t i0 = run * wv, i1 = i0 + run < nf ? i0 + run : nf;
@@ -283,25 +284,12 @@ __global__ __launch_bounds__(SETUP_FEW) void k_vis_setup(abt_vis_batch a, Work w
         uint32_t bits = 0;
         if (i < i1) {
             const double mx = fmid[3 * i], my = fmid[3 * i + 1];
-            const uint32_t f3 = nearest_box(bx, by, sbx, sby, finite, mx, my);
-            const int64_t o0 = a.f_off[i];
-            double px[3], py[3];
-#pragma unroll
-            for (int q = 0; q < 3; q++) {
-                const int64_t vq = vertex(o0 + q);
-                if (STAGE) {
-                    const double2 p = sxy[vq];
-                    px[q] = p.x;
-                    py[q] = p.y;
-                } else {
-                    px[q] = x[vq];
-                    py[q] = y[vq];
-                }
-                bits |= 1u << nearest_box(bx, by, sbx, sby, finite, px[q], py[q]);
-            }
             const double nz = a.f_nz[nf * b + i];
             const int64_t api = a.f_ap[i];
             const double apn = a.ap_nz[a.na * b + clampi(api - 1, a.na)];
+            const int64_t o0 = a.f_off[i];
+            const bool tri = a.f_off[i + 1] - o0 == 3;
+            const int v0 = (int)vertex(o0), v1 = (int)vertex(o0 + 1), v2 = (int)vertex(o0 + 2);
             bool vis = true;
             if (a.mode != ABT_VIS_INC) {   // midpoint outside the beam's extent (:2145-2155)
                 if (mx < sext[0]) vis = false;
@@ -319,11 +307,22 @@ __global__ __launch_bounds__(SETUP_FEW) void k_vis_setup(abt_vis_batch a, Work w
             a.id_beam[o] = 0;
             a.is_shad[o] = shad ? 1 : 0;
             w.mapping[o] = 0;
-            // the incident beam's blockers face up (:2553)
-            if (a.mode == ABT_VIS_INC && nz < C001) bits = 0;
-            if (a.f_off[i + 1] - o0 == 3 && faces_away(a.mode, px[0], py[0], px[1], py[1], px[2], py[2], ex, ey))
-                bits = w.keep_all ? bits | F_AWAY : 0;
-            if (tested) bits |= F_TESTED | (f3 << F_BOX);
+            // Neighbours agree, so a wave mostly skips the search of the midpoint's box or the vertices'.
+            // The incident beam's blockers face up (:2553).
+            bool away = false;
+            if (tri) {
+                const double2 p0 = at(v0), p1 = at(v1), p2 = at(v2);
+                away = faces_away(a.mode, p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, ex, ey);
+            }
+            if (tested) bits = F_TESTED | (uint32_t)nearest_box(bx, by, sbx, sby, finite, mx, my) << F_BOX;
+            if (!(a.mode == ABT_VIS_INC && nz < C001) && (w.keep_all || !away)) {
+                if (away) bits |= F_AWAY;
+#pragma unroll 1
+                for (int q = 0; q < 3; q++) {
+                    const double2 p = at(q == 0 ? v0 : (q == 1 ? v1 : v2));
+                    bits |= 1u << nearest_box(bx, by, sbx, sby, finite, p.x, p.y);
+                }
+            }
             fbits[i] = bits;
         }
         const uint32_t box = bits & F_TESTED ? (bits >> F_BOX) & (NB - 1) : NB;
