@@ -533,7 +533,7 @@ __host__ __device__ __forceinline__ void adj_bin_far(const AdjBeam& B, const Adj
                                                      const double* __restrict__ tab, double k, double kt,
                                                      AdjSum& acc)
 {
-    const FarGeom u = far_geometry_of(B.c, B.cc, kt, bn.f, far);
+    const FarGeom u = far_geometry(B.c, B.cc, kt, bn.f, far);
     const double kd = u.kd + bn.kr;
     const double k1 = fma(u.ux, B.ex[0], fma(u.uy, B.ex[1], u.uz * B.ex[2]));
     const double k2 = fma(u.ux, B.ey[0], fma(u.uy, B.ey[1], u.uz * B.ey[2]));

@@ -30,6 +30,15 @@ namespace abt {
 
 constexpr int BLOCK = 256;
 
+// A wave-uniform record through scalar loads: records are not written while a sweep runs, which the constant
+// address space says (barriers and LDS stores in the loop would otherwise rule them out).
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef const __attribute__((address_space(4))) double* ScalarRecord;
+#else
+typedef const double* ScalarRecord;
+#endif
+__device__ __forceinline__ ScalarRecord scalar_record(const double* r) { return (ScalarRecord)(uintptr_t)r; }
+
 // Bin inputs of one lane slot.
 template <int PREC>
 __device__ __forceinline__ BinIn load_bin(const DevGrid& g, int bc)
@@ -42,11 +51,11 @@ __device__ __forceinline__ BinIn load_bin(const DevGrid& g, int bc)
     return bi;
 }
 
-// Occupancy: 4 waves per SIMD (128 VGPRs) for the mixed body with up to 16-beam tiles and for
-// the FP64 bodies with 8-beam tiles, whose LDS (plain body: table with low parts 32 KB + tile 7 KB)
+// Occupancy: 4 waves per SIMD (128 VGPRs) for the mixed and the restructured body with up to 16-beam tiles and
+// for the other FP64 bodies with 8-beam tiles, whose LDS (plain body: table with low parts 32 KB + tile 7 KB)
 // lets 4 workgroups share a CU; else what the registers and LDS give (>= 2).
 template <int PREC, int TB, int BPT, int MODE>
-__global__ __launch_bounds__(BLOCK, (BPT == 1 && ((PREC == 1 && TB <= 16) || (PREC != 1 && TB <= 8))) ? 4 : 2)
+__global__ __launch_bounds__(BLOCK, (BPT == 1 && TB <= (PREC == 1 || PREC == 4 ? 16 : 8)) ? 4 : 2)
 void k_sweep(SweepArgs a)
 {
     constexpr bool INC = MODE == SWEEP_INC, LIST = MODE == SWEEP_LIST;
@@ -156,8 +165,8 @@ void k_sweep(SweepArgs a)
 #pragma unroll
                 for (int j = 0; j < BPT; j++) {
                     if (PREC == 4)
-                        beam_bin_fp64r_far(cur + bb * REC, vrecs, fb[j], bi[j].xt, bi[j].yt, etab, g.cc_far, a.fast_diff,
-                                           acc[j]);
+                        beam_bin_fp64r_far(cur + bb * REC, scalar_record(recs + (t0 + bb) * REC), vrecs, fb[j],
+                                           bi[j].xt, bi[j].yt, etab, g.cc_far, a.fast_diff, acc[j]);
                     else if (PREC == 3) {
                         AdjBeam B;
                         adj_beam_from_record(cur + bb * REC, B);
@@ -275,7 +284,7 @@ extern "C" int abt_launch_sweep(const abt::SweepArgs* a, int nseg, int prec, int
 }
 
 // One orientation's far field of nb prepared beams in nseg segments of `per` beams (a multiple
-// of 32, so that the mixed body's FP32 beam groups do not depend on the cut); prec: the ABI's
+// of 8, so that the mixed body's FP32 beam groups do not depend on the cut); prec: the ABI's
 // (0 plain FP64, 1 mixed, 3 restructured FP64) or 2, the incoherent sum (one segment).
 // work: nseg * 64 bytes per bin when nseg > 1.
 extern "C" int abt_launch_far_field(const abt::DevGrid* g, const double* recs, const double* vrecs,
@@ -296,7 +305,7 @@ extern "C" int abt_launch_far_field(const abt::DevGrid* g, const double* recs, c
     a.part = nseg > 1 ? work : nullptr;
     a.out = out;
     a.fast_diff = fast_diff;
-    int e = abt_launch_sweep(&a, nseg, kprec, kprec == 4 || kprec == 0 ? 8 : 16, 1, SWEEP_PLAIN, st);
+    int e = abt_launch_sweep(&a, nseg, kprec, kprec == 0 ? 8 : 16, 1, SWEEP_PLAIN, st);
     if (e) return e;
     if (nseg > 1) {
         const dim3 grid((g->nbins + BLOCK - 1) / BLOCK);

@@ -635,14 +635,14 @@ __host__ __device__ __forceinline__ double div_by(double a, double b, double y)
 }
 
 // f (gg I + hh J) A = w P A + w' Q A, w = f (gg + i hh), w' = f (gg - i hh)
-__host__ __device__ __forceinline__ void add_projectors(const double* __restrict__ r, double FR, double FI, double gg,
-                                                        double hh, double acc[8])
+template <class Rec>
+__host__ __device__ __forceinline__ void add_projectors(Rec r, double FR, double FI, double gg, double hh, double acc[8])
 {
     const double ta = FR * gg, tc = FR * hh;
     const double wr = fma(-FI, hh, ta), wi = fma(FI, gg, tc);
     const double vr = fma(FI, hh, ta), vi = fma(FI, gg, -tc);
-    const double* rp = r + R_RP64;
-    const double* rm = r + R_RM64;
+    const Rec rp = r + R_RP64;
+    const Rec rm = r + R_RM64;
     acc[0] = fma(wr, rp[0], fma(-wi, rp[1], acc[0]));
     acc[1] = fma(wr, rp[1], fma(wi, rp[0], acc[1]));
     acc[2] = fma(wr, rp[2], fma(-wi, rp[3], acc[2]));
@@ -915,20 +915,22 @@ __host__ __device__ __forceinline__ FarBin far_bin(const BinIn& bi)
 //     two FMAs and its table index is its rounding;
 //   * one reciprocal root 1 / (|inc x k| (1 - k_y^2) |d0 d1 d2|) for the polarisation's normalisation
 //     and the form factor's denominator together.
-// Tried: records through scalar loads instead of LDS (fewer instructions, but a wave waits for each of
-// the ~6 scalar loads of a beam: 24 orientations x 721 x 180 bins 116 ms against 104); the other branches
-// after each tile in a pass of their own, which frees registers for a fifth wave but recomputes the
-// beam (125 ms; 112 with 4 waves).  Measured against the body before: 24 orientations x 721 x 180 bins
-// 109.1 -> 90.6 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 41.0 -> 37.2 ms.  What is left of the issue
-// rate (14 % of the cycles) is waits that 4 waves do not cover.
+//   * the common path's 33 record values come through scalar loads: from LDS, 21 reads a beam and wave
+//     kept the LDS busy for 74 % of the time, in the way of the table's.  The record tiles stay: loading them
+//     brings the records into L2 ahead of the scalar loads, and their barriers keep a workgroup's waves on
+//     the same lines (without tiles 109 ms, with them 90.5, all from LDS 98.5, in one run of the 24
+//     orientations below).
+// Tried: the other branches after each tile in a pass of their own, which frees registers for a fifth wave but
+// recomputes the beam (125 ms against 104; 112 with 4 waves).  Measured against the body before, 24 orientations x
+// 721 x 180 bins 113.0 -> 86.7 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 43.8 -> 34.5 ms.
 struct FarGeom {
     double ux, uy, uz;   // direction of the bin from the aperture centre
     double kd;           // k (|x - c| - |x|) in table steps (the bin's own e^{i k |x|} follows the beam sum)
     double id;           // 1 / |x - c|
 };
 // c: the centre, cc = |c|^2, kt: table steps per um; far: cc is within the far geometry's limit
-__host__ __device__ __forceinline__ FarGeom far_geometry_of(const double* __restrict__ c, double cc, double kt,
-                                                            const FarBin& fb, bool far)
+template <class Rec>
+__host__ __device__ __forceinline__ FarGeom far_geometry(Rec c, double cc, double kt, const FarBin& fb, bool far)
 {
     FarGeom o;
     const double p = fma(fb.nx, c[0], fma(fb.ny, c[1], fb.nz * c[2]));
@@ -956,10 +958,6 @@ __host__ __device__ __forceinline__ FarGeom far_geometry_of(const double* __rest
     }
     return o;
 }
-__host__ __device__ __forceinline__ FarGeom far_geometry(const double* __restrict__ r, const FarBin& fb, double cc_far)
-{
-    return far_geometry_of(r + R_COM, r[R_CC], r[R_KT], fb, record_less(r[R_CC], cc_far));
-}
 
 // Outside the beam's field of view (fast_diff; diff_mod.f90:593-603)
 __host__ __device__ __forceinline__ bool far_culled(const double* __restrict__ r, const FarGeom& u, int fast_diff)
@@ -971,8 +969,8 @@ __host__ __device__ __forceinline__ bool far_culled(const double* __restrict__ r
 struct TriPhase {
     double Wr[3], Wi[3], d0, d1, d2;
 };
-__host__ __device__ __forceinline__ TriPhase tri_phases_of(const double* __restrict__ tx, const double* __restrict__ ty,
-                                                           double q1, double q2, double kd,
+template <class Rec>
+__host__ __device__ __forceinline__ TriPhase tri_phases_of(Rec tx, Rec ty, double q1, double q2, double kd,
                                                            const double* __restrict__ etab)
 {
     TriPhase o;
@@ -987,7 +985,8 @@ __host__ __device__ __forceinline__ TriPhase tri_phases_of(const double* __restr
     o.d2 = T[0] - T[2];
     return o;
 }
-__host__ __device__ __forceinline__ TriPhase tri_phases(const double* __restrict__ r, double q1, double q2, double kd,
+template <class Rec>
+__host__ __device__ __forceinline__ TriPhase tri_phases(Rec r, double q1, double q2, double kd,
                                                         const double* __restrict__ etab)
 {
     return tri_phases_of(r + R_TX, r + R_TY, q1, q2, kd, etab);
@@ -1007,25 +1006,27 @@ __host__ __device__ __forceinline__ bool one_denominator(const TriPhase& w, doub
     return fabs(d) > (1e-4 * (2 * ETAB_N) * (2 * ETAB_N)) * fmax(fabs(w.d0), fabs(w.d1));
 }
 
-// xt, yt: the theta_i bin of the same phi (forward fallback of hc).
-__host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __restrict__ r,
+// xt, yt: the theta_i bin of the same phi (forward fallback of hc).  h: the record again, where the common path
+// reads it from (on the device through scalar loads).
+template <class Rec>
+__host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __restrict__ r, Rec h,
                                                             const double* __restrict__ vrecs, const FarBin& fb,
                                                             double xt, double yt, const double* __restrict__ etab,
                                                             double cc_far, int fast_diff, double acc[8])
 {
-    const FarGeom u = far_geometry(r, fb, cc_far);
+    const FarGeom u = far_geometry(h + R_COM, h[R_CC], h[R_KT], fb, record_less(h[R_CC], cc_far));
     if (far_culled(r, u, fast_diff)) return;
-    const double* RR = r + R_RR;
+    const Rec RR = h + R_RR;
     const double k1 = fma(RR[0], u.ux, fma(RR[1], u.uy, RR[2] * u.uz));
     const double k2 = fma(RR[3], u.ux, fma(RR[4], u.uy, RR[5] * u.uz));
     const double k3 = fma(RR[6], u.ux, fma(RR[7], u.uy, RR[8] * u.uz));
-    const double q1 = r[R_PROP2] - k1, q2 = r[R_PROP2 + 1] - k2;   // q / k in the aperture plane
-    const bool nv3 = record_is3(r[R_NV]);
+    const double q1 = h[R_PROP2] - k1, q2 = h[R_PROP2 + 1] - k2;   // q / k in the aperture plane
+    const bool nv3 = record_is3(h[R_NV]);
     TriPhase w;
     double d = 0.0;
     bool one = false;
     if (nv3) {
-        w = tri_phases(r, q1, q2, u.kd, etab);
+        w = tri_phases(h, q1, q2, u.kd, etab);
         d = w.d0 * w.d1 * w.d2;
         one = one_denominator(w, d);
     }
@@ -1036,12 +1037,12 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __rest
     double FR, FI, gg, hh;
     if (one && !kclamp && !fwd) {
         // hc = unit(inc x khat) is normal to khat (see beam_bin_mixed)
-        const double* C = r + R_C64;
+        const Rec C = h + R_C64;
         const double P0 = fma(RR[3], u.uy, -RR[4] * u.ux);
         const double Q0 = fma(-u.uz, k2, RR[5]);
         const double m = s2 * d;
         const double ri = rsq64_1(fma(u.ux, u.ux, u.uy * u.uy) * (m * m));   // 1 / (|(ux, uy)| s2 |d|)
-        const double f = r[R_TA] * copysign(ri, d);
+        const double f = h[R_TA] * copysign(ri, d);
         const double A = fma(C[0], s2, C[1] * k3);
         const double B = fma(C[2], s2, C[1] * (k1 * k2));
         FR = f * fma(w.Wi[0], w.d1, fma(w.Wi[1], w.d2, w.Wi[2] * w.d0));
@@ -1170,7 +1171,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __rest
             hh = fma(pm, db, -qh * da);
         }
     }
-    add_projectors(r, FR, FI, gg, hh, acc);
+    add_projectors(h, FR, FI, gg, hh, acc);
 }
 
 // One beam, one bin from the bin's plain inputs (bi.rad = |x| is read); etab: the table, then
@@ -1182,7 +1183,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r(const double* __restrict
                                                         int fast_diff, double acc[8])
 {
     (void)g;
-    beam_bin_fp64r_far(r, vrecs, far_bin(bi), bi.xt, bi.yt, etab, etab[ETAB_CC_FAR], fast_diff, acc);
+    beam_bin_fp64r_far(r, r, vrecs, far_bin(bi), bi.xt, bi.yt, etab, etab[ETAB_CC_FAR], fast_diff, acc);
 }
 
 // Beams per FP32 partial sum of the mixed kernels: every MIXED_GROUP consecutive beams
