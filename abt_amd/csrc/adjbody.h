@@ -59,7 +59,7 @@ struct AdjBeam {
     double area;                // |N| / 2
     double qa2;                 // (aperture radius)^2: series branch when |q|^2 qa2 < SERIES_QA^2
     // FP64 body
-    const double* r;            // the record, for what only rare bins need
+    const double* r;            // the record, for what only rare bins need (FP64 adjoint)
     double tA;                  // 2 area / (lambda EXP_H^2)
     double Px, Py;              // P.e_x, P.e_y
     double tx[3], ty[3];        // in-plane coordinates of v_l - c in table steps times 1 / k
@@ -78,7 +78,8 @@ struct AdjAcc {
     double exb[3], eyb[3], ezb[3];
 };
 
-__host__ __device__ inline void adj_beam_from_record(const double* __restrict__ r, AdjBeam& B)
+template <class Rec>
+__host__ __device__ inline void adj_beam_from_record(Rec r, AdjBeam& B)
 {
     for (int i = 0; i < 3; i++) {
         B.c[i] = r[R_COM + i];
@@ -104,7 +105,7 @@ __host__ __device__ inline void adj_beam_from_record(const double* __restrict__ 
         B.V[2 * c + 1] = C[1] - C[2];
     }
     B.area = fabs(r[R_AREA]);
-    B.r = r;
+    B.r = (const double*)r;
     B.tA = 2.0 * B.area * r[R_IL] / (EXP_H * EXP_H);
     for (int i = 0; i < 3; i++) {
         B.tx[i] = r[R_TX + i];

@@ -239,9 +239,7 @@ int abt_batch_plan_create(const abt_dev_grid* g, int32_t norient, const int64_t*
     p->cus = cus;
     p->boff.assign(beam_off, beam_off + norient + 1);
     p->eoff.assign(ext_off, ext_off + norient + 1);
-    // (the plain FP64 body's LDS holds 4 waves per SIMD with 8-beam tiles; the restructured body's with 16, which
-    // where beams are mostly out of view halve the barriers: one large column 5.43 -> 5.36 ms)
-    rc = shape_for(p, precision == ABT_FP64 ? 8 : 16, 1, &p->shape);
+    rc = shape_for(p, 16, 1, &p->shape);
     if (rc) { delete p; return rc; }
     std::vector<abt::SweepSeg> segs;
     make_segments(p, segs);

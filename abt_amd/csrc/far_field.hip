@@ -2,9 +2,8 @@
 //
 // Work decomposition.  One lane per BPT far-field bins, bins contiguous with phi fastest (the
 // Fortran (nphi, ntheta) layout), 256 lanes per workgroup.  A workgroup sums one segment of
-// the beam list on one tile of 256 x BPT bins (grid: tiles x segments): beam records are staged
-// in LDS one tile at a time (cooperative coalesced loads, then broadcast reads) and every lane
-// walks them in beam order.  Segment sums are stored as the body forms them; k_finish_sum
+// the beam list on one tile of 256 x BPT bins (grid: tiles x segments): every lane walks the
+// beams in order, their records read through scalar loads.  Segment sums are stored as the body forms them; k_finish_sum
 // (one orientation) or the batched plan's epilogue (batch.hip) adds them in segment order and
 // finishes the sum, so each bin's sum is formed in a fixed order and repeats bit for bit.
 // Cutting the beam list is what fills the chip when there are few bins or few orientations,
@@ -31,7 +30,7 @@ namespace abt {
 constexpr int BLOCK = 256;
 
 // A wave-uniform record through scalar loads: records are not written while a sweep runs, which the constant
-// address space says (barriers and LDS stores in the loop would otherwise rule them out).
+// address space says (the loop's barriers would otherwise rule them out).
 #if defined(__HIP_DEVICE_COMPILE__)
 typedef const __attribute__((address_space(4))) double* ScalarRecord;
 #else
@@ -51,29 +50,29 @@ __device__ __forceinline__ BinIn load_bin(const DevGrid& g, int bc)
     return bi;
 }
 
-// Occupancy: 4 waves per SIMD (128 VGPRs) for the mixed and the restructured body with up to 16-beam tiles and
-// for the other FP64 bodies with 8-beam tiles, whose LDS (plain body: table with low parts 32 KB + tile 7 KB)
-// lets 4 workgroups share a CU; else what the registers and LDS give (>= 2).
+// Records.  A beam's record is the same for every lane, so it comes through scalar loads, straight into the
+// FP64 (and FP32) instructions' scalar operands; TB beams at a time, a barrier apart, so that a workgroup's waves
+// share the scalar cache's lines, and with the next TB records touched by one vector load a line, which
+// brings them into L2 ahead of the scalar loads.  Each of the three counts: records from LDS kept it busy
+// for 74 % of the time in the restructured body (42 % mixed, 51 % plain); scalar loads alone, or
+// with the barriers alone, run the orientation averages at 109 and 108 ms (mixed 39 ms).  16 orientations x 361 x
+// 180 bins, mixed: 30.8 -> 28.6 ms; 24 x 721 x 180, restructured: 98.5 -> 87.8 ms; 45 polygons x 721 x 180,
+// plain: 190 -> 184 us a step.
+// Occupancy: 4 waves per SIMD (128 VGPRs); 2 for two bins a lane and for the accurate body.
 template <int PREC, int TB, int BPT, int MODE>
-__global__ __launch_bounds__(BLOCK, (BPT == 1 && TB <= (PREC == 1 || PREC == 4 ? 16 : 8)) ? 4 : 2)
+__global__ __launch_bounds__(BLOCK, BPT == 1 && PREC != 3 ? 4 : 2)
 void k_sweep(SweepArgs a)
 {
     constexpr bool INC = MODE == SWEEP_INC, LIST = MODE == SWEEP_LIST;
-    // Mixed body: two record tiles; the next tile's records are loaded into registers while the
-    // current one is summed, then stored to the other buffer (one barrier per tile).  The FP64
-    // bodies need their registers: one tile, loaded between barriers.
-    constexpr bool DB = PREC == 1 && TB <= 16 && BPT == 1;
-    __shared__ double tile[(DB ? 2 : 1) * TB * REC];
     // the exponential table, or the table with its low parts
     constexpr bool TAB = PREC == 0 || PREC == 2 || PREC == 4;
     __shared__ double etab[PREC == 4 ? ETAB_DOUBLES : (TAB ? ETAB_GRID : 1)];
-    constexpr int PF = DB ? (TB * REC + BLOCK - 1) / BLOCK : 1;   // doubles per lane per tile
     const DevGrid& g = a.g;
     const int tid = threadIdx.x;
     const int nslots = LIST ? *a.list_count : g.nbins;
     const int slot0 = blockIdx.x * (BLOCK * BPT) + tid;   // slot of lane j: slot0 + j * BLOCK
     if ((int)blockIdx.x * (BLOCK * BPT) >= nslots) return;   // LIST: tiles past the listed bins
-    if (TAB) {   // published by the barriers of the tile loop before any use
+    if (TAB) {   // published by the barriers of the beam loop before any use
         for (int q = tid; q < (PREC == 4 ? ETAB_DOUBLES : ETAB_GRID); q += BLOCK) etab[q] = g.etab[q];
     }
     BinIn bi[BPT];
@@ -106,36 +105,18 @@ void k_sweep(SweepArgs a)
     }
     const double* __restrict__ recs = a.recs[tree];
     const double* __restrict__ vrecs = a.vrecs[tree];
-    if (DB) {
-        // the bin's inputs must have arrived before the tile loop: a use inside it would make
-        // the compiler wait there for the older loads, and with them for the prefetched tile
-        asm volatile("" : "+v"(bi[0].x), "+v"(bi[0].y), "+v"(bi[0].z), "+v"(bi[0].xt), "+v"(bi[0].yt), "+v"(bi[0].zt));
-    }
-    if (DB && b0 < b1) {
-        const int nt0 = (int)min((int64_t)TB, b1 - b0);
-        const double* src = recs + b0 * REC;
-        for (int q = tid; q < nt0 * REC; q += BLOCK) tile[q] = src[q];
-    }
-    if (DB) __syncthreads();
-    int buf = 0;
+    const auto touch = [&](int64_t t) {   // one lane per 128-byte line of the TB records from t
+        const int64_t bytes = t < b1 ? min((int64_t)TB, b1 - t) * (REC * 8) : 0;
+        int v = 0;
+        if (tid * 128 < bytes) v = *reinterpret_cast<const int*>(reinterpret_cast<const char*>(recs + t * REC) + tid * 128);
+        return v;
+    };
+    int line = touch(b0);
     for (int64_t t0 = b0; t0 < b1; t0 += TB) {
         const int nt = (int)min((int64_t)TB, b1 - t0);
-        const int64_t tn = t0 + TB;
-        const int ntn = DB && tn < b1 ? (int)min((int64_t)TB, b1 - tn) : 0;
-        const double* srcn = recs + (ntn ? tn : 0) * REC;
-        double pre[PF];
-#pragma unroll
-        for (int k = 0; k < PF; k++) {
-            const int q = tid + k * BLOCK;
-            pre[k] = q < ntn * REC ? srcn[q] : 0.0;
-        }
-        if (!DB) {
-            __syncthreads();
-            const double* src = recs + t0 * REC;
-            for (int q = tid; q < nt * REC; q += BLOCK) tile[q] = src[q];
-            __syncthreads();
-        }
-        const double* cur = tile + buf * (TB * REC);
+        asm volatile("" : : "v"(line));   // a use: the load is kept, and has ended
+        __syncthreads();
+        line = touch(t0 + TB);
         if (PREC == 1) {
             // FP32 partial sums over groups of MIXED_GROUP beams (segments start at multiples of
             // it from the tree's first beam), added into FP64
@@ -151,7 +132,8 @@ void k_sweep(SweepArgs a)
                 for (int bb = g0; bb < g1; bb++) {
 #pragma unroll
                     for (int j = 0; j < BPT; j++)
-                        beam_bin_mixed_t<INC>(cur + bb * REC, vrecs, g, bi[j], a.fast_diff, accf[j], incf[j]);
+                        beam_bin_mixed_t<INC>(scalar_record(recs + (t0 + bb) * REC), vrecs, g, bi[j], a.fast_diff,
+                                              accf[j], incf[j]);
                 }
 #pragma unroll
                 for (int j = 0; j < BPT; j++) {
@@ -165,27 +147,18 @@ void k_sweep(SweepArgs a)
 #pragma unroll
                 for (int j = 0; j < BPT; j++) {
                     if (PREC == 4)
-                        beam_bin_fp64r_far(cur + bb * REC, scalar_record(recs + (t0 + bb) * REC), vrecs, fb[j],
-                                           bi[j].xt, bi[j].yt, etab, g.cc_far, a.fast_diff, acc[j]);
+                        beam_bin_fp64r_far(scalar_record(recs + (t0 + bb) * REC), vrecs, fb[j], bi[j].xt, bi[j].yt, etab,
+                                           g.cc_far, a.fast_diff, acc[j]);
                     else if (PREC == 3) {
                         AdjBeam B;
-                        adj_beam_from_record(cur + bb * REC, B);
+                        adj_beam_from_record(scalar_record(recs + (t0 + bb) * REC), B);
                         model_bin_fp64(B, bi[j].x, bi[j].y, bi[j].z, bi[j].xt, bi[j].yt, bi[j].rad, g.waveno,
                                        g.lambda, acc[j]);
                     } else
-                        beam_bin_fp64p<PREC == 2>(cur + bb * REC, vrecs, g, bi[j], etab, a.fast_diff, acc[j]);
+                        beam_bin_fp64p<PREC == 2>(scalar_record(recs + (t0 + bb) * REC), vrecs, g, bi[j], etab,
+                                                  a.fast_diff, acc[j]);
                 }
             }
-        }
-        if (DB) {
-            double* nxt = tile + (buf ^ 1) * (TB * REC);
-#pragma unroll
-            for (int k = 0; k < PF; k++) {
-                const int q = tid + k * BLOCK;
-                if (q < ntn * REC) nxt[q] = pre[k];
-            }
-            __syncthreads();
-            buf ^= 1;
         }
     }
     const int nbins = g.nbins;
@@ -305,7 +278,7 @@ extern "C" int abt_launch_far_field(const abt::DevGrid* g, const double* recs, c
     a.part = nseg > 1 ? work : nullptr;
     a.out = out;
     a.fast_diff = fast_diff;
-    int e = abt_launch_sweep(&a, nseg, kprec, kprec == 0 ? 8 : 16, 1, SWEEP_PLAIN, st);
+    int e = abt_launch_sweep(&a, nseg, kprec, 16, 1, SWEEP_PLAIN, st);
     if (e) return e;
     if (nseg > 1) {
         const dim3 grid((g->nbins + BLOCK - 1) / BLOCK);

@@ -213,18 +213,30 @@ __host__ __device__ __forceinline__ void edge_exp(float wr0, float wi0, float wr
     ssi = fmaf(t, Ei, ssi);
 }
 
+// A record's FP32 blocks, in the address space of the record.
+template <class Rec>
+struct FloatsOf {
+    typedef const float* type;
+};
+#if defined(__HIP_DEVICE_COMPILE__)
+template <>
+struct FloatsOf<const __attribute__((address_space(4))) double*> {
+    typedef const __attribute__((address_space(4))) float* type;
+};
+#endif
+
+
 // Mixed-precision body: one beam, one bin.  Adds the beam's contribution to the FP32
 // projector sums accf: S+ (accf[0..3]) and S- (accf[4..7]), see mixed_finish; callers
 // add accf into FP64 sums every few beams.  INC: also adds the squared Frobenius norm of
 // the beam's amplitude, |f|^2 (gg^2 + hh^2) |A|_F^2 (the incoherent sum), to inc.
-template <bool INC>
-__host__ __device__ __forceinline__ void beam_bin_mixed_t(const double* __restrict__ r,
-                                                          const double* __restrict__ vrecs,
+template <bool INC, class Rec>
+__host__ __device__ __forceinline__ void beam_bin_mixed_t(Rec r, const double* __restrict__ vrecs,
                                                           const DevGrid& g, const BinIn& bi,
                                                           int fast_diff, float accf[8], float& inc)
 {
-    const float* rf = reinterpret_cast<const float*>(r + R_F32);
-    const float* rg = reinterpret_cast<const float*>(r + R_G32);
+    typedef typename FloatsOf<Rec>::type Floats;
+    const Floats rf = (Floats)(r + R_F32), rg = (Floats)(r + R_G32);
     // ---- FP64 geometry: bin direction from the aperture centre, |r - com| ----
     const double dx = bi.x - r[R_COM], dy = bi.y - r[R_COM + 1], dz = bi.z - r[R_COM + 2];
     const double s = fma(dx, dx, fma(dy, dy, dz * dz));
@@ -238,7 +250,7 @@ __host__ __device__ __forceinline__ void beam_bin_mixed_t(const double* __restri
         if (ux * r[R_PROP0] + uy * r[R_PROP0 + 1] + uz * r[R_PROP0 + 2] < r[R_COSFOV]) return;
     }
     // q = krev (prop2 - khat) in the aperture plane (revolutions per um); krev khat_x,y
-    const double* K = r + R_KRR;
+    const Rec K = r + R_KRR;
     const double qx = fma(-K[0], ux, fma(-K[1], uy, fma(-K[2], uz, r[R_KP2])));
     const double qy = fma(-K[3], ux, fma(-K[4], uy, fma(-K[5], uz, r[R_KP2 + 1])));
     const double k1r = r[R_KP2] - qx, k2r = r[R_KP2 + 1] - qy;
@@ -681,8 +693,8 @@ __host__ __device__ __forceinline__ void add_projectors(Rec r, double FR, double
 // before, 4.0 ms now; 5 orientations x 16,290 bins batched 7.9 -> 3.3 ms.
 // acc: the projector sums S+ (0..3) and S- (4..7).  tab: the exponential table (LDS).
 // INCOH: acc[0] += |amplC|_F^2 instead (temp_rot1 is orthogonal: the norm is final).
-template <bool INCOH>
-__host__ __device__ __forceinline__ void beam_bin_fp64p(const double* __restrict__ r,
+template <bool INCOH, class Rec>
+__host__ __device__ __forceinline__ void beam_bin_fp64p(Rec r,
                                                         const double* __restrict__ vrecs,
                                                         const DevGrid& g, const BinIn& bi,
                                                         const double* __restrict__ tab, int fast_diff,
@@ -696,7 +708,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64p(const double* __restrict
         const double vx = div_by(x1, r1, ir1), vy = div_by(y1, r1, ir1), vz = div_by(z1, r1, ir1);
         if (vx * r[R_PROP0] + vy * r[R_PROP0 + 1] + vz * r[R_PROP0 + 2] < r[R_COSFOV]) return;
     }
-    const double* R = r + R_RR;
+    const Rec R = r + R_RR;
     const double x3 = R[0] * x1 + R[1] * y1 + R[2] * z1;
     const double y3 = R[3] * x1 + R[4] * y1 + R[5] * z1;
     const double z3 = R[6] * x1 + R[7] * y1 + R[8] * z1;
@@ -714,7 +726,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64p(const double* __restrict
     // decides the clamp below
     const double k1 = div_by(x3, r1, ir1), k3 = div_by(z3, r1, ir1);
     const double k2 = div_by(y3, r1, ir1);
-    const double* C = r + R_C64;
+    const Rec C = r + R_C64;
     double gg, hj;   // rot4 . diff_ampl = gg I + hj J
     const double uz = z1 * ir1;
     const bool kclamp = fabs(k2) > K2CLAMP, fwd = !(fabs(uz) < FWD_DOT);
@@ -914,15 +926,11 @@ __host__ __device__ __forceinline__ FarBin far_bin(const BinIn& bi)
 //   * phases in table steps: the vertex coordinates carry krev and the table size, so a phase is
 //     two FMAs and its table index is its rounding;
 //   * one reciprocal root 1 / (|inc x k| (1 - k_y^2) |d0 d1 d2|) for the polarisation's normalisation
-//     and the form factor's denominator together.
-//   * the common path's 33 record values come through scalar loads: from LDS, 21 reads a beam and wave
-//     kept the LDS busy for 74 % of the time, in the way of the table's.  The record tiles stay: loading them
-//     brings the records into L2 ahead of the scalar loads, and their barriers keep a workgroup's waves on
-//     the same lines (without tiles 109 ms, with them 90.5, all from LDS 98.5, in one run of the 24
-//     orientations below).
+//     and the form factor's denominator together;
+//   * records through scalar loads (k_sweep).
 // Tried: the other branches after each tile in a pass of their own, which frees registers for a fifth wave but
 // recomputes the beam (125 ms against 104; 112 with 4 waves).  Measured against the body before, 24 orientations x
-// 721 x 180 bins 113.0 -> 86.7 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 43.8 -> 34.5 ms.
+// 721 x 180 bins 105.1 -> 77.8 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 40.9 -> 31.2 ms.
 struct FarGeom {
     double ux, uy, uz;   // direction of the bin from the aperture centre
     double kd;           // k (|x - c| - |x|) in table steps (the bin's own e^{i k |x|} follows the beam sum)
@@ -960,7 +968,8 @@ __host__ __device__ __forceinline__ FarGeom far_geometry(Rec c, double cc, doubl
 }
 
 // Outside the beam's field of view (fast_diff; diff_mod.f90:593-603)
-__host__ __device__ __forceinline__ bool far_culled(const double* __restrict__ r, const FarGeom& u, int fast_diff)
+template <class Rec>
+__host__ __device__ __forceinline__ bool far_culled(Rec r, const FarGeom& u, int fast_diff)
 {
     return fast_diff && u.ux * r[R_PROP0] + u.uy * r[R_PROP0 + 1] + u.uz * r[R_PROP0 + 2] < r[R_COSFOV];
 }
@@ -1006,27 +1015,26 @@ __host__ __device__ __forceinline__ bool one_denominator(const TriPhase& w, doub
     return fabs(d) > (1e-4 * (2 * ETAB_N) * (2 * ETAB_N)) * fmax(fabs(w.d0), fabs(w.d1));
 }
 
-// xt, yt: the theta_i bin of the same phi (forward fallback of hc).  h: the record again, where the common path
-// reads it from (on the device through scalar loads).
+// xt, yt: the theta_i bin of the same phi (forward fallback of hc).
 template <class Rec>
-__host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __restrict__ r, Rec h,
+__host__ __device__ __forceinline__ void beam_bin_fp64r_far(Rec r,
                                                             const double* __restrict__ vrecs, const FarBin& fb,
                                                             double xt, double yt, const double* __restrict__ etab,
                                                             double cc_far, int fast_diff, double acc[8])
 {
-    const FarGeom u = far_geometry(h + R_COM, h[R_CC], h[R_KT], fb, record_less(h[R_CC], cc_far));
+    const FarGeom u = far_geometry(r + R_COM, r[R_CC], r[R_KT], fb, record_less(r[R_CC], cc_far));
     if (far_culled(r, u, fast_diff)) return;
-    const Rec RR = h + R_RR;
+    const Rec RR = r + R_RR;
     const double k1 = fma(RR[0], u.ux, fma(RR[1], u.uy, RR[2] * u.uz));
     const double k2 = fma(RR[3], u.ux, fma(RR[4], u.uy, RR[5] * u.uz));
     const double k3 = fma(RR[6], u.ux, fma(RR[7], u.uy, RR[8] * u.uz));
-    const double q1 = h[R_PROP2] - k1, q2 = h[R_PROP2 + 1] - k2;   // q / k in the aperture plane
-    const bool nv3 = record_is3(h[R_NV]);
+    const double q1 = r[R_PROP2] - k1, q2 = r[R_PROP2 + 1] - k2;   // q / k in the aperture plane
+    const bool nv3 = record_is3(r[R_NV]);
     TriPhase w;
     double d = 0.0;
     bool one = false;
     if (nv3) {
-        w = tri_phases(h, q1, q2, u.kd, etab);
+        w = tri_phases(r, q1, q2, u.kd, etab);
         d = w.d0 * w.d1 * w.d2;
         one = one_denominator(w, d);
     }
@@ -1037,12 +1045,12 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __rest
     double FR, FI, gg, hh;
     if (one && !kclamp && !fwd) {
         // hc = unit(inc x khat) is normal to khat (see beam_bin_mixed)
-        const Rec C = h + R_C64;
+        const Rec C = r + R_C64;
         const double P0 = fma(RR[3], u.uy, -RR[4] * u.ux);
         const double Q0 = fma(-u.uz, k2, RR[5]);
         const double m = s2 * d;
         const double ri = rsq64_1(fma(u.ux, u.ux, u.uy * u.uy) * (m * m));   // 1 / (|(ux, uy)| s2 |d|)
-        const double f = h[R_TA] * copysign(ri, d);
+        const double f = r[R_TA] * copysign(ri, d);
         const double A = fma(C[0], s2, C[1] * k3);
         const double B = fma(C[2], s2, C[1] * (k1 * k2));
         FR = f * fma(w.Wi[0], w.d1, fma(w.Wi[1], w.d2, w.Wi[2] * w.d0));
@@ -1120,7 +1128,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __rest
             FI = ssi * sc;
         }
         if (!kclamp && !fwd) {
-            const double* C = r + R_C64;
+            const Rec C = r + R_C64;
             const double P0 = fma(RR[3], u.uy, -RR[4] * u.ux);
             const double Q0 = fma(-u.uz, k2, RR[5]);
             const double rh = rsq64_1(fma(u.ux, u.ux, u.uy * u.uy) * (s2 * s2));   // 1 / (|(ux, uy)| s2)
@@ -1171,7 +1179,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(const double* __rest
             hh = fma(pm, db, -qh * da);
         }
     }
-    add_projectors(h, FR, FI, gg, hh, acc);
+    add_projectors(r, FR, FI, gg, hh, acc);
 }
 
 // One beam, one bin from the bin's plain inputs (bi.rad = |x| is read); etab: the table, then
@@ -1183,7 +1191,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r(const double* __restrict
                                                         int fast_diff, double acc[8])
 {
     (void)g;
-    beam_bin_fp64r_far(r, r, vrecs, far_bin(bi), bi.xt, bi.yt, etab, etab[ETAB_CC_FAR], fast_diff, acc);
+    beam_bin_fp64r_far(r, vrecs, far_bin(bi), bi.xt, bi.yt, etab, etab[ETAB_CC_FAR], fast_diff, acc);
 }
 
 // Beams per FP32 partial sum of the mixed kernels: every MIXED_GROUP consecutive beams

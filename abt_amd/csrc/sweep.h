@@ -49,7 +49,7 @@ enum : int { SWEEP_PLAIN = 0, SWEEP_INC = 1, SWEEP_LIST = 2 };
 
 }  // namespace abt
 
-// Kernel instance for (kernel precision, beams per tile, bins per lane, variant); nullptr if none.
+// Kernel instance for (kernel precision, beams between barriers, bins per lane, variant); nullptr if none.
 // Kernel precisions: 0 plain FP64, 1 mixed, 2 incoherent FP64, 3 frame-free FP64 model, 4 restructured FP64.
 extern "C" const void* abt_sweep_kernel(int prec, int tb, int bpt, int mode);
 extern "C" int abt_launch_sweep(const abt::SweepArgs* a, int nseg, int prec, int tb, int bpt, int mode,

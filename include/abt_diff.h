@@ -229,8 +229,8 @@ int abt_batch_plan_destroy(abt_batch_plan* plan);
 /* Device bytes the plan holds (sums of beam segments: 64 bytes per bin per segment, up to 2 GiB
  * where one orientation's fit; Mueller partial sums; weights, tables). */
 int abt_batch_workspace(const abt_batch_plan* plan, size_t* bytes);
-/* Tile shape: beams staged per LDS tile (8, 16, 32) and bins per lane (1, 2).
- * Default 16 x 1 (ABT_FP64 and ABT_FP64_FAST 8 x 1) until set or autotuned (ABT_FP64_ACCURATE: 16 x 1 only;
+/* Tile shape: beams a workgroup sums between two barriers (8, 16, 32) and bins per lane (1, 2).
+ * Default 16 x 1 until set or autotuned (ABT_FP64_ACCURATE: 16 x 1 only;
  * ABT_FP64_FAST: 2 bins per lane with 8 or 16 beams per tile only).  Results do not depend on
  * it.  get_tiles: chunks is the number of Mueller partial sums, workgroups what the chip holds
  * at once. */
