@@ -76,7 +76,8 @@ int abt_find_vis(int mode, const abt_vis_geometry* geo, int64_t nf_in, const int
  * reference evaluates for them (nv of the blocker per pair passing the test).
  * phases: 0 (or 3) runs the whole evaluation; 1 runs only the set-up (boxes, flags,
  * candidate lists, blocker records), 2 only the blocker scan, which then reads the
- * set-up that the last phase-1 call left in the same workspace for the same inputs.
+ * set-up that the last phase-1 call left in the same workspace for the same inputs
+ * (with counts it repeats the set-up, since only a counted one lists every facet).
  * The workspace (abt_find_vis_workspace bytes, 256-byte aligned) is the caller's;
  * launches that share one must not overlap. */
 typedef struct abt_vis_batch {

@@ -36,6 +36,13 @@ def test_uncounted_scan_and_its_phases_match_oracle(mode, nbeam):
     B.run(phases=2)
     torch.cuda.synchronize()
     _same({k: x.cpu().numpy() for k, x in B.results().items()}, ref, f"{mode} in phases")
+    B.run(phases=2, counts=True)   # after a set-up that left facets out
+    in_phase = B.counts.clone()
+    B.counts.zero_()
+    B.run(counts=True)
+    torch.cuda.synchronize()
+    assert torch.equal(in_phase, B.counts) and int(B.counts[0]) > 0
+    _same({k: x.cpu().numpy() for k, x in B.results().items()}, ref, f"{mode} counted")
 
 
 @pytest.mark.parametrize("shape,lo,hi", [((14, 28), 3300, 3584), ((20, 40), 3585, 10000)])
