@@ -681,8 +681,7 @@ int launch_all(const abt_vis_batch& a, int64_t nvref, char* ws, int cus, hipStre
     w.mlist = (int32_t*)(ws + L.mlist);
     w.nvref = nvref;
     // A scan alone that counts sets up once more: the set-up before it need not have listed the facets that face
-    // away, which are half of a scan's entries (4096 beams x 2112 facets
-    // in phases: scan 1.08 -> 0.59 ms).
+    // away, which are half of a scan's entries (4096 beams x 2112 facets in phases: scan 1.08 -> 0.59 ms).
     w.keep_all = a.counts != nullptr;
     const bool stage = a.nv <= STAGE_NV;
     const size_t lds = stage ? sizeof(double2) * (size_t)a.nv : 0;
