@@ -49,12 +49,13 @@ def log(*a):
 
 
 def _traffic(kname):
-    """HBM bytes per launch of a kernel on its default workload, from the committed
-    rocprofv3 FETCH_SIZE / WRITE_SIZE passes scaled by the copy-kernel calibration."""
+    """HBM bytes of a kernel's launches in one step of its default workload (named by its beam.bins
+    where there are several), from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE passes scaled by the
+    copy-kernel calibration."""
     tpath = os.path.join(ROOT, "profiles", "traffic.json")
     if not os.path.exists(tpath):
         return None
-    return json.load(open(tpath)).get(kname, {}).get("bytes_per_launch")
+    return json.load(open(tpath)).get(kname, {}).get("bytes_per_step")
 
 
 def gate_report(M, M64, th=None, ph=None):
@@ -155,7 +156,7 @@ class OrientationCase:
         ms = (time.perf_counter() - t) * 1e3 / steps
         kms = None
         if with_kernel_ms:
-            # the persistent kernel and its short reductions, eager on the same stream
+            # the sweeps, epilogues and reductions, eager on the same stream
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             e0.record(s)
             p.run(self.rb, self.re, m, I, m1, self.vb, self.ve, stream=s)
@@ -208,15 +209,15 @@ def orientation_section(case, precision, steps, warmup, M64, plain_ms, gate=True
     ms, kms, M, Ih, info = case.timed_graph(precision, steps, warmup)
     value = case.bb / (ms * 1e-3)
     peak = PEAK[PEAK_OF[precision]]
-    kname = {"fp64_fast": "k_batch<4,%d,1>", "mixed": "k_batch<1,%d,%d>",
-             "mixed_gated": "k_batch<1,%d,%d> (estimate) + k_batch<4,16,1> (listed bins)"}[precision]
+    kname = {"fp64_fast": "k_sweep<4,%d,%d>", "mixed": "k_sweep<1,%d,%d>",
+             "mixed_gated": "k_sweep<1,%d,%d> (estimate) + k_sweep<4,16,1> (listed bins)"}[precision]
     t = info["tiles"]
-    kname = kname % ((t["beams_per_tile"],) if precision == "fp64_fast" else (t["beams_per_tile"], t["bins_per_thread"]))
+    kname = kname % (t["beams_per_tile"], t["bins_per_thread"])
     out = {"value": value, "unit": "beam·bin/s", "ms_per_step": ms, "steps": steps,
            "speedup_vs_fp64_plain": plain_ms / ms if np.isfinite(plain_ms) else None, **info,
            "roofline": {"bound": "valu", "achieved": F_ALG * case.bb / (kms * 1e-3) / 1e12, "peak": peak / 1e12,
                         "unit": "TFLOP/s", "frac": F_ALG * case.bb / (kms * 1e-3) / peak,
-                        "traffic": _traffic(kname), "kernel": kname, "kernel_ms": kms,
+                        "traffic": _traffic(f"{case.bb} beam.bins, {kname}"), "kernel": kname, "kernel_ms": kms,
                         "flop_per_beam_bin": F_ALG, "beam_bins_per_launch": case.bb}}
     if M64 is not None:
         out["accuracy"] = gate_report(M, M64, case.th, case.ph)
@@ -291,12 +292,12 @@ def stress_section(nbeam, steps, lam, dev, cpu_sample):
         k = float(np.mean([a for a, _ in kms]))
         s = float(np.mean([b for _, b in kms]))
         peak = PEAK[PEAK_OF[prec]]
-        kname = {"mixed": "k_far_field<1,16>", "fp64_fast": "k_far_field<4,16>", "fp64": "k_far_field<0,16>"}[prec]
+        kname = {"mixed": "k_sweep<1,16,1>", "fp64_fast": "k_sweep<4,16,1>", "fp64": "k_sweep<0,16,1>"}[prec]
         out[prec] = {"value": nbeam * nbins / (s * 1e-3), "ms_per_step": s, "kernel_ms": k,
                      "roofline": {"bound": "valu", "achieved": F_ALG * nbeam * nbins / (k * 1e-3) / 1e12,
                                   "peak": peak / 1e12, "unit": "TFLOP/s",
                                   "frac": F_ALG * nbeam * nbins / (k * 1e-3) / peak, "kernel": kname,
-                                  "traffic": _traffic(kname) if nbeam == 200_000 else None}}
+                                  "traffic": _traffic(f"{nbeam * nbins} beam.bins, {kname}")}}
         mus[prec] = mu[:16 * nbins].cpu().numpy().reshape(16, -1)
         log(f"  stress {prec}: {s:.1f} ms/step (kernel {k:.1f} ms), {nbeam * nbins / (s * 1e-3):.4e} beam.bin/s")
     for prec in ("mixed", "fp64_fast"):
@@ -415,7 +416,7 @@ def main():
                                      "2112 facets), m 1.31, 10 reflections, 721 theta x 180 phi bins, lambda 0.532 um",
                          "beams": case.nb, "ext_beams": case.ne, "beams_per_orientation": list(case.counts),
                          "bins": case.nbins, "beam_bins": case.bb, "precision": args.precision,
-                         "step": "one HIP-graph replay of the batched plan (persistent kernel + reductions)",
+                         "step": "one HIP-graph replay of the batched plan (sweeps, epilogues and reductions)",
                          "records": "prepared on the host (reference operation order and libm), resident in HBM"}
         out["roofline"] = head.pop("roofline")
         out.update(head)
@@ -613,8 +614,8 @@ def visibility_bench(nbeam, steps, warmup, dev, with_cpu=True):
                       "beams": nbeam, "facets": topo.nf, "candidate_pairs": pairs, "blocker_edges": edges},
            "setup_ms": setup_ms, "scan_ms": scan_ms,
            "roofline": {"bound": "valu", "achieved": ach / 1e12, "peak": PEAK["fp64"] / 1e12, "unit": "TFLOP/s",
-                        "frac": ach / PEAK["fp64"], "traffic": _traffic("k_vis_main<0,false>"),
-                        "kernel": "k_vis_main<0,false>", "kernel_ms": scan_ms, "flop_per_launch": flop}}
+                        "frac": ach / PEAK["fp64"], "traffic": _traffic("k_vis_main<0,false,true>"),
+                        "kernel": "k_vis_main<0,false,true>", "kernel_ms": scan_ms, "flop_per_launch": flop}}
     if with_cpu:
         out["cpu_baseline"] = vis_cpu_baseline(wl, min(nbeam, 4096), value)
     return out
