@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void k_adj_bins(DevGrid g, double* __restrict_
     }
 }
 
-// Bins of a unit's chunk
+// Bins of a unit's chunk: never none, since the plan cuts nbins into at most nbins / 256 chunks and at most 64
 __device__ __forceinline__ void chunk_bins(const AdjArgs& a, const AdjUnit& U, int* b0, int* b1)
 {
     const int n = (a.nbins + a.nchunks - 1) / a.nchunks;

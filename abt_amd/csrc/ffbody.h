@@ -918,8 +918,8 @@ __host__ __device__ __forceinline__ FarBin far_bin(const BinIn& bi)
 // Restructured FP64 body: one beam, one bin, added to the projector sums S+ (acc[0..3]) and
 // S- (acc[4..7]) that fp64r_finish turns into the amplitude matrix.  Bound by FP64 VALU issue (one
 // instruction of any kind takes 4 cycles of a SIMD); the common case -- a triangle seen away from its
-// edges' nulls, its forward direction, the k_y clamp and the forward fallback -- is kept to 138 FP64
-// instructions and ~25 others (207 in all before):
+// edges' nulls, its forward direction, the k_y clamp and the forward fallback -- is kept to 131 FP64
+// instructions and 26 others (207 in all before):
 //   * the far geometry: with h = (|c|^2 / 2 - x.c) / |x|^2 small, |x - c| - |x| and 1 / |x - c| are short
 //     series in h -- no root, no reciprocal; their cut is checked per beam against the grid's limit
 //     (g.cc_far, a scalar branch), beyond which both come from the distances;
@@ -930,7 +930,7 @@ __host__ __device__ __forceinline__ FarBin far_bin(const BinIn& bi)
 //   * records through scalar loads (k_sweep).
 // Tried: the other branches after each tile in a pass of their own, which frees registers for a fifth wave but
 // recomputes the beam (125 ms against 104; 112 with 4 waves).  Measured against the body before, 24 orientations x
-// 721 x 180 bins 105.1 -> 77.8 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 40.9 -> 31.2 ms.
+// 721 x 180 bins 105.8 -> 76.8 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 40.7 -> 30.6 ms.
 struct FarGeom {
     double ux, uy, uz;   // direction of the bin from the aperture centre
     double kd;           // k (|x - c| - |x|) in table steps (the bin's own e^{i k |x|} follows the beam sum)
