@@ -729,8 +729,13 @@ __host__ __device__ __forceinline__ void beam_bin_fp64p(Rec r,
     const Rec C = r + R_C64;
     double gg, hj;   // rot4 . diff_ampl = gg I + hj J
     const double uz = z1 * ir1;
-    const bool kclamp = fabs(k2) > K2CLAMP, fwd = !(fabs(uz) < FWD_DOT);
-    if (!kclamp && !fwd) {
+    // The reference's forward test is on inc . k with the clamped k_y (diff_mod.f90:151, 630).  Without the clamp
+    // that is -uz to rounding, with it at most 1.02e-6 off: bins near the threshold (4.3e-6 and less below it, 9 in
+    // the upper word) take the general branch, which forms it as the reference does.
+    constexpr uint32_t near_fwd = (uint32_t)(__builtin_bit_cast(uint64_t, FWD_DOT) >> 32) - 9;
+    const bool kclamp = fabs(k2) > K2CLAMP;
+    const bool away = (uint32_t)(__builtin_bit_cast(uint64_t, fabs(uz)) >> 32) < near_fwd;
+    if (!kclamp & away) {
         const double ux = x1 * ir1, uy = y1 * ir1;
         const double omk = fma(-k2, k2, 1.0);
         const double P0 = fma(R[3], uy, -(R[4] * ux));       // |inc x k| h_y
@@ -755,7 +760,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64p(Rec r,
         // scattering-plane vector hc (diff_mod.f90:630-635) and rot4 = p I - qh J
         const double i1 = r[R_INC2], i2 = r[R_INC2 + 1], i3 = r[R_INC2 + 2];
         double kk1 = k1, kk2 = k2c, kk3 = k3;
-        if (fwd) {
+        if (!(fabs(i1 * k1 + i2 * k2c + i3 * k3) < FWD_DOT)) {
             const double xt1 = bi.xt - r[R_COM], yt1 = bi.yt - r[R_COM + 1], zt1 = bi.zt - r[R_COM + 2];
             const double irt = rsq64_3(xt1 * xt1 + yt1 * yt1 + zt1 * zt1);
             kk1 = (R[0] * xt1 + R[1] * yt1 + R[2] * zt1) * irt;
