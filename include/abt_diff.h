@@ -159,8 +159,9 @@ size_t abt_far_field_workspace(const abt_dev_grid* g, int64_t nb, int precision)
 
 /* Coherent far-field sum of nb prepared beams: dev_out (complex, Fortran layout,
  * 8*nbins doubles) overwritten.  dev_work: abt_far_field_workspace bytes (NULL:
- * a buffer of the calling thread, ordered between the streams of its calls; nothing is
- * allocated while the stream is being captured and nb < 1024). */
+ * a buffer of the calling thread, ordered between the streams of its calls; while the stream is
+ * being captured the list runs uncut instead, which needs no memory but is slower where bins are
+ * few: give a workspace, which the graph's replays then use). */
 int abt_far_field_dev(const abt_dev_grid* g, const double* dev_recs, const double* dev_vrecs,
                       int64_t nb, int precision, int is_fast_diff, double* dev_out,
                       void* dev_work, size_t work_bytes, void* stream);
