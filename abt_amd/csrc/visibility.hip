@@ -138,7 +138,8 @@ __device__ __forceinline__ int nearest_box(const double* bx, const double* by, c
 // is at least a third of it when the area is negative (positive for find_vis_ext, whose checks have
 // the other sign): outside that edge.  A computed check is within 4 u (|m_x - x_e| |e_y| + |m_y - y_e| |e_x|)
 // of C_e, u = 1.1e-16, as is the computed area of its own; the extents of vertices and midpoints together, ex
-// and ey, bound the offsets.  64 u covers the factors 3, 4 and their sum four times over.
+// and ey, bound the offsets.  64 u covers the factors 3, 4 and their sum four times over.  A midpoint that is NaN
+// is outside no edge: with one among them, or one infinite, ex or ey is infinite and no triangle faces away.
 __device__ __forceinline__ bool faces_away(int mode, double x0, double y0, double x1, double y1, double x2, double y2,
                                            double ex, double ey)
 {
@@ -226,7 +227,11 @@ __global__ __launch_bounds__(SETUP_FEW) void k_vis_setup(abt_vis_batch a, Work w
                 }
             }
         }
-        for (int64_t i = tid; i < nf; i += nt) grow(8, fmid[3 * i], fmid[3 * i + 1]);
+        for (int64_t i = tid; i < nf; i += nt) {
+            const double px = fmid[3 * i], py = fmid[3 * i + 1];
+            grow(8, px, py);
+            if (px != px || py != py) r[9] = INFINITY;   // outside no edge: see faces_away
+        }
 #pragma unroll
         for (int q = 0; q < 12; q++) r[q] = (q & 1) ? wave_max(r[q]) : wave_min(r[q]);
         if (lane == 0) {
