@@ -144,8 +144,17 @@ __host__ __device__ __forceinline__ int record_int(double x)
 #endif
 }
 
-// A record field that holds the bits of a 64-bit integer.
-__host__ __device__ __forceinline__ int64_t record_int64(double x) { return __builtin_bit_cast(int64_t, x); }
+// A whole number of a beam record below 2^52 in scalar registers: the low bits of its sum with 2^52.
+__host__ __device__ __forceinline__ int64_t record_int64(double x)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, x + 4503599627370496.0);
+    uint32_t lo = (uint32_t)u, hi = (uint32_t)(u >> 32);
+#if defined(__HIP_DEVICE_COMPILE__)
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
+#endif
+    return (int64_t)((uint64_t)(hi & 0xfffffu) << 32 | lo);
+}
 
 // x == 3.0 for a value that is the same in every lane of a wave, as a scalar condition
 __host__ __device__ __forceinline__ bool record_is3(double x)
@@ -829,7 +838,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64p(Rec r,
             edge(d[j], s[j], c[j], d[n], v[n], s[n], c[n], r[R_EM + j], r[R_EN + j], r[R_EDX + j], r[R_EDY + j]);
         }
     } else {
-        const double* vr = vrecs + record_int64(r[R_VFIRST]) * VREC;
+        const double* vr = vrecs + record_int64(r[R_VOFF]) * VREC;
         const auto field = [&](int j, int f, int inl) { return nv > 3 ? vr[VREC * j + f] : r[inl + j]; };
         const auto phase = [&](int j) {
 #pragma clang fp contract(off)
@@ -1084,7 +1093,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(Rec r,
                 si = r[R_AREA] * ti;
             } else {
                 const int nv = record_int(r[R_NV]);
-                const double* vr = vrecs + record_int64(r[R_VFIRST]) * VREC;
+                const double* vr = vrecs + record_int64(r[R_VOFF]) * VREC;
                 for (int j = 0; j < nv; j++) {
                     const int jp = (j == nv - 1) ? 0 : j + 1;
                     const double xj = vr[VREC * j + V_X], yj = vr[VREC * j + V_Y];
@@ -1112,7 +1121,7 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(Rec r,
                 edge_diff64(w.Wr[2], w.Wi[2], w.Wr[0], w.Wi[0], turn * w.d2, qx, qy, r[R_EDX + 2], r[R_EDY + 2], ssr, ssi);
             } else {
                 const int nv = record_int(r[R_NV]);
-                const double* vr = vrecs + record_int64(r[R_VFIRST]) * VREC;
+                const double* vr = vrecs + record_int64(r[R_VOFF]) * VREC;
                 const double sx = (2 * ETAB_N) * qx, sy = (2 * ETAB_N) * qy;
                 const double T0 = fma(sx, vr[V_X], fma(sy, vr[V_Y], u.kd));
                 double Wr0, Wi0;

@@ -126,7 +126,6 @@ __host__ __device__ inline void make_beam_record(const double* ampl, const doubl
     rec[R_COSFOV] = cos(fov);
     rec[R_NV] = (double)nv;
     rec[R_VOFF] = (double)voff;
-    rec[R_VFIRST] = __builtin_bit_cast(double, (int64_t)voff);
     double waveno = 2.0 * PI_R4 / lambda;
     double krev = waveno / 6.283185307179586476925;
     rec[R_KREV] = krev;

@@ -43,7 +43,6 @@ enum : int {
     R_G32 = 76,     // second FP32 block (float index G_* below), 6 doubles
     R_F32 = 82,     // FP32 block (float index F_* below), 12 doubles
     R_SIGMA = 94,   // -1 when the amplitude matrix was sign-flipped (anti-parallel), else +1
-    R_VFIRST = 95,  // R_VOFF as the bits of an int64 (FP64 bodies: it stays in scalar registers, whole)
     // FP64 copies of the mixed kernel's per-beam constants, for the restructured FP64 body
     R_RP64 = 96,    // [4] r+ = (A(1,:) - i A(2,:)) / 2: re/im of columns 1, 2
     R_RM64 = 100,   // [4] r- = (A(1,:) + i A(2,:)) / 2

@@ -12,7 +12,7 @@ from abt_amd.workloads import grid, random_triangles
 from tests import emu
 
 LAM = 0.532
-R_NV, R_VOFF, R_VFIRST, VREC = 30, 31, 95, 12
+R_NV, R_VOFF, VREC = 30, 31, 12
 SHIFTS = [0, 1, 2**31 - 8, 2**31, 2**31 + 9, 5 * 2**31 - 3]
 
 
@@ -34,7 +34,6 @@ def _moved(recs, shift):
     r = recs.copy()
     assert (r[:, R_NV] > 3).sum() == 3
     r[:, R_VOFF] += shift
-    r.view(np.int64)[:, R_VFIRST] += shift           # the bits of a 64-bit integer
     return r
 
 
