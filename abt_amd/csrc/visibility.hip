@@ -424,6 +424,7 @@ __global__ __launch_bounds__(MW * WAVE, COUNT ? 4 : 8) void k_vis_main(abt_vis_b
     extern __shared__ double2 sxy[];
     __shared__ int s_res[SHARE ? MW : 1][WAVE];
     __shared__ int s_next;
+    __shared__ uint64_t s_work[COUNT ? MW : 1][2];
     // workgroups go round the XCDs: all of a beam's on one, next to each other, the one its set-up ran on
     const int k8 = blockIdx.x / XCDS, bi = k8 / w.parts * XCDS + blockIdx.x % XCDS, part = k8 % w.parts;
     if (bi >= w.nb) return;
@@ -584,15 +585,22 @@ __global__ __launch_bounds__(MW * WAVE, COUNT ? 4 : 8) void k_vis_main(abt_vis_b
             }
         }
     }
-    if (COUNT) {
+    if (COUNT) {   // one atomic of two lanes a workgroup: one a wave and counter queued for longer than the scan took
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1) {
             npair += __shfl_xor(npair, o, 64);
             nedge += __shfl_xor(nedge, o, 64);
         }
         if (lane == 0) {
-            atomicAdd(a.counts, (unsigned long long)npair);
-            atomicAdd(a.counts + 1, (unsigned long long)nedge);
+            s_work[wv][0] = npair;
+            s_work[wv][1] = nedge;
+        }
+        __syncthreads();
+        if (threadIdx.x < 2) {
+            uint64_t n = 0;
+#pragma unroll
+            for (int k = 0; k < MW; k++) n += s_work[k][threadIdx.x];
+            if (n) atomicAdd(a.counts + threadIdx.x, (unsigned long long)n);
         }
     }
 }
