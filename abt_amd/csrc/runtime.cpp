@@ -76,6 +76,11 @@ struct DevBuf {
 constexpr int PIN_SLOTS = 4;
 constexpr size_t PIN_SLOT = (size_t)1 << 20, PIN_RING = PIN_SLOTS * PIN_SLOT;
 constexpr size_t PIN_MAX = (size_t)64 << 20;   // a thread's pinned memory at most; larger inputs go unpinned
+// The second stream of abt_diff_main costs about 12 us (its wait, its own copies) and hides the beam tree's way back behind
+// the ext tree's sweep, whose length goes as its beams: 361 x 180 bins, us, without and with it, 1 + 1 beams 394 and
+// 403, 45 + 8 455 and 449, 600 + 100 1155 and 1060.  Results that fit one slot come in one copy: 3 x 3 bins 81 -> 34,
+// 181 x 45 121 -> 85.
+constexpr int64_t OVERLAP_BEAMS = 8;
 
 // per-thread staging: the host entry points may run concurrently on several threads
 struct ThreadState {
@@ -806,14 +811,15 @@ int abt_diff_main(const abt_grid* grid, double lambda, int is_fast_diff, const a
         double* d0 = (double*)ts.bufs[0].p;
         double* d1 = d0 + 8 * g->nbins;
         // Both trees' records in pinned memory: the ext tree's are prepared while the beam tree's kernel
-        // runs, and the beam tree's result comes back while the ext tree's does.
+        // runs, and with OVERLAP_BEAMS and more of them the beam tree's result comes back meanwhile.
         const bool pb = want_b && any_polygon(beams), pe = want_e && any_polygon(ext);
         const size_t rb = want_b ? record_bytes(beams, pb) : 0, re = want_e ? record_bytes(ext, pe) : 0;
         char* pin = pin_inputs(ts, rb + re);
         const auto hip = [&](hipError_t e, const char* what) {
             if (e != hipSuccess && !rc) rc = fail(ABT_ERR_HIP, "%s: %s", what, hipGetErrorString(e));
         };
-        bool apart = want_b && want_e && pin;
+        const bool both = want_b && want_e && pin, one_copy = both && 2 * ob <= PIN_SLOT;
+        const bool apart = both && !one_copy && ext->n >= OVERLAP_BEAMS;
         if (apart && !ts.back) hip(hipStreamCreateWithFlags(&ts.back, hipStreamNonBlocking), "stream");
         if (apart && !rc && !ts.first_done) hip(hipEventCreateWithFlags(&ts.first_done, hipEventDisableTiming), "event");
         if (!rc && want_b)
@@ -821,7 +827,7 @@ int abt_diff_main(const abt_grid* grid, double lambda, int is_fast_diff, const a
         if (!rc && apart) {
             hip(hipEventRecord(ts.first_done, ts.st), "event");
             if (!rc) hip(hipStreamWaitEvent(ts.back, ts.first_done, 0), "event");
-        } else if (!rc && want_b && want_e) {
+        } else if (!rc && want_b && want_e && !pin) {
             // the ext tree's staging must not overwrite the beam tree's still in flight
             hip(hipStreamSynchronize(ts.st), "stream sync");
         }
@@ -830,10 +836,19 @@ int abt_diff_main(const abt_grid* grid, double lambda, int is_fast_diff, const a
             abt_beams e2 = *ext;
             e2.fov = nullptr;
             rc = run_host_tree(g->d, &e2, pe, abt::PI_R4 / 2.0, precision, is_fast_diff, d1, ts,
-                               pin ? (double*)(pin + rb) : nullptr, apart ? 3 : 1);
+                               pin ? (double*)(pin + rb) : nullptr, both ? 3 : 1);
         }
-        if (!rc && want_b) hip(copy_back(ts, apart ? ts.back : ts.st, ampl_far_beam, d0, ob, pin != nullptr), "copy-back");
-        if (!rc && want_e) hip(copy_back(ts, ts.st, ampl_far_ext_diff, d1, ob, pin != nullptr), "copy-back");
+        if (!rc && one_copy) {   // the two results lie side by side
+            hip(hipMemcpyAsync(ts.pin, d0, 2 * ob, hipMemcpyDeviceToHost, ts.st), "copy-back");
+            if (!rc) hip(hipStreamSynchronize(ts.st), "copy-back");
+            if (!rc) {
+                memcpy(ampl_far_beam, ts.pin, ob);
+                memcpy(ampl_far_ext_diff, (char*)ts.pin + ob, ob);
+            }
+        } else {
+            if (!rc && want_b) hip(copy_back(ts, apart ? ts.back : ts.st, ampl_far_beam, d0, ob, pin != nullptr), "copy-back");
+            if (!rc && want_e) hip(copy_back(ts, ts.st, ampl_far_ext_diff, d1, ob, pin != nullptr), "copy-back");
+        }
         if (rc) {   // nothing may still read the staging
             (void)hipStreamSynchronize(ts.st);
             if (ts.back) (void)hipStreamSynchronize(ts.back);
