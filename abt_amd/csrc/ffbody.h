@@ -144,16 +144,17 @@ __host__ __device__ __forceinline__ int record_int(double x)
 #endif
 }
 
-// A whole number of a beam record below 2^52 in scalar registers: the low bits of its sum with 2^52.
+// A whole number of a beam record, below 2^52, in scalar registers: the upper 32 bits, then the rest, both exact.  Read
+// out of the bits of a sum with 2^52 instead, the polygons' branch took registers from the triangles': one orientation
+// x 162,360 bins 4.97 ms, 4.63 so.
 __host__ __device__ __forceinline__ int64_t record_int64(double x)
 {
-    const uint64_t u = __builtin_bit_cast(uint64_t, x + 4503599627370496.0);
-    uint32_t lo = (uint32_t)u, hi = (uint32_t)(u >> 32);
+    uint32_t hi = (uint32_t)(x * 0x1p-32), lo = (uint32_t)fma(-0x1p32, (double)hi, x);
 #if defined(__HIP_DEVICE_COMPILE__)
-    lo = __builtin_amdgcn_readfirstlane(lo);
     hi = __builtin_amdgcn_readfirstlane(hi);
+    lo = __builtin_amdgcn_readfirstlane(lo);
 #endif
-    return (int64_t)((uint64_t)(hi & 0xfffffu) << 32 | lo);
+    return (int64_t)((uint64_t)hi << 32 | lo);
 }
 
 // x == 3.0 for a value that is the same in every lane of a wave, as a scalar condition
