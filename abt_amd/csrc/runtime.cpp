@@ -333,9 +333,9 @@ static int grid_build(int64_t nth, const double* th, int64_t nph, const double* 
     if (rc) return rc;
     const int64_t nb = nth * nph;
     std::vector<double> h((size_t)(5 * nb + 4 * nph + 3 * nth + abt::ETAB_GRID));
-    double *x = h.data(), *y = x + nb, *z = y + nb, *rad = z + nb, *krr = rad + nb;
-    double *cp = krr + nb, *sp = cp + nph, *phv = sp + nph, *thv = phv + nph, *etab = thv + nth;
-    double *wph = etab + abt::ETAB_GRID, *wth = wph + nph;
+    // the table first, on the allocation's own alignment: kernels read it in pairs
+    double *etab = h.data(), *x = etab + abt::ETAB_GRID, *y = x + nb, *z = y + nb, *rad = z + nb, *krr = rad + nb;
+    double *cp = krr + nb, *sp = cp + nph, *phv = sp + nph, *thv = phv + nph, *wph = thv + nth, *wth = wph + nph;
     abt::fill_exp_table(etab);
     memcpy(phv, ph, sizeof(double) * nph);
     memcpy(thv, th, sizeof(double) * nth);
@@ -385,18 +385,19 @@ static int grid_build(int64_t nth, const double* th, int64_t nph, const double* 
     g->d.theta_i = theta_i_of(nth, th);
     abt::devgrid_constants(g->d, lambda);
     if (xs) g->d.cc_far = abt::far_limit(krev, *std::min_element(rad, rad + nb));   // the caller's bins
-    g->d.x = d;
-    g->d.y = d + nb;
-    g->d.z = d + 2 * nb;
-    g->d.rad = d + 3 * nb;
-    g->d.kr_rev = d + 4 * nb;
-    g->d.cphi = d + 5 * nb;
-    g->d.sphi = d + 5 * nb + nph;
-    g->d.phi = d + 5 * nb + 2 * nph;
-    g->d.theta = d + 5 * nb + 3 * nph;
-    g->d.etab = d + 5 * nb + 3 * nph + nth;
-    g->d.wphi = g->d.etab + abt::ETAB_GRID;
-    g->d.wth = g->d.wphi + nph;
+    const auto on_device = [&](const double* p) { return d + (p - h.data()); };
+    g->d.etab = on_device(etab);
+    g->d.x = on_device(x);
+    g->d.y = on_device(y);
+    g->d.z = on_device(z);
+    g->d.rad = on_device(rad);
+    g->d.kr_rev = on_device(krr);
+    g->d.cphi = on_device(cp);
+    g->d.sphi = on_device(sp);
+    g->d.phi = on_device(phv);
+    g->d.theta = on_device(thv);
+    g->d.wphi = on_device(wph);
+    g->d.wth = on_device(wth);
     g->d.theta_back = back;
     g->nbins = nb;
     *out = g;
