@@ -95,20 +95,51 @@ struct ThreadState {
     hipEvent_t slot_done[PIN_SLOTS] = {};
     hipStream_t back = nullptr;     // copies back while the stream's next kernel runs
     hipEvent_t first_done = nullptr;
+    ThreadState* next_idle = nullptr;
 };
 
-std::mutex g_reg_mu;
-std::vector<ThreadState*> g_threads;
+// Every state ever made, and those of threads that have ended, for threads that begin: a program that calls from
+// short-lived threads holds as much memory as it had threads at once (a state's device buffers are ordered by
+// its stream and ff_done, whoever holds it).  Never destroyed: threads may end after the process's statics.
+struct Registry {
+    std::mutex mu;
+    std::vector<ThreadState*> all;
+    ThreadState* idle = nullptr;
+};
+Registry& registry()
+{
+    static Registry* r = new Registry();
+    return *r;
+}
+
+struct ThreadHold {
+    ThreadState* ts = nullptr;
+    ~ThreadHold()
+    {
+        if (!ts) return;
+        Registry& r = registry();
+        std::lock_guard<std::mutex> lk(r.mu);
+        ts->next_idle = r.idle;
+        r.idle = ts;
+    }
+};
 
 ThreadState& tstate()
 {
-    static thread_local ThreadState* ts = nullptr;
-    if (!ts) {
-        ts = new ThreadState();
-        std::lock_guard<std::mutex> lk(g_reg_mu);
-        g_threads.push_back(ts);
+    static thread_local ThreadHold h;
+    if (!h.ts) {
+        Registry& r = registry();
+        std::lock_guard<std::mutex> lk(r.mu);
+        if (r.idle) {
+            h.ts = r.idle;
+            r.idle = h.ts->next_idle;
+        } else {
+            r.all.reserve(r.all.size() + 1);
+            h.ts = new ThreadState();
+            r.all.push_back(h.ts);
+        }
     }
-    return *ts;
+    return *h.ts;
 }
 
 int ensure_device()
@@ -149,11 +180,11 @@ int stream_of(ThreadState& ts)
     return 0;
 }
 
-// The thread's pinned memory with `inputs` bytes after the ring: their address, or null (too large, or no
-// memory to pin), for callers to do without.
-char* pin_inputs(ThreadState& ts, size_t inputs)
+// `inputs` bytes of the thread's pinned memory, after the ring where the call copies back through it: their
+// address, or null (too large, or no memory to pin), for callers to do without.
+char* pin_inputs(ThreadState& ts, size_t inputs, bool with_ring = true)
 {
-    const size_t need = PIN_RING + inputs;
+    const size_t ring = with_ring ? PIN_RING : 0, need = ring + inputs;
     if (inputs > PIN_MAX - PIN_RING) return nullptr;
     if (ts.pin_cap < need) {
         if (ts.pin) (void)hipHostFree(ts.pin);
@@ -168,12 +199,12 @@ char* pin_inputs(ThreadState& ts, size_t inputs)
         ts.pin_cap = cap;
     }
     for (hipEvent_t& e : ts.slot_done)
-        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        if (with_ring && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
             e = nullptr;
             (void)hipGetLastError();
             return nullptr;
         }
-    return (char*)ts.pin + PIN_RING;
+    return (char*)ts.pin + ring;
 }
 
 // dst (host) = src (device), after what is on the stream; returns when dst holds it.  pinned: pin_inputs has
@@ -299,7 +330,7 @@ int abt_thread_staging(int slot, size_t bytes, hipStream_t* st, void** p)
     return 0;
 }
 
-char* abt_thread_pinned(size_t bytes) { return pin_inputs(tstate(), bytes); }
+char* abt_thread_pinned(size_t bytes) { return pin_inputs(tstate(), bytes, false); }
 
 // ---------------------------------------------------------------------------
 // device grid
@@ -628,8 +659,9 @@ int abt_init(int device)
 int abt_finalize(void)
 {
     grid_cache_clear();
-    std::lock_guard<std::mutex> lk(g_reg_mu);
-    for (ThreadState* ts : g_threads) {
+    Registry& r = registry();
+    std::lock_guard<std::mutex> lk(r.mu);
+    for (ThreadState* ts : r.all) {
         for (auto& b : ts->bufs) {
             if (b.p) (void)hipFree(b.p);
             b.p = nullptr;
