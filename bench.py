@@ -17,12 +17,13 @@ orientation diff_main + finalise, summed).  Records are prepared on the host wit
 reference's operation order and libm (bit-identical to the oracle's frames) and are
 resident in HBM before the timed region.
 
-Sections in the same JSON line: the mixed-precision kernel (FP32 body) and the gated
-mixed plan on the same workload; the 200,000-aperture stress test (one orientation,
-1801 x 360 bins); the large absorbing column (a stated number of orientations); the
-adjoint; the reference-facing host entry points per call on the reference's CPU case;
-facet visibility; CPU baselines (the C restatement of the reference, OpenMP, on bounded
-samples).
+Sections in the same JSON line (their figures; --json-out FILE has them in full, with
+workloads, rooflines and every accuracy figure): the mixed-precision kernel (FP32 body)
+and the gated mixed plan on the same workload; the 200,000-aperture stress test (one
+orientation, 1801 x 360 bins); the large absorbing column (a stated number of
+orientations); the adjoint; the reference-facing host entry points per call on the
+reference's CPU case; facet visibility; CPU baselines (the C restatement of the
+reference, OpenMP, on bounded samples).
 """
 import argparse
 import json
@@ -473,12 +474,32 @@ def main():
         sections["dropin"] = dropin_section(LAM, dev)
     if args.vis_beams > 0:
         sections["visibility"] = visibility_bench(args.vis_beams, 20, 2, dev, args.cpu_sample > 0)
+    line = json_line(out, sections)
     out.update(sections)
-    line = json.dumps(out)
     if args.json_out:
         with open(args.json_out, "w") as f:
-            f.write(line + "\n")
+            f.write(json.dumps(out) + "\n")
     print(line, flush=True)
+
+
+# Left out of the printed line, which readers keep a few thousand characters of; --json-out has them.
+DETAIL = {"first_failing", "floored_per_element_max", "autotune_ms"}
+SECTION_DETAIL = DETAIL | {"p999", "norm_elem", "tiles", "roofline", "workload", "config", "sample", "model", "unit",
+                           "warmup", "beams", "ext_beams", "bins", "beam_bins", "kind", "cores", "loss",
+                           "grad_vertex_norm"}
+
+
+def _brief(x, leave_out):
+    """x without the keys of leave_out, floats to 6 digits."""
+    if isinstance(x, dict):
+        return {k: _brief(v, leave_out) for k, v in x.items() if k not in leave_out}
+    return float(f"{x:.6g}") if isinstance(x, float) else x
+
+
+def json_line(out, sections):
+    """The one line on stdout: the headline whole (less the lists of its accuracy check), the sections' figures."""
+    head = {k: v if k in ("value", "ms_per_step") else _brief(v, DETAIL) for k, v in out.items()}
+    return json.dumps({**head, **_brief(sections, SECTION_DETAIL)})
 
 
 def adjoint_bench(norient, lam, dev):
