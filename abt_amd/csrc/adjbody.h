@@ -526,7 +526,7 @@ __host__ __device__ __forceinline__ bool one_denominator_grad(const TriPhase& w,
 //   rho_0 = u_1 - u_2 - K_1 v_0 - Re(nu F) (1/K_2 - 1/K_0), and cyclic,
 // from which q_x and q_y gather sum_l rho_l x_l, rho_l y_l.  The amplitude side works in the
 // eigenvectors of g I + h J, U = C1 + i C2 (eigenvalue g - i h) and V = C1 - i C2 (g + i h): half the products.
-// 376 instructions a beam and bin where six edge terms, each with its own trigonometry, took 1634: 5 orientations
+// 396 instructions a beam and bin where six edge terms, each with its own trigonometry, took 1634: 5 orientations
 // of the rough column (209 blocks of 64 beams) x 16,290 bins 15.2 -> 5.2 ms, 3.3 ms with finer chunks of bins,
 // 3.1 ms with each bin's inputs loaded a bin ahead (k_adjoint64); the issue rate alone is 2.4 ms, the rest the last
 // round of waves and waits that two waves per SIMD leave open.

@@ -40,7 +40,7 @@ __device__ __forceinline__ ScalarRecord scalar_record(const double* r) { return 
 
 // A use of what the restructured body's geometry reads (centre, frame, direction, vertex count), so that it is
 // loaded at once and waited for once: left to itself each piece is loaded where it is first used, three waits in a row
-// before the phases.  24 orientations x 721 x 180 bins 86.8 -> 85.8 ms, 10,001 facets x 648,360 bins 30.85 ->
+// before the phases.  24 orientations x 721 x 180 bins 86.8 -> 85.8 ms (on a slower card than ffbody.h's figures), 10,001 facets x 648,360 bins 30.85 ->
 // 30.49.  With the vertices too 85.4, but 1 % slower where the field of view leaves most beams out; with the
 // polarisation's values 86.6; in the mixed body 0.5 %: left as they are.  In the incoherent sum, whose lists are
 // not cut and which waits for every record where bins are few, 5 % too: 4000 beams x 1332 bins 7.88 -> 7.13 ms.

@@ -40,35 +40,6 @@ __host__ __device__ __forceinline__ float abt_rcpf(float x)
 // ---------------------------------------------------------------------------
 // Mixed-precision kernel body.
 
-// sin/cos(2 pi t) for an FP64 revolution count t: quadrant reduction in FP64,
-// FP32 polynomial on the reduced octant (|r| <= 1/8 rev).
-__host__ __device__ __forceinline__ void sincos_rev64(double t, float* s, float* c)
-{
-    const double q = rint(4.0 * t);
-    const float r = (float)fma(-0.25, q, t);
-    const float z = r * r;
-    const float ps = fmaf(z, fmaf(z, fmaf(z, fmaf(z, ABT_SR4, ABT_SR3), ABT_SR2), ABT_SR1), ABT_SR0);
-    const float sn = r * ps;
-    const float cs = fmaf(z, fmaf(z, fmaf(z, fmaf(z, ABT_CR4, ABT_CR3), ABT_CR2), ABT_CR1), ABT_CR0);
-    const int qi = ((int)q) & 3;
-    float so = (qi & 1) ? cs : sn;
-    float co = (qi & 1) ? sn : cs;
-    co = (qi == 1 || qi == 2) ? -co : co;
-    so = (qi >= 2) ? -so : so;
-    *s = so;
-    *c = co;
-}
-
-// Half-period reduction of a revolution count t (FP64): t = r + m/2 with
-// |r| <= 1/4, so that e^{2 pi i t} = (-1)^m e^{2 pi i r}.  The parity of m is
-// returned as an FP32 sign mask (bit 31), which callers fold into one product.
-__host__ __device__ __forceinline__ float half_reduce(double t, unsigned* sgn)
-{
-    const double m = rint(2.0 * t);
-    *sgn = ((unsigned)(int)m) << 31;
-    return (float)fma(-0.5, m, t);
-}
-
 __host__ __device__ __forceinline__ float flipsign(float x, unsigned sgn)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -82,21 +53,9 @@ __host__ __device__ __forceinline__ float flipsign(float x, unsigned sgn)
 #endif
 }
 
-// sin(2 pi r) / r and cos(2 pi r) for |r| <= 1/4
-__host__ __device__ __forceinline__ float sin_over_r(float z)
-{
-    return fmaf(z, fmaf(z, fmaf(z, fmaf(z, ABT_HR4, ABT_HR3), ABT_HR2), ABT_HR1), ABT_HR0);
-}
-__host__ __device__ __forceinline__ float cos_poly(float z)
-{
-    return fmaf(z, fmaf(z, fmaf(z, fmaf(z, fmaf(z, ABT_KR5, ABT_KR4), ABT_KR3), ABT_KR2), ABT_KR1),
-                ABT_KR0);
-}
-
 // Polynomials in half revolutions: for |x| <= 1/2 and z = x^2,
 //   sinpi_over(z) = sin(pi x) / x,  cospi_poly(z) = cos(pi x),  sincpi_poly(z) = sin(pi x) / (pi x);
-// the first two are sin_over_r / cos_poly with the argument doubled (coefficients scaled
-// by powers of two, so the values are the same to the last bit).
+// the coefficients of sin(2 pi r) / r and cos(2 pi r) (trig.h) scaled by powers of two.
 __host__ __device__ __forceinline__ float sinpi_over(float z)
 {
     return fmaf(z, fmaf(z, fmaf(z, fmaf(z, ABT_HR4 / 512.f, ABT_HR3 / 128.f), ABT_HR2 / 32.f), ABT_HR1 / 8.f),
@@ -571,7 +530,7 @@ inline void fill_exp_table(double* tab)
     }
 }
 
-// What a caller keeps after the table for beam_bin_fp64r: the grid's far limit.
+// What a caller of beam_bin_fp64r keeps after the table: the grid's far limit.
 __host__ __device__ __forceinline__ void fp64r_constants(const DevGrid& g, double* c) { c[0] = g.cc_far; }
 
 // e^{2 pi i T / (2 ETAB_N)} for an FP64 T in table steps (|T| < 2^31), from the table (in LDS on the device): T = J + r with
@@ -703,7 +662,7 @@ __host__ __device__ __forceinline__ void add_projectors(Rec r, double FR, double
 // The edge terms of contour_integral cancel one another, so they keep the reference's
 // operations as well (the divisions included), in its order.
 // The default column's diff_main (3702 beams x 64,980 bins): 630 VALU instructions and 6.5 ms of kernels
-// before, 4.0 ms now; 5 orientations x 16,290 bins batched 7.9 -> 3.3 ms.
+// before, 3.4 ms now; 5 orientations x 16,290 bins batched 7.9 -> 3.3 ms.
 // acc: the projector sums S+ (0..3) and S- (4..7).  tab: the exponential table (LDS).
 // INCOH: acc[0] += |amplC|_F^2 instead (temp_rot1 is orthogonal: the norm is final).
 template <bool INCOH, class Rec>
@@ -884,7 +843,7 @@ __host__ __device__ __forceinline__ void projectors_to_matrix(double a[8])
     for (int q = 0; q < 8; q++) a[q] = x[q];
 }
 
-// One beam, one bin of the plain body, added to the amplitude matrix acc (before temp_rot1).
+// One beam, one bin of the plain body, added to the amplitude matrix acc (before temp_rot1): the CPU emulator's.
 __host__ __device__ __forceinline__ void beam_bin_fp64(const double* __restrict__ r,
                                                        const double* __restrict__ vrecs,
                                                        const DevGrid& g, const BinIn& bi,
@@ -947,8 +906,9 @@ __host__ __device__ __forceinline__ FarBin far_bin(const BinIn& bi)
 //     and the form factor's denominator together;
 //   * records through scalar loads (k_sweep).
 // Tried: the other branches after each tile in a pass of their own, which frees registers for a fifth wave but
-// recomputes the beam (125 ms against 104; 112 with 4 waves).  Measured against the body before, 24 orientations x
-// 721 x 180 bins 105.8 -> 76.8 ms (1.8e10 beam.bins), 10,001 facets x 648,360 bins 40.7 -> 30.6 ms.
+// recomputes the beam (125 ms against 104; 112 with 4 waves).  Measured against the body before, each pair on one card
+// (cards differ by up to 10 %), 24 orientations x 721 x 180 bins 112.7 -> 80.8 ms (1.8e10 beam.bins), 10,001 facets x
+// 648,360 bins 40.5 -> 30.0 ms.
 struct FarGeom {
     double ux, uy, uz;   // direction of the bin from the aperture centre
     double kd;           // k (|x - c| - |x|) in table steps (the bin's own e^{i k |x|} follows the beam sum)
@@ -1024,7 +984,7 @@ __host__ __device__ __forceinline__ TriPhase tri_phases(Rec r, double q1, double
 //   F = 2 A (W0 d1 + W1 d2 + W2 d0) / ((2 pi)^2 d0 d1 d2),  d_j = t_{j+1} - t_j,
 // and sum_ref / lambda = -i F / lambda.  The exponentials' rounding enters the numerator as ~1.7e-16 max |d|, so
 // F / A as ~9e-18 max |d| / |d0 d1 d2|: at most 1.7e-13 under the condition below (the two smaller |d_j| times
-// each other at least 1e-4 turns^2), what the phases carry anyway (half an ulp of ~10^5 table steps is
+// each other at least 5e-5 turns^2: |d2| is at most twice the larger of the others), what the phases carry anyway (half an ulp of ~10^5 table steps is
 // 5e-14 rad a vertex).  2 % of the waves have a lane beyond it (beams of the rough column); the earlier
 // condition, every |d_j| >= 1e-3 and |q| a >= 1.5, left 13 % of them a lane in the other branch.
 __host__ __device__ __forceinline__ bool one_denominator(const TriPhase& w, double d)
@@ -1200,8 +1160,8 @@ __host__ __device__ __forceinline__ void beam_bin_fp64r_far(Rec r,
     add_projectors(r, FR, FI, gg, hh, acc);
 }
 
-// One beam, one bin from the bin's plain inputs (bi.rad = |x| is read); etab: the table, then
-// fp64r_constants.
+// One beam, one bin from the bin's plain inputs (bi.rad = |x| is read), for the CPU emulator of the bodies; etab: the
+// table, then fp64r_constants.
 __host__ __device__ __forceinline__ void beam_bin_fp64r(const double* __restrict__ r,
                                                         const double* __restrict__ vrecs,
                                                         const DevGrid& g, const BinIn& bi,

@@ -8,7 +8,6 @@ result is close to minimax at these degrees.  Re-run to regenerate:
 
 Kernels fitted
   fp64:  sin(x) = x + x^3 * S(x^2),  cos(x) = 1 - x^2/2 + x^4 * C(x^2)   on |x| <= pi/4
-  fp32:  sin(2 pi r) = r * s(r^2),   cos(2 pi r) = c(r^2)                on |r| <= 1/8
   fp32:  sin(2 pi r) = r * h(r^2),   cos(2 pi r) = k(r^2)                on |r| <= 1/4
 """
 import mpmath as mp
@@ -35,8 +34,6 @@ def main():
     # fp64 sin: (sin x - x) / x^3 = S(x^2), relative to sin x
     S = lsq(lambda x: mp.sin(x) - x, lambda x: x ** 3, 6, mp.mpf("1e-4"), q)
     C = lsq(lambda x: mp.cos(x) - 1 + x * x / 2, lambda x: x ** 4, 6, mp.mpf("1e-4"), q)
-    s32 = lsq(lambda r: mp.sin(2 * mp.pi * r), lambda r: r, 5, mp.mpf("1e-6"), mp.mpf(1) / 8)
-    c32 = lsq(lambda r: mp.cos(2 * mp.pi * r), lambda r: mp.mpf(1), 5, mp.mpf("1e-6"), mp.mpf(1) / 8)
     h32 = lsq(lambda r: mp.sin(2 * mp.pi * r), lambda r: r, 5, mp.mpf("1e-6"), mp.mpf(1) / 4)
     # cos on |r| <= 1/4 passes through 0 at the end: fit the absolute error (weight 1)
     k32 = lsq(lambda r: mp.cos(2 * mp.pi * r), lambda r: mp.mpf(1), 6, mp.mpf("1e-6"), mp.mpf(1) / 4)
@@ -47,12 +44,6 @@ def main():
     print("// fp64 C(z), x^4 .. x^14")
     for i, v in enumerate(C):
         print(f"#define ABT_C{i + 1} {fmt(v)}")
-    print("// fp32 sin(2 pi r) = r * s(r^2)")
-    for i, v in enumerate(s32):
-        print(f"#define ABT_SR{i} {fmt(v)}f")
-    print("// fp32 cos(2 pi r) = c(r^2)")
-    for i, v in enumerate(c32):
-        print(f"#define ABT_CR{i} {fmt(v)}f")
     print("// fp32 sin(2 pi r) = r * h(r^2), |r| <= 1/4")
     for i, v in enumerate(h32):
         print(f"#define ABT_HR{i} {fmt(v)}f")

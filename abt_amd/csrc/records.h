@@ -121,7 +121,8 @@ constexpr int ETAB_N = 512;
 constexpr int ETAB_DOUBLES = 2 * (2 * ETAB_N);
 constexpr int ETAB_LO = ETAB_DOUBLES;       // offset of the low parts
 constexpr int ETAB_GRID = 2 * ETAB_DOUBLES;  // doubles of DevGrid::etab, and the plain body's LDS block
-// The FP64r body's LDS block: the table's high parts, then the grid's far limit (fp64r_constants).
+// The CPU emulator's block for the restructured body: the table's high parts, then the grid's far limit
+// (fp64r_constants).  The kernels keep the table in LDS and take the limit from the grid.
 constexpr int ETAB_CC_FAR = ETAB_DOUBLES, ETAB_LDS = ETAB_DOUBLES + 1;
 constexpr double BIN_RADIUS = 1e6;   // of make_far_field_bins (diff_mod.f90:846-852)
 

@@ -3,9 +3,6 @@
 // sincos_f64: Cody-Waite reduction by pi/2 with two fma steps (error ~2e-16
 //   absolute for |x| up to ~1e8, which covers the k*|r| ~ 1.2e7 rad far-field
 //   phase), then polynomials on |x| <= pi/4.  Used by the FP64 kernel.
-// sincos_rev_f32: sin/cos(2*pi*f) for a reduced revolution count f in
-//   [-0.5, 0.5] (from an FP64 phase reduction), FP32 polynomials on |r| <= 1/8.
-//   Used by the mixed-precision kernel.
 // Coefficients come from gen_trig_coeffs.py (least squares in 60-digit
 // arithmetic on Chebyshev nodes).
 #pragma once
@@ -26,20 +23,7 @@
 #define ABT_C4 -2.7557317412550660125e-7
 #define ABT_C5 2.0876170365636353732e-9
 #define ABT_C6 -1.1384108242074115052e-11
-// fp32 sin(2 pi r) = r * s(r^2)
-#define ABT_SR0 6.2831853071666184464f
-#define ABT_SR1 -4.1341702168545227836e+1f
-#define ABT_SR2 8.1605208488268080076e+1f
-#define ABT_SR3 -7.6698201365296159018e+1f
-#define ABT_SR4 4.1482575541750033494e+1f
-// fp32 cos(2 pi r) = c(r^2)
-#define ABT_CR0 9.9999999997439937953e-1f
-#define ABT_CR1 -1.9739208666567780209e+1f
-#define ABT_CR2 6.4939319231019713357e+1f
-#define ABT_CR3 -8.5443057786058814865e+1f
-#define ABT_CR4 5.9225039097985419551e+1f
-
-// fp32 sin(2 pi r) = r * h(r^2), cos(2 pi r) = k(r^2), |r| <= 1/4
+// fp32 sin(2 pi r) = r * h(r^2), cos(2 pi r) = k(r^2), |r| <= 1/4 (the mixed body's, in half revolutions: ffbody.h)
 // (max abs error in exact arithmetic 6.1e-9 and 8.3e-10)
 #define ABT_HR0 6.2831852918370438308f
 #define ABT_HR1 -4.1341682323056890963e+1f
@@ -78,31 +62,6 @@ __host__ __device__ inline void sincos_f64(double x, double* s, double* c)
     if (q >= 2) so = -so;
     *s = so;
     *c = co;
-}
-
-// sin(2 pi f), cos(2 pi f) for |f| <= 0.5 (any f works; the octant split assumes a
-// reduced input for full accuracy)
-__host__ __device__ inline void sincos_rev_f32(float f, float* s, float* c)
-{
-    float qf = rintf(4.0f * f);
-    float r = fmaf(-0.25f, qf, f);   // exact: |r| <= 1/8
-    float z = r * r;
-    float ps = fmaf(z, fmaf(z, fmaf(z, fmaf(z, ABT_SR4, ABT_SR3), ABT_SR2), ABT_SR1), ABT_SR0);
-    float sn = r * ps;
-    float cs = fmaf(z, fmaf(z, fmaf(z, fmaf(z, ABT_CR4, ABT_CR3), ABT_CR2), ABT_CR1), ABT_CR0);
-    int q = ((int)qf) & 3;
-    float so = (q & 1) ? cs : sn;
-    float co = (q & 1) ? sn : cs;
-    if (q == 1 || q == 2) co = -co;
-    if (q >= 2) so = -so;
-    *s = so;
-    *c = co;
-}
-
-// reduce an FP64 revolution count to its fractional part in [-0.5, 0.5]
-__host__ __device__ inline float frac_rev(double t)
-{
-    return (float)(t - rint(t));
 }
 
 }  // namespace abt

@@ -153,7 +153,7 @@ int abt_grid_destroy(abt_dev_grid* g);
 int64_t abt_grid_bins(const abt_dev_grid* g);
 
 /* Workspace bytes abt_far_field_dev needs for nb beams (0 when none): 64 bytes per bin
- * per beam segment, at most 32 segments of >= 32 beams (2048 bytes per bin).  With less than this
+ * per beam segment, at most 32 segments of >= 8 beams (2048 bytes per bin).  With less than this
  * the call still runs on segments of >= 512 beams where their sums fit. */
 size_t abt_far_field_workspace(const abt_dev_grid* g, int64_t nb, int precision);
 
