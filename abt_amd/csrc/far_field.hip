@@ -72,9 +72,10 @@ __device__ __forceinline__ BinIn load_bin(const DevGrid& g, int bc)
 // with the barriers alone, run the orientation averages at 109 and 108 ms (mixed 39 ms).  16 orientations x 361 x
 // 180 bins, mixed: 30.8 -> 28.6 ms; 24 x 721 x 180, restructured: 98.5 -> 87.8 ms; 45 polygons x 721 x 180,
 // plain: 190 -> 184 us a step.
-// Occupancy: 4 waves per SIMD (128 VGPRs); 2 for two bins a lane and for the accurate body.
+// Occupancy: 4 waves per SIMD (128 VGPRs); 2 for two bins a lane and for the accurate body.  Two bins fit 3 (168 VGPRs),
+// which the restructured body is told: with one register more it ran 32 orientations x 721 x 180 bins in 141 ms, not 115.
 template <int PREC, int TB, int BPT, int MODE>
-__global__ __launch_bounds__(BLOCK, BPT == 1 && PREC != 3 ? 4 : 2)
+__global__ __launch_bounds__(BLOCK, BPT == 1 && PREC != 3 ? 4 : (PREC == 4 ? 3 : 2))
 void k_sweep(SweepArgs a)
 {
     constexpr bool INC = MODE == SWEEP_INC, LIST = MODE == SWEEP_LIST;
