@@ -159,9 +159,18 @@ int ensure_device()
     return 0;
 }
 
+// Allocations of a call on one stream while another stream is captured (by default they would invalidate that
+// capture, of whatever thread): the buffers are no part of it.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 int buf_ensure(DevBuf& b, size_t bytes)
 {
     if (b.cap >= bytes) return 0;
+    const RelaxedCapture relaxed;
     if (b.p) HIPCHK(hipFree(b.p));
     b.p = nullptr;
     b.cap = 0;
@@ -187,6 +196,7 @@ char* pin_inputs(ThreadState& ts, size_t inputs, bool with_ring = true)
     const size_t ring = with_ring ? PIN_RING : 0, need = ring + inputs;
     if (inputs > PIN_MAX - PIN_RING) return nullptr;
     if (ts.pin_cap < need) {
+        const RelaxedCapture relaxed;
         if (ts.pin) (void)hipHostFree(ts.pin);
         ts.pin = nullptr;
         ts.pin_cap = 0;
